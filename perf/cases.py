@@ -1,0 +1,560 @@
+"""The work that performance is measured on: cases over the public entry points.
+
+A case is a dict of plain values with a "kind":
+
+  proj    one decode matvec (ss_hip_matvec_fused), RMSNorm in front or not
+  ffn     a decode MLP: ss_hip_ffn_gate_up with its RMSNorm, then the down matvec
+  head    the LM head of one token: RMSNorm + matvec, then ss_hip_argmax
+  attn    decode attention of one token over a cache (ss_hip_attention)
+  layer   the products and the attention of one decoder layer over a prompt
+          chunk (ss_hip_gemm, ss_hip_attention_rows, ss_hip_swiglu)
+  rows    the attention of a later prompt chunk over a long prefix
+  sample  one sampled token from device logits (ss_hip_sample_logits)
+  decode  eval-token steps of a whole model at a given context
+  prompt  a prompt through a whole model
+
+Weights are random blocks of the GGUF formats (Q4_0 2, Q8_0 8, Q4_K 12, Q6_K
+14), spread 1/sqrt(columns) as trained matrices roughly are; activations are
+N(0, 1), norm weights 1 + N(0, 0.01), cached K and V N(0, 1). A model is written
+as a GGUF file and loaded through the package, as a user's program does.
+`exact` restates each case in 64 bits with torch alone.
+"""
+import ctypes
+import math
+import os
+import struct
+import tempfile
+
+import numpy as np
+import torch
+
+import phonemap_amd as pm
+from phonemap_amd import api
+
+Q4_0, Q8_0, Q4_K, Q6_K = 2, 8, 12, 14
+BLOCK = {Q4_0: (32, 18), Q8_0: (32, 34), Q4_K: (256, 144), Q6_K: (256, 210)}   # weights, bytes
+EPS = 1e-5
+THETA = 10000.0
+
+
+def listed():
+    tiny = dict(layers=22, hidden=2048, heads=32, kv_heads=4, hd=64, ffn=5632, vocab=32000, type=Q4_0, head_type=Q4_0)
+    seven = dict(layers=4, hidden=4096, heads=32, kv_heads=32, hd=128, ffn=11008, vocab=32000, type=Q4_0, head_type=Q8_0)
+    return [
+        # the smallest call here: one attention output projection of a 7B-shape decode step
+        dict(name="proj-4096-q4_0", kind="proj", type=Q4_0, rows=4096, cols=4096, norm=False),
+        # the MLP of a 7B-shape decode step in Q4_0, the benchmark's own shape
+        dict(name="ffn-7b-q4_0", kind="ffn", type=Q4_0, down=Q4_0, hidden=4096, ffn=11008),
+        # the same for an 8B shape in the usual Q4_K / Q6_K mix of K-quant files
+        dict(name="ffn-8b-q4_k", kind="ffn", type=Q4_K, down=Q6_K, hidden=4096, ffn=14336),
+        # the 128k-vocabulary LM head and its greedy choice, the largest matrix of a decode step
+        dict(name="head-128k-q8_0", kind="head", type=Q8_0, vocab=128256, hidden=4096),
+        # decode attention of an 8B shape at the benchmark's long context
+        dict(name="attn-gqa4-4097", kind="attn", heads=32, kv_heads=8, hd=128, ctx=4097, max_seq=4608, kv=0),
+        # a full prompt chunk through one 7B-shape layer (the 512-token prompt of the benchmark)
+        dict(name="layer-7b-q4_0-512", kind="layer", type=Q4_0, hidden=4096, heads=32, kv_heads=32, hd=128, ffn=11008,
+             pos0=0, tokens=512),
+        # a chat turn of odd length continuing a conversation: 8B shape, Q4_K
+        dict(name="layer-8b-q4_k-77", kind="layer", type=Q4_K, hidden=4096, heads=32, kv_heads=8, hd=128, ffn=14336,
+             pos0=1000, tokens=77),
+        # the fourth chunk of a 2048-token prompt: its attention over the three before it
+        dict(name="rows-gqa4-2048", kind="rows", heads=32, kv_heads=8, hd=128, pos0=1536, tokens=512),
+        # a chat program's choice of the next token (the defaults of such programs)
+        dict(name="sample-128k", kind="sample", vocab=128256, temperature=0.8, top_k=40, top_p=0.95),
+        # token by token through the whole TinyLlama shape, as a generate loop does
+        dict(name="decode-tinyllama", kind="decode", kv=0, ctx=100, steps=8, **tiny),
+        # a short question through layers of the 7B shape
+        dict(name="prompt-7b-32", kind="prompt", kv=0, tokens=32, **seven),
+        # a question through TinyLlama with the int8 cache, the reference's own cache
+        dict(name="prompt-tinyllama-int8-64", kind="prompt", kv=1, tokens=64, **tiny),
+    ]
+
+
+def _log(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def _cols(rng, t, lo, hi):
+    unit = BLOCK[t][0]
+    return max(unit, _log(rng, lo, hi) // unit * unit)
+
+
+def draw(rng):
+    kind = rng.choice(["proj", "proj", "ffn", "ffn", "head", "attn", "attn", "layer", "layer", "rows", "sample", "decode",
+                       "prompt", "prompt"])
+    t = rng.choice([Q4_0, Q8_0, Q4_K, Q6_K])
+    if kind == "proj":
+        return dict(kind=kind, type=t, rows=_log(rng, 500, 28672), cols=_cols(rng, t, 1024, 14336), norm=rng.random() < 0.5)
+    if kind == "ffn":
+        d = rng.choice([t, Q6_K if t == Q4_K else t])
+        return dict(kind=kind, type=t, down=d, hidden=_cols(rng, t, 1024, 8192), ffn=_cols(rng, Q4_K, 2816, 16384))
+    if kind == "head":
+        return dict(kind=kind, type=rng.choice([Q4_0, Q8_0, Q6_K]), vocab=_log(rng, 32000, 128256), hidden=_cols(rng, Q4_K, 2048, 4096))
+    kvh, group, hd = rng.choice([(4, 8, 64), (8, 4, 128), (8, 8, 128), (32, 1, 128), (12, 1, 64), (4, 2, 128)])
+    if kind == "attn":
+        ctx = _log(rng, 24, 8000)
+        return dict(kind=kind, heads=kvh * group, kv_heads=kvh, hd=hd, ctx=ctx, max_seq=ctx + rng.randrange(0, 600),
+                    kv=int(rng.random() < 0.3))
+    if kind == "layer":
+        return dict(kind=kind, type=t, hidden=_cols(rng, Q4_K, 2048, 4096), heads=kvh * group, kv_heads=kvh, hd=hd,
+                    ffn=_cols(rng, Q4_K, 5632, 11008), pos0=rng.choice([0, rng.randrange(1, 1500)]), tokens=_log(rng, 8, 500))
+    if kind == "rows":
+        return dict(kind=kind, heads=kvh * group, kv_heads=kvh, hd=hd, pos0=rng.randrange(0, 3000), tokens=_log(rng, 16, 512))
+    if kind == "sample":
+        return dict(kind=kind, vocab=_log(rng, 32000, 128256), temperature=round(rng.uniform(0.5, 1.2), 2),
+                    top_k=rng.choice([0, 20, 40, 100]), top_p=rng.choice([0.8, 0.9, 0.95, 1.0]))
+    shape = rng.choice([
+        dict(layers=rng.randrange(4, 13), hidden=2048, heads=32, kv_heads=4, hd=64, ffn=5632, vocab=32000),
+        dict(layers=rng.randrange(2, 5), hidden=4096, heads=32, kv_heads=32, hd=128, ffn=11008, vocab=32000),
+        dict(layers=rng.randrange(2, 4), hidden=4096, heads=32, kv_heads=8, hd=128, ffn=14336, vocab=32000),
+    ])
+    shape.update(type=t, head_type=rng.choice([Q8_0, Q6_K]), kv=int(rng.random() < 0.3))
+    if kind == "decode":
+        return dict(kind=kind, ctx=_log(rng, 16, 2000), steps=4, **shape)
+    return dict(kind=kind, tokens=_log(rng, 2, 300 if shape["hidden"] == 2048 else 140), **shape)
+
+
+# ---- weights -----------------------------------------------------------------
+def _gen(seed):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    return g
+
+
+def _bytes(g, n, k):
+    return torch.randint(0, 256, (n, k), generator=g, device="cuda", dtype=torch.uint8)
+
+
+def _half(v):
+    return v.to(torch.float16).view(torch.uint8).reshape(v.shape[0], 2)
+
+
+def _blocks(g, t, rows, cols):
+    """Random GGUF blocks of a [rows x cols] matrix, spread 1/sqrt(cols): uint8 on the GPU."""
+    n, size = BLOCK[t]
+    nb = rows * cols // n
+    out = _bytes(g, nb, size)
+    z = torch.randn(nb, generator=g, device="cuda") / math.sqrt(cols)
+    if t == Q4_0:
+        out[:, :2] = _half(z / math.sqrt(21.5))
+    elif t == Q8_0:
+        out[:, :2] = _half(z / 73.6)
+        codes = out[:, 2:]
+        codes[codes == 128] = 129   # -127 .. 127
+    elif t == Q4_K:   # scale * nibble - min around zero
+        d = (0.5 + 0.5 * z.abs() * math.sqrt(cols)) / math.sqrt(cols) / 257.0
+        out[:, :2] = _half(d)
+        out[:, 2:4] = _half(7.5 * d)
+    else:
+        out[:, 208:] = _half(z / 1367.0)
+    return out
+
+
+def _dequant(b, t, rows, cols):
+    """The 64-bit weights of GGUF blocks."""
+    def half(x):
+        return x.contiguous().view(torch.float16).to(torch.float64).reshape(-1, 1)
+    nb = b.shape[0]
+    if t == Q4_0:
+        q = b[:, 2:]
+        w = torch.cat([q & 15, q >> 4], 1).to(torch.float64).sub_(8.0).mul_(half(b[:, :2]))
+    elif t == Q8_0:
+        w = b[:, 2:].contiguous().view(torch.int8).to(torch.float64) * half(b[:, :2])
+    elif t == Q4_K:
+        s = b[:, 4:16].to(torch.int32)
+        lo = torch.cat([s[:, 0:4] & 63, (s[:, 8:12] & 15) | ((s[:, 0:4] >> 6) << 4)], 1)
+        mn = torch.cat([s[:, 4:8] & 63, (s[:, 8:12] >> 4) | ((s[:, 4:8] >> 6) << 4)], 1)
+        q = b[:, 16:].reshape(nb, 4, 32)
+        q = torch.stack([q & 15, q >> 4], 2).reshape(nb, 8, 32).to(torch.float64)
+        w = q * (half(b[:, 0:2]) * lo).reshape(nb, 8, 1) - (half(b[:, 2:4]) * mn).reshape(nb, 8, 1)
+    else:
+        ql = b[:, :128].reshape(nb, 2, 2, 32)
+        qh = b[:, 128:192].reshape(nb, 2, 1, 32)
+        low = torch.cat([ql & 15, ql >> 4], 2)
+        high = torch.cat([(qh >> sh) & 3 for sh in (0, 2, 4, 6)], 2)
+        q = (low | (high << 4)).to(torch.float64).sub_(32.0).reshape(nb, 16, 16)
+        w = q * (half(b[:, 208:210]) * b[:, 192:208].contiguous().view(torch.int8)).reshape(nb, 16, 1)
+    return w.reshape(rows, cols)
+
+
+def _matmul64(x, b, t, rows, cols):
+    """x [n][cols] times the transposed matrix, in 64 bits, some rows at a time."""
+    n, out, step = BLOCK[t][0], [], max(1, (1 << 26) // cols)
+    for r in range(0, rows, step):
+        k = min(step, rows - r)
+        out.append(x @ _dequant(b[r * cols // n:(r + k) * cols // n], t, k, cols).T)
+    return torch.cat(out, 1)
+
+
+def _norm64(x, w):
+    return x / torch.sqrt((x * x).mean(-1, keepdim=True) + EPS) * w.double()
+
+
+def _attend64(q, k, v, pos0):
+    """Causal attention in 64 bits: q [n][H][hd], k and v [ctx][KVH][hd]."""
+    n, h, hd = q.shape
+    g = h // k.shape[1]
+    k, v = (z.double().repeat_interleave(g, 1).transpose(0, 1) for z in (k, v))      # [H][ctx][hd]
+    out, step = [], max(1, (1 << 27) // (h * k.shape[1]))
+    for r in range(0, n, step):
+        s = (q[r:r + step].transpose(0, 1).contiguous() @ k.transpose(1, 2).contiguous()) / math.sqrt(hd)
+        last = pos0 + r + torch.arange(s.shape[1], device=s.device).reshape(1, -1, 1)
+        s.masked_fill_(torch.arange(s.shape[2], device=s.device).reshape(1, 1, -1) > last, -math.inf)
+        out.append((torch.softmax(s, -1) @ v).transpose(0, 1))
+    return torch.cat(out, 0).reshape(n, h * hd)
+
+
+# ---- calls -------------------------------------------------------------------
+_ctx = None
+
+
+def _context():
+    global _ctx
+    if _ctx is None:
+        _ctx = pm.lib().ss_hip_init(0)
+        if not _ctx:
+            raise RuntimeError(pm.lib().ss_hip_last_error().decode())
+    return _ctx
+
+
+def _pack(b, t, rows, cols):
+    L, c = pm.lib(), _context()
+    dst = torch.empty(L.ss_hip_packed_bytes(t, rows, cols), dtype=torch.uint8, device="cuda")
+    src = b.cpu().numpy()
+    torch.cuda.synchronize()
+    pm.check(L.ss_hip_pack_matrix(c, dst.data_ptr(), src.ctypes.data, t, rows, cols))
+    return dst
+
+
+def _vec(g, *shape):
+    return torch.randn(*shape, generator=g, device="cuda")
+
+
+def _norm_w(g, n):
+    return 1.0 + 0.01 * _vec(g, n)
+
+
+class State:
+    pass
+
+
+def _inputs(c, seed):
+    """Everything random about a case, the same for prepare and exact."""
+    g, s = _gen(seed), State()
+    s.kind = c["kind"]
+    if s.kind == "proj":
+        s.w = _blocks(g, c["type"], c["rows"], c["cols"])
+        s.x, s.nw = _vec(g, c["cols"]), _norm_w(g, c["cols"])
+    elif s.kind == "ffn":
+        h, f = c["hidden"], c["ffn"]
+        s.gate, s.up, s.dn = _blocks(g, c["type"], f, h), _blocks(g, c["type"], f, h), _blocks(g, c["down"], h, f)
+        s.x, s.nw = _vec(g, h), _norm_w(g, h)
+    elif s.kind == "head":
+        s.w = _blocks(g, c["type"], c["vocab"], c["hidden"])
+        s.x, s.nw = _vec(g, c["hidden"]), _norm_w(g, c["hidden"])
+    elif s.kind in ("attn", "rows", "layer"):
+        n, ctx = (1, c["ctx"]) if s.kind == "attn" else (c["tokens"], c["pos0"] + c["tokens"])
+        s.n, s.ctx, s.max_seq = n, ctx, c.get("max_seq", ctx)
+        shape = (c["kv_heads"], s.max_seq, c["hd"])
+        if c.get("kv"):
+            s.k, s.v = (torch.randint(-127, 128, shape, generator=g, device="cuda", dtype=torch.int8) for _ in "kv")
+            s.ks, s.vs = (0.01 + 0.02 * torch.rand(s.max_seq, generator=g, device="cuda") for _ in "kv")
+        else:
+            s.k, s.v, s.ks, s.vs = _vec(g, *shape).half(), _vec(g, *shape).half(), None, None
+        if s.kind == "layer":
+            h, f, t = c["hidden"], c["ffn"], c["type"]
+            qd, kd = c["heads"] * c["hd"], c["kv_heads"] * c["hd"]
+            s.mats = [(qd, h), (kd, h), (kd, h), (h, qd), (f, h), (f, h), (h, f)]
+            s.ws = [_blocks(g, t, r, k) for r, k in s.mats]
+            s.x, s.an, s.fn = _vec(g, n, h), _norm_w(g, h), _norm_w(g, h)
+        else:
+            s.q = _vec(g, n, c["heads"] * c["hd"])
+    elif s.kind == "sample":
+        s.logits = 2.5 * _vec(g, c["vocab"])
+        s.rng = 0x9E3779B97F4A7C15 ^ (seed * 2654435761 + 1)
+    else:
+        h, f, t = c["hidden"], c["ffn"], c["type"]
+        qd, kd = c["heads"] * c["hd"], c["kv_heads"] * c["hd"]
+        s.emb, s.out = _blocks(g, c["head_type"], c["vocab"], h), _blocks(g, c["head_type"], c["vocab"], h)
+        s.on = _norm_w(g, h)
+        s.shapes = [("attn_q", qd, h), ("attn_k", kd, h), ("attn_v", kd, h), ("attn_output", h, qd),
+                    ("ffn_gate", f, h), ("ffn_up", f, h), ("ffn_down", h, f)]
+        s.layers = [dict(attn_norm=_norm_w(g, h), ffn_norm=_norm_w(g, h), **{n: _blocks(g, t, r, k) for n, r, k in s.shapes})
+                    for _ in range(c["layers"])]
+        s.n = c["steps"] if s.kind == "decode" else c["tokens"]
+        s.pos0 = c["ctx"] if s.kind == "decode" else 0
+        s.tokens = torch.randint(0, c["vocab"], (s.n,), generator=g, device="cuda")
+        s.cache = [(_vec(g, s.pos0, kd).half(), _vec(g, s.pos0, kd).half()) for _ in range(c["layers"])] if s.pos0 else None
+    return s
+
+
+def _gguf(path, c, s):
+    """The model as a GGUF file."""
+    def text(v):
+        return struct.pack("<Q", len(v)) + v.encode()
+
+    def u32(k, v):
+        return text("llama." + k) + struct.pack("<II", 4, v)
+
+    def f32(k, v):
+        return text("llama." + k) + struct.pack("<If", 6, v)
+    meta = [text("general.architecture") + struct.pack("<I", 8) + text("llama"),
+            u32("embedding_length", c["hidden"]), u32("block_count", c["layers"]),
+            u32("attention.head_count", c["heads"]), u32("attention.head_count_kv", c["kv_heads"]),
+            u32("attention.key_length", c["hd"]), u32("rope.dimension_count", c["hd"]),
+            u32("feed_forward_length", c["ffn"]), u32("context_length", 4096), u32("vocab_size", c["vocab"]),
+            f32("rope.freq_base", THETA), f32("attention.layer_norm_rms_epsilon", EPS)]
+    h, ht = c["hidden"], c["head_type"]
+    tensors = [("token_embd.weight", (h, c["vocab"]), ht, s.emb), ("output.weight", (h, c["vocab"]), ht, s.out),
+               ("output_norm.weight", (h,), 0, s.on)]
+    for i, ly in enumerate(s.layers):
+        tensors += [("blk.%d.%s.weight" % (i, n), (h,), 0, ly[n]) for n in ("attn_norm", "ffn_norm")]
+        tensors += [("blk.%d.%s.weight" % (i, n), (k, r), c["type"], ly[n]) for n, r, k in s.shapes]
+    info, at = b"", 0
+    for name, dims, t, data in tensors:
+        info += text(name) + struct.pack("<I%dQIQ" % len(dims), len(dims), *dims, t, at)
+        at += -(-data.numel() * data.element_size() // 32) * 32
+    head = b"GGUF" + struct.pack("<IQQ", 3, len(tensors), len(meta)) + b"".join(meta) + info
+    with open(path, "wb") as f:
+        f.write(head + bytes(-len(head) % 32))
+        for _, _, _, data in tensors:
+            raw = data.cpu().numpy()
+            raw.tofile(f)
+            f.write(bytes(-raw.nbytes % 32))
+
+
+def prepare(case, seed):
+    c, s = case, _inputs(case, seed)
+    s.case = c
+
+    def out(*shape):
+        return torch.empty(*shape, device="cuda")
+    if s.kind == "proj":
+        s.w, s.y = _pack(s.w, c["type"], c["rows"], c["cols"]), out(c["rows"])
+    elif s.kind == "ffn":
+        h, f = c["hidden"], c["ffn"]
+        s.gate, s.up, s.dn = _pack(s.gate, c["type"], f, h), _pack(s.up, c["type"], f, h), _pack(s.dn, c["down"], h, f)
+        s.act, s.y = out(f), out(h)
+    elif s.kind == "head":
+        s.w, s.y = _pack(s.w, c["type"], c["vocab"], c["hidden"]), out(c["vocab"])
+        s.best = torch.zeros(1, dtype=torch.int32, device="cuda")
+    elif s.kind in ("attn", "rows"):
+        s.y = out(s.n, c["heads"] * c["hd"])
+    elif s.kind == "layer":
+        s.ws = [_pack(b, c["type"], r, k) for b, (r, k) in zip(s.ws, s.mats)]
+        s.ys = [out(s.n, r) for r, _ in s.mats]
+        s.att, s.act = out(s.n, c["heads"] * c["hd"]), out(s.n, c["ffn"])
+    elif s.kind in ("decode", "prompt"):
+        fd, path = tempfile.mkstemp(suffix=".gguf")
+        os.close(fd)
+        try:
+            _gguf(path, c, s)
+            s.model = api.Model(path, max_context=s.pos0 + s.n + 64, kv="int8" if c["kv"] else "f16")
+        finally:
+            os.unlink(path)
+        if s.cache:
+            for i, (k, v) in enumerate(s.cache):
+                s.model.kv_write(i, 0, k.cpu().numpy().view(np.uint16), v.cpu().numpy().view(np.uint16))
+        s.ids = s.tokens.cpu().numpy().astype(np.int32)
+        s.ids_list = s.ids.tolist()
+        s.emb = s.out = s.layers = s.cache = None
+    torch.cuda.synchronize()
+    return s
+
+
+def _p(t):
+    return t.data_ptr() if t is not None else None
+
+
+def run(state):
+    s, c = state, state.case
+    L, ok = pm.lib(), pm.check
+    if s.kind in ("decode", "prompt"):
+        if s.kind == "prompt":
+            return s.model.eval_prompt(s.ids)[0]
+        for i in range(s.n - 1):
+            s.model.eval_token(s.ids_list[i], s.pos0 + i, want_logits=False)
+        return s.model.eval_token(s.ids_list[-1], s.pos0 + s.n - 1)[0]
+    x = _context()
+    if s.kind == "proj":
+        ok(L.ss_hip_matvec_fused(x, _p(s.y), _p(s.w), _p(s.x), _p(s.nw if c["norm"] else None), EPS, 0, c["rows"], c["cols"],
+                                 c["type"], None))
+        return s.y
+    if s.kind == "ffn":
+        ok(L.ss_hip_ffn_gate_up(x, _p(s.act), _p(s.gate), _p(s.up), _p(s.x), _p(s.nw), EPS, c["ffn"], c["hidden"], c["type"], None))
+        ok(L.ss_hip_matvec(x, _p(s.y), _p(s.dn), _p(s.act), c["hidden"], c["ffn"], c["down"], None))
+        return s.act, s.y
+    if s.kind == "head":
+        ok(L.ss_hip_matvec_fused(x, _p(s.y), _p(s.w), _p(s.x), _p(s.nw), EPS, 0, c["vocab"], c["hidden"], c["type"], None))
+        ok(L.ss_hip_argmax(x, _p(s.best), _p(s.y), c["vocab"], None))
+        return s.y, s.best
+    if s.kind == "attn":
+        ok(L.ss_hip_attention(x, _p(s.y), _p(s.q), _p(s.k), _p(s.v), _p(s.ks), _p(s.vs), c["heads"], c["kv_heads"], c["hd"],
+                              s.max_seq, s.ctx, c["kv"], None))
+        return s.y
+    if s.kind == "rows":
+        ok(L.ss_hip_attention_rows(x, _p(s.y), _p(s.q), _p(s.k), _p(s.v), c["heads"], c["kv_heads"], c["hd"], s.max_seq,
+                                   c["pos0"], s.n, None))
+        return s.y
+    if s.kind == "sample":
+        rng, tok = ctypes.c_uint64(s.rng), ctypes.c_int32(-1)
+        ok(L.ss_hip_sample_logits(x, _p(s.logits), c["vocab"], c["temperature"], c["top_p"], c["top_k"], ctypes.byref(rng),
+                                  ctypes.byref(tok)))
+        return tok.value, rng.value >> 32, rng.value & 0xFFFFFFFF
+
+    def product(i, inp, nw):
+        r, k = s.mats[i]
+        ok(L.ss_hip_gemm(x, _p(s.ys[i]), _p(s.ws[i]), _p(inp), _p(nw), EPS, 0, r, k, s.n, c["type"], None))
+    for i in range(3):
+        product(i, s.x, s.an)
+    ok(L.ss_hip_attention_rows(x, _p(s.att), _p(s.ys[0]), _p(s.k), _p(s.v), c["heads"], c["kv_heads"], c["hd"], s.max_seq,
+                               c["pos0"], s.n, None))
+    product(3, s.att, None)
+    product(4, s.x, s.fn)
+    product(5, s.x, s.fn)
+    ok(L.ss_hip_swiglu(x, _p(s.act), _p(s.ys[4]), _p(s.ys[5]), s.n * c["ffn"], None))
+    product(6, s.act, None)
+    return s.ys, s.att, s.act
+
+
+# ---- what a pass cannot do without ------------------------------------------
+def _mat_bytes(t, rows, cols):
+    return rows * cols * BLOCK[t][1] / BLOCK[t][0]
+
+
+def work(case):
+    c, k = case, case["kind"]
+    if k == "proj":
+        return dict(bytes=_mat_bytes(c["type"], c["rows"], c["cols"]) + 4 * (c["rows"] + c["cols"]), flops=2 * c["rows"] * c["cols"])
+    if k == "ffn":
+        n = c["hidden"] * c["ffn"]
+        return dict(bytes=2 * _mat_bytes(c["type"], c["ffn"], c["hidden"]) + _mat_bytes(c["down"], c["hidden"], c["ffn"]) +
+                    8 * (c["hidden"] + c["ffn"]), flops=6 * n)
+    if k == "head":
+        return dict(bytes=_mat_bytes(c["type"], c["vocab"], c["hidden"]) + 4 * (c["vocab"] + 2 * c["hidden"]),
+                    flops=2 * c["vocab"] * c["hidden"])
+    if k == "sample":
+        return dict(bytes=4 * c["vocab"], flops=4 * c["vocab"])
+    kd, qd = c["kv_heads"] * c["hd"], c["heads"] * c["hd"]
+    if k == "attn":
+        return dict(bytes=2 * c["ctx"] * kd * (1 if c["kv"] else 2) + 8 * qd, flops=4 * c["ctx"] * qd)
+    if k in ("rows", "layer"):
+        n, p = c["tokens"], c["pos0"]
+        seen = n * p + n * (n + 1) // 2
+        w = dict(bytes=4 * (p + n) * kd + 8 * n * qd, flops=4 * seen * qd)
+        if k == "layer":
+            h, f, t = c["hidden"], c["ffn"], c["type"]
+            m = 2 * h * qd + 2 * h * kd + 3 * h * f
+            w = dict(bytes=w["bytes"] + _mat_bytes(t, m // h, h) + 4 * n * (2 * h + 2 * kd + 4 * f),
+                     flops=w["flops"] + 2 * n * m)
+        return w
+    h, f = c["hidden"], c["ffn"]
+    m = 2 * h * qd + 2 * h * kd + 3 * h * f
+    n, p = (c["steps"], c["ctx"]) if k == "decode" else (c["tokens"], 0)
+    times, heads = (n, n) if k == "decode" else (1, 1)   # decode reads the weights at every step
+    seen = n * p + n * (n + 1) // 2
+    kvb = 2 * kd * (1 if c["kv"] else 2)
+    return dict(bytes=c["layers"] * (times * _mat_bytes(c["type"], m // h, h) + (seen if k == "decode" else n) * kvb) +
+                heads * _mat_bytes(c["head_type"], c["vocab"], h) + 4 * c["vocab"],
+                flops=c["layers"] * (2 * n * m + 4 * seen * qd) + heads * 2 * c["vocab"] * h)
+
+
+def tolerance(case):
+    k = case["kind"]
+    if k == "sample":
+        return "exact"   # a token and the generator's state
+    if k in ("decode", "prompt"):
+        # a K or V value on the edge of its 16-bit (int8) rounding falls either
+        # way, and what follows moves with it: 7e-5 (2e-3) measured against 64 bits
+        return dict(rel=1e-2, max=0.1) if case["kv"] else dict(rel=1e-3, max=1e-2)
+    if k == "layer":
+        return dict(rel=5e-6, max=2e-4)   # 32-bit sums, some of them of the ones before: 7e-7 measured
+    return dict(rel=4e-6, max=1e-4)       # 7e-7 measured
+
+
+# ---- the same in 64 bits -----------------------------------------------------
+def _round_half_away(x):
+    return torch.sign(x) * torch.floor(x.abs() + 0.5)
+
+
+def _cached64(x, kv):
+    """K or V rows [n][kd] as the cache holds them."""
+    if not kv:
+        return x.half().double()
+    s = x.abs().amax(1, keepdim=True) / 127.0
+    return _round_half_away(torch.where(s > 0, x / s, 0.0)) * s
+
+
+def _rope64(x, hd, pos0):
+    """Pairs (2i, 2i+1) turned by the angles of the 32-bit table."""
+    n = x.shape[0]
+    i = np.arange(0, hd, 2, dtype=np.float32)
+    freq = np.float32(1.0) / np.power(np.float32(THETA), i / np.float32(hd))
+    angle = (np.arange(pos0, pos0 + n, dtype=np.float32)[:, None] * freq).astype(np.float32)
+    cos, sin = (torch.from_numpy(f(angle)).double().to(x.device).reshape(n, 1, -1) for f in (np.cos, np.sin))
+    z = x.reshape(n, -1, hd)
+    a, b = z[..., 0::2], z[..., 1::2]
+    return torch.stack([a * cos - b * sin, a * sin + b * cos], -1).reshape(n, -1)
+
+
+def _model64(c, s):
+    h, f, hd, t = c["hidden"], c["ffn"], c["hd"], c["type"]
+    qd, kd = c["heads"] * hd, c["kv_heads"] * hd
+    nb = h // BLOCK[c["head_type"]][0]
+    rows = s.emb.reshape(c["vocab"], nb, -1)[s.tokens].reshape(s.n * nb, -1)
+    x = _dequant(rows, c["head_type"], s.n, h)
+
+    def mul(y, ly, name):
+        _, r, k = next(z for z in s.shapes if z[0] == name)
+        return _matmul64(y, ly[name], t, r, k)
+    for i, ly in enumerate(s.layers):
+        y = _norm64(x, ly["attn_norm"])
+        q = _rope64(mul(y, ly, "attn_q"), hd, s.pos0)
+        k = _cached64(_rope64(mul(y, ly, "attn_k"), hd, s.pos0), c["kv"])
+        v = _cached64(mul(y, ly, "attn_v"), c["kv"])
+        if s.cache:
+            k, v = (torch.cat([_cached64(old.double(), c["kv"]), new]) for old, new in zip(s.cache[i], (k, v)))
+        a = _attend64(q.reshape(s.n, c["heads"], hd), k.reshape(-1, c["kv_heads"], hd), v.reshape(-1, c["kv_heads"], hd), s.pos0)
+        x = x + mul(a, ly, "attn_output")
+        y = _norm64(x, ly["ffn_norm"])
+        gate = mul(y, ly, "ffn_gate")
+        x = x + mul(mul(y, ly, "ffn_up") * gate * torch.sigmoid(gate), ly, "ffn_down")
+    return _matmul64(_norm64(x[-1:], s.on), s.out, c["head_type"], c["vocab"], h)[0]
+
+
+def exact(case, seed):
+    c, s = case, _inputs(case, seed)
+    if s.kind == "sample":
+        return None   # whole numbers
+    if s.kind in ("decode", "prompt"):
+        return _model64(c, s)
+    if s.kind == "proj":
+        x = s.x.double().reshape(1, -1)
+        return _matmul64(_norm64(x, s.nw) if c["norm"] else x, s.w, c["type"], c["rows"], c["cols"])[0]
+    if s.kind == "head":
+        return _matmul64(_norm64(s.x.double().reshape(1, -1), s.nw), s.w, c["type"], c["vocab"], c["hidden"])[0], None
+    if s.kind == "ffn":
+        h, f = c["hidden"], c["ffn"]
+        x = _norm64(s.x.double().reshape(1, -1), s.nw)
+        gate, up = (_matmul64(x, b, c["type"], f, h) for b in (s.gate, s.up))
+        act = up * gate * torch.sigmoid(gate)
+        return act[0], _matmul64(act, s.dn, c["down"], h, f)[0]
+    hd = c["hd"]
+    k, v = (z[:, :s.ctx].double().transpose(0, 1) for z in (s.k, s.v))
+    if s.ks is not None:
+        k, v = (z * sc[:s.ctx].double().reshape(-1, 1, 1) for z, sc in ((k, s.ks), (v, s.vs)))
+    first = s.ctx - s.n
+    if s.kind in ("attn", "rows"):
+        return _attend64(s.q.double().reshape(s.n, c["heads"], hd), k, v, first)
+
+    def mul(i, x):
+        return _matmul64(x, s.ws[i], c["type"], *s.mats[i])
+    x = _norm64(s.x.double(), s.an)
+    ys = [mul(i, x) for i in range(3)]
+    att = _attend64(ys[0].reshape(s.n, c["heads"], hd), k, v, first)
+    ys.append(mul(3, att))
+    x = _norm64(s.x.double(), s.fn)
+    ys += [mul(4, x), mul(5, x)]
+    act = ys[5] * ys[4] * torch.sigmoid(ys[4])
+    ys.append(mul(6, act))
+    return ys, att, act
