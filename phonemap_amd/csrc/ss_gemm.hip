@@ -3,28 +3,40 @@
 // evaluates a prompt layer by layer; every token of a layer multiplies the
 // same matrices).
 //
-// v_mfma_f32_16x16x4f32: A is a 16-row x 4-column slice of the weights,
-// dequantised exactly in fp32 (d * (nibble - 8), quantize.c:60-72, or d *
-// code, quantize.c:139-149: an fp16 d times a small integer is exact in
-// fp32), B the 4 x 16 matching slice of 16 tokens' x (times the RMSNorm weight
-// when set), and the accumulator runs in fp32 over all blocks, as the
-// reference's fp32 dot product does. The RMSNorm scale 1/rms of each token
-// multiplies its outputs (tensor.c:114-131 applies it to x).
+// The products run on v_mfma_f32_32x32x16_f16 for every block format (Q4_0,
+// Q8_0, Q4_1, Q5_1, Q8_1, the K-quants; Q5_0 as Q8_0): the codes are exact
+// fp16 integers from a magic number (bits 0x6400 | u are 1024 + u; the
+// subtraction of the offset is exact), x is split into two fp16 parts under a
+// power-of-two scale per token and 256 columns (the largest |x s| in [2^13,
+// 2^14), so xh + xl is within 2^-22 |x| of x), every block's fp32 result is
+// scaled by its A into fp32 accumulators. The RMSNorm scale 1/rms of each
+// token multiplies its outputs (tensor.c:114-131 applies it to x).
 //
-// MFMA operand layout (checked on the device): lane l supplies A[l%16][l/16]
-// and B[l/16][l%16] and receives D[4*(l/16) + i][l%16], i = 0..3.
+// Two kernels share the arithmetic. k_gemm_ks, for short prompts, splits the
+// columns over the 8 waves of a workgroup and takes x straight into
+// registers; k_gemm_rs, for longer ones, has several waves read the same x
+// from LDS. pick_shape() chooses.
 //
-// The fast path (k_gemm_h, with a split-x scratch) runs the same products on
-// v_mfma_f32_16x16x32_f16 for every block format (Q4_0, Q8_0, Q4_1, Q5_1,
-// Q8_1, the K-quants; Q5_0 as Q8_0): the codes are exact fp16 integers, x is
-// split into two fp16 parts, and each block's (or 16-weight group's) fp32
-// result is scaled by its A, with B times the sum of x subtracted (see
-// below): eight times the fp32 MFMA rate per product, with x kept to 2^-22.
+// MFMA operands: lane l supplies A[l%32][8(l/32) + i] (x: token l%32) and
+// B[8(l/32) + i][l%32] (codes: row l%32), i = 0..7, and receives
+// D[8(j/4) + 4(l/32) + j%4][l%32] (token, row) in register j = 0..15. Step h
+// = 0, 1 of a block covers its columns 16h .. 16h + 15 (its two 16-weight
+// groups); slot i of lane half kg is column 16h + 8kg + 4(i/4) + p(i%4), p =
+// 0, 2, 1, 3: the order in which masking a code word gives fp16 pairs.
+//
+// K-quants other than Q6_K: weight = d * (sc * q) - dmin * m (Q3_K: d *
+// (s - 32)(q - 4), no minimum) with sc * q an integer of at most 2048, exact
+// in fp16. The codes are multiplied by their integer scale as fp16 pairs, a
+// whole unit (one super-block) runs as one chain of MFMAs, and d multiplies
+// its result once instead of every block's. The minima are one more MFMA per
+// unit (m exact, the unit's sums of x in two fp16 parts), times dmin. Q4_1
+// and Q5_1 take their minima the same way (m is an fp16).
 
 #include <hip/hip_runtime.h>
 #include <math.h>
 
 #include <atomic>
+#include <type_traits>
 
 #include "ss_device.h"
 #include "ss_kernels.h"
@@ -32,367 +44,27 @@
 namespace ssk {
 namespace {
 
-typedef float v4f __attribute__((ext_vector_type(4)));
-
-constexpr int kGemmWaves = 4;     // row groups of 16 per workgroup
-constexpr int kGemmTiles = 4;     // 16-token tiles per wave
-constexpr int kGemmTok = kGemmTiles * 16;
-constexpr int kXsPad = kGemmTok + 4;   // LDS row (one column of x for 64 tokens), padded
-
-// Sum of squares of each token's x (one workgroup per token), for the RMSNorm scale.
-__global__ void __launch_bounds__(256) k_sumsq(const float* __restrict__ x, int ldx, int cols,
-                                               float* __restrict__ ssq) {
-  __shared__ float red[4];
-  const float* xt = x + (size_t)blockIdx.x * ldx;
-  float ss = 0.f;
-  for (int c = threadIdx.x * 4; c < cols; c += 1024) {
-    const float4 v = *reinterpret_cast<const float4*>(xt + c);
-    ss = fmaf(v.x, v.x, ss);
-    ss = fmaf(v.y, v.y, ss);
-    ss = fmaf(v.z, v.z, ss);
-    ss = fmaf(v.w, v.w, ss);
-  }
-  ss = wave_sum(ss);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-  __syncthreads();
-  if (threadIdx.x == 0) ssq[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
-}
-
-// This lane's eight weights of block b, row m = l%16: columns kq + 4s,
-// s = 0..7, kq = l/16 (the A operands of the block's eight K=4 steps).
-template <int QT>
-struct WBlock {
-  uint32_t w[QT == 2 ? 4 : 8];
-  float d;
-};
-template <int QT>
-__device__ __forceinline__ void load_w(WBlock<QT>& f, const PackedMat& w, int g, int ntk, int b, int lane) {
-  const int tl = tile_lane(lane & 15, b);
-  const uint4* p = reinterpret_cast<const uint4*>(w.qs + tile_idx(g, ntk, b / kTB, tl) * QTraits<QT>::kQB);
-  const uint4 v0 = p[0];
-  f.w[0] = v0.x; f.w[1] = v0.y; f.w[2] = v0.z; f.w[3] = v0.w;
-  if constexpr (QT == 8) {
-    const uint4 v1 = p[1];
-    f.w[4] = v1.x; f.w[5] = v1.y; f.w[6] = v1.z; f.w[7] = v1.w;
-  }
-  f.d = h2f(w.ds[scale_idx(g, ntk, b / kTB, tl)]);
-}
-template <int QT>
-__device__ __forceinline__ float weight(const WBlock<QT>& f, int s, int kq) {
-  if constexpr (QT == 2) {   // column kq + 4s: byte kq of word s % 4, low nibble (s < 4) or high
-    const int nib = (int)((f.w[s & 3] >> (8 * kq + (s >= 4 ? 4 : 0))) & 0xFu);
-    return f.d * (float)(nib - 8);
-  } else {                   // byte kq of word s
-    return f.d * (float)(int8_t)((f.w[s] >> (8 * kq)) & 0xFFu);
-  }
-}
-
-// Rows r0 .. r0+3 of token t from the products g (and u, the up projection,
-// for EPI_SWIGLU): the RMSNorm scale of the token, the epilogue, the store.
-template <int EPI>
-__device__ __forceinline__ void gemm_epilogue(const GemmArgs& a, int t, int r0, const float (&g)[4],
-                                              const float (&u)[4]) {
-  const float scale = a.nw ? 1.0f / sqrtf(a.ssq[t] / (float)a.cols + a.eps) : 1.0f;
-  float* yp = a.y + (size_t)t * a.ldy + r0;
-  float v[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float x0 = g[i] * scale;
-    if constexpr (EPI == EPI_SWIGLU) {
-      const float up = u[i] * scale;
-      v[i] = up * (a.act == 1 ? gelu_tanh(x0) : silu(x0));   // layer_scheduler.c:529-547
-    } else {
-      v[i] = x0;
-    }
-  }
-  if (r0 + 3 < a.rows) {
-    float4 o = make_float4(v[0], v[1], v[2], v[3]);
-    if constexpr (EPI == EPI_ADD) {
-      const float4 p = *reinterpret_cast<const float4*>(yp);
-      o.x += p.x;
-      o.y += p.y;
-      o.z += p.z;
-      o.w += p.w;
-    }
-    *reinterpret_cast<float4*>(yp) = o;
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (r0 + i < a.rows) yp[i] = EPI == EPI_ADD ? yp[i] + v[i] : v[i];
-  }
-}
-
-template <int QT, int NMAT, int EPI>
-__global__ void __launch_bounds__(kGemmWaves * 64) k_gemm(const GemmArgs a) {
-  __shared__ float xs[2][32][kXsPad];   // x of the block: [column][token]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int g = blockIdx.x * kGemmWaves + wave;   // row group (past the last: computes, stores nothing)
-  const int ngroups = (a.rows + kRG - 1) / kRG;
-  const int gl = min(g, ngroups - 1);
-  const int nb = a.cols >> 5;
-  const int ntk = (nb + kTB - 1) / kTB;
-  const int t0 = blockIdx.y * kGemmTok;
-  const int n = lane & 15, kq = lane >> 4;
-
-  // staging: thread -> token t0 + tid/4, columns (tid%4)*8 .. +7 of the block
-  const int st = tid >> 2, sc = (tid & 3) * 8;
-  const float* xrow = a.x + (size_t)min(t0 + st, a.T - 1) * a.ldx;
-  float xv[8];
-  auto fetch_x = [&](int b) {
-    const float4 u = *reinterpret_cast<const float4*>(xrow + b * 32 + sc);
-    const float4 v = *reinterpret_cast<const float4*>(xrow + b * 32 + sc + 4);
-    xv[0] = u.x; xv[1] = u.y; xv[2] = u.z; xv[3] = u.w;
-    xv[4] = v.x; xv[5] = v.y; xv[6] = v.z; xv[7] = v.w;
-    if (a.nw) {
-      const float4 p = *reinterpret_cast<const float4*>(a.nw + b * 32 + sc);
-      const float4 q = *reinterpret_cast<const float4*>(a.nw + b * 32 + sc + 4);
-      xv[0] *= p.x; xv[1] *= p.y; xv[2] *= p.z; xv[3] *= p.w;
-      xv[4] *= q.x; xv[5] *= q.y; xv[6] *= q.z; xv[7] *= q.w;
-    }
-  };
-  auto put_x = [&](int buf) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) xs[buf][sc + j][st] = xv[j];
-  };
-
-  v4f acc[NMAT][kGemmTiles];
-#pragma unroll
-  for (int mt = 0; mt < NMAT; ++mt)
-#pragma unroll
-    for (int tt = 0; tt < kGemmTiles; ++tt) acc[mt][tt] = v4f{0.f, 0.f, 0.f, 0.f};
-
-  WBlock<QT> wb[NMAT];
-  fetch_x(0);
-#pragma unroll
-  for (int mt = 0; mt < NMAT; ++mt) load_w<QT>(wb[mt], mt == 0 ? a.w : a.w2, gl, ntk, 0, lane);
-  put_x(0);
-  __syncthreads();
-  for (int b = 0; b < nb; ++b) {
-    const int buf = b & 1;
-    const bool more = b + 1 < nb;
-    WBlock<QT> wn[NMAT];
-    if (more) {   // the next block's x and weights in flight during this block's products
-      fetch_x(b + 1);
-#pragma unroll
-      for (int mt = 0; mt < NMAT; ++mt) load_w<QT>(wn[mt], mt == 0 ? a.w : a.w2, gl, ntk, b + 1, lane);
-    }
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      float bx[kGemmTiles];
-#pragma unroll
-      for (int tt = 0; tt < kGemmTiles; ++tt) bx[tt] = xs[buf][4 * s + kq][tt * 16 + n];
-#pragma unroll
-      for (int mt = 0; mt < NMAT; ++mt) {
-        const float av = weight<QT>(wb[mt], s, kq);
-#pragma unroll
-        for (int tt = 0; tt < kGemmTiles; ++tt)
-          acc[mt][tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bx[tt], acc[mt][tt], 0, 0, 0);
-      }
-    }
-    if (more) {
-      put_x(buf ^ 1);
-#pragma unroll
-      for (int mt = 0; mt < NMAT; ++mt) wb[mt] = wn[mt];
-    }
-    __syncthreads();
-  }
-  if (g >= ngroups) return;
-
-  // epilogue: lane holds rows g*16 + 4kq + i of token t0 + 16tt + n
-  const int r0 = g * kRG + 4 * kq;
-#pragma unroll
-  for (int tt = 0; tt < kGemmTiles; ++tt) {
-    const int t = t0 + tt * 16 + n;
-    if (t >= a.T) continue;
-    float gv[4], uv[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      gv[i] = acc[0][tt][i];
-      uv[i] = acc[NMAT - 1][tt][i];
-    }
-    gemm_epilogue<EPI>(a, t, r0, gv, uv);
-  }
-}
-
-// ---- fp16 products -----------------------------------------------------------
-// Each 16x16x32 step is one 32-column block: B holds the block's codes as
-// exact fp16 integers (nibble - 8, or the Q8_0 code), A the 16 tokens' x as
-// two fp16 parts, and the step's fp32 result is scaled by the block's d (one
-// per output row) into the accumulator. Codes come from a magic number: the
-// fp16 with bits 0x6400 | u is 1024 + u for u < 1024, and subtracting 1032
-// (Q4_0) or 1152 (Q8_0, u = code + 128) is exact.
-//
-// x of each token is scaled by a power of two s_t (its largest |x| then lies
-// in [2^13, 2^14)) and split into xh = fp16(x s_t) and xl = fp16(x s_t - xh):
-// xh + xl is within 2^-22 |x| of x (or 2^-25 / s_t absolute for the small
-// elements), against 2^-24 for fp32 itself; 1/s_t is applied in the epilogue.
-//
-// Slot order: lane group kq (= lane/16) supplies slots 8kq .. 8kq+7 of the
-// step. Q4_0: the 8 nibbles of 32-bit word kq of the block, two per fp16 pair
-// (bits 4k and 4k+16: slot 2k and 2k+1), i.e. slot s is column
-// 4kq + 2(s&1) + (s>>2) + 16((s>>1)&1). Q8_0: bytes 8kq .. 8kq+7, slot s is
-// column 8kq + 4(s>>2) + 2(s&1) + ((s>>1)&1). The split x holds each block in
-// slot order, so lane group kq reads 16 contiguous bytes.
+typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 
-constexpr int kHWaves = 4;
-constexpr int kHTiles = 4;                // 16-token tiles per workgroup
-constexpr int kHTok = kHTiles * 16;
-constexpr int kHChunks = 16;              // 16-byte chunks of one token's 128 columns
-
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-typedef __attribute__((address_space(1))) void* gbl_ptr_t;
-
-constexpr v8h kOnes = {1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16};
-
-template <int QT>
-__host__ __device__ constexpr int slot_col(int s) {   // column within the block of slot s (s < 32)
-  return QT == 2 ? 4 * (s >> 3) + 2 * (s & 1) + ((s >> 2) & 1) + 16 * ((s >> 1) & 1)
-                 : 8 * (s >> 3) + 4 * ((s >> 2) & 1) + 2 * (s & 1) + ((s >> 1) & 1);
-}
-
-// Token blockIdx.x of x (times nw): the scale 1/s_t into xinv[t], then the
-// fp16 parts in slot order (ldxs: row length, a multiple of 128; columns past
-// cols are zero); with ssq set, first its sum of squares (of x alone).
-// Thread i takes the 32-column blocks i, i + 256, ...: a block is 8 float4 of
-// x (and of nw), all requested before any is used, so each pass over the row
-// is one round trip per block a thread holds; a block's four 16-byte chunks
-// of each part are then formed in registers, in slot order.
-template <int QT>
-__global__ void __launch_bounds__(256) k_split_x(const float* __restrict__ x, int ldx, const float* __restrict__ nw,
-                                                 int cols, float* __restrict__ ssq, uint16_t* __restrict__ xh,
-                                                 uint16_t* __restrict__ xl, float* __restrict__ xinv, int ldxs) {
-  __shared__ float red[2][4];
-  const int t = blockIdx.x;
-  const float* xt = x + (size_t)t * ldx;
-  const int nb = cols >> 5;   // cols is a multiple of 32: whole blocks
-  // block blk: v = x, u = x * nw (x when nw is null)
-  auto load_block = [&](int blk, float (&v)[32], float (&u)[32]) {
-    const float4* xp = reinterpret_cast<const float4*>(xt + 32 * blk);
-    float4 xv[8], wv[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) xv[i] = xp[i];
-    if (nw) {
-      const float4* wp = reinterpret_cast<const float4*>(nw + 32 * blk);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) wv[i] = wp[i];
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      v[4 * i] = xv[i].x;
-      v[4 * i + 1] = xv[i].y;
-      v[4 * i + 2] = xv[i].z;
-      v[4 * i + 3] = xv[i].w;
-      if (nw) {
-        u[4 * i] = xv[i].x * wv[i].x;
-        u[4 * i + 1] = xv[i].y * wv[i].y;
-        u[4 * i + 2] = xv[i].z * wv[i].z;
-        u[4 * i + 3] = xv[i].w * wv[i].w;
-      } else {
-        u[4 * i] = xv[i].x;
-        u[4 * i + 1] = xv[i].y;
-        u[4 * i + 2] = xv[i].z;
-        u[4 * i + 3] = xv[i].w;
-      }
-    }
-  };
-  float ss = 0.f, mx = 0.f;
-  for (int blk = threadIdx.x; blk < nb; blk += 256) {
-    float v[32], u[32];
-    load_block(blk, v, u);
-#pragma unroll
-    for (int j = 0; j < 32; ++j) {
-      ss = fmaf(v[j], v[j], ss);
-      mx = fmaxf(mx, fabsf(u[j]));
-    }
-  }
-  ss = wave_sum(ss);
-  mx = wave_max(mx);
-  if ((threadIdx.x & 63) == 0) {
-    red[0][threadIdx.x >> 6] = ss;
-    red[1][threadIdx.x >> 6] = mx;
-  }
-  __syncthreads();
-  mx = fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3]));
-  int e = 0;
-  if (mx > 0.f && mx <= 3.0e38f) frexpf(mx, &e);        // mx < 2^e
-  const float sc = ldexpf(1.0f, 14 - e);                // largest |x s| in [2^13, 2^14)
-  if (threadIdx.x == 0) {
-    if (ssq) ssq[t] = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
-    xinv[t] = ldexpf(1.0f, e - 14);
-  }
-  uint4* oh = reinterpret_cast<uint4*>(xh + (size_t)t * ldxs);
-  uint4* ol = reinterpret_cast<uint4*>(xl + (size_t)t * ldxs);
-  for (int blk = threadIdx.x; blk < ldxs / 32; blk += 256) {
-    float u[32];
-    if (blk < nb) {
-      float v[32];
-      load_block(blk, v, u);
-    } else {
-#pragma unroll
-      for (int j = 0; j < 32; ++j) u[j] = 0.f;   // padding columns past cols
-    }
-#pragma unroll
-    for (int kq = 0; kq < 4; ++kq) {   // chunk 4 blk + kq: slots 8 kq .. 8 kq + 7
-      uint32_t h[4], l[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const float v0 = u[slot_col<QT>(8 * kq + 2 * k)] * sc;
-        const float v1 = u[slot_col<QT>(8 * kq + 2 * k + 1)] * sc;
-        const _Float16 a = (_Float16)v0, b = (_Float16)v1;
-        const _Float16 la = (_Float16)(v0 - (float)a), lb = (_Float16)(v1 - (float)b);
-        h[k] = __builtin_bit_cast(uint32_t, h2{a, b});
-        l[k] = __builtin_bit_cast(uint32_t, h2{la, lb});
-      }
-      oh[4 * blk + kq] = make_uint4(h[0], h[1], h[2], h[3]);
-      ol[4 * blk + kq] = make_uint4(l[0], l[1], l[2], l[3]);
-    }
-  }
-}
-
-// The weight formats of the products. Every 32-weight block is
-// sum_g (A_g * sum c x - B_g * sum x) over its two 16-weight groups g, c
-// being the stored code (an exact fp16 integer) and A, B exact fp32:
+// Every 32-weight block is sum_g (A_g * sum c x - B_g * sum x) over its two
+// 16-weight groups g, c being the stored code (an exact fp16 integer) and A,
+// B exact fp32:
 //   Q4_0, Q8_0: A = d, B = 0 (Q4_0 codes are nibble - 8)
 //   Q4_1, Q5_1: A = d, B = -m (nibbles; 5-bit codes as int8)
 //   Q8_1:       A = fp32 d, B = 0
 //   K-quants:   kq_affine (Q4_K and Q5_K one (A, B) pair per block; Q2_K,
 //               Q3_K and Q6_K one per 16-weight group)
-// kLay: the code layout, and so the slot order of the split x (2: nibbles
-// as Q4_0's, 8: int8 codes as Q8_0's).
+// kLay: the code layout (2: nibbles as Q4_0's, 8: int8 codes as Q8_0's).
 template <int QT>
 struct PQ {
   static constexpr int kLay = code_bytes_of(QT) == 16 ? 2 : 8;
   static constexpr bool kGroups = QT == kQ2K || QT == kQ3K || QT == kQ6K;
   static constexpr bool kMin =
       QT == kQ4_1 || QT == kQ5_1 || QT == kQ2K || QT == kQ3K || QT == kQ4K || QT == kQ5K;
-  static constexpr float kNibOff = QT == 2 ? -1032.0f : -1024.0f;   // 0x6400 | u is 1024 + u
 };
-
-// A lane's 8 codes of one block as exact fp16 values in slot order (nibble
-// layout: w0 = 32-bit word kq of the block; int8 layout: w0, w1 = words 2kq,
-// 2kq+1).
-template <int QT>
-__device__ __forceinline__ v8h codes_f16(uint32_t w0, uint32_t w1) {
-  v4u r;
-  if constexpr (PQ<QT>::kLay == 2) {
-    const h2 off = {(_Float16)PQ<QT>::kNibOff, (_Float16)PQ<QT>::kNibOff};
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-      r[k] = __builtin_bit_cast(uint32_t,
-                                __builtin_bit_cast(h2, ((w0 >> (4 * k)) & 0x000F000Fu) | 0x64006400u) + off);
-  } else {
-    const h2 off = {(_Float16)-1152.0f, (_Float16)-1152.0f};
-    const uint32_t u0 = w0 ^ 0x80808080u, u1 = w1 ^ 0x80808080u;
-    r[0] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, (u0 & 0x00FF00FFu) | 0x64006400u) + off);
-    r[1] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, ((u0 >> 8) & 0x00FF00FFu) | 0x64006400u) + off);
-    r[2] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, (u1 & 0x00FF00FFu) | 0x64006400u) + off);
-    r[3] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, ((u1 >> 8) & 0x00FF00FFu) | 0x64006400u) + off);
-  }
-  return __builtin_bit_cast(v8h, r);
-}
 
 // (A_g, B_g) of a block from its scale entry e (16 bits, or 32 for Q4_1 /
 // Q5_1 / Q8_1) and, for the K-quants, its super-block word sup.
@@ -412,291 +84,864 @@ __device__ __forceinline__ void block_affine(uint32_t e, uint32_t sup, float (&A
   }
 }
 
-// The slots of 16-weight group g among a lane's 8 (slot order above): nibble
-// layout, slots 2, 3, 6, 7 are the block's weights 16..31 (pairs 1 and 3 of
-// the four fp16 pairs); int8 layout, lane groups kq 2 and 3 hold them.
+
+// Sum of squares of each token's x (one workgroup per token), for the
+// embedding's RMSNorm scale.
+__global__ void __launch_bounds__(256) k_sumsq(const float* __restrict__ x, int ldx, int cols,
+                                               float* __restrict__ ssq) {
+  __shared__ float red[4];
+  const float* xt = x + (size_t)blockIdx.x * ldx;
+  float ss = 0.f;
+  for (int c = threadIdx.x * 4; c < cols; c += 1024) {
+    const float4 v = *reinterpret_cast<const float4*>(xt + c);
+    ss = fmaf(v.x, v.x, ss);
+    ss = fmaf(v.y, v.y, ss);
+    ss = fmaf(v.z, v.z, ss);
+    ss = fmaf(v.w, v.w, ss);
+  }
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  if (threadIdx.x == 0) ssq[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+// a * x + y
+__device__ __forceinline__ v16f fma16(float a, v16f x, v16f y) { return __builtin_elementwise_fma(v16f(a), x, y); }
+
+constexpr int kSW = 8;            // waves per workgroup
+constexpr int kSUnit = 8;         // 32-column blocks of a unit (2 tiles, one super-block)
+constexpr int kSTok = 32;         // tokens of a tile
+constexpr float kSumScale = 1.0f / 32.0f;   // |x s_t| < 2^14, so a block's sum times this is below 2^14 too
+
+// MFMA steps of a unit's minima (8 sums each): none, one per block, one per 16-weight group
 template <int QT>
-__device__ __forceinline__ v8h group_part(v8h v, int g, int kq) {
-  if constexpr (PQ<QT>::kLay == 2) {
-    v4u r = __builtin_bit_cast(v4u, v);
-    if (g == 0) {
-      r[1] = 0u;
-      r[3] = 0u;
-    } else {
-      r[0] = 0u;
-      r[2] = 0u;
+constexpr int sum_steps() {
+  return QT == kQ2K ? 2 : QT == kQ4_1 || QT == kQ5_1 || QT == kQ4K || QT == kQ5K ? 1 : 0;
+}
+// the integer scale is multiplied into the codes
+template <int QT>
+constexpr bool folded() { return QT == kQ2K || QT == kQ3K || QT == kQ4K || QT == kQ5K; }
+
+__host__ __device__ constexpr int slot_col_ks(int i) {   // column of slot i (i < 8) within a lane half's 8
+  return 4 * (i >> 2) + ((i & 1) << 1 | ((i >> 1) & 1));
+}
+
+// The split x of ntile token tiles and nu units: the fragments, then per
+// (tile, unit) of 32 tokens the inverse scales, the sums of squares, and the
+// block sums' fragments.
+struct KsView {
+  uint4* x;        // fragment (tile, block, step, part): 64 chunks of 16 bytes
+  float* inv;      // [tile][unit][32]
+  float* ssq;      // [tile][unit][32]
+  uint4* sum;      // fragment (tile, unit, step): 64 chunks
+};
+__host__ __device__ inline KsView ks_view(uint16_t* xs, int ntile, int nu) {
+  KsView v;
+  v.x = reinterpret_cast<uint4*>(xs);
+  v.inv = reinterpret_cast<float*>(v.x + (size_t)ntile * nu * kSUnit * 4 * 64);
+  v.ssq = v.inv + (size_t)ntile * nu * kSTok;
+  v.sum = reinterpret_cast<uint4*>(v.ssq + (size_t)ntile * nu * kSTok);
+  return v;
+}
+
+// One wave: 8 tokens (lane % 8) x the 8 blocks (lane / 8) of unit blockIdx.y
+// of x (times nw). The unit's inverse scale 1/s per token (the largest |x s|
+// of the unit lies in [2^13, 2^14)) and its sum of squares of x, then x s as
+// two fp16 parts in fragment order: part p of step h of block b is the 1 KB
+// fragment 2h + p of (tile, b), lane half kg and token t%32 at chunk 32 kg +
+// t%32. So 8 lanes write 128 contiguous bytes, and no reduction leaves the
+// wave. Blocks past the row are zero; tokens past T are not written (nor
+// used). SUMS: also the sums of each block (1) or 16-column group (2), times
+// kSumScale, as two fp16 parts: fragment (tile, unit, step), part and token
+// as kg and token above, 8 sums each.
+template <int SUMS>
+__global__ void __launch_bounds__(64) k_split_ks(const float* __restrict__ x, int ldx, const float* __restrict__ nw,
+                                                 int T, int nb, KsView o) {
+  const int lane = threadIdx.x, b = lane >> 3;
+  const int t = blockIdx.x * 8 + (lane & 7), unit = blockIdx.y, nu = gridDim.y;
+  const int blk = unit * kSUnit + b, tile = t / kSTok, tok = t % kSTok;
+  const bool in = t < T && blk < nb;
+  float u[32], ss = 0.f, mx = 0.f;
+  {
+    const float4* xq = reinterpret_cast<const float4*>(x + (size_t)min(t, T - 1) * ldx + 32 * min(blk, nb - 1));
+    const float4* wq = nw ? reinterpret_cast<const float4*>(nw + 32 * min(blk, nb - 1)) : xq;
+    float4 xv[8], wv[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) xv[i] = xq[i];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) wv[i] = wq[i];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float a[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w};
+      const float w[4] = {wv[i].x, wv[i].y, wv[i].z, wv[i].w};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float v = in ? a[k] : 0.f;
+        ss = fmaf(v, v, ss);
+        u[4 * i + k] = nw ? v * w[k] : v;
+        mx = fmaxf(mx, fabsf(u[4 * i + k]));
+      }
     }
-    return __builtin_bit_cast(v8h, r);
-  } else {
-    return (kq >= 2) == (g == 1) ? v : v8h{};
+  }
+#pragma unroll
+  for (int off = 8; off < 64; off <<= 1) {
+    ss += __shfl_xor(ss, off, kWave);
+    mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
+  }
+  int e = 0;
+  if (mx > 0.f && mx <= 3.0e38f) frexpf(mx, &e);        // mx < 2^e
+  e = max(e, -100);                                     // (2^(14 - e) stays finite)
+  const float sc = ldexpf(1.0f, 14 - e);                // largest |x s| in [2^13, 2^14)
+  if (t >= T) return;
+  const size_t at = (size_t)tile * nu + unit;
+  if (b == 0) {
+    o.inv[at * kSTok + tok] = ldexpf(1.0f, e - 14);
+    o.ssq[at * kSTok + tok] = ss;
+  }
+  uint4* q = o.x + (at * kSUnit + b) * 4 * kWave + tok;
+  float sum[2] = {0.f, 0.f};
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int kg = 0; kg < 2; ++kg) {
+      uint32_t hi[4], lo[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float v0 = u[16 * h + 8 * kg + slot_col_ks(2 * k)] * sc;
+        const float v1 = u[16 * h + 8 * kg + slot_col_ks(2 * k + 1)] * sc;
+        const _Float16 p = (_Float16)v0, r = (_Float16)v1;
+        const _Float16 lp = (_Float16)(v0 - (float)p), lr = (_Float16)(v1 - (float)r);
+        hi[k] = __builtin_bit_cast(uint32_t, h2{p, r});
+        lo[k] = __builtin_bit_cast(uint32_t, h2{lp, lr});
+        if constexpr (SUMS > 0) sum[SUMS == 2 ? h : 0] += ((float)p + (float)lp) + ((float)r + (float)lr);
+      }
+      q[(2 * h) * kWave + 32 * kg] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+      q[(2 * h + 1) * kWave + 32 * kg] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+    }
+#pragma unroll
+  for (int g = 0; g < SUMS; ++g) {
+    const int i = SUMS * b + g;   // sum i of the unit
+    const float v = sum[g] * kSumScale;
+    const _Float16 p = (_Float16)v;
+    const _Float16 r = (_Float16)(v - (float)p);
+    uint16_t* z = reinterpret_cast<uint16_t*>(o.sum + (at * SUMS + i / 8) * kWave + tok) + i % 8;
+    z[0] = __builtin_bit_cast(uint16_t, p);
+    z[32 * 8] = __builtin_bit_cast(uint16_t, r);
   }
 }
 
-// Workgroup: 4 waves x kHRG row groups of 16 rows x 64 tokens. Per packed tile
-// (4 blocks, 128 columns) the split x of the 64 tokens is copied into LDS by
-// direct global-to-LDS loads (double buffered; the next tile's x, codes and
-// scales in flight during this tile's products). Chunk q of token r sits at
-// slot q ^ (r % 16) of its LDS row, so the 16 tokens of a tile read one
-// chunk each from distinct banks. Lane (n, kq): weight row n of each row
-// group, token rows 4kq .. 4kq+3 of each 16-token tile in the results.
-template <int QT, int NMAT, int EPI, int kHRG>
-__global__ void __launch_bounds__(kHWaves * 64, 2) k_gemm_h(const GemmArgs a, int ldxs) {
-  __shared__ v4u xs[2][2][kHTok][kHChunks];   // [buffer][high, low][token][slot]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int ngroups = (a.rows + kRG - 1) / kRG;
-  const int g0 = (blockIdx.x * kHWaves + wave) * kHRG;
-  const int nb = a.cols >> 5;
-  const int ntk = (nb + kTB - 1) / kTB;
-  const int t0 = blockIdx.y * kHTok;
-  const int n = lane & 15, kq = lane >> 4;
-  constexpr int kQW = PQ<QT>::kLay == 2 ? 1 : 2;   // code words per lane per block
-  const uint16_t* xlo = a.xs + (size_t)a.T * ldxs;
-  const float* xinv = reinterpret_cast<const float*>(a.xs + 2 * (size_t)a.T * ldxs);
-
-  // staging: 2 parts x 64 tokens x 16 chunks per tile = 32 rows of 1 KB; wave
-  // w copies rows 8w .. 8w+7 (part R / 16, tokens 4(R % 16) .. +3), lane i
-  // token 4(R % 16) + i/16, slot i % 16
-  auto stage_x = [&](int tk, int buf) {
+// A lane's 8 codes of step h of a block as exact fp16 values in slot order.
+// Nibble layout: words 2kg and 2kg+1 of the block's chunk serve both steps
+// (low nibbles, then high). int8 layout: words 4h + 2kg and + 1.
+// magic: 0x64006400 in a vector register, so that mask and or are one
+// instruction (it takes one constant beside its registers).
+template <int QT>
+__device__ __forceinline__ v8h codes_ks(uint2 w, int h, uint32_t magic) {
+  v4u r;
+  const uint32_t q[2] = {w.x, w.y};
+  if constexpr (PQ<QT>::kLay == 2) {
+    // Q4_0: nibble - 8; Q3_K: its code + 4 - 4; the others' nibble as it is
+    constexpr float kOff = QT == 2 ? -1032.0f : QT == kQ3K ? -1028.0f : -1024.0f;
+    const h2 off = {(_Float16)kOff, (_Float16)kOff};
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int R = 8 * wave + k, part = R >> 4, r = 4 * (R & 15) + (lane >> 4), slot = lane & 15;
-      const int t = min(t0 + r, a.T - 1);
-      const uint16_t* src = (part ? xlo : a.xs) + (size_t)t * ldxs + tk * 128 + 8 * (slot ^ (r & 15));
-      __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)&xs[buf][part][4 * (R & 15)][0], 16, 0, 0);
+    for (int k = 0; k < 4; ++k)
+      r[k] = __builtin_bit_cast(
+          uint32_t, __builtin_bit_cast(h2, ((q[k >> 1] >> (8 * (k & 1) + 4 * h)) & 0x000F000Fu) | magic) + off);
+  } else {
+    const h2 off = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      // bytes 0, 2 (k even) or 1, 3 of the word, each below a 0x64
+      const uint32_t u = q[k >> 1] ^ 0x80808080u;
+      r[k] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, __builtin_amdgcn_perm(magic, u, k & 1 ? 0x05030501u : 0x05020500u)) + off);
+    }
+  }
+  return __builtin_bit_cast(v8h, r);
+}
+// times an integer scale (the products are integers of at most 2048: exact)
+__device__ __forceinline__ v8h times(v8h c, int sc) {
+  const h2 s = {(_Float16)sc, (_Float16)sc};
+  v4u r = __builtin_bit_cast(v4u, c);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) r[k] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, (uint32_t)r[k]) * s);
+  return __builtin_bit_cast(v8h, r);
+}
+// the integer scale of 16-weight group h from a block's scale entry (kq_affine)
+template <int QT>
+__device__ __forceinline__ int int_scale(uint32_t e, int h) {
+  if constexpr (QT == kQ2K) return (int)((e >> (8 * h)) & 15u);
+  if constexpr (QT == kQ3K) return (int)((e >> (8 * h)) & 0xffu) - 32;
+  return (int)(e & 0xffu);
+}
+
+// One unit's codes and scale entries of one 32-row tile: lane (row n = l%32,
+// half kg).
+template <int QT>
+struct KCodes {
+  static constexpr int kQ = PQ<QT>::kLay == 2 ? 1 : 2;
+  uint2 q[kSUnit][kQ];
+};
+template <int QT>
+struct KScale {
+  static constexpr int kE = is_wide(QT) ? kSUnit : kSUnit / 2;
+  uint32_t e[kE];   // entries of (block b, both tiles)
+  uint32_t su;      // K-quants: the unit is one super-block
+  __device__ __forceinline__ uint32_t entry(int k) const {
+    if constexpr (is_wide(QT)) return e[k];
+    return k / kTB ? e[k % kTB] >> 16 : e[k % kTB] & 0xffffu;
+  }
+};
+
+// The planes of one 32-row tile (row groups gb and gb + 1 of the matrix) as
+// buffer views: a lane's offset is loop-invariant, the tile and unit a scalar.
+template <int QT>
+struct KView {
+  static constexpr int kQB = QTraits<QT>::kQB, kEB = is_wide(QT) ? 4 : 2;
+  __amdgpu_buffer_rsrc_t q, e, su;
+  uint32_t qo, eo, so;
+  int ntk;
+  __device__ __forceinline__ void init(const PackedMat& w, int gb, int ngroups, int ntk_, int n, int kg) {
+    ntk = ntk_;
+    gb = min(gb, ngroups - 1);
+    const int g = min(n / kRG, ngroups - 1 - gb);   // a missing second group: the first again, not stored
+    const uint32_t qg = (uint32_t)ntk * kWave * kQB;
+    const uint32_t eg = (uint32_t)((ntk + kUT - 1) / kUT) * kWave * kUT * kEB;
+    const uint32_t sg = (uint32_t)(ntk / 2) * kRG * 4;
+    q = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(w.qs) + (size_t)gb * qg, (short)0, (int)(2 * qg), kBufferFlags);
+    e = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(reinterpret_cast<const uint8_t*>(w.ds)) + (size_t)gb * eg, (short)0, (int)(2 * eg), kBufferFlags);
+    if constexpr (is_kq(QT))
+      su = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<uint8_t*>(reinterpret_cast<const uint8_t*>(w.su)) + (size_t)gb * sg, (short)0, (int)(2 * sg), kBufferFlags);
+    qo = g * qg + (n % kRG) * kQB + 8 * kg;
+    eo = g * eg + (n % kRG) * kUT * kEB;
+    so = g * sg + (n % kRG) * 4;
+  }
+};
+
+typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+
+// tile h (blocks 4h .. 4h + 3) of unit u, or with h = -1 both
+template <int QT>
+__device__ __forceinline__ void load_codes(KCodes<QT>& f, const KView<QT>& w, int u, int h) {
+  constexpr int kQB = KView<QT>::kQB;
+#pragma unroll
+  for (int k = 0; k < kSUnit; ++k) {
+    if (h >= 0 && k / kTB != h) continue;
+    // a tile past the row (the last unit's) reloads the last one: its x is zero
+    const int t = min(2 * u + k / kTB, w.ntk - 1);
+#pragma unroll
+    for (int i = 0; i < KCodes<QT>::kQ; ++i) {
+      const v2u v = __builtin_amdgcn_raw_buffer_load_b64(w.q, w.qo + (k % kTB) * kRG * kQB + 16 * i, t * kWave * kQB, 0);
+      f.q[k][i] = make_uint2(v.x, v.y);
+    }
+  }
+}
+template <int QT>
+__device__ __forceinline__ void load_scales(KScale<QT>& f, const KView<QT>& w, int u) {
+  constexpr int kEB = KView<QT>::kEB;
+  const int es = ((2 * u / kUT) * kWave * kUT + 2 * u % kUT) * kEB;
+#pragma unroll
+  for (int b = 0; b < kTB; ++b) {
+    if constexpr (is_wide(QT)) {
+      const v2u v = __builtin_amdgcn_raw_buffer_load_b64(w.e, w.eo + b * kRG * kUT * kEB, es, 0);
+      f.e[b] = v.x;
+      f.e[kTB + b] = v.y;
+    } else {
+      f.e[b] = __builtin_amdgcn_raw_buffer_load_b32(w.e, w.eo + b * kRG * kUT * kEB, es, 0);
+    }
+  }
+  f.su = 0u;
+  if constexpr (is_kq(QT)) f.su = __builtin_amdgcn_raw_buffer_load_b32(w.su, w.so, u * kRG * 4, 0);
+}
+
+// The minima of a unit as an MFMA operand: sum i of the unit times its m, in
+// both lane halves (the sums' two parts).
+template <int QT, int S>
+__device__ __forceinline__ void unit_minima(const KScale<QT>& w, v8h (&mv)[S]) {
+#pragma unroll
+  for (int s = 0; s < sum_steps<QT>(); ++s)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t e = w.entry(QT == kQ2K ? (8 * s + j) / 2 : j);
+      if constexpr (QT == kQ2K)
+        mv[s][j] = (_Float16)(int)((e >> (8 * (j & 1) + 4)) & 15u);
+      else if constexpr (is_wide(QT))
+        mv[s][j] = __builtin_bit_cast(_Float16, (uint16_t)(e >> 16));
+      else
+        mv[s][j] = (_Float16)(int)(e >> 8);
+    }
+}
+// acc += (part * d + mins * f) / s for the 16 tokens of a lane half, whose
+// inverse scales are inv[8 (j/4) + j%4]
+template <int QT>
+__device__ __forceinline__ void unit_scale(v16f& acc, const v16f& part, const v16f& mins, float d, float f,
+                                           const float* inv, bool live) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float4 s4 = *reinterpret_cast<const float4*>(inv + 8 * q);
+    const float s[4] = {s4.x, s4.y, s4.z, s4.w};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int j = 4 * q + c;
+      float v = part[j];
+      if constexpr (folded<QT>()) v *= d;
+      if constexpr (sum_steps<QT>() > 0) v = fmaf(f, mins[j], v);
+      if (live) acc[j] = fmaf(s[c], v, acc[j]);
+    }
+  }
+}
+
+// One wave's products of a 32-row tile with TT token tiles, block by block.
+// A block is 4 TT MFMAs; the matrix core takes 32 cycles for each, in which
+// the wave can issue 8 other vector instructions, so what a block needs
+// besides is put between them: the codes of the next block, the scaling of
+// the first token tiles' products while the last one's run, and the scaling
+// of the last one's of the block before.
+template <int QT, int TT>
+struct Pipe {
+  v16f part[TT];   // the unit's sums, to be scaled by 1/s (and d)
+  v8h c0, c1;      // codes of the block to come
+  v16f p;          // the last token tile's product of the block before, not yet scaled
+  float A;         // and its scale
+  uint32_t magic;
+
+  static constexpr bool kDelay = !folded<QT>() && QT != kQ6K;   // p and A are used
+  __device__ __forceinline__ void codes(const KCodes<QT>& q, const KScale<QT>& w, int blk, v8h& n0, v8h& n1) const {
+    n0 = codes_ks<QT>(q.q[blk][0], 0, magic);
+    n1 = codes_ks<QT>(q.q[blk][KCodes<QT>::kQ - 1], 1, magic);
+    if constexpr (folded<QT>()) {
+      n0 = times(n0, int_scale<QT>(w.entry(blk), 0));
+      n1 = times(n1, int_scale<QT>(w.entry(blk), 1));
+    }
+  }
+  __device__ __forceinline__ void init(const KCodes<QT>& q, const KScale<QT>& w) {
+    magic = 0x64006400u;
+    asm("" : "+v"(magic));
+    codes(q, w, 0, c0, c1);
+  }
+  // block BLK of the unit with scales w and x fragments x; wc: the unit's
+  // codes, qn, wn: codes and scales of the unit after it
+  template <int BLK>
+  __device__ __forceinline__ void block(const KCodes<QT>& wc, const KScale<QT>& w, const KCodes<QT>& qn, const KScale<QT>& wn,
+                                        const v8h (&x)[TT][4]) {
+    v8h n0, n1;
+    if constexpr (BLK + 1 < kSUnit)
+      codes(wc, w, BLK + 1, n0, n1);
+    else
+      codes(qn, wn, 0, n0, n1);
+    if constexpr (QT == kQ6K) {   // one scale per 16-weight group
+      float S[2], Z[2];
+      block_affine<QT>(w.entry(BLK), w.su, S, Z);
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt) {
+        v16f q = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[tt][0], c0, v16f{}, 0, 0, 0);
+        v16f r = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[tt][2], c1, v16f{}, 0, 0, 0);
+        q = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[tt][1], c0, q, 0, 0, 0);
+        r = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[tt][3], c1, r, 0, 0, 0);
+        part[tt] = fma16(S[1], r, BLK > 0 ? fma16(S[0], q, part[tt]) : q * S[0]);
+      }
+    } else {
+      v16f q[TT];
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt) {
+        q[tt] = folded<QT>() && BLK > 0 ? part[tt] : v16f{};
+        q[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[tt][0], c0, q[tt], 0, 0, 0);
+        q[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[tt][1], c0, q[tt], 0, 0, 0);
+        q[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[tt][2], c1, q[tt], 0, 0, 0);
+        q[tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[tt][3], c1, q[tt], 0, 0, 0);
+      }
+      if constexpr (folded<QT>()) {
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) part[tt] = q[tt];
+      } else {
+        if constexpr (BLK > 0) add_last<BLK>();
+        float S[2], Z[2];
+        block_affine<QT>(w.entry(BLK), 0u, S, Z);
+#pragma unroll
+        for (int tt = 0; tt + 1 < TT; ++tt) part[tt] = BLK > 0 ? fma16(S[0], q[tt], part[tt]) : q[tt] * S[0];
+        p = q[TT - 1];
+        A = S[0];
+      }
+    }
+    c0 = n0;
+    c1 = n1;
+    constexpr int kValu = (24 + (folded<QT>() ? 10 : QT == kQ6K ? 32 * TT : 16 * TT)) / (4 * TT);
+#pragma unroll
+    for (int i = 0; i < 4 * TT; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);       // an MFMA
+      __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);   // then vector instructions
+    }
+    // the sums stay where they are: the compiler would otherwise put off the
+    // scaling of several blocks
+    if constexpr (!folded<QT>()) {
+      if constexpr (TT == 2 && (BLK > 0 || QT == kQ6K))
+        asm volatile("" : "+v"(part[0]), "+v"(part[TT - 1]));
+      else if constexpr (TT == 2 || BLK > 0 || QT == kQ6K)
+        asm volatile("" : "+v"(part[0]));
+      if constexpr (kDelay) asm volatile("" : "+v"(p));
+    }
+  }
+  template <int BLK>
+  __device__ __forceinline__ void add_last() {   // block BLK - 1's last product
+    part[TT - 1] = BLK > 1 ? fma16(A, p, part[TT - 1]) : p * A;
+  }
+  // The unit is done: acc += its sums, scaled, with its minima. sum: the
+  // fragments of its block sums; inv: the inverse scales of the lane half's
+  // tokens, 8 (j/4) + j%4 for register j of token tile 0, stride ld per tile.
+  template <int S>
+  __device__ __forceinline__ void finish(v16f (&acc)[TT], const KScale<QT>& w, const v8h (&sum)[S][TT], const float* inv,
+                                         int ld, bool live) {
+    if constexpr (kDelay) add_last<kSUnit>();
+    const float d = folded<QT>() ? h2f((uint16_t)(w.su & 0xffffu)) : 1.f, dm = h2f((uint16_t)(w.su >> 16));
+    v8h mv[S];
+    unit_minima<QT>(w, mv);
+    const float fm = is_wide(QT) ? 32.0f : -32.0f * dm;   // Q4_1, Q5_1: + m
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) {
+      v16f r = v16f{};
+#pragma unroll
+      for (int s = 0; s < sum_steps<QT>(); ++s) r = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum[s][tt], mv[s], r, 0, 0, 0);
+      unit_scale<QT>(acc[tt], part[tt], r, d, fm, inv + tt * ld, live);
+    }
+  }
+};
+
+// Codes of one unit, and the fragments of its block sums.
+template <int QT, int TT>
+struct KWork {
+  KCodes<QT> q;
+  KScale<QT> w;
+  v8h sum[sum_steps<QT>() > 0 ? sum_steps<QT>() : 1][TT];
+};
+
+// ---- short prompts: the columns split over the waves ------------------------
+// A workgroup of 8 waves owns 32 rows x 32 tokens (NMAT 2: of both matrices,
+// the first half of the waves taking w (gate), the second w2 (up)); wave w
+// takes the units w, w + 8, ... (w + 4). A wave shares nothing with another
+// until the end: no barrier and no LDS in the loop, x and codes straight into
+// registers. At the end the partial sums of every output are added in LDS in
+// wave order. What bounds it at these sizes is the latency of the chain codes
+// -> x -> products -> sum, not a rate: a 4096 x 4096 Q4_0 matrix takes 10 us
+// per round of workgroups (32 to 64 tokens: 14.4 and 15.9 us with the split,
+// 46.4 us with the 64-row workgroups that staged x in LDS for every matrix
+// before; Q4_K at 77 tokens 58 -> 26.5 us).
+constexpr int kKsUnits = 128;   // units whose inverse scales go through LDS; past them, from memory
+
+template <int QT, int NMAT, int EPI, int TT, int KW>
+__global__ void __launch_bounds__(KW * 64) k_gemm_ks(const GemmArgs a, int nu) {
+  constexpr int SUMS = sum_steps<QT>();
+  constexpr int KS = KW / NMAT;   // column slices
+  constexpr int kThreads = KW * 64, kPer = 1024 / kThreads;   // outputs of a tile per thread
+  __shared__ float red[KW][16][kWave];
+  __shared__ float rn[TT][kThreads];
+  __shared__ float inv_lds[TT * kKsUnits * kSTok];   // [TT][nu][32]
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int slice = wave % KS;
+  const int n = lane & 31, kg = lane >> 5;
+  const int ntk = ((a.cols >> 5) + kTB - 1) / kTB;
+  const int ngroups = (a.rows + kRG - 1) / kRG;
+  const int row0 = blockIdx.x * 32;
+  const int tile0 = blockIdx.y * TT, ntile = (a.T + kSTok - 1) / kSTok;
+  const KsView xs = ks_view(a.xs, ntile, nu);
+
+  KView<QT> wv;
+  wv.init(NMAT == 2 && wave >= KS ? a.w2 : a.w, row0 / kRG, ngroups, ntk, n, kg);
+
+  // this workgroup's token tiles as buffer views: a lane whose token is past
+  // T has an offset past the view and reads zero without touching memory
+  __amdgpu_buffer_rsrc_t xr[TT], sr[TT];
+  uint32_t xo[TT];
+#pragma unroll
+  for (int tt = 0; tt < TT; ++tt) {
+    const size_t at = (size_t)min(tile0 + tt, ntile - 1) * nu;
+    xr[tt] = __builtin_amdgcn_make_buffer_rsrc(xs.x + at * kSUnit * 4 * kWave, (short)0, nu * kSUnit * 4096, kBufferFlags);
+    if constexpr (SUMS > 0)
+      sr[tt] = __builtin_amdgcn_make_buffer_rsrc(xs.sum + at * SUMS * kWave, (short)0, nu * SUMS * 1024, kBufferFlags);
+    xo[tt] = (tile0 + tt) * kSTok + n < a.T ? lane * 16u : 0x7fffff00u;
+  }
+  struct Frags {
+    v8h v[TT][4];   // (step, part) fragments of one block
+  };
+  auto load_x = [&](Frags& f, int blk) {
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        f.v[tt][i] = __builtin_bit_cast(v8h, __builtin_amdgcn_raw_buffer_load_b128(xr[tt], xo[tt] + i * 1024, blk * 4096, 0));
+  };
+  // two units of codes, used in turn: each is refilled with the unit two
+  // turns on as soon as it is used up
+  KWork<QT, TT> wa, wb;
+  auto load_w = [&](KWork<QT, TT>& f, int u) {
+    u = min(u, nu - 1);   // past the end: reloaded, not used
+    load_scales<QT>(f.w, wv, u);
+    load_codes<QT>(f.q, wv, u, -1);
+#pragma unroll
+    for (int s = 0; s < SUMS; ++s)
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt)
+        f.sum[s][tt] =
+            __builtin_bit_cast(v8h, __builtin_amdgcn_raw_buffer_load_b128(sr[tt], xo[tt], (u * SUMS + s) * 1024, 0));
+  };
+  v16f acc[TT];
+#pragma unroll
+  for (int tt = 0; tt < TT; ++tt) acc[tt] = v16f{};
+  Frags xa, xb;   // blocks of even and odd index
+  const int u0 = min(slice, nu - 1);
+  load_w(wa, u0);
+  load_x(xa, u0 * kSUnit);
+  load_x(xb, u0 * kSUnit + 1);
+  load_w(wb, u0 + KS);
+  // while those are in flight: the inverse scales into LDS, and each token's
+  // sum of squares (thread: token tid % 32, units tid / 32, + KW * 2, ...)
+#pragma unroll
+  for (int tt = 0; tt < TT; ++tt) {
+    const size_t at = (size_t)min(tile0 + tt, ntile - 1) * nu * kSTok;
+    float ss = 0.f;
+    for (int i = tid; i < nu * kSTok; i += kThreads) {
+      if (nu <= kKsUnits) inv_lds[tt * nu * kSTok + i] = xs.inv[at + i];
+      ss += xs.ssq[at + i];
+    }
+    rn[tt][tid] = ss;
+  }
+  __syncthreads();
+  Pipe<QT, TT> pipe;
+  pipe.init(wa.q, wa.w);
+  auto unit = [&](int u, KWork<QT, TT>& f, const KWork<QT, TT>& next) {
+    const int un = min(u + KS, nu - 1);
+    auto blocks = [&](auto kc) {   // blocks 2k and 2k + 1, then the x two on
+      constexpr int k = 2 * decltype(kc)::value;
+      pipe.template block<k>(f.q, f.w, next.q, next.w, xa.v);
+      load_x(xa, k + 2 < kSUnit ? u * kSUnit + k + 2 : un * kSUnit);
+      __builtin_amdgcn_sched_barrier(0);
+      pipe.template block<k + 1>(f.q, f.w, next.q, next.w, xb.v);
+      load_x(xb, k + 3 < kSUnit ? u * kSUnit + k + 3 : un * kSUnit + 1);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    blocks(std::integral_constant<int, 0>{});
+    blocks(std::integral_constant<int, 1>{});
+    blocks(std::integral_constant<int, 2>{});
+    blocks(std::integral_constant<int, 3>{});
+    if (nu <= kKsUnits)
+      pipe.finish(acc, f.w, f.sum, inv_lds + u * kSTok + 4 * kg, nu * kSTok, true);
+    else
+      pipe.finish(acc, f.w, f.sum, xs.inv + ((size_t)tile0 * nu + u) * kSTok + 4 * kg, nu * kSTok, true);
+    load_w(f, u + 2 * KS);
+  };
+  int u = slice;
+#pragma unroll 1
+  for (; u + KS < nu; u += 2 * KS) {   // (no branch inside: the compiler then counts the loads exactly)
+    unit(u, wa, wb);
+    unit(u + KS, wb, wa);
+  }
+  if (u < nu) unit(u, wa, wb);
+
+  // the slices' partial sums, tile by tile, added in slice order: output
+  // tid + kThreads k of a tile is register j = wave + KW k, lane `lane`
+  float v[NMAT][TT][kPer];
+#pragma unroll
+  for (int tt = 0; tt < TT; ++tt) {
+    if (tt) __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 16; ++j) red[wave][j][lane] = acc[tt][j];
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < NMAT; ++m)
+#pragma unroll
+      for (int k = 0; k < kPer; ++k) {
+        float s = 0.f;
+#pragma unroll
+        for (int q = 0; q < KS; ++q) s += red[m * KS + q][wave + KW * k][lane];
+        v[m][tt][k] = s;
+      }
+  }
+#pragma unroll
+  for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int j = wave + KW * k;
+      const int tok = 8 * (j >> 2) + 4 * kg + (j & 3), t = (tile0 + tt) * kSTok + tok, row = row0 + n;
+      if (t >= a.T || row >= a.rows) continue;
+      float scale = 1.f;   // the RMSNorm scale of tensor.c:114-131
+      if (a.nw) {
+        float ss = 0.f;
+#pragma unroll
+        for (int q = 0; q < 2 * KW; ++q) ss += rn[tt][q * kSTok + tok];
+        scale = 1.0f / sqrtf(ss / (float)a.cols + a.eps);
+      }
+      float* yp = a.y + (size_t)t * a.ldy + row;
+      const float y = v[0][tt][k] * scale;
+      if constexpr (EPI == EPI_SWIGLU)
+        *yp = v[NMAT - 1][tt][k] * scale * (a.act == 1 ? gelu_tanh(y) : silu(y));   // layer_scheduler.c:529-547
+      else if constexpr (EPI == EPI_ADD)
+        *yp += y;
+      else
+        *yp = y;
+    }
+}
+
+// ---- longer prompts: x shared through LDS -----------------------------------
+// The same products for more tokens. A workgroup of 8 waves owns RW row
+// tiles (32 rows each; NMAT 2: RW / 2 of each matrix) x 64 tokens, its waves
+// being KG = 8 / RW column groups of RW row tiles: column group g takes the
+// units g, g + KG, .... The RW waves of a group read the same x, so it goes
+// through LDS: 32 KB per stage for all groups (SB = RW / 2 blocks of each
+// group's unit), by direct global-to-LDS loads, four stages in four arrays
+// named at compile time, three of them in flight ahead of the one in use.
+// One barrier per stage: past it every wave's loads of the next stage have
+// landed, and every wave has the last of the stage before in registers, so
+// that its array can be refilled.
+//
+// Bound: the vector and matrix instructions of two waves per SIMD. A block of
+// 8 waves takes 0.30 us with nothing but its LDS reads, MFMAs and vector
+// instructions, 0.36 us with the whole chip busy (the clock drops), and about
+// 0.45 us here; a round of workgroups adds the first loads and the last sum.
+// 512 tokens, split included, against 64-row (128-row) workgroups of 16x16x32
+// MFMAs with one tile of x ahead and a full drain per barrier: Q4_0 4096 x
+// 4096 71.8 -> 49.7 us, 11008 x 4096 149 -> 124 us, 4096 x 11008 164 -> 117
+// us; Q4_K 4096 x 4096 93 -> 53.5 us.
+constexpr int kRsUnits = 112;   // columns / 256 at most (the inverse scales' share of LDS)
+
+template <int N>
+__device__ __forceinline__ void wait_loads() {   // all but the N youngest loads, and every LDS access
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4));   // the builtin: the compiler counts it
+}
+
+template <int QT, int NMAT, int EPI, int RW>
+__global__ void __launch_bounds__(kSW * 64) k_gemm_rs(const GemmArgs a, int nu) {
+  constexpr int KG = kSW / RW, SB = RW / 2, NS = kSUnit / SB, TT = 2;
+  constexpr int RT = RW / NMAT;   // row tiles of each matrix
+  constexpr int SUMS = sum_steps<QT>();
+  static_assert(RW >= 2 && NS % 4 == 0, "whole turns of the four stages per unit");
+  // vector memory instructions of a unit's two loads of codes
+  constexpr bool kSumLate = is_wide(QT);   // the block sums at the unit's end (Q4_1, Q5_1: registers)
+  constexpr int kN1 = kTB + (is_kq(QT) ? 1 : 0) + kTB * KCodes<QT>::kQ + (kSumLate ? 0 : SUMS * TT), kN2 = kTB * KCodes<QT>::kQ;
+  constexpr int kStage = 2048;   // 16-byte chunks
+  __shared__ v4u s0[kStage], s1[kStage], s2[kStage], s3[kStage];
+  __shared__ float rn[TT * kSTok], psum[TT][kSW][kSTok];
+  __shared__ float inv_lds[TT * kRsUnits * kSTok];   // [TT][nu][32]
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rt = wave % RW, kgrp = wave / RW;
+  const int n = lane & 31, kg = lane >> 5;
+  const int ntk = ((a.cols >> 5) + kTB - 1) / kTB;
+  const int ngroups = (a.rows + kRG - 1) / kRG;
+  const int row0 = blockIdx.x * 32 * RT;
+  const int tile0 = blockIdx.y * TT, ntile = (a.T + kSTok - 1) / kSTok;
+  const KsView xs = ks_view(a.xs, ntile, nu);
+
+  KView<QT> wv;
+  wv.init(NMAT == 2 && rt >= RT ? a.w2 : a.w, (row0 + 32 * (rt % RT)) / kRG, ngroups, ntk, n, kg);
+  __amdgpu_buffer_rsrc_t sr[TT];
+  if constexpr (SUMS > 0) {
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+      sr[tt] = __builtin_amdgcn_make_buffer_rsrc(xs.sum + (size_t)min(tile0 + tt, ntile - 1) * nu * SUMS * kWave, (short)0,
+                                                 nu * SUMS * 1024, kBufferFlags);
+  }
+  const int nit = (nu + KG - 1) / KG;
+  auto unit_of = [&](int it) { return min(kgrp + it * KG, nu - 1); };
+  // this wave's 4 of the stage's fragments: 8 SB per group, (tt, block, i)
+  auto issue = [&](int u, int stage, v4u* buf) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int f = 4 * rt + k, tt = f / (4 * SB), b = f / 4 % SB, i = f % 4;
+      const uint4* src = xs.x + ((((size_t)min(tile0 + tt, ntile - 1) * nu + u) * kSUnit + stage * SB + b) * 4 + i) * kWave + lane;
+      __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)&buf[(kgrp * 8 * SB + f) * kWave], 16, 0, 0);
     }
   };
-  // per block: codes, the raw scale entry; per tile: the K-quants' super-block word
-  uint32_t wq[NMAT][kHRG][kTB][kQW];
-  uint32_t we[NMAT][kHRG][kTB];
-  uint32_t wsu[NMAT][kHRG];
-  // Blocks past the row (the last tile's padding of a 32-weight type) are
-  // read and weighted 0 (entry 0: A = B = 0). Where that selection sits
-  // decides where the compiler waits for the next tile: made at load, it
-  // waits for the whole next tile (its loads complete in order) inside the
-  // current tile's first block; made at use, those loads overlap all four
-  // blocks. Measured per variant at the 7B and 70B shapes (512-token chunks):
-  // at use, the stores and the one-row-group accumulation ran 9-13% faster
-  // (7B QKV 179 -> 160 us, Wo + down 118 -> 105 us, 70B QKV 319 -> 279 us);
-  // gate+up (1191 -> 1228 us at 70B) and the two-row-group accumulation
-  // (377 -> 426 us) ran slower, so those keep the selection at load.
-  constexpr bool kMaskAtLoad = EPI == EPI_SWIGLU || (EPI == EPI_ADD && kHRG == 2);
-  auto load_w = [&](int tk, uint32_t (&q)[NMAT][kHRG][kTB][kQW], uint32_t (&e)[NMAT][kHRG][kTB],
-                    uint32_t (&su)[NMAT][kHRG]) {
+
+  v16f acc[TT];
 #pragma unroll
-    for (int mt = 0; mt < NMAT; ++mt)
+  for (int tt = 0; tt < TT; ++tt) acc[tt] = v16f{};
+  // One unit of codes: its first tile is refilled with the next unit's after
+  // block 3, with that unit's scales and this one's block sums, its second
+  // tile after block 7 (a second unit in registers would spill)
+  KCodes<QT> q;
+  KScale<QT> w, wn;
+  v8h sum[SUMS > 0 ? SUMS : 1][TT];
+  auto load_sums = [&](int it) {
 #pragma unroll
-      for (int r = 0; r < kHRG; ++r) {
-        const PackedMat& w = mt == 0 ? a.w : a.w2;
-        const int g = min(g0 + r, ngroups - 1);
+    for (int s = 0; s < SUMS; ++s)
 #pragma unroll
-        for (int b = 0; b < kTB; ++b) {
-          const int tl = tile_lane(n, b);
-          const uint32_t* p =
-              reinterpret_cast<const uint32_t*>(w.qs + tile_idx(g, ntk, tk, tl) * QTraits<QT>::kQB) + kQW * kq;
-#pragma unroll
-          for (int k = 0; k < kQW; ++k) q[mt][r][b][k] = p[k];
-          const uint32_t ev = is_wide(QT) ? reinterpret_cast<const uint32_t*>(w.ds)[scale_idx(g, ntk, tk, tl)]
-                                          : (uint32_t)w.ds[scale_idx(g, ntk, tk, tl)];
-          e[mt][r][b] = !kMaskAtLoad || tk * kTB + b < nb ? ev : 0u;
-        }
-        // K-quants: the 4 blocks of a tile lie in super-block tk / 2 (nb is a multiple of 8)
-        su[mt][r] = is_kq(QT) ? w.su[((size_t)g * (ntk / 2) + tk / 2) * kRG + n] : 0u;
-      }
+      for (int tt = 0; tt < TT; ++tt)
+        sum[s][tt] = __builtin_bit_cast(
+            v8h, __builtin_amdgcn_raw_buffer_load_b128(sr[tt], lane * 16, (unit_of(it) * SUMS + s) * 1024, 0));
   };
+  auto load_first = [&](int it) {
+    asm volatile("" ::: "memory");   // the count of wait_loads: not before the loads ahead, not after those behind
+    load_codes<QT>(q, wv, unit_of(it + 1), 0);
+    load_scales<QT>(wn, wv, unit_of(it + 1));
+    if constexpr (!kSumLate) load_sums(it);
+    asm volatile("" ::: "memory");
+  };
+  auto load_second = [&](int it) {
+    asm volatile("" ::: "memory");
+    load_codes<QT>(q, wv, unit_of(it + 1), 1);
+    asm volatile("" ::: "memory");
+  };
+  load_codes<QT>(q, wv, unit_of(0), -1);
+  load_scales<QT>(w, wv, unit_of(0));
+  issue(unit_of(0), 0, s0);
+  issue(unit_of(0), 1, s1);
+  issue(unit_of(0), 2, s2);
+  issue(unit_of(0), 3, s3);
+  // inverse scales and sums of squares: as in k_gemm_ks
+#pragma unroll
+  for (int tt = 0; tt < TT; ++tt) {
+    const size_t at = (size_t)min(tile0 + tt, ntile - 1) * nu * kSTok;
+    float ss = 0.f;
+    for (int i = tid; i < nu * kSTok; i += kSW * 64) {
+      inv_lds[tt * nu * kSTok + i] = xs.inv[at + i];
+      ss += xs.ssq[at + i];
+    }
+    ss += __shfl_xor(ss, 32, kWave);
+    if (lane < kSTok) psum[tt][wave][lane] = ss;
+  }
+  __syncthreads();   // waits for every load so far, the four stages among them
+  if (tid < TT * kSTok) {
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < kSW; ++i) ss += psum[tid / kSTok][i][tid % kSTok];
+    // the RMSNorm scale of tensor.c:114-131 (read after the loop's barriers)
+    rn[tid] = a.nw ? 1.0f / sqrtf(ss / (float)a.cols + a.eps) : 1.0f;
+  }
+  // x fragments of one block: read from LDS while the block before is used
+  struct Frags {
+    v8h v[TT][4];
+  };
+  Frags fa, fb;
+  auto read = [&](Frags& x, const v4u* buf, int b) {
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        x.v[tt][i] = __builtin_bit_cast(v8h, buf[(kgrp * 8 * SB + (tt * SB + b) * 4 + i) * kWave + lane]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  read(fa, s0, 0);
+  Pipe<QT, TT> pipe;
+  pipe.init(q, w);
+#pragma unroll 1
+  for (int it = 0; it < nit; ++it) {
+    const int u = unit_of(it);
+    // a group without a unit in the last turn: its sums are dropped
+    const bool live = kgrp + it * KG < nu;
+    // stage k of the unit from cur (its first block's x read already), the
+    // next stage in nxt: past the barrier, cur is read by no one any more
+    // (every wave has its last block in registers) and takes the stage four on
+    auto stage = [&](auto kc, v4u* cur, const v4u* nxt) {
+      constexpr int k = decltype(kc)::value;
+      if constexpr (SB == 2) {
+        // the first block's x (read a block ago) is here: said before the next
+        // reads, or the compiler waits for those too
+        __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));
+        read(fb, cur, 1);
+        pipe.template block<k * SB>(q, w, q, wn, fa.v);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // the next stage was requested three stages ago; since then two more
+      // (4 loads each) and the codes loaded at the end of the three stages
+      // before this one
+      constexpr int kEnd1 = NS / 2 - 1, kEnd2 = NS - 1;   // the stages that end with them
+      constexpr auto among = [](int e) { return e == (k + NS - 1) % NS || e == (k + NS - 2) % NS || e == (k + NS - 3) % NS; };
+      wait_loads<8 + (among(kEnd1) ? kN1 : 0) + (among(kEnd2) ? kN2 : 0)>();
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if constexpr (k + 4 < NS)
+        issue(u, k + 4, cur);
+      else
+        issue(unit_of(it + 1), k + 4 - NS, cur);
+      asm volatile("" ::: "memory");
+      if constexpr (SB == 2) {
+        read(fa, nxt, 0);
+        pipe.template block<k * SB + 1>(q, w, q, wn, fb.v);
+      } else if constexpr (k % 2 == 0) {
+        read(fb, nxt, 0);
+        pipe.template block<k>(q, w, q, wn, fa.v);
+      } else {
+        read(fa, nxt, 0);
+        pipe.template block<k>(q, w, q, wn, fb.v);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (k == NS / 2 - 1) load_first(it);
+    };
+    auto turn = [&](auto qc) {   // four stages
+      constexpr int q = 4 * decltype(qc)::value;
+      stage(std::integral_constant<int, q>{}, s0, s1);
+      stage(std::integral_constant<int, q + 1>{}, s1, s2);
+      stage(std::integral_constant<int, q + 2>{}, s2, s3);
+      stage(std::integral_constant<int, q + 3>{}, s3, s0);
+    };
+    turn(std::integral_constant<int, 0>{});
+    if constexpr (NS == 8) turn(std::integral_constant<int, 1>{});
+    if constexpr (kSumLate) load_sums(it);   // (not among the counted: wait_loads then waits for more)
+    load_second(it);
+    pipe.finish(acc, w, sum, inv_lds + u * kSTok + 4 * kg, nu * kSTok, live);
+    w = wn;
+  }
 
-  v4f acc[NMAT][kHRG][kHTiles];
-#pragma unroll
-  for (int mt = 0; mt < NMAT; ++mt)
-#pragma unroll
-    for (int r = 0; r < kHRG; ++r)
-#pragma unroll
-      for (int tt = 0; tt < kHTiles; ++tt) acc[mt][r][tt] = v4f{0.f, 0.f, 0.f, 0.f};
-
-  stage_x(0, 0);
-  load_w(0, wq, we, wsu);
+  // the column groups' sums of each row tile, added in group order
   vm_drain();
   __syncthreads();
-#pragma unroll 1
-  for (int tk = 0; tk < ntk; ++tk) {
-    const int buf = tk & 1;
-    // the next tile in flight (the last iteration reloads its own tile into
-    // the idle buffer: branch-free, read by no one)
-    const int tn = min(tk + 1, ntk - 1);
-    uint32_t nq[NMAT][kHRG][kTB][kQW];
-    uint32_t ne[NMAT][kHRG][kTB];
-    uint32_t nsu[NMAT][kHRG];
-    stage_x(tn, buf ^ 1);
-    load_w(tn, nq, ne, nsu);
+  float* red[TT] = {reinterpret_cast<float*>(s0), reinterpret_cast<float*>(s1)};   // [wave][16][64]
 #pragma unroll
-    for (int b = 0; b < kTB; ++b) {
-      constexpr int NG = PQ<QT>::kGroups ? 2 : 1;   // codes split by 16-weight group
-      v8h wc[NMAT][kHRG][NG];
-      float A[NMAT][kHRG][2], B[NMAT][kHRG][2];
+  for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
-      for (int mt = 0; mt < NMAT; ++mt)
+    for (int j = 0; j < 16; ++j) red[tt][(wave * 16 + j) * kWave + lane] = acc[tt][j];
+  __syncthreads();
 #pragma unroll
-        for (int r = 0; r < kHRG; ++r) {
-          const v8h c = codes_f16<QT>(wq[mt][r][b][0], wq[mt][r][b][kQW - 1]);
+  for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
-          for (int gg = 0; gg < NG; ++gg) wc[mt][r][gg] = NG == 1 ? c : group_part<QT>(c, gg, kq);
-          block_affine<QT>(kMaskAtLoad || tk * kTB + b < nb ? we[mt][r][b] : 0u, wsu[mt][r], A[mt][r], B[mt][r]);
-        }
+    for (int q = 0; q < 2 * RT; ++q) {   // row tile q / 2, register j, lane
+      const int j = wave + kSW * (q & 1), r = q >> 1;
+      const int tok = 8 * (j >> 2) + 4 * kg + (j & 3), t = (tile0 + tt) * kSTok + tok;
+      const int row = row0 + 32 * r + n;
+      if (t >= a.T || row >= a.rows) continue;
+      float v[NMAT];
 #pragma unroll
-      for (int tt = 0; tt < kHTiles; ++tt) {
-        const v8h xh = __builtin_bit_cast(v8h, xs[buf][0][tt * 16 + n][(4 * b + kq) ^ n]);
-        const v8h xl = __builtin_bit_cast(v8h, xs[buf][1][tt * 16 + n][(4 * b + kq) ^ n]);
-        v4f sx[NG];   // sum of x over the block (or group), for the B terms
-        if constexpr (PQ<QT>::kMin) {
+      for (int m = 0; m < NMAT; ++m) {
+        v[m] = 0.f;
 #pragma unroll
-          for (int gg = 0; gg < NG; ++gg) {
-            const v8h one = NG == 1 ? kOnes : group_part<QT>(kOnes, gg, kq);
-            sx[gg] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, one, v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-            sx[gg] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, one, sx[gg], 0, 0, 0);
-          }
-        }
-#pragma unroll
-        for (int mt = 0; mt < NMAT; ++mt)
-#pragma unroll
-          for (int r = 0; r < kHRG; ++r)
-#pragma unroll
-            for (int gg = 0; gg < NG; ++gg) {
-              v4f c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, wc[mt][r][gg], v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-              c = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, wc[mt][r][gg], c, 0, 0, 0);
-              const float ag = A[mt][r][gg];
-#pragma unroll
-              for (int i = 0; i < 4; ++i) acc[mt][r][tt][i] = fmaf(ag, c[i], acc[mt][r][tt][i]);
-              if constexpr (PQ<QT>::kMin) {
-                const float bg = -B[mt][r][gg];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) acc[mt][r][tt][i] = fmaf(bg, sx[gg][i], acc[mt][r][tt][i]);
-              }
-            }
+        for (int g = 0; g < KG; ++g) v[m] += red[tt][((g * RW + m * RT + r) * 16 + j) * kWave + lane];
+        v[m] *= rn[tt * kSTok + tok];
       }
-      __builtin_amdgcn_sched_barrier(0);   // one block's operands live at a time
+      float* yp = a.y + (size_t)t * a.ldy + row;
+      if constexpr (EPI == EPI_SWIGLU)
+        *yp = v[NMAT - 1] * (a.act == 1 ? gelu_tanh(v[0]) : silu(v[0]));   // layer_scheduler.c:529-547
+      else if constexpr (EPI == EPI_ADD)
+        *yp += v[0];
+      else
+        *yp = v[0];
     }
-#pragma unroll
-    for (int mt = 0; mt < NMAT; ++mt)
-#pragma unroll
-      for (int r = 0; r < kHRG; ++r) {
-#pragma unroll
-        for (int b = 0; b < kTB; ++b) {
-#pragma unroll
-          for (int k = 0; k < kQW; ++k) wq[mt][r][b][k] = nq[mt][r][b][k];
-          we[mt][r][b] = ne[mt][r][b];
-        }
-        wsu[mt][r] = nsu[mt][r];
-      }
-    vm_drain();   // this wave's direct LDS loads of the next tile have landed
-    __syncthreads();
-  }
+}
 
-  // epilogue: lane holds row g*16 + n of tokens t0 + 16tt + 4kq + i
-  // per token: 1/s_t, times the RMSNorm scale. The sums of squares come
-  // through a buffer view (empty without a norm weight: reads return 0 and
-  // the scale is 1), so no branch separates the loads and all are in flight
-  // together.
-  const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float*>(a.ssq), (short)0, a.nw ? a.T * 4 : 0, kBufferFlags);
-  float tsc[kHTiles][4];
-#pragma unroll
-  for (int tt = 0; tt < kHTiles; ++tt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int t = min(t0 + tt * 16 + 4 * kq + i, a.T - 1);
-      const float ss = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sr, t * 4, 0, 0));
-      const float rn = 1.0f / sqrtf(ss / (float)a.cols + a.eps);
-      tsc[tt][i] = xinv[t] * (a.nw ? rn : 1.0f);
-    }
-  // the accumulating form reads every old value before it writes any (a
-  // load after a store to y would wait for it: the compiler cannot tell the
-  // addresses apart); clamped addresses, used only where the output exists
-  float yo[kHRG][kHTiles][4];
-  if constexpr (EPI == EPI_ADD) {
-#pragma unroll
-    for (int r = 0; r < kHRG; ++r) {
-      const int row = min((g0 + r) * kRG + n, a.rows - 1);
-#pragma unroll
-      for (int tt = 0; tt < kHTiles; ++tt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          yo[r][tt][i] = a.y[(size_t)min(t0 + tt * 16 + 4 * kq + i, a.T - 1) * a.ldy + row];
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < kHRG; ++r) {
-    const int g = g0 + r;
-    const int row = g * kRG + n;
-    if (g >= ngroups || row >= a.rows) continue;
-#pragma unroll
-    for (int tt = 0; tt < kHTiles; ++tt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int t = t0 + tt * 16 + 4 * kq + i;
-        if (t >= a.T) continue;
-        const float scale = tsc[tt][i];
-        const float x0 = acc[0][r][tt][i] * scale;
-        float v;
-        if constexpr (EPI == EPI_SWIGLU) {
-          const float up = acc[NMAT - 1][r][tt][i] * scale;
-          v = up * (a.act == 1 ? gelu_tanh(x0) : silu(x0));   // layer_scheduler.c:529-547
-        } else {
-          v = x0;
-        }
-        float* yp = a.y + (size_t)t * a.ldy + row;
-        if constexpr (EPI == EPI_ADD)
-          *yp = yo[r][tt][i] + v;
-        else
-          *yp = v;
-      }
-  }
+// launches per epilogue and kernel (k_gemm_ks, k_gemm_rs)
+std::atomic<int64_t> g_gemm_launches[kGemmVariants];
+template <int EPI>
+void count_launch(int kernel) {
+  constexpr int slot = EPI == EPI_STORE ? 0 : EPI == EPI_ADD ? 1 : 2;
+  g_gemm_launches[2 * slot + kernel].fetch_add(1, std::memory_order_relaxed);
 }
 
 template <int QT, int NMAT, int EPI>
-hipError_t launch_gemm_t(const GemmArgs& a, hipStream_t s) {
-  const int ngroups = (a.rows + kRG - 1) / kRG;
-  const dim3 grid((ngroups + kGemmWaves - 1) / kGemmWaves, (a.T + kGemmTok - 1) / kGemmTok);
-  hipLaunchKernelGGL((k_gemm<QT, NMAT, EPI>), grid, dim3(kGemmWaves * 64), 0, s, a);
+hipError_t launch_ks(const GemmArgs& a, int nu, hipStream_t s) {
+  count_launch<EPI>(0);
+  const dim3 grid((a.rows + 31) / 32, (a.T + kSTok - 1) / kSTok);
+  hipLaunchKernelGGL((k_gemm_ks<QT, NMAT, EPI, 1, kSW>), grid, dim3(kSW * 64), 0, s, a, nu);
   return hipGetLastError();
 }
 
-std::atomic<int64_t> g_gemm_h_launches[kGemmVariants];
-
-template <int QT, int NMAT, int EPI, int RG>
-hipError_t launch_gemm_h_t(const GemmArgs& a, int ldxs, hipStream_t s) {
-  constexpr int slot = EPI == EPI_STORE ? 0 : EPI == EPI_ADD ? 1 : 2;
-  g_gemm_h_launches[2 * slot + RG - 1].fetch_add(1, std::memory_order_relaxed);
-  const int ngroups = (a.rows + kRG - 1) / kRG;
-  const dim3 grid((ngroups + kHWaves * RG - 1) / (kHWaves * RG), (a.T + kHTok - 1) / kHTok);
-  hipLaunchKernelGGL((k_gemm_h<QT, NMAT, EPI, RG>), grid, dim3(kHWaves * 64), 0, s, a, ldxs);
+template <int QT, int NMAT, int EPI, int RW>
+hipError_t launch_rs(const GemmArgs& a, int nu, hipStream_t s) {
+  count_launch<EPI>(1);
+  const int rows = 32 * RW / NMAT;
+  const dim3 grid((a.rows + rows - 1) / rows, (a.T + 2 * kSTok - 1) / (2 * kSTok));
+  hipLaunchKernelGGL((k_gemm_rs<QT, NMAT, EPI, RW>), grid, dim3(kSW * 64), 0, s, a, nu);
   return hipGetLastError();
-}
-
-template <int QT>
-hipError_t launch_gemm_q(int epi, const GemmArgs& a, hipStream_t s) {
-  switch (epi) {
-    case EPI_STORE: return launch_gemm_t<QT, 1, EPI_STORE>(a, s);
-    case EPI_ADD: return launch_gemm_t<QT, 1, EPI_ADD>(a, s);
-    case EPI_SWIGLU: return launch_gemm_t<QT, 2, EPI_SWIGLU>(a, s);
-    default: return hipErrorInvalidValue;
-  }
-}
-
-// Two matrices (gate/up) take one row group of each per wave; one matrix two
-// row groups per wave, or one when that leaves fewer than two workgroups per
-// compute unit.
-template <int QT>
-hipError_t launch_gemm_h(int epi, const GemmArgs& a, int ldxs, int n_cu, hipStream_t s) {
-  const int ngroups = (a.rows + kRG - 1) / kRG;
-  const long wg2 = (long)((ngroups + 2 * kHWaves - 1) / (2 * kHWaves)) * ((a.T + kHTok - 1) / kHTok);
-  const bool one = wg2 < 2L * n_cu;
-  switch (epi) {
-    case EPI_STORE:
-      return one ? launch_gemm_h_t<QT, 1, EPI_STORE, 1>(a, ldxs, s) : launch_gemm_h_t<QT, 1, EPI_STORE, 2>(a, ldxs, s);
-    case EPI_ADD:
-      return one ? launch_gemm_h_t<QT, 1, EPI_ADD, 1>(a, ldxs, s) : launch_gemm_h_t<QT, 1, EPI_ADD, 2>(a, ldxs, s);
-    case EPI_SWIGLU: return launch_gemm_h_t<QT, 2, EPI_SWIGLU, 1>(a, ldxs, s);
-    default: return hipErrorInvalidValue;
-  }
 }
 
 int device_cus() {
@@ -710,11 +955,54 @@ int device_cus() {
   return n;
 }
 
+// The workgroup shape: 1 for k_gemm_ks, else k_gemm_rs's RW. Every shape runs
+// one workgroup per compute unit at a time, so a launch takes its rounds of
+// workgroups times what one round takes: at 4096 columns 10 us (two matrices
+// 18: half the waves for each), 24 us (RW 2) and 38 us (RW 4), and in the
+// same ratio at others. The least of the three was the fastest measured at
+// every token count from 8 to 512 of 4096, 11008 and 1024 rows but for ties
+// (4096 rows, 77 / 128 / 256 / 512 tokens: 25.1, 27.1, 48.8, 89.3 us with 1;
+// 26.3, 27.3, 32.7, 58.3 with 2; 36.8, 37.5, 40.9, 49.7 with 4).
+int pick_shape(int rows, int T, int nmat, int nu, int n_cu) {
+  auto rounds = [&](int r, int t) {
+    const long wg = (long)((rows + r - 1) / r) * ((T + t - 1) / t);
+    return (wg + n_cu - 1) / n_cu;
+  };
+  const long c1 = rounds(32, 32) * (nmat == 2 ? 18 : 10);
+  const long c2 = rounds(64 / nmat, 64) * 24, c4 = rounds(128 / nmat, 64) * 38;
+  if (nu > kRsUnits || (c1 <= c2 && c1 <= c4)) return 1;
+  return c2 <= c4 ? 2 : 4;
+}
+
+template <int QT, int NMAT, int EPI>
+hipError_t launch_shape(const GemmArgs& a, int nu, hipStream_t s) {
+  switch (pick_shape(a.rows, a.T, NMAT, nu, device_cus())) {
+    case 1: return launch_ks<QT, NMAT, EPI>(a, nu, s);
+    case 2: return launch_rs<QT, NMAT, EPI, 2>(a, nu, s);
+    default:
+      // Q4_1 and Q5_1 (a scale and a minimum of 16 bits per block) would spill with RW 4
+      return launch_rs<QT, NMAT, EPI, QT == kQ4_1 || QT == kQ5_1 ? 2 : 4>(a, nu, s);
+  }
+}
+
+template <int QT>
+hipError_t launch_type(int epi, const GemmArgs& a, hipStream_t s) {
+  const int nb = a.cols / 32, nu = (nb + kSUnit - 1) / kSUnit;
+  const KsView v = ks_view(a.xs, (a.T + kSTok - 1) / kSTok, nu);
+  hipLaunchKernelGGL(k_split_ks<sum_steps<QT>()>, dim3((a.T + 7) / 8, nu), dim3(64), 0, s, a.x, a.ldx, a.nw, a.T, nb, v);
+  if (hipError_t e = hipGetLastError()) return e;
+  switch (epi) {
+    case EPI_STORE: return launch_shape<QT, 1, EPI_STORE>(a, nu, s);
+    case EPI_ADD: return launch_shape<QT, 1, EPI_ADD>(a, nu, s);
+    default: return launch_shape<QT, 2, EPI_SWIGLU>(a, nu, s);
+  }
+}
+
 }  // namespace
 
-const int64_t* gemm_h_launch_counts() {
+const int64_t* gemm_launch_counts() {
   static int64_t snap[kGemmVariants];
-  for (int i = 0; i < kGemmVariants; ++i) snap[i] = g_gemm_h_launches[i].load(std::memory_order_relaxed);
+  for (int i = 0; i < kGemmVariants; ++i) snap[i] = g_gemm_launches[i].load(std::memory_order_relaxed);
   return snap;
 }
 
@@ -725,43 +1013,24 @@ hipError_t launch_sumsq(const float* x, int cols, int T, float* ssq, hipStream_t
 }
 
 hipError_t launch_gemm(int epi, const GemmArgs& a, hipStream_t s) {
-  if (a.T <= 0 || a.rows <= 0 || a.cols <= 0 || a.cols % 32 || a.ldy < a.rows || a.ldx < a.cols || a.ldx % 4 ||
-      (a.nw && !a.ssq))
+  if (a.T <= 0 || a.rows <= 0 || a.cols <= 0 || a.cols % 32 || a.ldy < a.rows || a.ldx < a.cols || a.ldx % 4 || !a.xs)
     return hipErrorInvalidValue;
   if (epi != EPI_STORE && epi != EPI_ADD && epi != EPI_SWIGLU) return hipErrorInvalidValue;
   const int t = dev_type(a.type);
-  if (a.xs && product_format(t)) {
-    if (is_kq(t) && a.cols % 256) return hipErrorInvalidValue;   // whole super-blocks
-    const int ldxs = (a.cols + 127) / 128 * 128;
-    uint16_t* xl = a.xs + (size_t)a.T * ldxs;
-    float* xinv = reinterpret_cast<float*>(a.xs + 2 * (size_t)a.T * ldxs);
-    float* ssq = a.nw ? a.ssq : nullptr;
-    if (code_bytes_of(t) == 16)   // nibble layouts: Q4_0's slot order
-      hipLaunchKernelGGL(k_split_x<2>, dim3(a.T), dim3(256), 0, s, a.x, a.ldx, a.nw, a.cols, ssq, a.xs, xl, xinv, ldxs);
-    else
-      hipLaunchKernelGGL(k_split_x<8>, dim3(a.T), dim3(256), 0, s, a.x, a.ldx, a.nw, a.cols, ssq, a.xs, xl, xinv, ldxs);
-    if (hipError_t e = hipGetLastError()) return e;
-    const int n_cu = device_cus();
-    switch (t) {
-      case 2: return launch_gemm_h<2>(epi, a, ldxs, n_cu, s);
-      case 8: return launch_gemm_h<8>(epi, a, ldxs, n_cu, s);
-      case kQ4_1: return launch_gemm_h<kQ4_1>(epi, a, ldxs, n_cu, s);
-      case kQ5_1: return launch_gemm_h<kQ5_1>(epi, a, ldxs, n_cu, s);
-      case kQ8_1: return launch_gemm_h<kQ8_1>(epi, a, ldxs, n_cu, s);
-      case kQ2K: return launch_gemm_h<kQ2K>(epi, a, ldxs, n_cu, s);
-      case kQ3K: return launch_gemm_h<kQ3K>(epi, a, ldxs, n_cu, s);
-      case kQ4K: return launch_gemm_h<kQ4K>(epi, a, ldxs, n_cu, s);
-      case kQ5K: return launch_gemm_h<kQ5K>(epi, a, ldxs, n_cu, s);
-      default: return launch_gemm_h<kQ6K>(epi, a, ldxs, n_cu, s);
-    }
+  if (is_kq(t) && a.cols % 256) return hipErrorInvalidValue;   // whole super-blocks
+  switch (t) {
+    case 2: return launch_type<2>(epi, a, s);
+    case 8: return launch_type<8>(epi, a, s);
+    case kQ4_1: return launch_type<kQ4_1>(epi, a, s);
+    case kQ5_1: return launch_type<kQ5_1>(epi, a, s);
+    case kQ8_1: return launch_type<kQ8_1>(epi, a, s);
+    case kQ2K: return launch_type<kQ2K>(epi, a, s);
+    case kQ3K: return launch_type<kQ3K>(epi, a, s);
+    case kQ4K: return launch_type<kQ4K>(epi, a, s);
+    case kQ5K: return launch_type<kQ5K>(epi, a, s);
+    case kQ6K: return launch_type<kQ6K>(epi, a, s);
+    default: return hipErrorInvalidValue;
   }
-  if (a.nw) {
-    hipLaunchKernelGGL(k_sumsq, dim3(a.T), dim3(256), 0, s, a.x, a.ldx, a.cols, a.ssq);
-    if (hipError_t e = hipGetLastError()) return e;
-  }
-  if (t == 2) return launch_gemm_q<2>(epi, a, s);
-  if (t == 8) return launch_gemm_q<8>(epi, a, s);
-  return hipErrorInvalidValue;
 }
 
 }  // namespace ssk

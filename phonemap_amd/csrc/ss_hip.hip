@@ -106,10 +106,9 @@ struct ss_hip_ctx {
   float* att_o = nullptr;
   float* att_ml = nullptr;
   uint32_t* att_cnt = nullptr;
-  float* g_ssq = nullptr;      // prompt products: sums of squares of x
   uint16_t* g_xs = nullptr;    // prompt products: x split into fp16 parts
 
-  size_t att_o_floats = 0, att_ml_floats = 0, att_cnt_bytes = 0, g_ssq_bytes = 0, g_xs_bytes = 0;
+  size_t att_o_floats = 0, att_ml_floats = 0, att_cnt_bytes = 0, g_xs_bytes = 0;
   float* smp = nullptr;        // sampling: probabilities [n]
   size_t smp_bytes = 0;
   uint64_t* smp_io = nullptr;  // sampling: [0] index, [1] advanced state
@@ -308,7 +307,7 @@ void ss_hip_free(ss_hip_ctx_t* c) {
   if (c->stream) hipStreamSynchronize(c->stream);
   for (auto& kv : c->registry) hipFree(kv.second);
   void* bufs[] = {c->staging, c->am_part, c->rope_row, c->att_o, c->att_ml, c->att_cnt,
-                  c->g_ssq, c->g_xs, c->plug_x, c->plug_y, c->smp, c->smp_io};
+                  c->g_xs, c->plug_x, c->plug_y, c->smp, c->smp_io};
   for (void* b : bufs)
     if (b) hipFree(b);
   for (int i = 0; i < ss_hip_ctx::kBatchSlots; ++i) {
@@ -408,8 +407,7 @@ int32_t ss_hip_gemm(ss_hip_ctx_t* c, float* y, const void* w, const float* x, co
       !quant_type_ok(type) || !product_type(type))
     return fail(kErrParams, "gemm: bad argument (rows %d cols %d tokens %d type %d)", rows, cols, n_tokens, type);
   if (set_device(c)) return kErrBackend;
-  int32_t rc = ensure(c, (void**)&c->g_ssq, &c->g_ssq_bytes, sizeof(float) * n_tokens, false);
-  if (!rc) rc = ensure(c, (void**)&c->g_xs, &c->g_xs_bytes, 2 * ssk::gemm_split_elems(n_tokens, cols), false);
+  int32_t rc = ensure(c, (void**)&c->g_xs, &c->g_xs_bytes, 2 * ssk::gemm_split_elems(n_tokens, cols), false);
   if (rc) return rc;
   hipStream_t s = pick(c, stream);
   ssk::GemmArgs a;
@@ -417,7 +415,6 @@ int32_t ss_hip_gemm(ss_hip_ctx_t* c, float* y, const void* w, const float* x, co
   a.w = view(w, type, rows, cols);
   a.x = x;
   a.nw = nw;
-  a.ssq = c->g_ssq;
   a.xs = c->g_xs;
   a.eps = eps;
   a.y = y;
@@ -1482,7 +1479,6 @@ ssk::GemmArgs gemm_args(ss_hip_model* m, const void* w, int type, int rows, int 
   a.w = view(w, type, rows, cols);
   a.x = x;
   a.y = y;
-  a.ssq = m->pf_ssq;
   a.xs = m->pf_xs;
   a.ldx = cols;
   a.ldy = rows;
@@ -1958,7 +1954,7 @@ int32_t ss_hip_model_launch(const ss_hip_model_t* m) { return m ? m->launch : -1
 
 int32_t ss_hip_gemm_launch_counts(int64_t* out, int32_t n) {
   if (!out || n < 0) return fail(kErrParams, "gemm_launch_counts: null output");
-  const int64_t* c = ssk::gemm_h_launch_counts();
+  const int64_t* c = ssk::gemm_launch_counts();
   for (int i = 0; i < n && i < ssk::kGemmVariants; ++i) out[i] = c[i];
   return 0;
 }

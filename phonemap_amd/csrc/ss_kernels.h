@@ -101,18 +101,19 @@ struct GemmArgs {
   PackedMat w, w2;           // w2: up projection for EPI_SWIGLU
   const float* x;            // [T][ldx] token-major
   const float* nw;           // RMSNorm weight [cols]: x is normalised (tensor.c:114-131), or nullptr
-  float* ssq;                // [T] scratch for the sums of squares of x (required with nw)
   float eps;
   float* y;                  // [T][ldy] (EPI_ADD: accumulated into)
   uint16_t* xs;              // scratch of gemm_split_elems(T, cols) 16-bit words: x split into
-                             // two fp16 parts and a scale per token (fp16 products), or
-                             // nullptr (fp32 products)
+                             // two fp16 parts, with their scales and sums
   int ldx, ldy, rows, cols, T, type;
   int act;                   // EPI_SWIGLU: 0 SiLU, 1 GELU (Gemma's GeGLU)
 };
 // 16-bit words of GemmArgs::xs for T tokens of cols columns
+// (whole tiles of 32 tokens and units of 256 columns: x in two parts, and per
+// token and unit two fp32 values and up to 16 sums in two parts)
 inline size_t gemm_split_elems(int T, int cols) {
-  return 2 * (size_t)T * (size_t)((cols + 127) / 128 * 128) + 2 * (size_t)T;
+  const size_t t = (size_t)((T + 31) / 32 * 32), nu = (size_t)((cols + 255) / 256);
+  return t * nu * (2 * 256 + 4 + 32);
 }
 
 struct AttnArgs {
@@ -178,16 +179,15 @@ hipError_t launch_attention_merge(int head_dim, int group, const AttnArgs& a, hi
 hipError_t launch_attention_rows(int head_dim, int group, const AttnArgs& a, hipStream_t s);
 // ssq[t] = sum of x[t][c]^2 (x [T][cols])
 hipError_t launch_sumsq(const float* x, int cols, int T, float* ssq, hipStream_t s);
-// Y = W X over T tokens with EPI_STORE, EPI_ADD or EPI_SWIGLU; with nw set,
-// first the sums of squares of X into a.ssq. With a.xs: X is split into fp16
-// parts first and the products run in fp16 (exact codes, fp32 accumulation
-// and scales); otherwise in fp32.
+// Y = W X over T tokens with EPI_STORE, EPI_ADD or EPI_SWIGLU: X is split into
+// fp16 parts in a.xs, and the products run on them (exact codes, fp32
+// accumulation and scales).
 hipError_t launch_gemm(int epi, const GemmArgs& a, hipStream_t s);
-// Launches of the fp16-MFMA products since the library was loaded, per
-// epilogue (EPI_STORE, EPI_ADD, EPI_SWIGLU) and row groups per wave (1, 2):
-// index 2 * epilogue_slot + RG - 1.
+// Launches of the prompt products since the library was loaded, per epilogue
+// (EPI_STORE, EPI_ADD, EPI_SWIGLU) and kernel (0: one row tile per workgroup,
+// 1: several): index 2 * epilogue_slot + kernel.
 constexpr int kGemmVariants = 6;
-const int64_t* gemm_h_launch_counts();
+const int64_t* gemm_launch_counts();
 bool attention_supported(int head_dim, int group);
 // positions one attention workgroup covers in one round of loads
 int attn_round_positions(int head_dim, int group);

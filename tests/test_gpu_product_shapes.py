@@ -1,0 +1,72 @@
+"""The prompt products at the edges of their kernels' tiles: token counts and
+row counts that take each workgroup shape (one row tile, two, four), with
+ragged token tiles (32 tokens), row tiles (32 rows, of row groups of 16) and
+units (256 columns), fewer units than column groups, and rows so long that the
+inverse scales are read from memory. Every token against the exact product
+(fp64 over the dequantised weights).
+
+Bound per output: |y - e| <= 1e-6 sum_j |w_j x_j|. x in two fp16 parts is within
+2^-22 = 2.4e-7 of x, and the fp32 sums add up to 2^-24 per term of a chain of
+at most 256 (a few 1e-7 in all as roundings go either way).
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from tests.util import Q2_K, Q3_K, Q4_0, Q4_1, Q4_K, Q5_1, Q5_K, Q6_K, Q8_0, Q8_1, dequant_np, make_blocks
+
+pytestmark = pytest.mark.gpu
+TYPES32 = [Q4_0, Q8_0, Q4_1, Q5_1, Q8_1]
+TYPES_K = [Q2_K, Q3_K, Q4_K, Q5_K, Q6_K]
+
+
+def _counts(hip):
+    out = (C.c_int64 * 6)()
+    assert hip.L.ss_hip_gemm_launch_counts(out, 6) == 0
+    return np.array(out[:])
+
+
+def _check(hip, qtype, rows, cols, T, kernel):
+    print("product shape", qtype, rows, cols, T, flush=True)
+    rng = np.random.default_rng(rows + 3 * cols + 7 * T + qtype)
+    w = make_blocks(qtype, rows, cols, rng)
+    x = rng.standard_normal((T, cols)).astype(np.float32)
+    x[:, : cols // 2] *= 1e-3 * 10.0 ** rng.integers(0, 7, (T, 1))   # units of different magnitude
+    nw = (1.0 + 0.1 * rng.standard_normal(cols)).astype(np.float32)
+    y0 = rng.standard_normal((T, rows)).astype(np.float32)
+    W, X, NW, Y = hip.packed(w, qtype, rows, cols), hip.upload(x), hip.upload(nw), hip.upload(y0)
+    wd = dequant_np(w, rows, cols, qtype)
+    xn = x.astype(np.float64) * nw
+    k = 1.0 / np.sqrt(np.mean(x.astype(np.float64) ** 2, 1, keepdims=True) + 1e-5)
+    before = _counts(hip)
+    assert hip.L.ss_hip_gemm(hip.ctx, Y.ptr, W.ptr, X.ptr, NW.ptr, C.c_float(1e-5), 1, rows, cols, T, qtype, None) == 0, hip.err()
+    got = Y.read(np.float32, T * rows).reshape(T, rows)
+    exact, mag = xn @ wd.T * k + y0, np.abs(xn) @ np.abs(wd).T * k + np.abs(y0)
+    assert np.max(np.abs(got - exact) / mag) <= 1e-6
+    assert hip.L.ss_hip_gemm(hip.ctx, Y.ptr, W.ptr, X.ptr, None, C.c_float(1e-5), 0, rows, cols, T, qtype, None) == 0, hip.err()
+    got = Y.read(np.float32, T * rows).reshape(T, rows)
+    xd = x.astype(np.float64)
+    assert np.max(np.abs(got - xd @ wd.T) / (np.abs(xd) @ np.abs(wd).T)) <= 1e-6
+    ran = _counts(hip) - before
+    assert ran[2 + kernel] == 1 and ran[kernel] == 1 and ran.sum() == 2, ran
+    for b in (W, X, NW, Y):
+        b.free()
+
+
+@pytest.mark.parametrize("qtype", TYPES32)
+@pytest.mark.parametrize("rows,cols,T,kernel", [
+    (17, 32, 2, 0), (40, 2080, 33, 0), (16, 33056, 3, 0),     # one row tile; 130 units
+    (4100, 288, 130, 1),                                       # two row tiles, 2 units for 4 column groups
+    (4100, 1056, 200, 1),                                      # four row tiles, 5 units for 2 column groups
+])
+def test_product_shapes_block32(hip, qtype, rows, cols, T, kernel):
+    _check(hip, qtype, rows, cols, T, kernel)
+
+
+@pytest.mark.parametrize("qtype", TYPES_K)
+@pytest.mark.parametrize("rows,cols,T,kernel", [
+    (17, 256, 2, 0), (40, 2304, 33, 0), (4100, 512, 130, 1), (4100, 1280, 200, 1),
+])
+def test_product_shapes_kquants(hip, qtype, rows, cols, T, kernel):
+    _check(hip, qtype, rows, cols, T, kernel)
