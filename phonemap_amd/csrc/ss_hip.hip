@@ -109,9 +109,9 @@ struct ss_hip_ctx {
   uint16_t* g_xs = nullptr;    // prompt products: x split into fp16 parts
 
   size_t att_o_floats = 0, att_ml_floats = 0, att_cnt_bytes = 0, g_xs_bytes = 0;
-  float* smp = nullptr;        // sampling: probabilities [n]
+  float* smp = nullptr;        // sampling: scratch
   size_t smp_bytes = 0;
-  uint64_t* smp_io = nullptr;  // sampling: [0] index, [1] advanced state
+  uint64_t* smp_io = nullptr;  // sampling: [0] index, [1] advanced state (pinned host memory the kernel writes)
 
   // device address of this device's copy of `scratch` (ss_hip_attention_noalloc)
   void* scratch = nullptr;
@@ -307,9 +307,10 @@ void ss_hip_free(ss_hip_ctx_t* c) {
   if (c->stream) hipStreamSynchronize(c->stream);
   for (auto& kv : c->registry) hipFree(kv.second);
   void* bufs[] = {c->staging, c->am_part, c->rope_row, c->att_o, c->att_ml, c->att_cnt,
-                  c->g_xs, c->plug_x, c->plug_y, c->smp, c->smp_io};
+                  c->g_xs, c->plug_x, c->plug_y, c->smp};
   for (void* b : bufs)
     if (b) hipFree(b);
+  if (c->smp_io) hipHostFree(c->smp_io);
   for (int i = 0; i < ss_hip_ctx::kBatchSlots; ++i) {
     if (c->batch_x[i]) hipFree(c->batch_x[i]);
     if (c->batch_y[i]) hipFree(c->batch_y[i]);
@@ -642,12 +643,12 @@ int32_t ss_hip_sample_logits(ss_hip_ctx_t* c, const float* logits, int32_t n, fl
                              int32_t top_k, uint64_t* rng_state, int32_t* out_host) {
   if (!c || !logits || n <= 0 || !rng_state || !out_host) return fail(kErrParams, "sample: bad argument");
   if (int32_t rc = set_device(c)) return rc;
-  if (!c->smp_io) HIP_TRY(hipMalloc((void**)&c->smp_io, 2 * sizeof(uint64_t)));
+  if (!c->smp_io) HIP_TRY(hipHostMalloc((void**)&c->smp_io, 2 * sizeof(uint64_t), hipHostMallocDefault));
   hipStream_t s = c->stream;
   if (!(temperature > 0.0f)) {   // tensor.c:366-368
     HIP_TRY(ssk::launch_argmax(reinterpret_cast<int*>(c->smp_io), logits, n, c->am_part, s));
   } else {
-    if (int32_t rc = ensure(c, (void**)&c->smp, &c->smp_bytes, sizeof(float) * (size_t)n, false)) return rc;
+    if (int32_t rc = ensure(c, (void**)&c->smp, &c->smp_bytes, ssk::sample_scratch_bytes(n), false)) return rc;
     ssk::SampleArgs a;
     memset(&a, 0, sizeof(a));
     a.logits = logits;
@@ -661,11 +662,9 @@ int32_t ss_hip_sample_logits(ss_hip_ctx_t* c, const float* logits, int32_t n, fl
     a.rng_out = c->smp_io + 1;
     HIP_TRY(ssk::launch_sample(a, s));
   }
-  uint64_t io[2];
-  HIP_TRY(hipMemcpyAsync(io, c->smp_io, sizeof(io), hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
-  *out_host = (int32_t)(uint32_t)(io[0] & 0xffffffffu);
-  if (temperature > 0.0f) *rng_state = io[1];
+  *out_host = (int32_t)(uint32_t)(c->smp_io[0] & 0xffffffffu);
+  if (temperature > 0.0f) *rng_state = c->smp_io[1];
   return 0;
 }
 

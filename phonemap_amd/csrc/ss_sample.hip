@@ -21,6 +21,13 @@
 // one sequential walk inside the chunk that holds r. The index differs from
 // the reference's only when r lies within the reference's fp32 rounding of a
 // cumulative boundary.
+//
+// One workgroup reads a 128256-entry row some 15 times, 25 us each: 373 us.
+// Rows of more than kOneGroup entries go over many workgroups instead, in a
+// few short launches (launch_sample), with the same fixed-point sums and the
+// same comparisons, so the same index. A softmax term e = exp(x - max) is
+// computed before its probability p = e * inv is known; p does not decrease
+// with e, so the k-th largest p is that of the k-th largest e.
 
 #include <float.h>
 #include <math.h>
@@ -33,6 +40,12 @@ namespace {
 
 constexpr int kThreads = 1024;
 constexpr int kWaves = kThreads / kWave;
+constexpr int kOneGroup = 1024;                // rows up to this: k_sample alone
+constexpr int kTile = 1024;                    // entries per workgroup of the others
+constexpr int kTileThreads = 256;
+constexpr int kBins = 2048;                    // by key >> 19 (sign 0, exponent, 4 bits of the mantissa): e, p <= 1
+constexpr int kCand = 2048;                    // candidates the top-k path keeps in LDS
+constexpr int kMaxTopK = 1024;                 // top_k it takes
 constexpr double kFix = 4503599627370496.0;   // 2^52: probabilities (each <= 1, sums <= ~1)
 constexpr double kFixE = 1099511627776.0;     // 2^40: softmax terms (each <= 1, up to 2^18 of them)
 
@@ -40,6 +53,11 @@ constexpr double kFixE = 1099511627776.0;     // 2^40: softmax terms (each <= 1,
 // are clamped to 2 (a probability never exceeds 1 + rounding)
 __device__ __forceinline__ uint64_t fix(float p) {
   return p > 0.f ? (uint64_t)((double)fminf(p, 2.0f) * kFix) : 0ull;
+}
+// the sum at which top-p cuts off (at least one step: the largest value always stays)
+__device__ __forceinline__ uint64_t top_p_target(float top_p) {
+  const uint64_t t = (uint64_t)((double)top_p * kFix);
+  return t > 0 ? t : 1ull;
 }
 // sort key of tensor.c:384-385 (NaN ranks as 0)
 __device__ __forceinline__ uint32_t key(float p) { return __float_as_uint(p == p ? p : 0.f); }
@@ -157,8 +175,29 @@ __device__ float top_p_cutoff(const float* p, int V, uint64_t target, Shared& sh
   return __uint_as_float(prefix);
 }
 
-__global__ void __launch_bounds__(kThreads) k_sample(const SampleArgs a) {
-  __shared__ Shared sh;
+__device__ uint64_t advance(uint64_t st) {   // xorshift64, tensor.c:341-343
+  st ^= st << 13;
+  st ^= st >> 7;
+  st ^= st << 17;
+  return st;
+}
+// r as fixed point: (float)(st >> 11) / (float)2^53
+__device__ uint64_t draw_fix(uint64_t st) {
+  const float r = (float)(st >> 11) / (float)(1ull << 53);
+  return (uint64_t)((double)r * kFix);
+}
+__device__ void put_result(const SampleArgs& a, int idx, uint64_t st) {
+  *a.out = idx;
+  *a.rng_out = st;
+  if (a.tokens) {
+    const int pos = *a.dpos;
+    a.tokens[pos + 1] = idx;
+    *a.dpos = pos + 1;
+  }
+}
+
+// the whole of ss_sample in one workgroup
+__device__ void sample_one_group(const SampleArgs& a, Shared& sh) {
   const int V = a.V, tid = threadIdx.x;
   float* p = a.probs;
 
@@ -195,7 +234,7 @@ __global__ void __launch_bounds__(kThreads) k_sample(const SampleArgs a) {
 
   // 3. top-p (tensor.c:398-417)
   if (a.top_p > 0.f && a.top_p < 1.0f) {
-    const uint64_t target = (uint64_t)((double)a.top_p * kFix);
+    const uint64_t target = top_p_target(a.top_p);
     const float cutoff = top_p_cutoff(p, V, target, sh);
     for (int i = tid; i < V; i += kThreads)
       if (p[i] < cutoff) p[i] = 0.f;
@@ -220,12 +259,7 @@ __global__ void __launch_bounds__(kThreads) k_sample(const SampleArgs a) {
 
   // 5. draw (tensor.c:341-343, 431-442): first i with r < cdf_i, i before any
   // NaN (a NaN term makes every later comparison false)
-  uint64_t st = a.rng;
-  st ^= st << 13;
-  st ^= st >> 7;
-  st ^= st << 17;
-  const float r = (float)(st >> 11) / (float)(1ull << 53);
-  const uint64_t rf = (uint64_t)((double)r * kFix);
+  const uint64_t st = advance(a.rng), rf = draw_fix(st);
   const int C = (V + kThreads - 1) / kThreads;   // contiguous chunk per thread
   const int i0 = min(tid * C, V), i1 = min(i0 + C, V);
   uint64_t cs = 0;
@@ -256,23 +290,503 @@ __global__ void __launch_bounds__(kThreads) k_sample(const SampleArgs a) {
   }
   found = block_min_i(found, sh);
   if (tid != 0) return;
-  const int idx = found < first_nan && found < V ? found : V - 1;
-  *a.out = idx;
-  *a.rng_out = st;
-  if (a.tokens) {
-    const int pos = *a.dpos;
-    a.tokens[pos + 1] = idx;
-    *a.dpos = pos + 1;
+  put_result(a, found < first_nan && found < V ? found : V - 1, st);
+}
+
+__global__ void __launch_bounds__(kThreads) k_sample(const SampleArgs a) {
+  __shared__ Shared sh;
+  sample_one_group(a, sh);
+}
+
+// ---- many workgroups ---------------------------------------------------------
+// Scratch of a row (SampleArgs::probs): p or e per entry, the boundary list or
+// the candidates, the histogram, and the per-workgroup values.
+struct Work {
+  float* e;            // [V] softmax terms
+  float* list;         // [V] values of the boundary bin (top-p), or [2 * kCand] candidates (index, e)
+  uint64_t* hist;      // [kBins] counts of e (top-k) or sums of p (top-p) per bin
+  uint64_t* esum;      // [nb] fixed-point sums of e
+  uint64_t* psum;      // [nb] of the kept p, then of their renormalised values
+  float* mx;           // [nb]
+  uint32_t* nan;       // [nb] nonzero: a term is NaN
+  uint32_t* count;     // [1] list entries
+  float* cut;          // [2] cutoff, renormalisation factor
+};
+__host__ __device__ inline size_t up256(size_t n) { return (n + 255) & ~(size_t)255; }
+__host__ __device__ inline Work work_of(float* base, int V, size_t* bytes) {
+  const int nb = (V + kTile - 1) / kTile;
+  uint8_t* p = reinterpret_cast<uint8_t*>(base);
+  size_t o = 0;
+  auto take = [&](size_t n) {
+    uint8_t* q = p + o;
+    o += up256(n);
+    return q;
+  };
+  Work w;
+  w.e = reinterpret_cast<float*>(take(sizeof(float) * (size_t)V));
+  w.list = reinterpret_cast<float*>(take(sizeof(float) * (size_t)(V > 2 * kCand ? V : 2 * kCand)));
+  w.hist = reinterpret_cast<uint64_t*>(take(sizeof(uint64_t) * kBins));
+  w.esum = reinterpret_cast<uint64_t*>(take(sizeof(uint64_t) * nb));
+  w.psum = reinterpret_cast<uint64_t*>(take(sizeof(uint64_t) * nb));
+  w.mx = reinterpret_cast<float*>(take(sizeof(float) * nb));
+  w.nan = reinterpret_cast<uint32_t*>(take(sizeof(uint32_t) * nb));
+  w.count = reinterpret_cast<uint32_t*>(take(sizeof(uint32_t)));
+  w.cut = reinterpret_cast<float*>(take(2 * sizeof(float)));
+  if (bytes) *bytes = o;
+  return w;
+}
+
+// sum, maximum or or over a workgroup of W waves (red: W slots), in every thread
+template <int W>
+__device__ __forceinline__ uint64_t group_sum(uint64_t v, uint64_t* red) {
+  v = wave_sum_u64(v);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  uint64_t t = 0;
+#pragma unroll
+  for (int i = 0; i < W; ++i) t += red[i];
+  return t;
+}
+// sum of n values (the per-workgroup sums of an earlier launch)
+template <int W>
+__device__ __forceinline__ uint64_t total(const uint64_t* p, int n, uint64_t* red) {
+  uint64_t v = 0;
+  for (int i = threadIdx.x; i < n; i += W * kWave) v += p[i];
+  return group_sum<W>(v, red);
+}
+template <int W>
+__device__ __forceinline__ bool any_nan(const Work& w, int nb, uint64_t* red) {
+  uint64_t v = 0;
+  for (int i = threadIdx.x; i < nb; i += W * kWave) v += w.nan[i];
+  return group_sum<W>(v, red) != 0;
+}
+__device__ __forceinline__ float inv_of(uint64_t esum) { return 1.0f / (float)((double)esum / kFixE); }
+
+constexpr int kTW = kTileThreads / kWave, kTK = kTile / kTileThreads;
+
+// 1. the row's maximum of logit / temperature; the histogram starts at zero
+__global__ void __launch_bounds__(kTileThreads) k_smp_max(const SampleArgs a) {
+  __shared__ float red[kTW];
+  const Work w = work_of(a.probs, a.V, nullptr);
+  const int i0 = blockIdx.x * kTile + threadIdx.x;
+  float mx = -FLT_MAX;
+#pragma unroll
+  for (int k = 0; k < kTK; ++k) {
+    const float l = a.logits[min(i0 + k * kTileThreads, a.V - 1)];
+    mx = fmaxf(mx, l != l ? -FLT_MAX : l / a.temperature);
+  }
+  mx = wave_max(mx);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+  for (int i = blockIdx.x * kTileThreads + threadIdx.x; i < kBins; i += gridDim.x * kTileThreads) w.hist[i] = 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *w.count = 0;
+  __syncthreads();
+  if (threadIdx.x == 0) w.mx[blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+}
+
+// 2. the softmax terms, their sum, and (COUNT) how many fall into each bin
+template <bool COUNT>
+__global__ void __launch_bounds__(kTileThreads) k_smp_exp(const SampleArgs a) {
+  __shared__ float redf[kTW];
+  __shared__ uint64_t red[kTW];
+  __shared__ uint32_t hist[COUNT ? kBins : 1];
+  const Work w = work_of(a.probs, a.V, nullptr);
+  const int tid = threadIdx.x;
+  float l[kTK];
+#pragma unroll
+  for (int k = 0; k < kTK; ++k) l[k] = a.logits[min((int)blockIdx.x * kTile + k * kTileThreads + tid, a.V - 1)];
+  float mx = -FLT_MAX;
+  for (int i = tid; i < (int)gridDim.x; i += kTileThreads) mx = fmaxf(mx, w.mx[i]);
+  mx = wave_max(mx);
+  if ((tid & 63) == 0) redf[tid >> 6] = mx;
+  if constexpr (COUNT)
+    for (int i = tid; i < kBins; i += kTileThreads) hist[i] = 0;
+  __syncthreads();
+  mx = fmaxf(fmaxf(redf[0], redf[1]), fmaxf(redf[2], redf[3]));
+  uint64_t s = 0;
+  bool nan = false;
+#pragma unroll
+  for (int k = 0; k < kTK; ++k) {
+    const int i = blockIdx.x * kTile + k * kTileThreads + tid;
+    if (i >= a.V) break;
+    const float x = l[k] != l[k] ? -FLT_MAX : l[k] / a.temperature;
+    const float e = expf(x - mx);
+    w.e[i] = e;
+    s += e > 0.f ? (uint64_t)((double)e * kFixE) : 0ull;   // e <= 1
+    nan = nan || e != e;
+    if constexpr (COUNT)
+      if (e > 0.f) atomicAdd(&hist[__float_as_uint(e) >> 19], 1u);
+  }
+  s = group_sum<kTW>(s, red);
+  const bool nans = group_sum<kTW>(nan ? 1 : 0, red) != 0;
+  if (tid == 0) {
+    w.esum[blockIdx.x] = s;
+    w.nan[blockIdx.x] = nans;
+  }
+  if constexpr (COUNT)
+    for (int i = tid; i < kBins; i += kTileThreads)
+      if (hist[i]) atomicAdd(reinterpret_cast<unsigned long long*>(&w.hist[i]), (unsigned long long)hist[i]);
+}
+
+// The largest bin at which the sum of hist over it and the bins above reaches
+// target, or -1; above: the sum over the bins above it (over all when -1).
+// 256 threads, 8 bins each.
+__device__ int find_bin(const uint64_t* hist, uint64_t target, uint64_t* red, int* sel, uint64_t* sel_above, uint64_t& above) {
+  static_assert(kBins == 8 * kTileThreads, "eight bins per thread");
+  const int tid = threadIdx.x, top = kBins - 1 - 8 * tid;   // thread 0 takes the highest bins
+  uint64_t h[8], s = 0;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    h[k] = hist[top - k];
+    s += h[k];
+  }
+  uint64_t incl = s;   // inclusive scan over the workgroup
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const uint64_t o = __shfl_up(incl, off, kWave);
+    if ((tid & 63) >= off) incl += o;
+  }
+  if (tid == 0) *sel = -1;
+  if ((tid & 63) == 63) red[tid >> 6] = incl;
+  __syncthreads();
+  uint64_t base = incl - s;
+  for (int i = 0; i < tid >> 6; ++i) base += red[i];
+  if (tid == kTileThreads - 1) *sel_above = base + s;   // everything; replaced below when a bin reaches the target
+  __syncthreads();
+  if (base < target && base + s >= target) {
+    int k = 0;
+    while (base + h[k] < target) base += h[k++];
+    *sel = top - k;
+    *sel_above = base;
+  }
+  __syncthreads();
+  above = *sel_above;
+  return *sel;
+}
+
+// ---- 0 < top_k <= kMaxTopK: the candidates ---------------------------------
+// 3. every term that may belong to the k largest: those of the bin the k-th
+// falls into and above (and a few rounding steps below: their p may equal
+// the k-th's). Terms of 0 are left out: their probability is 0 in any case.
+__global__ void __launch_bounds__(kTileThreads) k_smp_gather(const SampleArgs a) {
+  __shared__ uint64_t red[kTW], sa;
+  __shared__ int sel;
+  const Work w = work_of(a.probs, a.V, nullptr);
+  float e[kTK];
+#pragma unroll
+  for (int k = 0; k < kTK; ++k) e[k] = w.e[min((int)blockIdx.x * kTile + k * kTileThreads + (int)threadIdx.x, a.V - 1)];
+  uint64_t above;
+  const int bin = find_bin(w.hist, (uint64_t)a.top_k, red, &sel, &sa, above);
+  const uint32_t low = bin <= 0 ? 1u : ((uint32_t)bin << 19) - 8u;
+#pragma unroll
+  for (int k = 0; k < kTK; ++k) {
+    const int i = blockIdx.x * kTile + k * kTileThreads + threadIdx.x;
+    if (i < a.V && e[k] > 0.f && __float_as_uint(e[k]) >= low) {
+      const uint32_t at = atomicAdd(w.count, 1u);
+      if (at < (uint32_t)kCand) {
+        w.list[2 * at] = __int_as_float(i);
+        w.list[2 * at + 1] = e[k];
+      }
+    }
   }
 }
 
+// 4. the k-th largest, the top-p cutoff, the renormalisation and the draw over
+// the candidates, whose order in the list does not matter: each is compared
+// with all others by 8 threads. More than kCand candidates (ties, a flat
+// row): the whole row in this workgroup.
+__global__ void __launch_bounds__(kThreads) k_smp_topk(const SampleArgs a) {
+  __shared__ Shared sh;
+  __shared__ int idx[kCand];
+  __shared__ float p[kCand];
+  __shared__ uint32_t th, cut;
+  __shared__ int found;
+  const Work w = work_of(a.probs, a.V, nullptr);
+  const int tid = threadIdx.x, nb = (a.V + kTile - 1) / kTile;
+  const uint32_t n = *w.count;
+  if (n > (uint32_t)kCand) {
+    sample_one_group(a, sh);
+    return;
+  }
+  const uint64_t st = advance(a.rng), rf = draw_fix(st);
+  const bool nan = any_nan<kWaves>(w, nb, sh.u);
+  const float inv = inv_of(total<kWaves>(w.esum, nb, sh.u));
+  for (int i = tid; i < (int)n; i += kThreads) {
+    idx[i] = __float_as_int(w.list[2 * i]);
+    p[i] = w.list[2 * i + 1] * inv;
+  }
+  if (tid == 0) {
+    th = 0;
+    cut = 0;
+    found = 0x7fffffff;
+  }
+  __syncthreads();
+  const int part = tid & 7;
+  // f(i) for every candidate, by the 8 threads of an aligned group
+  auto each = [&](auto f) {
+    for (int i = tid >> 3; i < (int)n; i += kThreads / 8) f(i);
+  };
+  auto sum8u = [](uint64_t v) {
+    v += __shfl_xor(v, 1, kWave);
+    v += __shfl_xor(v, 2, kWave);
+    return v + __shfl_xor(v, 4, kWave);
+  };
+  each([&](int i) {   // the k-th largest p (p >= 0: its bits order like its value)
+    uint64_t c = 0;   // greater ones, and (high half) equal ones
+    for (int j = part; j < (int)n; j += 8) c += p[j] > p[i] ? 1ull : p[j] == p[i] ? 1ull << 32 : 0ull;
+    c = sum8u(c);
+    const uint32_t gt = (uint32_t)c, eq = (uint32_t)(c >> 32);
+    if (part == 0 && gt < (uint32_t)a.top_k && gt + eq >= (uint32_t)a.top_k) th = __float_as_uint(p[i]);
+  });
+  __syncthreads();
+  const float tk = __uint_as_float(th);
+  if (a.top_p > 0.f && a.top_p < 1.0f) {
+    const uint64_t target = top_p_target(a.top_p);
+    each([&](int i) {   // the largest p whose sum with those above it reaches the target
+      uint64_t s = 0;
+      for (int j = part; j < (int)n; j += 8) s += p[j] >= tk && p[j] >= p[i] ? fix(p[j]) : 0ull;
+      s = sum8u(s);
+      if (part == 0 && p[i] >= tk && s >= target) atomicMax(&cut, __float_as_uint(p[i]));
+    });
+    __syncthreads();
+  }
+  const float low = fmaxf(tk, __uint_as_float(cut));
+  uint64_t s = 0;
+  for (int i = tid; i < (int)n; i += kThreads) s += p[i] >= low ? fix(p[i]) : 0ull;
+  s = group_sum<kWaves>(s, sh.u);
+  const float pinv = s > 0 ? 1.0f / (float)((double)s / kFix) : 1.0f;
+  each([&](int i) {   // the first index whose cumulative probability exceeds r
+    uint64_t c = 0;
+    for (int j = part; j < (int)n; j += 8) c += p[j] >= low && idx[j] <= idx[i] ? fix(p[j] * pinv) : 0ull;
+    c = sum8u(c);
+    if (part == 0 && p[i] >= low && rf < c) atomicMin(&found, idx[i]);
+  });
+  __syncthreads();
+  if (tid == 0) put_result(a, !nan && found < a.V ? found : a.V - 1, st);
+}
+
+// ---- no top-k: the whole distribution ----------------------------------------
+// 3. the probabilities and (HIST) their sums per bin, or their whole sum
+template <bool HIST>
+__global__ void __launch_bounds__(kTileThreads) k_smp_prob(const SampleArgs a) {
+  __shared__ uint64_t red[kTW];
+  __shared__ uint64_t hist[HIST ? kBins : 1];
+  const Work w = work_of(a.probs, a.V, nullptr);
+  const int tid = threadIdx.x;
+  if constexpr (HIST)
+    for (int i = tid; i < kBins; i += kTileThreads) hist[i] = 0;
+  const float inv = inv_of(total<kTW>(w.esum, gridDim.x, red));
+  uint64_t s = 0;
+#pragma unroll
+  for (int k = 0; k < kTK; ++k) {
+    const int i = blockIdx.x * kTile + k * kTileThreads + tid;
+    if (i >= a.V) break;
+    const float p = w.e[i] * inv;
+    w.e[i] = p;
+    s += fix(p);
+    if constexpr (HIST)
+      if (p > 0.f)
+        atomicAdd(reinterpret_cast<unsigned long long*>(&hist[__float_as_uint(p) >> 19]), (unsigned long long)fix(p));
+  }
+  s = group_sum<kTW>(s, red);
+  if (tid == 0) w.psum[blockIdx.x] = s;
+  if constexpr (HIST)
+    for (int i = tid; i < kBins; i += kTileThreads)
+      if (hist[i]) atomicAdd(reinterpret_cast<unsigned long long*>(&w.hist[i]), (unsigned long long)hist[i]);
+}
+
+// 4. the values of the bin the top-p cutoff lies in
+__global__ void __launch_bounds__(kTileThreads) k_smp_boundary(const SampleArgs a) {
+  __shared__ uint64_t red[kTW], sa;
+  __shared__ int sel;
+  const Work w = work_of(a.probs, a.V, nullptr);
+  float p[kTK];
+#pragma unroll
+  for (int k = 0; k < kTK; ++k) p[k] = w.e[min((int)blockIdx.x * kTile + k * kTileThreads + (int)threadIdx.x, a.V - 1)];
+  uint64_t above;
+  const int bin = find_bin(w.hist, top_p_target(a.top_p), red, &sel, &sa, above);
+#pragma unroll
+  for (int k = 0; k < kTK; ++k) {
+    const int i = blockIdx.x * kTile + k * kTileThreads + threadIdx.x;
+    if (i < a.V && p[k] > 0.f && (int)(__float_as_uint(p[k]) >> 19) == bin) w.list[atomicAdd(w.count, 1u)] = p[k];
+  }
+}
+
+// 5. the cutoff within that bin, and the renormalisation (CUT false: of everything)
+template <bool CUT>
+__global__ void __launch_bounds__(kTileThreads) k_smp_cutoff(const SampleArgs a) {
+  __shared__ uint64_t red[kTW], sa, bins[256];
+  __shared__ int sel;
+  const Work w = work_of(a.probs, a.V, nullptr);
+  const int tid = threadIdx.x, nb = (a.V + kTile - 1) / kTile;
+  uint64_t s = 0;
+  uint32_t prefix = 0;
+  if constexpr (CUT) {
+    const uint64_t target = top_p_target(a.top_p);
+    uint64_t above;
+    const int bin = find_bin(w.hist, target, red, &sel, &sa, above);
+    s = above;   // everything when no bin reaches the target: the cutoff is 0
+    if (bin >= 0) {
+      // the remaining 19 bits of the key, 7, 6 and 6 at a time
+      const int n = (int)*w.count;
+      prefix = (uint32_t)bin << 19;
+      uint32_t mask = ~0u << 19;
+      for (int shift = 12; shift >= 0; shift -= 6) {
+        const uint32_t width = shift == 12 ? 128 : 64;
+        __syncthreads();
+        bins[tid] = 0;
+        __syncthreads();
+        for (int i = tid; i < n; i += kTileThreads) {
+          const uint32_t u = __float_as_uint(w.list[i]);
+          if ((u & mask) == prefix)
+            atomicAdd(reinterpret_cast<unsigned long long*>(&bins[(u >> shift) & (width - 1)]),
+                      (unsigned long long)fix(__uint_as_float(u)));
+        }
+        __syncthreads();
+        if (tid == 0) {
+          int b = (int)width - 1;
+          uint64_t acc = above;
+          for (; b > 0; --b) {   // some bin reaches the target: their sum does
+            if (acc + bins[b] >= target) break;
+            acc += bins[b];
+          }
+          sel = b;
+          sa = acc;
+        }
+        __syncthreads();
+        prefix |= (uint32_t)sel << shift;
+        mask |= (width - 1) << shift;
+        above = sa;
+      }
+      // all keys of the last bin are equal: its sum is the cutoff's own
+      s = above + bins[sel];
+    }
+  } else {
+    s = total<kTW>(w.psum, nb, red);
+  }
+  if (tid == 0) {
+    w.cut[0] = __uint_as_float(prefix);
+    w.cut[1] = s > 0 ? 1.0f / (float)((double)s / kFix) : 1.0f;
+  }
+}
+
+// 6. the renormalised sum of each tile
+__global__ void __launch_bounds__(kTileThreads) k_smp_sums(const SampleArgs a) {
+  __shared__ uint64_t red[kTW];
+  const Work w = work_of(a.probs, a.V, nullptr);
+  const float low = w.cut[0], pinv = w.cut[1];
+  uint64_t s = 0;
+#pragma unroll
+  for (int k = 0; k < kTK; ++k) {
+    const int i = blockIdx.x * kTile + k * kTileThreads + threadIdx.x;
+    const float p = w.e[min(i, a.V - 1)];
+    s += i < a.V && p >= low ? fix(p * pinv) : 0ull;
+  }
+  s = group_sum<kTW>(s, red);
+  if (threadIdx.x == 0) w.psum[blockIdx.x] = s;
+}
+
+// 7. the tile the draw falls into, and the entry in it
+__global__ void __launch_bounds__(kThreads) k_smp_draw(const SampleArgs a) {
+  __shared__ uint64_t red[kWaves], base;
+  __shared__ int tile, found;
+  const Work w = work_of(a.probs, a.V, nullptr);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nb = (a.V + kTile - 1) / kTile;
+  const uint64_t st = advance(a.rng), rf = draw_fix(st);
+  const bool nan = any_nan<kWaves>(w, nb, red);
+  const float low = w.cut[0], pinv = w.cut[1];
+  // exclusive sum of v over the threads before this one; total in all
+  auto scan = [&](uint64_t v, uint64_t& total_out) {
+    uint64_t incl = v;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const uint64_t o = __shfl_up(incl, off, kWave);
+      if (lane >= off) incl += o;
+    }
+    __syncthreads();
+    if (lane == 63) red[wave] = incl;
+    __syncthreads();
+    uint64_t before = incl - v;
+    total_out = 0;
+    for (int i = 0; i < kWaves; ++i) {
+      if (i < wave) before += red[i];
+      total_out += red[i];
+    }
+    return before;
+  };
+  if (tid == 0) {
+    tile = -1;
+    found = 0x7fffffff;
+  }
+  uint64_t done = 0;
+  for (int b0 = 0; b0 < nb; b0 += kThreads) {
+    const uint64_t v = b0 + tid < nb ? w.psum[b0 + tid] : 0ull;
+    uint64_t all;
+    const uint64_t before = done + scan(v, all);
+    if (v > 0 && rf >= before && rf < before + v) {
+      tile = b0 + tid;
+      base = before;
+    }
+    done += all;
+    __syncthreads();
+  }
+  const int t = tile;
+  if (t >= 0) {   // uniform
+    const int i = t * kTile + tid;
+    const float p = w.e[min(i, a.V - 1)];
+    const uint64_t v = i < a.V && p >= low ? fix(p * pinv) : 0ull;
+    uint64_t all;
+    const uint64_t c = base + scan(v, all) + v;
+    if (i < a.V && rf < c) atomicMin(&found, i);
+  }
+  __syncthreads();
+  if (tid == 0) put_result(a, !nan && found < a.V ? found : a.V - 1, st);
+}
+static_assert(kTile == kThreads, "k_smp_draw: one entry per thread");
+
 }  // namespace
+
+size_t sample_scratch_bytes(int V) {
+  if (V <= kOneGroup) return sizeof(float) * (size_t)V;
+  size_t bytes = 0;
+  work_of(nullptr, V, &bytes);
+  return bytes;
+}
 
 hipError_t launch_sample(const SampleArgs& a, hipStream_t s) {
   if (a.V <= 0 || !a.logits || !a.probs || !a.out || !a.rng_out || !(a.temperature > 0.f) ||
       (a.tokens && !a.dpos))
     return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_sample, dim3(1), dim3(kThreads), 0, s, a);
+  // Rows of up to kOneGroup entries (one per thread) and a top_k past the
+  // candidates' space stay with one workgroup. The whole call, one workgroup
+  // and many: 128256 entries with top_k 40 and top_p 0.95 407 and 33 us, with
+  // top_p alone 341 and 56 us, with neither 200 and 36 us; 4097 entries 98 and
+  // 30, 73 and 46, 41 and 35 us. What remains is four (six) launches and the
+  // wait for them.
+  const bool topk = a.top_k > 0 && a.top_k < a.V, topp = a.top_p > 0.f && a.top_p < 1.0f;
+  if (a.V <= kOneGroup || (topk && a.top_k > kMaxTopK)) {
+    hipLaunchKernelGGL(k_sample, dim3(1), dim3(kThreads), 0, s, a);
+    return hipGetLastError();
+  }
+  const dim3 nb((a.V + kTile - 1) / kTile), th(kTileThreads);
+  hipLaunchKernelGGL(k_smp_max, nb, th, 0, s, a);
+  if (topk) {
+    hipLaunchKernelGGL(k_smp_exp<true>, nb, th, 0, s, a);
+    hipLaunchKernelGGL(k_smp_gather, nb, th, 0, s, a);
+    hipLaunchKernelGGL(k_smp_topk, dim3(1), dim3(kThreads), 0, s, a);
+    return hipGetLastError();
+  }
+  hipLaunchKernelGGL(k_smp_exp<false>, nb, th, 0, s, a);
+  if (topp) {
+    hipLaunchKernelGGL(k_smp_prob<true>, nb, th, 0, s, a);
+    hipLaunchKernelGGL(k_smp_boundary, nb, th, 0, s, a);
+    hipLaunchKernelGGL(k_smp_cutoff<true>, dim3(1), th, 0, s, a);
+  } else {
+    hipLaunchKernelGGL(k_smp_prob<false>, nb, th, 0, s, a);
+    hipLaunchKernelGGL(k_smp_cutoff<false>, dim3(1), th, 0, s, a);
+  }
+  hipLaunchKernelGGL(k_smp_sums, nb, th, 0, s, a);
+  hipLaunchKernelGGL(k_smp_draw, dim3(1), dim3(kThreads), 0, s, a);
   return hipGetLastError();
 }
 

@@ -1,0 +1,35 @@
+"""Device sampling at the sizes where its launches change: rows of one
+workgroup (up to 1024 entries) and of many, at the edges of their 1024-entry
+tiles; the top-k candidates just within and past their space (ties); no top-k
+with a cutoff that keeps one value, most of the row, or everything; infinite
+logits. Bars as in test_gpu_sample.py.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from tests.test_gpu_sample import _check_index, _device_sample
+
+pytestmark = pytest.mark.gpu
+PARAMS = [(0.8, 0.95, 40), (1.0, 0.9, 0), (1.2, 1.0, 0), (0.9, 1.0, 1024), (0.9, 0.7, 1025), (1.0, 1e-6, 0), (1.0, 0.9999, 0)]
+
+
+@pytest.mark.parametrize("V", [1024, 1025, 4096, 5119, 5120, 5121, 70001])
+@pytest.mark.parametrize("kind", ["normal", "flat", "steps", "inf"])
+def test_sample_sizes(hip, V, kind):
+    print("sample", V, kind, flush=True)
+    rng = np.random.default_rng(V)
+    for T, top_p, top_k in PARAMS:
+        x = (2.5 * rng.standard_normal(V)).astype(np.float32)
+        if kind == "flat":
+            x[:] = 0.25
+        elif kind == "steps":   # 2048 ties at the top: the candidates' space, and one more
+            x[rng.permutation(V)[: 2048 + (top_k == 40)]] = 11.0
+        elif kind == "inf":
+            x[rng.integers(0, V, V // 2)] = -np.inf
+        for _ in range(2):
+            seed = int(rng.integers(1, 2 ** 63))
+            want, want_st, p, r = oracle.sample(x, T, top_p, top_k, seed)
+            got, got_st = _device_sample(hip, x, T, top_p, top_k, seed)
+            assert got_st == want_st and 0 <= got < V
+            _check_index(got, want, p, r)
