@@ -3,32 +3,49 @@
 // The reference evaluates a prompt token by token, each token attending to
 // positions 0..its own over the fp16 cache (layer_scheduler.c:415-468, called
 // per token from ss_scheduler_prefill, :681-803). Here the tokens of a prompt
-// chunk attend together, one workgroup per 64 query rows of one KV head
-// (row r: token z0 + r / G, head r % G), on v_mfma_f32_16x16x32_f16.
+// chunk attend together, 32 query rows of one KV head to a tile (row r: token
+// r / G, head r % G), on v_mfma_f32_32x32x16_f16.
 //
-// Operand layout of v_mfma_f32_16x16x32_f16 (checked on the device by the
-// prompt products): lane l supplies A[l%16][8(l/16) + i] and B[8(l/16) + i][l%16],
-// i = 0..7, and receives D[4(l/16) + i][l%16], i = 0..3.
+// Operand layout of v_mfma_f32_32x32x16_f16 (checked on the device by the
+// prompt products): lane l supplies A[l%32][8(l/32) + i] and B[8(l/32) + i][l%32],
+// i = 0..7, and receives D[8(j/4) + 4(l/32) + j%4][l%32], j = 0..15.
 //
-// Each wave owns 16 query rows and computes transposed tiles: S^T = K Q^T
-// (A = 16 keys of K, B = Q^T), so lane (n, kq) receives the scores of query
-// row n, and O^T = V^T P^T (A = V^T, B = P^T), whose B operand is exactly
-// the scores' D registers once the keys of S^T tile t are ordered
-// key(t, r) = 8(r / 4) + 4t + r % 4: lane (n, kq) then holds keys 8kq + j,
-// j = 0..7, of query row n, the B layout. Softmax statistics of a row live in
-// the 4 lanes n, n+16, n+32, n+48 (two shuffles per reduction).
+// Each wave owns 32 query rows and, per 32-key block, computes transposed
+// tiles: S^T = K Q^T (A = the keys' K rows, B = Q^T), so lane (n, h) = (l%32,
+// l/32) receives scores of query row n, and O^T = V^T P^T (A = V^T, B = P^T),
+// whose B operand is exactly the scores' D registers once row 16c + 8b + 4h + i
+// of the S^T tile is key 16c + 8h + 4b + i: elements 8c..8c+7 of lane (n, h)
+// are then keys 16c + 8h + 0..7 of query row n, the B layout. A row's softmax
+// statistics live in lanes n and n + 32 (one v_permlane32_swap per reduction).
 //
 // Precision: K and V are fp16 in the cache (exact MFMA operands). q is
 // scaled per row by a power of two (its largest magnitude to [2^13, 2^14))
-// and split into two fp16 parts, hi + lo = q to 2^-22; P (in [0, 1], times
-// 2^12) is split the same way; each product is two MFMAs accumulating in
-// fp32. The softmax is the online form (running max and sum per row) in fp32.
+// and split into two fp16 parts, hi + lo = q to 2^-22; P (times 2^12) is split
+// the same way; each product is two MFMAs accumulating in fp32. The softmax is
+// the online form (running maximum and sum per row) in fp32, in base 2: the
+// scores' scale carries log2(e), rounded once like 1/sqrt(hd) itself. The
+// running maximum may lag the true one by up to 3 (P <= 2^3: 2^15 after the
+// scale, inside fp16's range), so most blocks skip rescaling O.
 //
-// Staging, per 64-key block, double buffered: K rows go to LDS by direct
-// global-to-LDS loads (16-byte chunk c of key k at slot c ^ kswz(k) of its
-// row); V is loaded into registers and written to LDS transposed (V^T rows
-// of 64 keys, 8-key chunk c of row d at slot c ^ (d % 8)). Both swizzles
-// spread one MFMA operand read over all banks.
+// Bound and split. At 32 rows per wave one LDS operand read feeds two MFMAs of
+// 32 cycles, so a block is 1024 matrix cycles per wave at head_dim 128 against
+// 512 of LDS and about as many of softmax as of products. A workgroup is RT row
+// tiles x KG key groups, the groups taking every KG-th block and merged through
+// LDS at the end, so a short prompt over a long prefix walks KG times fewer
+// steps. With 16 rows per wave, four waves walking all keys and V transposed
+// in registers, 512 tokens over 1536 (32 heads on 8, head_dim 128) took 94 us
+// and 77 over 1000 50 us; now 41 and 18, the first 1.6 times what a large
+// fp16 product takes for the same operations. At head_dim 256 the O and q of
+// 32 rows would leave one wave per SIMD pair, so DS = 2 waves share a row tile:
+// each scores half of the head dimension and the halves are added through LDS,
+// and each holds half of O (64 tokens over 700, 16 heads on 8: 31 us; one
+// wave 44; before 60).
+//
+// Staging, per block and key group, double buffered, by direct global-to-LDS
+// loads: K rows in tile-row order (16-byte chunk c of row r at slot c ^ kswz),
+// V rows as they are (chunk c at slot c ^ vswz(key)), read transposed by
+// ds_read_b64_tr_b16 (lane i of 16 addresses key i/4, dims 4(i%4)..+3, and
+// receives dim i of the four keys). Both swizzles spread a read over all banks.
 
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -39,34 +56,33 @@
 namespace ssk {
 namespace {
 
-typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef short v4s __attribute__((ext_vector_type(4)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
+typedef __attribute__((address_space(3))) v4s* lds_v4s_t;
 typedef __attribute__((address_space(1))) void* gbl_ptr_t;
 
-constexpr int kFWaves = 4;               // waves per workgroup, 16 query rows each
-constexpr int kFRows = 16 * kFWaves;     // query rows per workgroup
-// keys per block: 64, or 32 at head_dim 256 (the K and V^T tiles stay 64 KB)
-__host__ __device__ constexpr int flash_keys(int hd) { return hd == 256 ? 32 : 64; }
-constexpr float kPScale = 4096.0f;       // P is split as P * 2^12
+constexpr int kBlk = 32;            // keys per block, query rows per tile
+constexpr int kCompute = 256;       // compute units
+constexpr float kLog2e = 1.44269504088896340736f;
+constexpr float kPExp = 12.0f;      // P is held times 2^12
+constexpr float kLag = 3.0f;        // the running maximum's lag (base 2)
 
-// K row slot swizzle: the 16 keys of one S^T operand read (8(r/4) + 4t + r%4)
-// take 8 distinct values, two keys each.
-__device__ __forceinline__ int kswz(int key) { return (key & 3) | ((key >> 1) & 4); }
-
-__device__ __forceinline__ float max4(float v) {   // over lanes n, n+16, n+32, n+48
-  v = fmaxf(v, __shfl_xor(v, 16, kWave));
-  return fmaxf(v, __shfl_xor(v, 32, kWave));
+// the value of the lane with the same query row (lane ^ 32) joined to this one's
+__device__ __forceinline__ float max_pair(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
-__device__ __forceinline__ float sum4(float v) {
-  v += __shfl_xor(v, 16, kWave);
-  return v + __shfl_xor(v, 32, kWave);
+__device__ __forceinline__ float sum_pair(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 __device__ __forceinline__ int wave_max_int(int v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, kWave));
-  return v;
+  return __builtin_amdgcn_readfirstlane(v);
 }
 
 // hi + lo = v (to 2^-22 of |v| for normal values) as two fp16 vectors
@@ -79,63 +95,114 @@ __device__ __forceinline__ void split8(const float (&v)[8], v8h& hi, v8h& lo) {
   }
 }
 
-template <int HD, int G>
-__global__ void __launch_bounds__(kFWaves * 64) k_flash_rows(const AttnArgs a) {
-  constexpr int CH = HD / 8;             // 16-byte chunks per K row
-  constexpr int NC = HD / 32;            // 32-wide slices of the head dimension
-  constexpr int NDT = HD / 16;           // 16-dim tiles of O^T
-  constexpr int kTQ = kFRows / G;        // tokens per workgroup
-  constexpr int kFKeys = flash_keys(HD);  // keys per block
-  constexpr int NS = kFKeys / 32;         // 32-key halves per block
-  constexpr int kVC = kFKeys / 8;         // 8-key chunks per V^T row
-  constexpr int kKG = kFKeys / 4;         // 4-key groups per block
-  constexpr int kVItems = kKG * CH;       // (4-key group, chunk) staging items of V
+// tile row -> key of the block: bits 2 and 3 change places (its own inverse)
+__host__ __device__ constexpr int tile_key(int r) { return (r & 19) | ((r & 4) << 1) | ((r & 8) >> 1); }
+// slot swizzles (16-byte chunks of a row of CH): 16 neighbouring tile rows take
+// 16 places of 256 bytes; the 4 keys of a transposed read take 4 groups of 4
+template <int CH> __device__ __forceinline__ int kswz(int row) { return CH == 8 ? (row >> 1) & 7 : row & 15; }
+template <int CH> __device__ __forceinline__ int vswz(int key) { return CH == 8 ? 2 * (key & 2) : 4 * (key & 3); }
+
+template <int HD, int G, int RT, int KG, int DS>
+__global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs a) {
+  constexpr int CH = HD / 8;             // 16-byte chunks per row
+  constexpr int NC = HD / 16 / DS;       // a wave's 16-wide slices of the head dimension
+  constexpr int NDT = HD / 32 / DS;      // and 32-dim tiles of O^T
+  constexpr int NT = RT * KG * DS * 64;
+  constexpr int kGrp = kBlk * CH;        // chunks of one key group's block
+  constexpr int kLoads = kGrp / (64 * RT * DS);   // direct loads per wave, K and V each
   static_assert(HD == 64 || HD == 128 || HD == 256, "head_dim 64, 128 or 256");
-  static_assert(kFKeys * CH % (kFWaves * 64) == 0, "K staging rounds");
-  static_assert(kVItems <= kFWaves * 64, "V staging items");
+  static_assert(kBlk % G == 0 && RT <= 2 && KG % 2 == 0 && kGrp % (64 * RT * DS) == 0, "shape");
 
   // two buffers of each, as separate arrays: the loop names them at compile
   // time, so the compiler can tell the buffer being read from the one the
   // direct global-to-LDS loads of the next block fill, and does not wait for
   // those loads before the current block's reads
-  __shared__ v4u ks0[kFKeys * CH], ks1[kFKeys * CH];   // K rows, swizzled slots
-  __shared__ v4u vt0[HD * kVC], vt1[HD * kVC];         // V^T rows of the block's keys, swizzled slots
+  __shared__ v4u ks0[KG * kGrp], ks1[KG * kGrp];
+  __shared__ v4u vs0[KG * kGrp], vs1[KG * kGrp];
+  __shared__ float xs[DS > 1 ? RT * KG * DS : 1][DS > 1 ? 16 * 64 : 1];   // the waves' shares of S^T
+  __shared__ float gm[KG][RT * 32], gl[KG][RT * 32];   // each group's maximum and sum of a row
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int n = lane & 15, kq = lane >> 4;
-  const int kvh = blockIdx.y;
-  const int z0 = (gridDim.x - 1 - blockIdx.x) * kTQ;   // the longest prefixes first
-  auto pos_of = [&](int z) { return a.dpos ? a.dpos[z] : a.pos0 + z; };
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ds = wave % DS, rt = wave / DS % RT, g = wave / (DS * RT);
+  const int n = lane & 31, h = lane >> 5;
+  // neighbouring workgroups take the KV heads in turn, so the workgroups of
+  // one head meet in one XCD's L2; the longest prefixes come first
+  const int kvh = blockIdx.x % a.n_kv_heads;
+  const int row0 = (gridDim.x / a.n_kv_heads - 1 - blockIdx.x / a.n_kv_heads) * (RT * 32);
 
-  // this lane's query row: token z, head h of the KV head's group
-  const int r = 16 * wave + n;
-  const int z = z0 + r / G, h = r % G;
-  const int zc = min(z, a.n_tok - 1);
-  const int lim = z < a.n_tok ? pos_of(zc) : -1;   // last position the row sees
-  // positions 0..ctx-1 serve every token of the workgroup; wlim bounds this wave's rows
-  const int ctx = wave_max_int(pos_of(min(z0 + lane % kTQ, a.n_tok - 1))) + 1;
-  const int wlim = __builtin_amdgcn_readfirstlane(wave_max_int(lim));
-  const int nblk = (ctx + kFKeys - 1) / kFKeys;
+  // this lane's query row: token z, head hq of the KV head's group
+  const int row = row0 + 32 * rt + n;
+  const int z = row / G, hq = row % G;
+  const int lim = a.pos0 + z;   // last position the row sees (rows past the last token are not stored)
+  // positions 0..ctx-1 serve every token of the workgroup; wmin..wmax are this wave's rows' limits
+  const int ctx = a.pos0 + min((row0 + RT * 32 - 1) / G, a.n_tok - 1) + 1;
+  const int wmin = a.pos0 + (row0 + 32 * rt) / G, wmax = min(wmin + 32 / G, ctx) - 1;
+  const int nstep = (ctx + KG * kBlk - 1) / (KG * kBlk);
 
-  // q as the B operand of S^T: lane (n, kq) holds q[32c + 8kq + i] of row n
+  float qv[NC][8];
+  float amax = 0.f;
+  {
+    const float* qp = a.q + (size_t)min(z, a.n_tok - 1) * a.tok_q + ((size_t)kvh * G + hq) * HD + 8 * h;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const float4 x0 = *reinterpret_cast<const float4*>(qp + 16 * (ds * NC + c));
+      const float4 x1 = *reinterpret_cast<const float4*>(qp + 16 * (ds * NC + c) + 4);
+      qv[c][0] = x0.x, qv[c][1] = x0.y, qv[c][2] = x0.z, qv[c][3] = x0.w;
+      qv[c][4] = x1.x, qv[c][5] = x1.y, qv[c][6] = x1.z, qv[c][7] = x1.w;
+    }
+  }
+  const size_t head_base = (size_t)kvh * a.max_seq * HD;
+  const uint16_t* kc = static_cast<const uint16_t*>(a.kc) + head_base;
+  const uint16_t* vc = static_cast<const uint16_t*>(a.vc) + head_base;
+
+  // this group's block of a step -> LDS, each of its RT * DS waves a share
+  // (positions past ctx - 1 reload ctx - 1: finite, masked)
+  auto stage = [&](int step, v4u* kd, v4u* vd) {
+    const int kb = (step * KG + g) * kBlk;
+    if (kb >= ctx) return;
+    int ln = lane;
+    if (HD == 256) asm volatile("" : "+v"(ln));   // places computed again each step, not kept in registers
+#pragma unroll
+    for (int k = 0; k < kLoads; ++k) {
+      const int base = ((rt * DS + ds) * kLoads + k) * 64;
+      const int r = (base + ln) / CH, slot = (base + ln) % CH;
+      const int pk = min(kb + tile_key(r), ctx - 1);
+      __builtin_amdgcn_global_load_lds((gbl_ptr_t)(kc + (size_t)pk * HD + 8 * (slot ^ kswz<CH>(r))),
+                                       (lds_ptr_t)&kd[g * kGrp + base], 16, 0, 0);
+    }
+#pragma unroll
+    for (int k = 0; k < kLoads; ++k) {
+      const int base = ((rt * DS + ds) * kLoads + k) * 64;
+      const int r = (base + ln) / CH, slot = (base + ln) % CH;
+      const int pv = min(kb + r, ctx - 1);
+      __builtin_amdgcn_global_load_lds((gbl_ptr_t)(vc + (size_t)pv * HD + 8 * (slot ^ vswz<CH>(r))),
+                                       (lds_ptr_t)&vd[g * kGrp + base], 16, 0, 0);
+    }
+  };
+  // the staged loads have landed and the other buffer's reads are done, for
+  // this wave, and for the others where waves share the staging
+  auto turn = [&] {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    if (RT * DS > 1) __syncthreads();
+  };
+
+  stage(0, ks0, vs0);
+
+  // q as the B operand of S^T: lane (n, h) holds q[16c + 8h + i] of row n
   v8h qh[NC], ql[NC];
   float qscale;
   {
-    const float* qp = a.q + (size_t)zc * a.tok_q + ((size_t)kvh * G + h) * HD + 8 * kq;
-    float qv[NC][8];
-    float amax = 0.f;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const float4 x0 = *reinterpret_cast<const float4*>(qp + 32 * c);
-      const float4 x1 = *reinterpret_cast<const float4*>(qp + 32 * c + 4);
-      const float t[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+    for (int c = 0; c < NC; ++c)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        qv[c][i] = t[i];
-        amax = fmaxf(amax, fabsf(t[i]));
-      }
+      for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(qv[c][i]));
+    amax = max_pair(amax);
+    if (DS > 1) {   // the row's other half counts too
+      xs[wave][lane] = amax;
+      __syncthreads();
+      amax = fmaxf(amax, xs[wave ^ 1][lane]);
     }
-    amax = max4(amax);
     int e = 0;
     frexpf(amax, &e);   // amax = f * 2^e, f in [0.5, 1); 0 gives e = 0
     const int shift = min(max(14 - e, -100), 100);
@@ -148,166 +215,162 @@ __global__ void __launch_bounds__(kFWaves * 64) k_flash_rows(const AttnArgs a) {
       split8(qv[c], qh[c], ql[c]);
     }
   }
+  const bool cap = a.softcap > 0.f;
+  const float qs = cap ? 1.0f : qscale * kLog2e;   // scores of the tile -> base-2 exponents
 
-  const size_t head_base = (size_t)kvh * a.max_seq * HD;
-  const uint16_t* kc = static_cast<const uint16_t*>(a.kc) + head_base;
-  const uint16_t* vc = static_cast<const uint16_t*>(a.vc) + head_base;
+  v16f o[NDT];
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt) o[dt] = v16f{};
+  float m = -INFINITY, l = 0.f;   // l: this lane's share of the row's sum, times 2^12
 
-  // K block -> LDS (positions past ctx - 1 reload ctx - 1: finite, masked)
-  auto stage_k = [&](int blk, v4u* dst) {
+  // transposed V read: lane's key of 4 and its 8 bytes of a 32-dim tile
+  const int vkey = 8 * h + ((lane >> 2) & 3);
+  const int vch = 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1);
+
+  auto step = [&](int st, const v4u* kall, const v4u* vall, v4u* knxt, v4u* vnxt) {
+    if (st + 1 < nstep) stage(st + 1, knxt, vnxt);
+    const int kb = (st * KG + g) * kBlk;
+    const v4u* kcur = kall + g * kGrp;
+    const v4u* vcur = vall + g * kGrp;
+    v16f acc = v16f{};
+    if (kb <= wmax) {
 #pragma unroll
-    for (int k = 0; k < kFKeys * CH / (kFWaves * 64); ++k) {
-      const int P = k * kFWaves * 64 + wave * 64 + lane;   // LDS chunk this lane fills
-      const int key = P / CH, slot = P % CH;
-      const int p = min(blk * kFKeys + key, ctx - 1);
-      const uint16_t* src = kc + (size_t)p * HD + 8 * (slot ^ kswz(key));
-      __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)&dst[k * kFWaves * 64 + wave * 64], 16, 0, 0);
-    }
-  };
-  // V block: thread (kg, c) loads dims 8c..8c+7 of keys 4kg..4kg+3
-  const int vkg = tid % kKG, vch = tid / kKG;
-  uint4 vr[4];
-  auto load_v = [&](int blk) {
-    if (tid < kVItems) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int p = min(blk * kFKeys + 4 * vkg + u, ctx - 1);
-        vr[u] = *reinterpret_cast<const uint4*>(vc + (size_t)p * HD + 8 * vch);
+      for (int c = 0; c < NC; ++c) {
+        const v8h kv = __builtin_bit_cast(v8h, kcur[n * CH + ((2 * (ds * NC + c) + h) ^ kswz<CH>(n))]);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv, qh[c], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv, ql[c], acc, 0, 0, 0);
       }
     }
-  };
-  auto store_v = [&](v4u* vdst) {   // dim 8c + j of the 4 keys -> V^T row 8c + j
-    if (tid < kVItems) {
+    if (DS > 1) {   // the sum of the two waves' shares, the same in both
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        uint32_t w[4];
+      for (int j = 0; j < 16; ++j) xs[wave][64 * j + lane] = acc[j];
+      __syncthreads();
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const uint32_t word = j < 2 ? vr[u].x : j < 4 ? vr[u].y : j < 6 ? vr[u].z : vr[u].w;
-          w[u] = (j & 1) ? word >> 16 : word & 0xffffu;
-        }
-        uint8_t* row = reinterpret_cast<uint8_t*>(&vdst[(8 * vch + j) * kVC]);
-        *reinterpret_cast<uint2*>(row + 16 * ((vkg >> 1) ^ (j & (kVC - 1))) + 8 * (vkg & 1)) =
-            make_uint2(w[0] | (w[1] << 16), w[2] | (w[3] << 16));
+      for (int j = 0; j < 16; ++j) acc[j] += xs[wave ^ 1][64 * j + lane];
+    }
+    if (kb <= wmax) {
+      // element j is key kb + 16(j/8) + 8h + j%8 of row n
+      float sc[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) sc[j] = acc[j];
+      if (cap) {   // (q . k) / sqrt(hd), softcapped (layer_scheduler.c:442-448)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) sc[j] = softcap(sc[j] * qscale, a) * kLog2e;
       }
-    }
-  };
-
-  v4f o[NDT];
+      if (kb + kBlk - 1 > wmin) {   // causal limit
 #pragma unroll
-  for (int dt = 0; dt < NDT; ++dt) o[dt] = v4f{0.f, 0.f, 0.f, 0.f};
-  float m = -INFINITY, l = 0.f;   // l: this lane's share of the row's sum
-
-  stage_k(0, ks0);
-  load_v(0);
-  store_v(vt0);
-  vm_drain();
-  __syncthreads();
-  // one block: the next block's K and V requested into the other buffers,
-  // this block's keys used from kcur / vcur
-  auto step = [&](int blk, const v4u* kcur, const v4u* vcur, v4u* knxt, v4u* vnxt) {
-    const bool next = blk + 1 < nblk;
-    if (next) {
-      load_v(blk + 1);
-      stage_k(blk + 1, knxt);
-    }
-    const int kb = blk * kFKeys;
-    if (kb <= wlim) {
-      // S^T tiles (s, t): keys kb + 32s + 8(n/4) + 4t + n%4 against the wave's 16 rows
-      v4f st[NS][2];
+        for (int j = 0; j < 16; ++j)
+          if (kb + 16 * (j / 8) + 8 * h + j % 8 > lim) sc[j] = -INFINITY;
+      }
+      float bmax = sc[0];
 #pragma unroll
-      for (int s = 0; s < NS; ++s)
+      for (int j = 1; j < 16; ++j) bmax = fmaxf(bmax, sc[j]);
+      bmax = max_pair(bmax) * qs;
+      if (__any(bmax > m + kLag)) {
+        const float mn = fmaxf(m, bmax);
+        const float corr = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
+        l *= corr;
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const int key = 32 * s + 8 * (n >> 2) + 4 * t + (n & 3);
-          v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
+        for (int dt = 0; dt < NDT; ++dt) o[dt] *= corr;
+        m = mn;
+      }
+      const float mo = (m == -INFINITY ? 0.f : m) - kPExp;   // nothing seen yet: weights stay 0
+      v8h ph[2], pl[2];
 #pragma unroll
-          for (int c = 0; c < NC; ++c) {
-            const v8h kv = __builtin_bit_cast(v8h, kcur[key * CH + ((4 * c + kq) ^ kswz(key))]);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kv, qh[c], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kv, ql[c], acc, 0, 0, 0);
-          }
-          st[s][t] = acc;
-        }
-      // lane (n, kq): element i of tile (s, t) is key kb + 32s + 8kq + 4t + i of row n
-      float sc[NS][2][4];
-      float bmax = -INFINITY;
-#pragma unroll
-      for (int s = 0; s < NS; ++s)
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int key = kb + 32 * s + 8 * kq + 4 * t + i;
-            // (q . k) / sqrt(hd), softcapped when set (layer_scheduler.c:442-448); causal limit
-            const float v = key <= lim ? softcap(st[s][t][i] * qscale, a) : -INFINITY;
-            sc[s][t][i] = v;
-            bmax = fmaxf(bmax, v);
-          }
-      bmax = max4(bmax);
-      const float mn = fmaxf(m, bmax);
-      const float ms = mn == -INFINITY ? 0.f : mn;   // nothing seen yet: weights stay 0
-      const float corr = expf(m - ms);
-      l *= corr;
-#pragma unroll
-      for (int dt = 0; dt < NDT; ++dt) o[dt] *= corr;
-      v8h ph[NS], pl[NS];
-#pragma unroll
-      for (int s = 0; s < NS; ++s) {
+      for (int c = 0; c < 2; ++c) {
         float pv[8];
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float p = expf(sc[s][t][i] - ms);   // layer_scheduler.c:450-458
-            l += p;
-            pv[4 * t + i] = p * kPScale;
-          }
-        split8(pv, ph[s], pl[s]);
+        for (int i = 0; i < 8; ++i) {
+          pv[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[8 * c + i], qs, -mo));   // layer_scheduler.c:450-458
+          l += pv[i];
+        }
+        split8(pv, ph[c], pl[c]);
       }
-      m = mn;
-      // O^T += V^T P^T over the block's 32-key halves
+      // O^T += V^T P^T
 #pragma unroll
-      for (int dt = 0; dt < NDT; ++dt)
+      for (int c = 0; c < 2; ++c)
 #pragma unroll
-        for (int s = 0; s < NS; ++s) {
-          const int d = 16 * dt + n;
-          const v8h vv = __builtin_bit_cast(v8h, vcur[d * kVC + ((4 * s + kq) ^ (d & (kVC - 1)))]);
-          o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv, ph[s], o[dt], 0, 0, 0);
-          o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vv, pl[s], o[dt], 0, 0, 0);
+        for (int dt = 0; dt < NDT; ++dt) {
+          union { v4s t[2]; v8h v; } vv;
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const int key = 16 * c + 4 * u + vkey;
+            const v4u* p = &vcur[key * CH + ((4 * (ds * NDT + dt) + vch) ^ vswz<CH>(vkey))];
+            vv.t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t)(reinterpret_cast<const v4s*>(p) + (lane & 1)));
+          }
+          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vv.v, ph[c], o[dt], 0, 0, 0);
+          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vv.v, pl[c], o[dt], 0, 0, 0);
         }
     }
-    if (next) store_v(vnxt);
-    vm_drain();   // this wave's direct LDS loads of the next block have landed
-    __syncthreads();
+    turn();
   };
+  turn();
 #pragma unroll 1
-  for (int blk = 0; blk < nblk; blk += 2) {
-    step(blk, ks0, vt0, ks1, vt1);
-    if (blk + 1 < nblk) step(blk + 1, ks1, vt1, ks0, vt0);
+  for (int st = 0; st < nstep; st += 2) {
+    step(st, ks0, vs0, ks1, vs1);
+    if (st + 1 < nstep) step(st + 1, ks1, vs1, ks0, vs0);
   }
 
-  // lane (n, kq) holds dims 16dt + 4kq .. +3 of row n   (layer_scheduler.c:460-466)
-  l = sum4(l);
-  if (z < a.n_tok) {
-    const float inv = 1.0f / (l * kPScale);
-    float* op = a.out + (size_t)z * a.tok_o + ((size_t)kvh * G + h) * HD + 4 * kq;
+  // the groups' rows -> one: every group's O at the common maximum through
+  // LDS (the staging buffers: RT * KG tiles of 32 rows x HD floats, KG / 2 in
+  // each), then summed row by row   (layer_scheduler.c:460-466)
+  l = sum_pair(l);
+  if (h == 0 && ds == 0) {
+    gm[g][32 * rt + n] = m;
+    gl[g][32 * rt + n] = l;
+  }
+  __syncthreads();
+  {
+    float mx = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < KG; ++k) mx = fmaxf(mx, gm[k][32 * rt + n]);
+    float lt = 0.f;
+#pragma unroll
+    for (int k = 0; k < KG; ++k) {
+      const float mk = gm[k][32 * rt + n];
+      lt += mk == -INFINITY ? 0.f : gl[k][32 * rt + n] * __builtin_amdgcn_exp2f(mk - mx);
+    }
+    const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mx) / lt;
+    auto bank = [&](int w) { return w == 0 ? ks0 : w == 1 ? vs0 : w == 2 ? ks1 : vs1; };
+    const int tile = wave / DS;
+    float4* dst = reinterpret_cast<float4*>(bank(tile / (KG / 2))) + (tile % (KG / 2)) * (32 * HD / 4);
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt)
-      *reinterpret_cast<float4*>(op + 16 * dt) =
-          make_float4(o[dt][0] * inv, o[dt][1] * inv, o[dt][2] * inv, o[dt][3] * inv);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)   // dims 32dt + 8q + 4h .. +3 of row n
+        dst[n * (HD / 4) + ((8 * (ds * NDT + dt) + 2 * q + h) ^ (n & 15))] =
+            make_float4(o[dt][4 * q] * f, o[dt][4 * q + 1] * f, o[dt][4 * q + 2] * f, o[dt][4 * q + 3] * f);
+    __syncthreads();
+    for (int i = tid; i < RT * 32 * (HD / 4); i += NT) {
+      const int r = i / (HD / 4), c = i % (HD / 4);
+      const int zr = (row0 + r) / G, hr = (row0 + r) % G;
+      if (zr >= a.n_tok) continue;
+      float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (int k = 0; k < KG; ++k) {
+        const int w = k * RT + r / 32;
+        const float4* src = reinterpret_cast<const float4*>(bank(w / (KG / 2))) + (w % (KG / 2)) * (32 * HD / 4);
+        const float4 v = src[(r % 32) * (HD / 4) + (c ^ (r & 15))];
+        s.x += v.x;
+        s.y += v.y;
+        s.z += v.z;
+        s.w += v.w;
+      }
+      *reinterpret_cast<float4*>(a.out + (size_t)zr * a.tok_o + ((size_t)kvh * G + hr) * HD + 4 * c) = s;
+    }
   }
 }
 
-template <int HD>
-hipError_t launch_flash_hd(int group, const AttnArgs& a, hipStream_t s) {
-  const dim3 block(kFWaves * 64);
-  auto grid = [&](int g) { return dim3((a.n_tok * g + kFRows - 1) / kFRows, a.n_kv_heads); };
+template <int HD, int RT, int KG, int DS = 1>
+hipError_t launch_flash(int group, const AttnArgs& a, hipStream_t s) {
+  const int64_t tiles = ((int64_t)a.n_tok * group + 32 * RT - 1) / (32 * RT);
+  if (tiles * a.n_kv_heads > INT32_MAX) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)(tiles * a.n_kv_heads)), block(RT * KG * DS * 64);
   switch (group) {
-    case 1: hipLaunchKernelGGL((k_flash_rows<HD, 1>), grid(1), block, 0, s, a); break;
-    case 2: hipLaunchKernelGGL((k_flash_rows<HD, 2>), grid(2), block, 0, s, a); break;
-    case 4: hipLaunchKernelGGL((k_flash_rows<HD, 4>), grid(4), block, 0, s, a); break;
-    case 8: hipLaunchKernelGGL((k_flash_rows<HD, 8>), grid(8), block, 0, s, a); break;
+    case 1: hipLaunchKernelGGL((k_flash_rows<HD, 1, RT, KG, DS>), grid, block, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((k_flash_rows<HD, 2, RT, KG, DS>), grid, block, 0, s, a); break;
+    case 4: hipLaunchKernelGGL((k_flash_rows<HD, 4, RT, KG, DS>), grid, block, 0, s, a); break;
+    case 8: hipLaunchKernelGGL((k_flash_rows<HD, 8, RT, KG, DS>), grid, block, 0, s, a); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -319,9 +382,21 @@ hipError_t launch_attention_rows(int head_dim, int group, const AttnArgs& a, hip
   if (a.n_tok < 1 || a.n_kv_heads < 1 || a.max_seq < 1 || !a.q || !a.out || !a.kc || !a.vc || a.tok_q % 4 ||
       a.tok_o % 4)
     return hipErrorInvalidValue;
-  if (head_dim == 64) return launch_flash_hd<64>(group, a, s);
-  if (head_dim == 128) return launch_flash_hd<128>(group, a, s);
-  if (head_dim == 256) return launch_flash_hd<256>(group, a, s);   // Gemma
+  // Up to 64 keys: two key groups, one step (32 heads x 32 tokens at head_dim
+  // 128: 6.5 us, with four groups 7.8). More row tiles than compute units at
+  // head_dim 128: two tiles share a workgroup's staging (512 tokens over 1536,
+  // 32 heads on 8: 41 us against 55 with one; 77 tokens over 1000, 80 tiles:
+  // 18 against 23 the other way round). head_dim 64 keeps one tile, as two
+  // such workgroups fit a compute unit (2000 tokens, 8 heads: 22 against 24).
+  // head_dim 256 has LDS for two key groups only.
+  const bool two_blocks = (int64_t)a.pos0 + a.n_tok <= 2 * kBlk;
+  const int64_t tiles = ((int64_t)a.n_tok * group + 31) / 32 * a.n_kv_heads;
+  if (head_dim == 64) return two_blocks ? launch_flash<64, 1, 2>(group, a, s) : launch_flash<64, 1, 4>(group, a, s);
+  if (head_dim == 128) {
+    if (two_blocks) return launch_flash<128, 1, 2>(group, a, s);
+    return tiles > kCompute ? launch_flash<128, 2, 4>(group, a, s) : launch_flash<128, 1, 4>(group, a, s);
+  }
+  if (head_dim == 256) return launch_flash<256, 1, 2, 2>(group, a, s);   // Gemma
   return hipErrorInvalidValue;
 }
 

@@ -1515,7 +1515,7 @@ int32_t enqueue_layer_rows(ss_hip_model* m, int l, const DevLayer& ly, int T, in
   at.tok_q = ldq;
   at.kc = kc;
   at.vc = vc;
-  at.dpos = dpos;
+  at.pos0 = p0;
   at.max_seq = m->max_seq;
   at.ns = 1;
   at.n_kv_heads = m->KVH;

@@ -136,8 +136,8 @@ struct AttnArgs {
   int split_fill;            // attn_chunks' fill (0: none)
   int wo_merge;              // with cnt set: when at most kMergeSplits splits are active, leave
                              // them in part_o/part_ml for the Wo matvec (which then merges them)
-  int n_tok;                 // prompt rows (launch_attention_rows): token z at position dpos[z]
-  int pos0;                  // (or pos0 + z when dpos is null),
+  int n_tok;                 // prompt rows (launch_attention_rows): token z at position
+  int pos0;                  // pos0 + z,
   int tok_q, tok_o;          // its query at q + z*tok_q, its output at out + z*tok_o
 };
 
@@ -174,7 +174,7 @@ hipError_t launch_attention(int head_dim, int group, int kv_type, const AttnArgs
 // nothing when one split is active (the attention wrote the output).
 hipError_t launch_attention_merge(int head_dim, int group, const AttnArgs& a, hipStream_t s);
 // Causal attention of a.n_tok prompt rows (token z: query a.q + z*a.tok_q,
-// positions 0..a.dpos[z] (or a.pos0 + z), output a.out + z*a.tok_o), fp16
+// positions 0..a.pos0 + z, output a.out + z*a.tok_o), fp16
 // cache, head_dim 64, 128 or 256, on MFMA (ss_flash.hip).
 hipError_t launch_attention_rows(int head_dim, int group, const AttnArgs& a, hipStream_t s);
 // ssq[t] = sum of x[t][c]^2 (x [T][cols])
