@@ -47,6 +47,11 @@
 // ds_read_b64_tr_b16 (lane i of 16 addresses key i/4, dims 4(i%4)..+3, and
 // receives dim i of the four keys). Both swizzles spread a read over all banks.
 
+// An int8 cache's codes are exact in fp16: a block passes through registers,
+// where codes become fp16 (requested before the current block's products,
+// written to LDS after them), a position's K scale multiplies its scores and
+// its V scale the weights after the row's sum took them.
+
 #include <hip/hip_runtime.h>
 #include <math.h>
 
@@ -57,6 +62,7 @@ namespace ssk {
 namespace {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
@@ -95,6 +101,19 @@ __device__ __forceinline__ void split8(const float (&v)[8], v8h& hi, v8h& lo) {
   }
 }
 
+// 8 int8 codes -> fp16, exact: 1024 + (code + 128) by placing the byte, less 1152
+__device__ __forceinline__ v4u codes8(uint32_t lo, uint32_t hi) {
+  const v2h off = {(_Float16)1152.f, (_Float16)1152.f};
+  v4u r;
+  lo ^= 0x80808080u;
+  hi ^= 0x80808080u;
+  r[0] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, lo, 0x04010400u)) - off);
+  r[1] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, lo, 0x04030402u)) - off);
+  r[2] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, hi, 0x04010400u)) - off);
+  r[3] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, hi, 0x04030402u)) - off);
+  return r;
+}
+
 // tile row -> key of the block: bits 2 and 3 change places (its own inverse)
 __host__ __device__ constexpr int tile_key(int r) { return (r & 19) | ((r & 4) << 1) | ((r & 8) >> 1); }
 // slot swizzles (16-byte chunks of a row of CH): 16 neighbouring tile rows take
@@ -102,7 +121,7 @@ __host__ __device__ constexpr int tile_key(int r) { return (r & 19) | ((r & 4) <
 template <int CH> __device__ __forceinline__ int kswz(int row) { return CH == 8 ? (row >> 1) & 7 : row & 15; }
 template <int CH> __device__ __forceinline__ int vswz(int key) { return CH == 8 ? 2 * (key & 2) : 4 * (key & 3); }
 
-template <int HD, int G, int RT, int KG, int DS>
+template <int HD, int G, int RT, int KG, int DS, bool Q8>
 __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs a) {
   constexpr int CH = HD / 8;             // 16-byte chunks per row
   constexpr int NC = HD / 16 / DS;       // a wave's 16-wide slices of the head dimension
@@ -120,6 +139,8 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
   __shared__ v4u ks0[KG * kGrp], ks1[KG * kGrp];
   __shared__ v4u vs0[KG * kGrp], vs1[KG * kGrp];
   __shared__ float xs[DS > 1 ? RT * KG * DS : 1][DS > 1 ? 16 * 64 : 1];   // the waves' shares of S^T
+  __shared__ float sc0[Q8 ? KG : 1][64], sc1[Q8 ? KG : 1][64];   // int8: the block's K scales, then its V scales
+  __shared__ float vred[RT * KG * DS];
   __shared__ float gm[KG][RT * 32], gl[KG][RT * 32];   // each group's maximum and sum of a row
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -153,8 +174,8 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
     }
   }
   const size_t head_base = (size_t)kvh * a.max_seq * HD;
-  const uint16_t* kc = static_cast<const uint16_t*>(a.kc) + head_base;
-  const uint16_t* vc = static_cast<const uint16_t*>(a.vc) + head_base;
+  const uint16_t* kc = static_cast<const uint16_t*>(a.kc) + (Q8 ? 0 : head_base);
+  const uint16_t* vc = static_cast<const uint16_t*>(a.vc) + (Q8 ? 0 : head_base);
 
   // this group's block of a step -> LDS, each of its RT * DS waves a share
   // (positions past ctx - 1 reload ctx - 1: finite, masked)
@@ -180,6 +201,41 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
                                        (lds_ptr_t)&vd[g * kGrp + base], 16, 0, 0);
     }
   };
+  // an int8 block passes through registers: 16 codes are two chunks of fp16
+  constexpr int kQLoads = Q8 ? kLoads / 2 : 1, kQRow = HD / 16;
+  static_assert(kLoads % 2 == 0, "pairs of chunks");
+  v4u kq[kQLoads], vq[kQLoads];
+  float qsc = 0.f;
+  auto load_q = [&](int step) {
+    const int kb = (step * KG + g) * kBlk;
+    if (kb >= ctx) return;
+    const int8_t* k8 = static_cast<const int8_t*>(a.kc) + head_base;
+    const int8_t* v8 = static_cast<const int8_t*>(a.vc) + head_base;
+#pragma unroll
+    for (int k = 0; k < kQLoads; ++k) {
+      const int i = ((rt * DS + ds) * kQLoads + k) * 64 + lane;
+      const int pk = min(kb + tile_key(i / kQRow), ctx - 1), pv = min(kb + i / kQRow, ctx - 1);
+      kq[k] = *reinterpret_cast<const v4u*>(k8 + (size_t)pk * HD + 16 * (i % kQRow));
+      vq[k] = *reinterpret_cast<const v4u*>(v8 + (size_t)pv * HD + 16 * (i % kQRow));
+    }
+    qsc = (h ? a.vs : a.ks)[min(kb + n, ctx - 1)];
+  };
+  float vnorm = 1.f, vscale = 1.f;
+  auto store_q = [&](int step, v4u* kd, v4u* vd, float (*scd)[64]) {
+    if ((step * KG + g) * kBlk >= ctx) return;
+#pragma unroll
+    for (int k = 0; k < kQLoads; ++k) {
+      const int i = ((rt * DS + ds) * kQLoads + k) * 64 + lane;
+      const int r = i / kQRow, c = 2 * (i % kQRow);
+      v4u* kr = kd + g * kGrp + r * CH;
+      v4u* vr = vd + g * kGrp + r * CH;
+      kr[c ^ kswz<CH>(r)] = codes8(kq[k][0], kq[k][1]);
+      kr[(c + 1) ^ kswz<CH>(r)] = codes8(kq[k][2], kq[k][3]);
+      vr[c ^ vswz<CH>(r)] = codes8(vq[k][0], vq[k][1]);
+      vr[(c + 1) ^ vswz<CH>(r)] = codes8(vq[k][2], vq[k][3]);
+    }
+    if (rt == 0 && ds == 0) scd[g][lane] = h ? qsc * vnorm : qsc;
+  };
   // the staged loads have landed and the other buffer's reads are done, for
   // this wave, and for the others where waves share the staging
   auto turn = [&] {
@@ -187,7 +243,28 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
     if (RT * DS > 1) __syncthreads();
   };
 
-  stage(0, ks0, vs0);
+  if (Q8) {
+    load_q(0);
+    // the V scales by the power of two of the largest one, so that P times
+    // them keeps its two fp16 parts (a scale 2^-k of the largest loses bits
+    // below 2^-37 of the largest)
+    float vm = 0.f;
+    for (int p = tid; p < ctx; p += NT) vm = fmaxf(vm, a.vs[p]);
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) vm = fmaxf(vm, __shfl_xor(vm, off, kWave));
+    if (lane == 0) vred[wave] = vm;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) vm = fmaxf(vm, vred[w]);
+    int e = 0;
+    frexpf(vm, &e);
+    e = min(max(e, -120), 120);
+    vnorm = ldexpf(1.0f, -e);
+    vscale = ldexpf(1.0f, e);
+    store_q(0, ks0, vs0, sc0);
+  } else {
+    stage(0, ks0, vs0);
+  }
 
   // q as the B operand of S^T: lane (n, h) holds q[16c + 8h + i] of row n
   v8h qh[NC], ql[NC];
@@ -227,8 +304,12 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
   const int vkey = 8 * h + ((lane >> 2) & 3);
   const int vch = 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1);
 
-  auto step = [&](int st, const v4u* kall, const v4u* vall, v4u* knxt, v4u* vnxt) {
-    if (st + 1 < nstep) stage(st + 1, knxt, vnxt);
+  auto step = [&](int st, const v4u* kall, const v4u* vall, const float (*scl)[64], v4u* knxt, v4u* vnxt,
+                  float (*scn)[64]) {
+    if (st + 1 < nstep) {
+      if (Q8) load_q(st + 1);
+      else stage(st + 1, knxt, vnxt);
+    }
     const int kb = (st * KG + g) * kBlk;
     const v4u* kcur = kall + g * kGrp;
     const v4u* vcur = vall + g * kGrp;
@@ -252,7 +333,7 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
       // element j is key kb + 16(j/8) + 8h + j%8 of row n
       float sc[16];
 #pragma unroll
-      for (int j = 0; j < 16; ++j) sc[j] = acc[j];
+      for (int j = 0; j < 16; ++j) sc[j] = Q8 ? acc[j] * scl[g][16 * (j / 8) + 8 * h + j % 8] : acc[j];
       if (cap) {   // (q . k) / sqrt(hd), softcapped (layer_scheduler.c:442-448)
 #pragma unroll
         for (int j = 0; j < 16; ++j) sc[j] = softcap(sc[j] * qscale, a) * kLog2e;
@@ -283,6 +364,7 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
         for (int i = 0; i < 8; ++i) {
           pv[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[8 * c + i], qs, -mo));   // layer_scheduler.c:450-458
           l += pv[i];
+          if (Q8) pv[i] *= scl[g][32 + 16 * c + 8 * h + i];
         }
         split8(pv, ph[c], pl[c]);
       }
@@ -302,13 +384,14 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
           o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vv.v, pl[c], o[dt], 0, 0, 0);
         }
     }
+    if (Q8 && st + 1 < nstep) store_q(st + 1, knxt, vnxt, scn);
     turn();
   };
   turn();
 #pragma unroll 1
   for (int st = 0; st < nstep; st += 2) {
-    step(st, ks0, vs0, ks1, vs1);
-    if (st + 1 < nstep) step(st + 1, ks1, vs1, ks0, vs0);
+    step(st, ks0, vs0, sc0, ks1, vs1, sc1);
+    if (st + 1 < nstep) step(st + 1, ks1, vs1, sc1, ks0, vs0, sc0);
   }
 
   // the groups' rows -> one: every group's O at the common maximum through
@@ -330,7 +413,7 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
       const float mk = gm[k][32 * rt + n];
       lt += mk == -INFINITY ? 0.f : gl[k][32 * rt + n] * __builtin_amdgcn_exp2f(mk - mx);
     }
-    const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mx) / lt;
+    const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mx) / lt * vscale;
     auto bank = [&](int w) { return w == 0 ? ks0 : w == 1 ? vs0 : w == 2 ? ks1 : vs1; };
     const int tile = wave / DS;
     float4* dst = reinterpret_cast<float4*>(bank(tile / (KG / 2))) + (tile % (KG / 2)) * (32 * HD / 4);
@@ -361,25 +444,31 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
   }
 }
 
-template <int HD, int RT, int KG, int DS = 1>
-hipError_t launch_flash(int group, const AttnArgs& a, hipStream_t s) {
+template <int HD, int RT, int KG, int DS, bool Q8>
+hipError_t launch_flash_kv(int group, const AttnArgs& a, hipStream_t s) {
   const int64_t tiles = ((int64_t)a.n_tok * group + 32 * RT - 1) / (32 * RT);
   if (tiles * a.n_kv_heads > INT32_MAX) return hipErrorInvalidValue;
   const dim3 grid((unsigned)(tiles * a.n_kv_heads)), block(RT * KG * DS * 64);
   switch (group) {
-    case 1: hipLaunchKernelGGL((k_flash_rows<HD, 1, RT, KG, DS>), grid, block, 0, s, a); break;
-    case 2: hipLaunchKernelGGL((k_flash_rows<HD, 2, RT, KG, DS>), grid, block, 0, s, a); break;
-    case 4: hipLaunchKernelGGL((k_flash_rows<HD, 4, RT, KG, DS>), grid, block, 0, s, a); break;
-    case 8: hipLaunchKernelGGL((k_flash_rows<HD, 8, RT, KG, DS>), grid, block, 0, s, a); break;
+    case 1: hipLaunchKernelGGL((k_flash_rows<HD, 1, RT, KG, DS, Q8>), grid, block, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((k_flash_rows<HD, 2, RT, KG, DS, Q8>), grid, block, 0, s, a); break;
+    case 4: hipLaunchKernelGGL((k_flash_rows<HD, 4, RT, KG, DS, Q8>), grid, block, 0, s, a); break;
+    case 8: hipLaunchKernelGGL((k_flash_rows<HD, 8, RT, KG, DS, Q8>), grid, block, 0, s, a); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
+template <int HD, int RT, int KG, int DS = 1>
+hipError_t launch_flash(int group, int kv_type, const AttnArgs& a, hipStream_t s) {
+  return kv_type ? launch_flash_kv<HD, RT, KG, DS, true>(group, a, s)
+                 : launch_flash_kv<HD, RT, KG, DS, false>(group, a, s);
+}
 
 }  // namespace
 
-hipError_t launch_attention_rows(int head_dim, int group, const AttnArgs& a, hipStream_t s) {
-  if (a.n_tok < 1 || a.n_kv_heads < 1 || a.max_seq < 1 || !a.q || !a.out || !a.kc || !a.vc || a.tok_q % 4 ||
+hipError_t launch_attention_rows(int head_dim, int group, int kv_type, const AttnArgs& a, hipStream_t s) {
+  if (a.n_tok < 1 || a.n_kv_heads < 1 || a.max_seq < 1 || !a.q || !a.out || !a.kc || !a.vc ||
+      (kv_type && (!a.ks || !a.vs)) || a.tok_q % 4 ||
       a.tok_o % 4)
     return hipErrorInvalidValue;
   // Up to 64 keys: two key groups, one step (32 heads x 32 tokens at head_dim
@@ -391,12 +480,12 @@ hipError_t launch_attention_rows(int head_dim, int group, const AttnArgs& a, hip
   // head_dim 256 has LDS for two key groups only.
   const bool two_blocks = (int64_t)a.pos0 + a.n_tok <= 2 * kBlk;
   const int64_t tiles = ((int64_t)a.n_tok * group + 31) / 32 * a.n_kv_heads;
-  if (head_dim == 64) return two_blocks ? launch_flash<64, 1, 2>(group, a, s) : launch_flash<64, 1, 4>(group, a, s);
+  if (head_dim == 64) return two_blocks ? launch_flash<64, 1, 2>(group, kv_type, a, s) : launch_flash<64, 1, 4>(group, kv_type, a, s);
   if (head_dim == 128) {
-    if (two_blocks) return launch_flash<128, 1, 2>(group, a, s);
-    return tiles > kCompute ? launch_flash<128, 2, 4>(group, a, s) : launch_flash<128, 1, 4>(group, a, s);
+    if (two_blocks) return launch_flash<128, 1, 2>(group, kv_type, a, s);
+    return tiles > kCompute ? launch_flash<128, 2, 4>(group, kv_type, a, s) : launch_flash<128, 1, 4>(group, kv_type, a, s);
   }
-  if (head_dim == 256) return launch_flash<256, 1, 2, 2>(group, a, s);   // Gemma
+  if (head_dim == 256) return launch_flash<256, 1, 2, 2>(group, kv_type, a, s);   // Gemma
   return hipErrorInvalidValue;
 }
 

@@ -175,8 +175,8 @@ hipError_t launch_attention(int head_dim, int group, int kv_type, const AttnArgs
 hipError_t launch_attention_merge(int head_dim, int group, const AttnArgs& a, hipStream_t s);
 // Causal attention of a.n_tok prompt rows (token z: query a.q + z*a.tok_q,
 // positions 0..a.pos0 + z, output a.out + z*a.tok_o), fp16
-// cache, head_dim 64, 128 or 256, on MFMA (ss_flash.hip).
-hipError_t launch_attention_rows(int head_dim, int group, const AttnArgs& a, hipStream_t s);
+// or int8 cache, head_dim 64, 128 or 256, on MFMA (ss_flash.hip).
+hipError_t launch_attention_rows(int head_dim, int group, int kv_type, const AttnArgs& a, hipStream_t s);
 // ssq[t] = sum of x[t][c]^2 (x [T][cols])
 hipError_t launch_sumsq(const float* x, int cols, int T, float* ssq, hipStream_t s);
 // Y = W X over T tokens with EPI_STORE, EPI_ADD or EPI_SWIGLU: X is split into
@@ -221,8 +221,8 @@ hipError_t launch_kv_append(void* kc, void* vc, float* ksc, float* vsc, const fl
 // RoPE of the q and k parts of n prompt rows [q | k | v] (stride ld; token z
 // at position dpos[z]) and the fp16 cache append of k and v.
 hipError_t launch_rope_kv_rows(float* qkv, const float* bias, int ld, int qdim, int kvdim, int head_dim, int rope_dim,
-                               const float* cs, const int* dpos, uint16_t* kc, uint16_t* vc, int max_seq,
-                               int n, hipStream_t s);
+                               const float* cs, const int* dpos, void* kc, void* vc, float* ksc, float* vsc,
+                               int max_seq, int kv_type, int n, hipStream_t s);
 // acc[j] += sum over the T rows x[t] (stride d) of x[t][j] * k_t * w[j] (the
 // output RMSNorm, k_t from ssq[t]), or of x[t][j] when w is null
 hipError_t launch_pool_rows(const float* x, int T, int d, const float* w, const float* ssq, float eps, float* acc,

@@ -968,6 +968,56 @@ __global__ void k_rope_kv_rows(float* qkv, const float* bias, int ld, int qdim, 
   }
 }
 
+// The same for the int8 cache: workgroups 0 .. gridDim.x - 3 of a row take its
+// queries, the last two its K and V, whose scale is the largest magnitude over
+// all KV heads (layer_scheduler.c:101-118): the values go back to the row,
+// then, once that is known, as codes to the cache, like k_kv_append's.
+__global__ void __launch_bounds__(256) k_rope_kv_rows_q8(float* qkv, const float* bias, int ld, int qdim, int kvdim,
+                                                         int head_dim, int rope_dim, const float* cs, const int* dpos,
+                                                         int8_t* kc, int8_t* vc, float* ksc, float* vsc, int max_seq) {
+  const int pos = dpos[blockIdx.y];
+  const int ng = gridDim.x - 2, part = (int)blockIdx.x - ng;   // < 0: queries, 0: K, 1: V
+  const int begin = part < 0 ? 0 : qdim + part * kvdim, width = part < 0 ? qdim : kvdim;
+  const int first = part < 0 ? blockIdx.x * 256 : 0, step = part < 0 ? ng * 256 : 256;
+  float* row = qkv + (size_t)blockIdx.y * ld + begin;
+  float m = 0.f;
+  for (int p = first + threadIdx.x; p < width / 2; p += step) {
+    const float2 v = reinterpret_cast<const float2*>(row)[p];
+    float a = v.x, b = v.y;
+    if (bias) {   // layer_scheduler.c:367-402, before RoPE
+      const float2 bb = reinterpret_cast<const float2*>(bias + begin)[p];
+      a = a + bb.x;
+      b = b + bb.y;
+    }
+    const int i0 = 2 * p % head_dim;
+    if (part < 1 && i0 < rope_dim) {
+      const float c = cs[(size_t)pos * rope_dim + i0], s = cs[(size_t)pos * rope_dim + i0 + 1];
+      const float ra = a * c - b * s;
+      const float rb = a * s + b * c;
+      a = ra;
+      b = rb;
+    }
+    reinterpret_cast<float2*>(row)[p] = make_float2(a, b);
+    m = fmaxf(m, fmaxf(fabsf(a), fabsf(b)));
+  }
+  if (part < 0) return;
+  __shared__ float red[4];
+  m = wave_max(m);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  const float amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  const float s = amax / 127.0f;
+  const float inv = s > 0.0f ? 1.0f / s : 0.0f;
+  int8_t* c = part ? vc : kc;
+  for (int p = threadIdx.x; p < width / 2; p += 256) {   // each thread its own pairs
+    const float2 v = reinterpret_cast<const float2*>(row)[p];
+    const int g = 2 * p / head_dim, d = 2 * p % head_dim;
+    *reinterpret_cast<char2*>(c + ((size_t)g * max_seq + pos) * head_dim + d) =
+        make_char2((signed char)roundf(v.x * inv), (signed char)roundf(v.y * inv));
+  }
+  if (threadIdx.x == 0) (part ? vsc : ksc)[pos] = s;
+}
+
 // KV append: fp16 (one thread per element) or the int8 absmax encoding of
 // layer_scheduler.c:101-118 (one workgroup each for K and V).
 __global__ void k_kv_append(void* kc, void* vc, float* ksc, float* vsc, const float* k,
@@ -1250,13 +1300,19 @@ hipError_t launch_kv_append(void* kc, void* vc, float* ksc, float* vsc, const fl
 }
 
 hipError_t launch_rope_kv_rows(float* qkv, const float* bias, int ld, int qdim, int kvdim, int head_dim, int rope_dim,
-                               const float* cs, const int* dpos, uint16_t* kc, uint16_t* vc, int max_seq,
-                               int n, hipStream_t s) {
+                               const float* cs, const int* dpos, void* kc, void* vc, float* ksc, float* vsc,
+                               int max_seq, int kv_type, int n, hipStream_t s) {
   if (n <= 0 || ld % 2 || qdim % 2 || kvdim % 2 || head_dim % 2 || ld < qdim + 2 * kvdim) return hipErrorInvalidValue;
+  if (kv_type) {
+    hipLaunchKernelGGL(k_rope_kv_rows_q8, dim3((qdim / 2 + 255) / 256 + 2, n), dim3(256), 0, s, qkv, bias, ld, qdim,
+                       kvdim, head_dim, rope_dim, cs, dpos, static_cast<int8_t*>(kc), static_cast<int8_t*>(vc), ksc,
+                       vsc, max_seq);
+    return hipGetLastError();
+  }
   const int npairs = (qdim + 2 * kvdim) / 2;
   const int gx = (npairs + 255) / 256;
   hipLaunchKernelGGL(k_rope_kv_rows, dim3(gx, n), dim3(256), 0, s, qkv, bias, ld, qdim, kvdim, head_dim, rope_dim,
-                     cs, dpos, kc, vc, max_seq);
+                     cs, dpos, static_cast<uint16_t*>(kc), static_cast<uint16_t*>(vc), max_seq);
   return hipGetLastError();
 }
 
