@@ -296,8 +296,9 @@ void ss_hip_model_free(ss_hip_model_t *m);
 int32_t ss_hip_eval_token(ss_hip_model_t *m, int32_t token, int32_t pos, float *logits_host,
                           int32_t *argmax_out);
 /* ss_scheduler_prefill (layer_scheduler.h:119). A prompt of at least the
- * batch threshold (default 8 tokens) runs as matrix products over chunks of
- * up to 512 tokens; shorter prompts run token by token. */
+ * batch threshold runs as matrix products over chunks of up to 512 tokens;
+ * shorter prompts run token by token. The default threshold is 4 tokens, more
+ * over a prefix longer than 4096 positions (up to 8 with the fp16 cache). */
 int32_t ss_hip_eval_prompt(ss_hip_model_t *m, const int32_t *tokens, int32_t n,
                            int32_t start_pos, float *logits_host, int32_t *argmax_out);
 /* Batch threshold of ss_hip_eval_prompt: 0 restores the default, a negative

@@ -1445,9 +1445,27 @@ int32_t enqueue_prompt_layer_major(ss_hip_model* m, const int32_t* tokens, int n
 // chunk's K/V having been appended first). Later chunks read the earlier
 // chunks' cache. Both caches take it: token by token, 64 tokens of a
 // 22-layer TinyLlama with the int8 cache took 40.5 ms, as products 1.6.
-// Prompts shorter than kPrefillMin tokens run token by token.
+//
+// Where tokens become products. The products' launches cost the same from 1
+// to 16 tokens, a token by itself 0.3-0.45 of them: 7B Q4_0 layers at 3 / 4 / 8
+// tokens run in 564 / 732 / 1410 us per 4 layers token by token, 538 us as
+// products; 8B Q4_K 633 / 820 / 1590 against 550; two 256-wide layers 171 /
+// 216 / 395 against 135. Over a long prefix the rows' attention has few
+// workgroups and its walk costs 10 us (int8: 16) per 1000 positions and layer,
+// a token's own attention 1.2: at 8000 positions 4 tokens break even with the
+// int8 cache and 8 still run in half the time, so the prefix may grow by 2048
+// positions per token above two. From kPrefillAlways tokens on an fp16 cache
+// any prefix goes (8 tokens over 8000: 871 us against 1790).
 constexpr int kPrefillChunk = 512;
-constexpr int kPrefillMin = 8;
+constexpr int kPrefillMin = 4, kPrefillAlways = 8;
+constexpr int kPrefillPrefix = 2048;
+
+bool prompt_as_products(const ss_hip_model* m, int n, int start) {
+  if (m->pf_min < 0 || m->token_only) return false;
+  if (m->pf_min > 0) return n >= m->pf_min;
+  if (m->kv_type == SS_HIP_KV_F16 && n >= kPrefillAlways) return true;
+  return n >= kPrefillMin && start <= (int64_t)kPrefillPrefix * (n - 2);
+}
 
 int32_t prefill_setup(ss_hip_model* m) {
   if (m->pf_cap) return 0;
@@ -2029,8 +2047,7 @@ int32_t ss_hip_eval_prompt(ss_hip_model_t* m, const int32_t* tokens, int32_t n, 
   HIP_TRY(hipStreamSynchronize(s));
   HIP_TRY(hipMemcpy(m->tokens + start, tokens, sizeof(int) * n, hipMemcpyHostToDevice));
   HIP_TRY(ssk::launch_set_state(m->dpos, m->tokens, start, tokens[0], s));
-  const int pf_min = m->pf_min > 0 ? m->pf_min : kPrefillMin;
-  if (m->pf_min >= 0 && n >= pf_min && !m->token_only) {
+  if (prompt_as_products(m, n, start)) {
     if (int32_t rc = prefill_setup(m)) return rc;
     if (int32_t rc = enqueue_prompt_rows(m, tokens, n, start)) {
       hipStreamSynchronize(s);
