@@ -369,40 +369,6 @@ __device__ __forceinline__ float q4_dot(const uint4 q, const uint32_t* ra, const
   return fmaf((float)(a - (int)ta.x), __uint_as_float(ta.y), (float)(b - (int)tb.x) * __uint_as_float(tb.y));
 }
 
-// Q4_K sub-block (quantize.c:265-310: weight = dsc * q - dmn with q the
-// nibble, dsc = d * scale and dmn = dmin * min of the sub-block, both exact
-// in fp32), packed like a Q4_0 block (nibble j of weight j, j + 16 in the
-// high nibble) but without the -8 offset: sum w x = dsc * sum q X s3 -
-// dmn * sum X s3 per 16-value record, sum X being the records' [12] / 8.
-__device__ __forceinline__ float q4k_dot(const uint4 q, const uint32_t* ra, const uint32_t* rb, float dsc,
-                                         float dmn) {
-  const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-  int a = 0, b = 0;
-#pragma unroll
-  for (int l = 0; l < 3; ++l) {
-    const uint4 xa = *reinterpret_cast<const uint4*>(ra + 4 * l);
-    const uint4 xb = *reinterpret_cast<const uint4*>(rb + 4 * l);
-    if (l) {
-      a <<= 7;
-      b <<= 7;
-    }
-    a = sdot4(w[0] & 0x0F0F0F0Fu, (int)xa.x, a);
-    a = sdot4(w[1] & 0x0F0F0F0Fu, (int)xa.y, a);
-    a = sdot4(w[2] & 0x0F0F0F0Fu, (int)xa.z, a);
-    a = sdot4(w[3] & 0x0F0F0F0Fu, (int)xa.w, a);
-    b = sdot4((w[0] >> 4) & 0x0F0F0F0Fu, (int)xb.x, b);
-    b = sdot4((w[1] >> 4) & 0x0F0F0F0Fu, (int)xb.y, b);
-    b = sdot4((w[2] >> 4) & 0x0F0F0F0Fu, (int)xb.z, b);
-    b = sdot4((w[3] >> 4) & 0x0F0F0F0Fu, (int)xb.w, b);
-  }
-  const uint2 ta = *reinterpret_cast<const uint2*>(ra + 12);
-  const uint2 tb = *reinterpret_cast<const uint2*>(rb + 12);
-  const float sa = __uint_as_float(ta.y), sb = __uint_as_float(tb.y);
-  const float qx = fmaf((float)a, sa, (float)b * sb);
-  const float sx = fmaf((float)((int)ta.x >> 3), sa, (float)((int)tb.x >> 3) * sb);
-  return fmaf(dsc, qx, -dmn * sx);
-}
-
 // The K-quants other than Q4_K: a 32-weight block is two 16-weight groups,
 // each with weight = A * c - B (A = d * scale, B = dmin * min, or B = 4 A for
 // Q3_K's codes stored + 4, B = 0 for Q6_K; all exact in fp32). The block's
@@ -410,7 +376,7 @@ __device__ __forceinline__ float q4k_dot(const uint4 q, const uint32_t* ra, cons
 //   Q2_K (quantize.c:180-215)  e = scale byte of each group (scale | min << 4)
 //   Q3_K (:219-263)            e = the groups' 6-bit scales; A = d (s - 32)
 //   Q5_K (:312-346)            e = scale | min << 8, one pair for the block
-//   Q4_K (:265-310)            as Q5_K (the prompt products; the matvec uses q4k_dot)
+//   Q4_K (:265-310)            as Q5_K (the prompt products; the matvec forms it from nibbles)
 //   Q6_K (:350-383)            e = the groups' int8 scales
 template <int QT>
 __device__ __forceinline__ void kq_affine(uint32_t e, uint32_t sup, float (&A)[2], float (&B)[2]) {
@@ -432,51 +398,6 @@ __device__ __forceinline__ void kq_affine(uint32_t e, uint32_t sup, float (&A)[2
       B[g] = 0.f;
     }
   }
-}
-
-// sum over one 16-value record of code * X, exact: X = 16384 q1 + 128 q2 + q3
-// from the record's three int8 levels; nibble codes (w[i] & 0x0F0F0F0F or
-// >> 4) or int8 codes (|code| <= 32 keeps the sum inside int32)
-template <bool NIB, bool HIGH>
-__device__ __forceinline__ int rec_sum(const uint32_t (&w)[4], const uint32_t* r) {
-  int a = 0;
-#pragma unroll
-  for (int l = 0; l < 3; ++l) {
-    const uint4 x = *reinterpret_cast<const uint4*>(r + 4 * l);
-    if (l) a <<= 7;
-    const uint32_t xs[4] = {x.x, x.y, x.z, x.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t c = NIB ? (HIGH ? (w[i] >> 4) & 0x0F0F0F0Fu : w[i] & 0x0F0F0F0Fu) : w[i];
-      a = sdot4(c, (int)xs[i], a);
-    }
-  }
-  return a;
-}
-
-// One 32-weight block of a K-quant other than Q4_K: sum over both groups of
-// A * (sum c X) s3 - B * (sum X) s3, sum X being the record's word 12 / 8.
-template <int QT>
-__device__ __forceinline__ float kq_dot(const uint4 qa, const uint4 qb, const uint32_t* ra, const uint32_t* rb,
-                                        uint32_t e, uint32_t sup) {
-  float A[2], B[2];
-  kq_affine<QT>(e, sup, A, B);
-  int a, b;
-  if constexpr (QT == 10 || QT == 11) {   // nibbles: weight j low, j + 16 high
-    const uint32_t w[4] = {qa.x, qa.y, qa.z, qa.w};
-    a = rec_sum<true, false>(w, ra);
-    b = rec_sum<true, true>(w, rb);
-  } else {                                // int8 codes: 16 per record
-    const uint32_t wa[4] = {qa.x, qa.y, qa.z, qa.w}, wb[4] = {qb.x, qb.y, qb.z, qb.w};
-    a = rec_sum<false, false>(wa, ra);
-    b = rec_sum<false, false>(wb, rb);
-  }
-  const uint2 ta = *reinterpret_cast<const uint2*>(ra + 12);
-  const uint2 tb = *reinterpret_cast<const uint2*>(rb + 12);
-  const float sa = __uint_as_float(ta.y), sb = __uint_as_float(tb.y);
-  const float qx = fmaf(A[0], (float)a * sa, A[1] * ((float)b * sb));
-  const float sx = fmaf(B[0], (float)((int)ta.x >> 3) * sa, B[1] * ((float)((int)tb.x >> 3) * sb));
-  return qx - sx;
 }
 
 // Q8_0 block (quantize.c:139-149: 32 int8 codes, value d * code); levels 1-2
@@ -507,19 +428,6 @@ __device__ __forceinline__ float q8_dot(const uint4 qa, const uint4 qb, const ui
   }
   const float sa3 = __uint_as_float(ra[13]), sb3 = __uint_as_float(rb[13]);
   return fmaf(fmaf((float)a12, 128.0f, (float)a3), sa3, fmaf((float)b12, 128.0f, (float)b3) * sb3);
-}
-
-// Q5_1 block (quantize.c:114-137: weight = q * d + m, q = 0..31, stored as
-// int8 codes): d * sum q X s3 + m * sum X s3 per 16-value record, sum X
-// being the records' [12] / 8.
-__device__ __forceinline__ float q51_dot(const uint4 qa, const uint4 qb, const uint32_t* ra, const uint32_t* rb,
-                                         float d, float m) {
-  const float qx = q8_dot(qa, qb, ra, rb);
-  const uint2 ta = *reinterpret_cast<const uint2*>(ra + 12);
-  const uint2 tb = *reinterpret_cast<const uint2*>(rb + 12);
-  const float sx = fmaf((float)((int)ta.x >> 3), __uint_as_float(ta.y),
-                        (float)((int)tb.x >> 3) * __uint_as_float(tb.y));
-  return fmaf(d, qx, m * sx);
 }
 
 

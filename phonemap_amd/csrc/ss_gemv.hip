@@ -343,20 +343,26 @@ __device__ __forceinline__ void load_round(Round<QT, NMAT, UT>& f, const GemvArg
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 
-// Q4_0 and Q8_0 tiles on the matrix cores. Lane l holds block l/16 of row
-// l%16 (Q4_0: weight j in the low nibble of byte j and weight j+16 in its
-// high nibble; Q8_0: weights 0-15, then 16-31, as int8). Each 16-value half
-// of the tile is one v_mfma_i32_16x16x64_i8: lane l gives its half's 16
-// weights as column l%16 of B at k = 16(l/16) .. +15, and A is block
-// diagonal, row 4b + i holding level i of block b's x record at the same k
-// (lanes l%16 = 4(l/16) + i, i < 3; every other lane gives zeros), so
+// The block types' tiles on the matrix cores (all but F16 / F32). Lane l holds
+// block l/16 of row l%16 (nibble types: weight j in the low nibble of byte j
+// and weight j+16 in its high nibble; the others: codes 0-15, then 16-31, as
+// int8). Each 16-value half of the tile is one v_mfma_i32_16x16x64_i8: lane l
+// gives its half's 16 codes as column l%16 of B at k = 16(l/16) .. +15, and A
+// is block diagonal, row 4b + i holding level i of block b's x record at the
+// same k (lanes l%16 = 4(l/16) + i, i < 3; every other lane gives zeros), so
 // D[4b + i][n], register i of lane l, is the lane's own level-i sum over its
-// half: the integers the sdot4 form (q4_dot, q8_dot) adds, combined the same
-// way, so the results are bit for bit the same. zero: kZeroPad<UT> zero
-// words in LDS (the A rows of the other lanes: every tile's offset from it
-// stays inside it, so the addresses differ by constants alone).
+// half: the integers that v_dot4 over the records would add, combined the
+// same way, so the results are bit for bit those of the dot-product form.
+// The vector units bound that form for the K-quants: 24 v_dot4 a block on top
+// of unpacking. Q4_K gate and up of 14336 x 4096: 16.5 us with v_dot4, 13.9
+// here (4.9 TB/s); Q6_K 4096 x 14336 14.8 and 13.1 (4.9 TB/s of its int8
+// codes). zero: kZeroPad<UT> zero words in LDS (the A rows of the other lanes:
+// every tile's offset from it stays inside it, so the addresses differ by
+// constants alone).
 template <int UT>
 constexpr int kZeroPad = ((UT - 1) * kTB * kXW + kRW + 4 + 3) / 4 * 4;
+
+constexpr bool nibble_codes(int t) { return t == 2 || t == kQ4_1 || t == kQ4K || t == kQ2K || t == kQ3K; }
 
 template <int QT, int NMAT, int UT>
 __device__ __forceinline__ void mfma_round(float (&acc)[NMAT], const Round<QT, NMAT, UT>& f, const int* xs,
@@ -376,10 +382,10 @@ __device__ __forceinline__ void mfma_round(float (&acc)[NMAT], const Round<QT, N
     const uint2 tb = *reinterpret_cast<const uint2*>(ra + kRW + 12);
 #pragma unroll
     for (int m = 0; m < NMAT; ++m) {
-      const uint32_t sw = f.sc[m][k / 2];
-      const uint32_t e = k & 1 ? sw >> 16 : sw & 0xffffu;
+      const uint32_t sw = f.sc[m][is_wide(QT) ? k : k / 2];
+      const uint32_t e = is_wide(QT) ? sw : k & 1 ? sw >> 16 : sw & 0xffffu;
       v4i blo, bhi;
-      if constexpr (QT == 2) {
+      if constexpr (nibble_codes(QT)) {
         const uint4 q = f.q[m][k][0];
         blo = v4i{(int)(q.x & 0x0F0F0F0Fu), (int)(q.y & 0x0F0F0F0Fu), (int)(q.z & 0x0F0F0F0Fu),
                   (int)(q.w & 0x0F0F0F0Fu)};
@@ -387,21 +393,48 @@ __device__ __forceinline__ void mfma_round(float (&acc)[NMAT], const Round<QT, N
                   (int)((q.z >> 4) & 0x0F0F0F0Fu), (int)((q.w >> 4) & 0x0F0F0F0Fu)};
       } else {
         blo = __builtin_bit_cast(v4i, f.q[m][k][0]);
-        bhi = __builtin_bit_cast(v4i, f.q[m][k][1]);
+        bhi = __builtin_bit_cast(v4i, f.q[m][k][Round<QT, NMAT, UT>::kNV - 1]);
       }
       const v4i dl = __builtin_amdgcn_mfma_i32_16x16x64_i8(alo, blo, z, 0, 0, 0);
       const v4i dh = __builtin_amdgcn_mfma_i32_16x16x64_i8(ahi, bhi, z, 0, 0, 0);
-      float s;
-      if constexpr (QT == 2) {   // q4_dot: sum X * nibble - 8 sum X, |.| < 2^31 per half
+      const float sa = __uint_as_float(ta.y), sb = __uint_as_float(tb.y);
+      if constexpr (QT == 8 || QT == kQ5_1 || QT == kQ8_1) {
+        // levels 1-2 in one integer (|.| < 2^31), level 3 added in fp32
+        const int a12 = (dl[0] << 7) + dl[1], b12 = (dh[0] << 7) + dh[1];
+        const float s = fmaf(fmaf((float)a12, 128.0f, (float)dl[2]), sa, fmaf((float)b12, 128.0f, (float)dh[2]) * sb);
+        if constexpr (QT == kQ5_1) {   // d * q + m (quantize.c:114-137); the records' word 12 is 8 * sum X
+          const float sx = fmaf((float)((int)ta.x >> 3), sa, (float)((int)tb.x >> 3) * sb);
+          acc[m] += fmaf(h2f((uint16_t)(e & 0xffffu)), s, h2f((uint16_t)(e >> 16)) * sx);
+        } else {
+          acc[m] = fmaf(QT == kQ8_1 ? __uint_as_float(e) : h2f((uint16_t)e), s, acc[m]);
+        }
+      } else {                         // |sum code * X| < 2^31 per half
         const int a = (dl[0] << 14) + (dl[1] << 7) + dl[2];
         const int b = (dh[0] << 14) + (dh[1] << 7) + dh[2];
-        s = fmaf((float)(a - (int)ta.x), __uint_as_float(ta.y), (float)(b - (int)tb.x) * __uint_as_float(tb.y));
-      } else {                   // q8_dot: levels 1-2 in one integer, level 3 added in fp32
-        const int a12 = (dl[0] << 7) + dl[1], b12 = (dh[0] << 7) + dh[1];
-        s = fmaf(fmaf((float)a12, 128.0f, (float)dl[2]), __uint_as_float(ta.y),
-                 fmaf((float)b12, 128.0f, (float)dh[2]) * __uint_as_float(tb.y));
+        if constexpr (QT == 2) {       // sum X * nibble - 8 sum X (quantize.c:60-72)
+          const float s = fmaf((float)(a - (int)ta.x), sa, (float)(b - (int)tb.x) * sb);
+          acc[m] = fmaf(h2f((uint16_t)e), s, acc[m]);
+        } else if constexpr (QT == kQ4K || QT == kQ4_1) {   // dsc * q - dmn (quantize.c:265-310; Q4_1: d, -m)
+          float dsc, dmn;
+          if constexpr (QT == kQ4K) {
+            const uint32_t sup = f.su[m][k / 2];
+            dsc = h2f((uint16_t)(sup & 0xffffu)) * (float)(e & 0xffu);   // exact
+            dmn = h2f((uint16_t)(sup >> 16)) * (float)(e >> 8);
+          } else {
+            dsc = h2f((uint16_t)(e & 0xffffu));
+            dmn = -h2f((uint16_t)(e >> 16));
+          }
+          const float qx = fmaf((float)a, sa, (float)b * sb);
+          const float sx = fmaf((float)((int)ta.x >> 3), sa, (float)((int)tb.x >> 3) * sb);
+          acc[m] += fmaf(dsc, qx, -dmn * sx);
+        } else {                       // an (A, B) pair per 16 weights
+          float A[2], B[2];
+          kq_affine<QT>(e, f.su[m][k / 2], A, B);
+          const float qx = fmaf(A[0], (float)a * sa, A[1] * ((float)b * sb));
+          const float sx = fmaf(B[0], (float)((int)ta.x >> 3) * sa, B[1] * ((float)((int)tb.x >> 3) * sb));
+          acc[m] += qx - sx;
+        }
       }
-      acc[m] = fmaf(h2f((uint16_t)e), s, acc[m]);
     }
   }
 }
@@ -413,42 +446,14 @@ __device__ __forceinline__ void mfma_round(float (&acc)[NMAT], const Round<QT, N
 template <int QT, int NMAT, int UT>
 __device__ __forceinline__ void fma_round(float (&acc)[NMAT], const Round<QT, NMAT, UT>& f, const int* xs,
                                           int kb, const int* zero, int lane) {
-  if constexpr (QT == 2 || QT == 8) {
+  if constexpr (is_float(QT)) {
+#pragma unroll
+    for (int k = 0; k < UT; ++k)
+#pragma unroll
+      for (int m = 0; m < NMAT; ++m)
+        acc[m] += float_dot<QT>(f.q[m][k], reinterpret_cast<const float*>(xs + (k * kTB + kb) * kXW));
+  } else {
     mfma_round<QT, NMAT, UT>(acc, f, xs, zero, lane);
-    return;
-  }
-#pragma unroll
-  for (int k = 0; k < UT; ++k) {
-    const uint32_t* ra = reinterpret_cast<const uint32_t*>(xs + (k * kTB + kb) * kXW);
-#pragma unroll
-    for (int m = 0; m < NMAT; ++m) {
-      const uint32_t sw = f.sc[m][is_wide(QT) ? k : k / 2];
-      const uint32_t e = is_wide(QT) ? sw : k & 1 ? sw >> 16 : sw & 0xffffu;
-      if constexpr (is_float(QT)) {
-        acc[m] += float_dot<QT>(f.q[m][k], reinterpret_cast<const float*>(ra));
-      } else if constexpr (QT == kQ4_1) {   // d * q + m: Q4_K's dot with dsc = d, dmn = -m
-        acc[m] += q4k_dot(f.q[m][k][0], ra, ra + kRW, h2f((uint16_t)(e & 0xffffu)), -h2f((uint16_t)(e >> 16)));
-      } else if constexpr (QT == kQ5_1) {
-        acc[m] += q51_dot(f.q[m][k][0], f.q[m][k][1], ra, ra + kRW, h2f((uint16_t)(e & 0xffffu)),
-                          h2f((uint16_t)(e >> 16)));
-      } else if constexpr (QT == kQ8_1) {
-        acc[m] = fmaf(__uint_as_float(e), q8_dot(f.q[m][k][0], f.q[m][k][1], ra, ra + kRW), acc[m]);
-      } else if constexpr (QT == kQ4K) {
-        const uint32_t sup = f.su[m][k / 2];
-        const float dsc = h2f((uint16_t)(sup & 0xffffu)) * (float)(e & 0xffu);   // exact
-        const float dmn = h2f((uint16_t)(sup >> 16)) * (float)(e >> 8);
-        acc[m] += q4k_dot(f.q[m][k][0], ra, ra + kRW, dsc, dmn);
-      } else if constexpr (is_kq(QT)) {
-        acc[m] += kq_dot<QT>(f.q[m][k][0], f.q[m][k][Round<QT, NMAT, UT>::kNV - 1], ra, ra + kRW, e, f.su[m][k / 2]);
-      } else {
-        float s;
-        if constexpr (QT == 2)
-          s = q4_dot(f.q[m][k][0], ra, ra + kRW);
-        else
-          s = q8_dot(f.q[m][k][0], f.q[m][k][1], ra, ra + kRW);
-        acc[m] = fmaf(h2f((uint16_t)e), s, acc[m]);
-      }
-    }
   }
 }
 
@@ -612,15 +617,15 @@ constexpr int kMergeNone = 0, kMergeEarly = 1, kMergeLate = 2;
 template <int QT, int NMAT, int EPI, int UT, int MERGE, bool PX, int NR>
 __global__ void __launch_bounds__((gemv_max_waves<QT, NMAT>() * 64)) k_gemv(const GemvArgs a) {
   extern __shared__ float4 smem4[];
-  // zeros per wave for the matrix-core A rows (Q4_0, Q8_0)
-  __shared__ v4i zpad[gemv_max_waves<QT, NMAT>()][(QT == 2 || QT == 8) ? kZeroPad<UT> / 4 : 1];
+  // zeros per wave for the matrix-core A rows
+  __shared__ v4i zpad[gemv_max_waves<QT, NMAT>()][is_float(QT) ? 1 : kZeroPad<UT> / 4];
   int* xs = reinterpret_cast<int*>(smem4);
   static_assert(NR == 0 || PX, "rounds issued up front take x from the records");
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform (scalar)
   // written by its own wave before any use (fences below order the accesses)
-  if constexpr (QT == 2 || QT == 8) {
+  if constexpr (!is_float(QT)) {
     for (int i = lane; i < kZeroPad<UT> / 4; i += kWave) zpad[wave][i] = v4i{0, 0, 0, 0};
   }
   const int S = blockDim.x >> 6;
@@ -1177,13 +1182,15 @@ hipError_t launch_k(const GemvArgs& a, const GemvPlan& p, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Records path of Q4_0 / Q8_0 matrices with two-tile units whose rows take
-// 2 to 4 units per wave: every unit of a wave requested at once (NR rounds;
-// four-tile units would keep their records in scratch memory).
+// Records path of Q4_0, Q8_0, Q4_K and Q6_K matrices with two-tile units whose
+// rows take 2 to 4 units per wave: every unit of a wave requested at once (NR
+// rounds; four-tile units would keep their records in scratch memory). A token
+// through 12 layers of hidden 2048, ffn 8192: Q4_K 403 us with the loop over
+// units, 386 here; Q6_K 445 and 438.
 template <int QT, int NMAT, int EPI, int MERGE = kMergeNone, bool PX = false, int UT = kGemvUnit>
 hipError_t launch_t(const GemvArgs& a, hipStream_t s) {
   const GemvPlan p = gemv_plan(a.rows, a.cols, QT, NMAT, UT);
-  if constexpr (PX && MERGE == kMergeNone && (QT == 2 || QT == 8) && UT == 2) {   // four-tile units keep their records in scratch
+  if constexpr (PX && MERGE == kMergeNone && (QT == 2 || QT == 8 || QT == kQ4K || QT == kQ6K) && UT == 2) {   // four-tile units keep their records in scratch
     const int ntk = (a.cols / 32 + kTB - 1) / kTB;
     const int S = p.threads / kWave, nr = ((ntk + UT - 1) / UT + S - 1) / S;
     // more rounds per wave (up to 7 for the 8B down projection, fewer and
