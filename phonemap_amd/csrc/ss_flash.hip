@@ -413,7 +413,8 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
       const float mk = gm[k][32 * rt + n];
       lt += mk == -INFINITY ? 0.f : gl[k][32 * rt + n] * __builtin_amdgcn_exp2f(mk - mx);
     }
-    const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mx) / lt * vscale;
+    // (a row whose scores are all -inf keeps its 0 / 0)
+    const float f = (m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mx)) / lt * vscale;
     auto bank = [&](int w) { return w == 0 ? ks0 : w == 1 ? vs0 : w == 2 ? ks1 : vs1; };
     const int tile = wave / DS;
     float4* dst = reinterpret_cast<float4*>(bank(tile / (KG / 2))) + (tile % (KG / 2)) * (32 * HD / 4);

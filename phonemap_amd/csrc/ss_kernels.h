@@ -219,7 +219,8 @@ hipError_t launch_kv_append(void* kc, void* vc, float* ksc, float* vsc, const fl
                             const float* v, int n_kv_heads, int head_dim, int max_seq,
                             const int* dpos, int pos, int kv_type, hipStream_t s);
 // RoPE of the q and k parts of n prompt rows [q | k | v] (stride ld; token z
-// at position dpos[z]) and the fp16 cache append of k and v.
+// at position dpos[z]) and the append of k and v to the fp16 or int8 cache
+// (ksc, vsc: its scales).
 hipError_t launch_rope_kv_rows(float* qkv, const float* bias, int ld, int qdim, int kvdim, int head_dim, int rope_dim,
                                const float* cs, const int* dpos, void* kc, void* vc, float* ksc, float* vsc,
                                int max_seq, int kv_type, int n, hipStream_t s);
