@@ -1182,15 +1182,16 @@ hipError_t launch_k(const GemvArgs& a, const GemvPlan& p, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Records path of Q4_0, Q8_0, Q4_K and Q6_K matrices with two-tile units whose
+// Records path of Q4_0, Q8_0 and K-quant matrices with two-tile units whose
 // rows take 2 to 4 units per wave: every unit of a wave requested at once (NR
 // rounds; four-tile units would keep their records in scratch memory). A token
 // through 12 layers of hidden 2048, ffn 8192: Q4_K 403 us with the loop over
-// units, 386 here; Q6_K 445 and 438.
+// units, 386 here; Q2_K 411 and 397, Q3_K 407 and 393, Q5_K 444 and 441, Q6_K
+// 445 and 438.
 template <int QT, int NMAT, int EPI, int MERGE = kMergeNone, bool PX = false, int UT = kGemvUnit>
 hipError_t launch_t(const GemvArgs& a, hipStream_t s) {
   const GemvPlan p = gemv_plan(a.rows, a.cols, QT, NMAT, UT);
-  if constexpr (PX && MERGE == kMergeNone && (QT == 2 || QT == 8 || QT == kQ4K || QT == kQ6K) && UT == 2) {   // four-tile units keep their records in scratch
+  if constexpr (PX && MERGE == kMergeNone && (QT == 2 || QT == 8 || is_kq(QT)) && UT == 2) {   // four-tile units keep their records in scratch
     const int ntk = (a.cols / 32 + kTB - 1) / kTB;
     const int S = p.threads / kWave, nr = ((ntk + UT - 1) / UT + S - 1) / S;
     // more rounds per wave (up to 7 for the 8B down projection, fewer and

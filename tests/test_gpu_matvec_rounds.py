@@ -15,7 +15,7 @@ from tests.util import rel_err
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("qtype", [12, 14])
+@pytest.mark.parametrize("qtype", [10, 11, 12, 13, 14])
 @pytest.mark.parametrize("hidden,ffn", [(2304, 4352), (2304, 6400), (2048, 8192)])
 def test_decode_steps(qtype, hidden, ffn):
     spec = dict(n_layers=1, hidden=hidden, n_heads=hidden // 64, n_kv_heads=hidden // 256, head_dim=64, ffn=ffn,
