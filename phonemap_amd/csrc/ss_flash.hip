@@ -364,7 +364,14 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
         for (int i = 0; i < 8; ++i) {
           pv[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[8 * c + i], qs, -mo));   // layer_scheduler.c:450-458
           l += pv[i];
-          if (Q8) pv[i] *= scl[g][32 + 16 * c + 8 * h + i];
+          if (Q8) {
+            // rounded to fp32 before it is split: as a factor of the split's
+            // conversions it would give hi two values, one to multiply and
+            // another to take lo from, an fp16 step apart where they round to
+            // different sides
+            pv[i] *= scl[g][32 + 16 * c + 8 * h + i];
+            asm("" : "+v"(pv[i]));
+          }
         }
         split8(pv, ph[c], pl[c]);
       }

@@ -541,6 +541,36 @@ int32_t attention_setup(ss_hip_ctx_t* c, const char* what, ssk::AttnArgs& a, int
   return 0;
 }
 
+int32_t attention_rows(ss_hip_ctx_t* c, float* out, const float* q, const void* kc, const void* vc, const float* ksc,
+                       const float* vsc, int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, int32_t max_seq,
+                       int32_t pos0, int32_t n_tokens, int32_t kv_type, void* stream) {
+  if (!c || !out || !q || !kc || !vc || n_kv_heads <= 0 || n_heads % n_kv_heads || pos0 < 0 || n_tokens <= 0 ||
+      (int64_t)pos0 + n_tokens > max_seq)
+    return fail(kErrParams, "attention_rows: bad argument (pos0 %d, %d tokens, max_seq %d)", pos0, n_tokens,
+                max_seq);
+  const int group = n_heads / n_kv_heads;
+  if (!ssk::attention_supported(head_dim, group))
+    return fail(kErrParams, "attention_rows: head_dim %d / group %d not supported", head_dim, group);
+  if (set_device(c)) return kErrBackend;
+  ssk::AttnArgs a;
+  memset(&a, 0, sizeof(a));
+  a.q = q;
+  a.kc = kc;
+  a.vc = vc;
+  a.ks = ksc;
+  a.vs = vsc;
+  a.max_seq = max_seq;
+  a.ns = 1;
+  a.n_kv_heads = n_kv_heads;
+  a.scale = 1.0f / sqrtf((float)head_dim);
+  a.out = out;
+  a.n_tok = n_tokens;
+  a.pos0 = pos0;
+  a.tok_q = a.tok_o = n_heads * head_dim;
+  HIP_TRY(ssk::launch_attention_rows(head_dim, group, kv_type, a, pick(c, stream)));
+  return 0;
+}
+
 size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 }  // namespace
@@ -572,29 +602,16 @@ int32_t ss_hip_attention(ss_hip_ctx_t* c, float* out, const float* q, const void
 int32_t ss_hip_attention_rows(ss_hip_ctx_t* c, float* out, const float* q, const void* kc, const void* vc,
                               int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, int32_t max_seq,
                               int32_t pos0, int32_t n_tokens, void* stream) {
-  if (!c || !out || !q || !kc || !vc || n_kv_heads <= 0 || n_heads % n_kv_heads || pos0 < 0 || n_tokens <= 0 ||
-      (int64_t)pos0 + n_tokens > max_seq)
-    return fail(kErrParams, "attention_rows: bad argument (pos0 %d, %d tokens, max_seq %d)", pos0, n_tokens,
-                max_seq);
-  const int group = n_heads / n_kv_heads;
-  if (!ssk::attention_supported(head_dim, group))
-    return fail(kErrParams, "attention_rows: head_dim %d / group %d not supported", head_dim, group);
-  if (set_device(c)) return kErrBackend;
-  ssk::AttnArgs a;
-  memset(&a, 0, sizeof(a));
-  a.q = q;
-  a.kc = kc;
-  a.vc = vc;
-  a.max_seq = max_seq;
-  a.ns = 1;
-  a.n_kv_heads = n_kv_heads;
-  a.scale = 1.0f / sqrtf((float)head_dim);
-  a.out = out;
-  a.n_tok = n_tokens;
-  a.pos0 = pos0;
-  a.tok_q = a.tok_o = n_heads * head_dim;
-  HIP_TRY(ssk::launch_attention_rows(head_dim, group, 0, a, pick(c, stream)));
-  return 0;
+  return attention_rows(c, out, q, kc, vc, nullptr, nullptr, n_heads, n_kv_heads, head_dim, max_seq, pos0, n_tokens,
+                        SS_HIP_KV_F16, stream);
+}
+
+int32_t ss_hip_attention_rows_int8(ss_hip_ctx_t* c, float* out, const float* q, const void* kc, const void* vc,
+                                   const float* ksc, const float* vsc, int32_t n_heads, int32_t n_kv_heads,
+                                   int32_t head_dim, int32_t max_seq, int32_t pos0, int32_t n_tokens, void* stream) {
+  if (!ksc || !vsc) return fail(kErrParams, "attention_rows: no scales");
+  return attention_rows(c, out, q, kc, vc, ksc, vsc, n_heads, n_kv_heads, head_dim, max_seq, pos0, n_tokens,
+                        SS_HIP_KV_INT8, stream);
 }
 
 int32_t ss_hip_attention_noalloc(ss_hip_ctx_t* c, float* out, const float* q, const void* kc,
