@@ -174,14 +174,6 @@ int32_t ss_hip_attention_rows(ss_hip_ctx_t *ctx, float *out_dev, const float *q_
                               int32_t n_kv_heads, int32_t head_dim, int32_t max_seq, int32_t pos0,
                               int32_t n_tokens, void *stream);
 
-/* The same over one layer's int8 cache with its per-position scales, as
- * ss_hip_eval_prompt runs it for a model with that cache. */
-int32_t ss_hip_attention_rows_int8(ss_hip_ctx_t *ctx, float *out_dev, const float *q_dev,
-                                   const void *k_cache, const void *v_cache, const float *k_scale,
-                                   const float *v_scale, int32_t n_heads, int32_t n_kv_heads,
-                                   int32_t head_dim, int32_t max_seq, int32_t pos0,
-                                   int32_t n_tokens, void *stream);
-
 /* ss_hip_attention with no device allocation. No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving loops, harnesses that forbid

@@ -606,6 +606,9 @@ int32_t ss_hip_attention_rows(ss_hip_ctx_t* c, float* out, const float* q, const
                         SS_HIP_KV_F16, stream);
 }
 
+// The same over given codes and scales of an int8 cache, as ss_hip_eval_prompt
+// runs it for a model with that cache. Not in the public header: it holds that
+// kernel to 64 bits without a model around it.
 int32_t ss_hip_attention_rows_int8(ss_hip_ctx_t* c, float* out, const float* q, const void* kc, const void* vc,
                                    const float* ksc, const float* vsc, int32_t n_heads, int32_t n_kv_heads,
                                    int32_t head_dim, int32_t max_seq, int32_t pos0, int32_t n_tokens, void* stream) {
