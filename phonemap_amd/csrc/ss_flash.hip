@@ -47,10 +47,16 @@
 // ds_read_b64_tr_b16 (lane i of 16 addresses key i/4, dims 4(i%4)..+3, and
 // receives dim i of the four keys). Both swizzles spread a read over all banks.
 
+//
 // An int8 cache's codes are exact in fp16: a block passes through registers,
 // where codes become fp16 (requested before the current block's products,
 // written to LDS after them), a position's K scale multiplies its scores and
-// its V scale the weights after the row's sum took them.
+// its V scale the weights after the row's sum took them. Weight times V scale
+// has no bound of its own, so each row also keeps the binary exponent of its
+// largest one (lagging by 2 at most) and holds P, and so O, relative to that:
+// a row's precision depends on the positions it sees alone. Maxima are whole
+// numbers there, so that moving either is exact. A position the row does not
+// see has V scale 0 (its own may be infinite).
 
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -75,6 +81,7 @@ constexpr int kCompute = 256;       // compute units
 constexpr float kLog2e = 1.44269504088896340736f;
 constexpr float kPExp = 12.0f;      // P is held times 2^12
 constexpr float kLag = 3.0f;        // the running maximum's lag (base 2)
+constexpr float kLagX = 2.0f;       // int8: the lag of the exponent of weight times V scale
 
 // the value of the lane with the same query row (lane ^ 32) joined to this one's
 __device__ __forceinline__ float max_pair(float v) {
@@ -85,14 +92,11 @@ __device__ __forceinline__ float sum_pair(float v) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
-__device__ __forceinline__ int wave_max_int(int v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, kWave));
-  return __builtin_amdgcn_readfirstlane(v);
-}
+// 2^e of a whole number (or -inf: 0)
+__device__ __forceinline__ float pow2(float e) { return ldexpf(1.0f, (int)fmaxf(e, -200.f)); }
 
 // hi + lo = v (to 2^-22 of |v| for normal values) as two fp16 vectors
-__device__ __forceinline__ void split8(const float (&v)[8], v8h& hi, v8h& lo) {
+__device__ __forceinline__ void split8(const float* v, v8h& hi, v8h& lo) {
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const _Float16 h = (_Float16)v[i];
@@ -140,7 +144,6 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
   __shared__ v4u vs0[KG * kGrp], vs1[KG * kGrp];
   __shared__ float xs[DS > 1 ? RT * KG * DS : 1][DS > 1 ? 16 * 64 : 1];   // the waves' shares of S^T
   __shared__ float sc0[Q8 ? KG : 1][64], sc1[Q8 ? KG : 1][64];   // int8: the block's K scales, then its V scales
-  __shared__ float vred[RT * KG * DS];
   __shared__ float gm[KG][RT * 32], gl[KG][RT * 32];   // each group's maximum and sum of a row
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -220,7 +223,6 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
     }
     qsc = (h ? a.vs : a.ks)[min(kb + n, ctx - 1)];
   };
-  float vnorm = 1.f, vscale = 1.f;
   auto store_q = [&](int step, v4u* kd, v4u* vd, float (*scd)[64]) {
     if ((step * KG + g) * kBlk >= ctx) return;
 #pragma unroll
@@ -234,7 +236,7 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
       vr[c ^ vswz<CH>(r)] = codes8(vq[k][0], vq[k][1]);
       vr[(c + 1) ^ vswz<CH>(r)] = codes8(vq[k][2], vq[k][3]);
     }
-    if (rt == 0 && ds == 0) scd[g][lane] = h ? qsc * vnorm : qsc;
+    if (rt == 0 && ds == 0) scd[g][lane] = qsc;
   };
   // the staged loads have landed and the other buffer's reads are done, for
   // this wave, and for the others where waves share the staging
@@ -245,22 +247,6 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
 
   if (Q8) {
     load_q(0);
-    // the V scales by the power of two of the largest one, so that P times
-    // them keeps its two fp16 parts (a scale 2^-k of the largest loses bits
-    // below 2^-37 of the largest)
-    float vm = 0.f;
-    for (int p = tid; p < ctx; p += NT) vm = fmaxf(vm, a.vs[p]);
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) vm = fmaxf(vm, __shfl_xor(vm, off, kWave));
-    if (lane == 0) vred[wave] = vm;
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < NT / 64; ++w) vm = fmaxf(vm, vred[w]);
-    int e = 0;
-    frexpf(vm, &e);
-    e = min(max(e, -120), 120);
-    vnorm = ldexpf(1.0f, -e);
-    vscale = ldexpf(1.0f, e);
     store_q(0, ks0, vs0, sc0);
   } else {
     stage(0, ks0, vs0);
@@ -298,7 +284,8 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
   v16f o[NDT];
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt) o[dt] = v16f{};
-  float m = -INFINITY, l = 0.f;   // l: this lane's share of the row's sum, times 2^12
+  float m = -INFINITY, l = 0.f;   // l: this lane's share of the row's sum, times 2^12 (int8: the sum)
+  float ex = -INFINITY;           // int8: the exponent O is held relative to, times 2^12
 
   // transposed V read: lane's key of 4 and its 8 bytes of a 32-dim tile
   const int vkey = 8 * h + ((lane >> 2) & 3);
@@ -334,6 +321,11 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
       float sc[16];
 #pragma unroll
       for (int j = 0; j < 16; ++j) sc[j] = Q8 ? acc[j] * scl[g][16 * (j / 8) + 8 * h + j % 8] : acc[j];
+      float vsc[Q8 ? 16 : 1];
+      if constexpr (Q8) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) vsc[j] = scl[g][32 + 16 * (j / 8) + 8 * h + j % 8];
+      }
       if (cap) {   // (q . k) / sqrt(hd), softcapped (layer_scheduler.c:442-448)
 #pragma unroll
         for (int j = 0; j < 16; ++j) sc[j] = softcap(sc[j] * qscale, a) * kLog2e;
@@ -341,40 +333,63 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
       if (kb + kBlk - 1 > wmin) {   // causal limit
 #pragma unroll
         for (int j = 0; j < 16; ++j)
-          if (kb + 16 * (j / 8) + 8 * h + j % 8 > lim) sc[j] = -INFINITY;
+          if (kb + 16 * (j / 8) + 8 * h + j % 8 > lim) {
+            sc[j] = -INFINITY;
+            if constexpr (Q8) vsc[j] = 0.f;
+          }
       }
       float bmax = sc[0];
 #pragma unroll
       for (int j = 1; j < 16; ++j) bmax = fmaxf(bmax, sc[j]);
       bmax = max_pair(bmax) * qs;
       if (__any(bmax > m + kLag)) {
-        const float mn = fmaxf(m, bmax);
-        const float corr = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
+        const float mn = Q8 ? ceilf(fmaxf(m, bmax)) : fmaxf(m, bmax);
+        const float by = m - (mn == -INFINITY ? 0.f : mn);
+        const float corr = Q8 ? pow2(by) : __builtin_amdgcn_exp2f(by);
         l *= corr;
+        if constexpr (!Q8) {
 #pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) o[dt] *= corr;
+          for (int dt = 0; dt < NDT; ++dt) o[dt] *= corr;
+        }
         m = mn;
       }
-      const float mo = (m == -INFINITY ? 0.f : m) - kPExp;   // nothing seen yet: weights stay 0
-      v8h ph[2], pl[2];
+      const float mo = (m == -INFINITY ? 0.f : m) - (Q8 ? 0.f : kPExp);   // nothing seen yet: weights stay 0
+      float pv[16];
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        float pv[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          pv[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[8 * c + i], qs, -mo));   // layer_scheduler.c:450-458
-          l += pv[i];
-          if (Q8) {
-            // rounded to fp32 before it is split: as a factor of the split's
-            // conversions it would give hi two values, one to multiply and
-            // another to take lo from, an fp16 step apart where they round to
-            // different sides
-            pv[i] *= scl[g][32 + 16 * c + 8 * h + i];
-            asm("" : "+v"(pv[i]));
-          }
-        }
-        split8(pv, ph[c], pl[c]);
+      for (int j = 0; j < 16; ++j) {
+        pv[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j], qs, -mo));   // layer_scheduler.c:450-458
+        l += pv[j];
       }
+      if constexpr (Q8) {
+        float bx = 0.f;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          pv[j] *= vsc[j];
+          bx = fmaxf(bx, pv[j]);
+        }
+        bx = max_pair(bx);   // below 2^(e + 1)
+        const float t = m + (float)max((int)(__float_as_uint(bx) >> 23) - 127, -100);
+        if (__any(bx > 0.f && t > ex + kLagX)) {
+          const float en = bx > 0.f ? fmaxf(ex, t) : ex;
+          const float corr = en == ex ? 1.f : pow2(ex - en);
+#pragma unroll
+          for (int dt = 0; dt < NDT; ++dt) o[dt] *= corr;
+          ex = en;
+        }
+        const int up = (int)fminf(kPExp + m - ex, 126.f);   // (past 126 with every pv 0 only)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          pv[j] = ldexpf(pv[j], up);
+          // rounded to fp32 before it is split: as a factor of the split's
+          // conversions it would give hi two values, one to multiply and
+          // another to take lo from, an fp16 step apart where they round to
+          // different sides
+          asm("" : "+v"(pv[j]));
+        }
+      }
+      v8h ph[2], pl[2];
+      split8(pv, ph[0], pl[0]);
+      split8(pv + 8, ph[1], pl[1]);
       // O^T += V^T P^T
 #pragma unroll
       for (int c = 0; c < 2; ++c)
@@ -421,7 +436,7 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
       lt += mk == -INFINITY ? 0.f : gl[k][32 * rt + n] * __builtin_amdgcn_exp2f(mk - mx);
     }
     // (a row whose scores are all -inf keeps its 0 / 0)
-    const float f = (m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mx)) / lt * vscale;
+    const float f = (m == -INFINITY ? 0.f : Q8 ? pow2(ex - kPExp - mx) : __builtin_amdgcn_exp2f(m - mx)) / lt;
     auto bank = [&](int w) { return w == 0 ? ks0 : w == 1 ? vs0 : w == 2 ? ks1 : vs1; };
     const int tile = wave / DS;
     float4* dst = reinterpret_cast<float4*>(bank(tile / (KG / 2))) + (tile % (KG / 2)) * (32 * HD / 4);

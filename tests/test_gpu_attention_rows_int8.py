@@ -74,3 +74,25 @@ def test_rows_against_64_bits(hip, H, KVH, hd, pos0, n):
     err = _row_err(_rows(hip, *c, pos0), _exact(*c, pos0))
     print("worst row %.2e, all rows %.2e" % (err.max(), np.sqrt(np.mean(err ** 2))), flush=True)
     assert err.max() <= TOL
+
+
+@pytest.mark.parametrize("H,KVH,hd,pos0,n", SHAPES)
+@pytest.mark.parametrize("last", [1e6, np.inf])
+def test_rows_do_not_depend_on_later_scales(hip, H, KVH, hd, pos0, n, last):
+    """V scales spread over 8 decades, each position's above the next one's by
+    chance only, and the last position's far above all (or infinite): the rows
+    before it do not see it."""
+    print("int8 attention rows, wide scales", H, KVH, hd, pos0, n, last, flush=True)
+    q, k, v, ks, vs = _case(H, KVH, hd, pos0, n, 1000 + H + hd + pos0 + n)
+    vs *= 10.0 ** np.random.default_rng(n).uniform(-8, 0, vs.size).astype(np.float32)
+    vs[pos0 + n - 1] = last
+    got = _rows(hip, q, k, v, ks, vs, pos0)
+    if np.isinf(last):
+        # weight * inf * code in every element (0 codes: NaN)
+        assert not np.isfinite(got[-1]).any()
+        got, q, vs = got[:-1], q[:-1], vs.copy()
+    else:
+        assert np.isfinite(got).all()
+    err = _row_err(got, _exact(q, k, v, ks, vs, pos0))
+    print("worst row %.2e" % err.max(), flush=True)
+    assert err.max() <= TOL
