@@ -18,14 +18,26 @@
 // are then keys 16c + 8h + 0..7 of query row n, the B layout. A row's softmax
 // statistics live in lanes n and n + 32 (one v_permlane32_swap per reduction).
 //
-// Precision: K and V are fp16 in the cache (exact MFMA operands). q is
-// scaled per row by a power of two (its largest magnitude to [2^13, 2^14))
-// and split into two fp16 parts, hi + lo = q to 2^-22; P (times 2^12) is split
-// the same way; each product is two MFMAs accumulating in fp32. The softmax is
-// the online form (running maximum and sum per row) in fp32, in base 2: the
-// scores' scale carries log2(e), rounded once like 1/sqrt(hd) itself. The
-// running maximum may lag the true one by up to 3 (P <= 2^3: 2^15 after the
-// scale, inside fp16's range), so most blocks skip rescaling O.
+// Precision: K and V are fp16 in the cache (exact MFMA operands). q, times the
+// softmax's scale and log2(e) (that product to 2^-48), is scaled per row by a
+// power of two (its largest magnitude to [2^13, 2^14)) and held as two fp16
+// parts, to 2^-23 of the value; P (times 2^12) is held the same way; each
+// product is two MFMAs accumulating in fp32. The softmax is the online form
+// (running maximum and sum per row) in fp32, in base 2; maxima are whole
+// numbers, so moving one is exact, and one may lag the true maximum by up to 3
+// (P <= 2^3: 2^15 after the scale, inside fp16's range), so most blocks skip
+// rescaling O. What else rounds are the sums, in two forms. FULL adds a
+// score's high parts in two chains and a block's share of O from zero: each
+// sum rounds a few times per block, and over 4 to 7 tokens (fp16) and 4 to 64
+// (int8), contexts 4 to 4008 and every head dimension its error against 64
+// bits is that of the attention of single tokens, which sums in fp32
+// throughout (0.98 and 0.89 of it, geometric means; 1.8 and 1.4 with one chain
+// of sixteen MFMAs per score, a scale rounded to fp32 and weights' exponents
+// up to 15). It is used where such tokens would otherwise be attended one by
+// one. The other form runs longer fp16 prompts: the score's parts in one
+// chain, the low ones first, and O one chain over all blocks (1.2 of that
+// error, up to 1.8 at 4000 positions; 100 tokens over 3000, 32 heads on 8,
+// head_dim 128: 38 us, FULL 43).
 //
 // Bound and split. At 32 rows per wave one LDS operand read feeds two MFMAs of
 // 32 cycles, so a block is 1024 matrix cycles per wave at head_dim 128 against
@@ -46,7 +58,6 @@
 // V rows as they are (chunk c at slot c ^ vswz(key)), read transposed by
 // ds_read_b64_tr_b16 (lane i of 16 addresses key i/4, dims 4(i%4)..+3, and
 // receives dim i of the four keys). Both swizzles spread a read over all banks.
-
 //
 // An int8 cache's codes are exact in fp16: a block passes through registers,
 // where codes become fp16 (requested before the current block's products,
@@ -54,9 +65,8 @@
 // its V scale the weights after the row's sum took them. Weight times V scale
 // has no bound of its own, so each row also keeps the binary exponent of its
 // largest one (lagging by 2 at most) and holds P, and so O, relative to that:
-// a row's precision depends on the positions it sees alone. Maxima are whole
-// numbers there, so that moving either is exact. A position the row does not
-// see has V scale 0 (its own may be infinite).
+// a row's precision depends on the positions it sees alone. A position the row
+// does not see has V scale 0 (its own may be infinite).
 
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -78,8 +88,9 @@ typedef __attribute__((address_space(1))) void* gbl_ptr_t;
 
 constexpr int kBlk = 32;            // keys per block, query rows per tile
 constexpr int kCompute = 256;       // compute units
-constexpr float kLog2e = 1.44269504088896340736f;
-constexpr float kPExp = 12.0f;      // P is held times 2^12
+constexpr int kFullRows = 8;        // fp16 launches of fewer tokens sum in the FULL form
+constexpr float kLog2e = 1.44269504088896340736f, kLog2eLow = 1.92596299e-8f;   // log2 e = their sum
+constexpr float kPExp = 12.0f, kPScale = 4096.0f;   // P is held times 2^12
 constexpr float kLag = 3.0f;        // the running maximum's lag (base 2)
 constexpr float kLagX = 2.0f;       // int8: the lag of the exponent of weight times V scale
 
@@ -95,7 +106,7 @@ __device__ __forceinline__ float sum_pair(float v) {
 // 2^e of a whole number (or -inf: 0)
 __device__ __forceinline__ float pow2(float e) { return ldexpf(1.0f, (int)fmaxf(e, -200.f)); }
 
-// hi + lo = v (to 2^-22 of |v| for normal values) as two fp16 vectors
+// hi + lo = v (to 2^-23 of |v| for normal values) as two fp16 vectors
 __device__ __forceinline__ void split8(const float* v, v8h& hi, v8h& lo) {
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
@@ -125,7 +136,7 @@ __host__ __device__ constexpr int tile_key(int r) { return (r & 19) | ((r & 4) <
 template <int CH> __device__ __forceinline__ int kswz(int row) { return CH == 8 ? (row >> 1) & 7 : row & 15; }
 template <int CH> __device__ __forceinline__ int vswz(int key) { return CH == 8 ? 2 * (key & 2) : 4 * (key & 3); }
 
-template <int HD, int G, int RT, int KG, int DS, bool Q8>
+template <int HD, int G, int RT, int KG, int DS, bool Q8, bool FULL>
 __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs a) {
   constexpr int CH = HD / 8;             // 16-byte chunks per row
   constexpr int NC = HD / 16 / DS;       // a wave's 16-wide slices of the head dimension
@@ -164,6 +175,7 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
   const int wmin = a.pos0 + (row0 + 32 * rt) / G, wmax = min(wmin + 32 / G, ctx) - 1;
   const int nstep = (ctx + KG * kBlk - 1) / (KG * kBlk);
 
+  const bool cap = a.softcap > 0.f;
   float qv[NC][8];
   float amax = 0.f;
   {
@@ -267,19 +279,26 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
       amax = fmaxf(amax, xs[wave ^ 1][lane]);
     }
     int e = 0;
-    frexpf(amax, &e);   // amax = f * 2^e, f in [0.5, 1); 0 gives e = 0
+    // q times the softmax's scale (and log2 e), as sh + sl, keeps what its two
+    // parts hold
+    const float c0 = cap ? a.scale : a.scale * kLog2e;
+    const float c1 = cap ? 0.f : __builtin_fmaf(a.scale, kLog2e, -c0) + a.scale * kLog2eLow;
+    frexpf(amax * c0, &e);
     const int shift = min(max(14 - e, -100), 100);
-    const float sc = ldexpf(1.0f, shift);
-    qscale = a.scale * ldexpf(1.0f, -shift);   // S^T holds (q . k) * 2^shift
+    const float sh = ldexpf(c0, shift), sl = ldexpf(c1, shift);
+    qscale = ldexpf(1.0f, -shift);   // S^T holds the scores * 2^shift
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
+    for (int c = 0; c < NC; ++c)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) qv[c][i] *= sc;
-      split8(qv[c], qh[c], ql[c]);
-    }
+      for (int i = 0; i < 8; ++i) {
+        float p = qv[c][i] * sh;
+        asm("" : "+v"(p));   // one value for both parts (see the weights below)
+        const _Float16 hi = (_Float16)p;
+        qh[c][i] = hi;
+        ql[c][i] = (_Float16)__builtin_fmaf(qv[c][i], sl, __builtin_fmaf(qv[c][i], sh, -(float)hi));
+      }
   }
-  const bool cap = a.softcap > 0.f;
-  const float qs = cap ? 1.0f : qscale * kLog2e;   // scores of the tile -> base-2 exponents
+  const float qs = cap ? kLog2e : qscale;   // scores of the tile -> base-2 exponents
 
   v16f o[NDT];
 #pragma unroll
@@ -302,11 +321,23 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
     const v4u* vcur = vall + g * kGrp;
     v16f acc = v16f{};
     if (kb <= wmax) {
+      v8h kv[NC];
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
-        const v8h kv = __builtin_bit_cast(v8h, kcur[n * CH + ((2 * (ds * NC + c) + h) ^ kswz<CH>(n))]);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv, qh[c], acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv, ql[c], acc, 0, 0, 0);
+        kv[c] = __builtin_bit_cast(v8h, kcur[n * CH + ((2 * (ds * NC + c) + h) ^ kswz<CH>(n))]);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv[c], ql[c], acc, 0, 0, 0);
+      }
+      if constexpr (FULL) {
+        v16f odd = v16f{};
+#pragma unroll
+        for (int c = 0; c < NC; c += 2) {
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv[c], qh[c], acc, 0, 0, 0);
+          odd = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv[c + 1], qh[c + 1], odd, 0, 0, 0);
+        }
+        acc += odd;
+      } else {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv[c], qh[c], acc, 0, 0, 0);
       }
     }
     if (DS > 1) {   // the sum of the two waves' shares, the same in both
@@ -328,7 +359,7 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
       }
       if (cap) {   // (q . k) / sqrt(hd), softcapped (layer_scheduler.c:442-448)
 #pragma unroll
-        for (int j = 0; j < 16; ++j) sc[j] = softcap(sc[j] * qscale, a) * kLog2e;
+        for (int j = 0; j < 16; ++j) sc[j] = softcap(sc[j] * qscale, a);
       }
       if (kb + kBlk - 1 > wmin) {   // causal limit
 #pragma unroll
@@ -343,9 +374,8 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
       for (int j = 1; j < 16; ++j) bmax = fmaxf(bmax, sc[j]);
       bmax = max_pair(bmax) * qs;
       if (__any(bmax > m + kLag)) {
-        const float mn = Q8 ? ceilf(fmaxf(m, bmax)) : fmaxf(m, bmax);
-        const float by = m - (mn == -INFINITY ? 0.f : mn);
-        const float corr = Q8 ? pow2(by) : __builtin_amdgcn_exp2f(by);
+        const float mn = ceilf(fmaxf(m, bmax));
+        const float corr = pow2(m - (mn == -INFINITY ? 0.f : mn));
         l *= corr;
         if constexpr (!Q8) {
 #pragma unroll
@@ -353,12 +383,15 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
         }
         m = mn;
       }
-      const float mo = (m == -INFINITY ? 0.f : m) - (Q8 ? 0.f : kPExp);   // nothing seen yet: weights stay 0
+      const float mo = m == -INFINITY ? 0.f : m;   // nothing seen yet: weights stay 0
       float pv[16];
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        pv[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j], qs, -mo));   // layer_scheduler.c:450-458
-        l += pv[j];
+      for (int j = 0; j < 16; ++j) pv[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j], qs, -mo));   // layer_scheduler.c:450-458
+      {
+        float t[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) t[j] = pv[j] + pv[j + 8];
+        l += ((t[0] + t[4]) + (t[1] + t[5])) + ((t[2] + t[6]) + (t[3] + t[7]));
       }
       if constexpr (Q8) {
         float bx = 0.f;
@@ -387,24 +420,44 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
           asm("" : "+v"(pv[j]));
         }
       }
+      if constexpr (!Q8) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) pv[j] *= kPScale;   // (exact: part of the split's conversions)
+      }
       v8h ph[2], pl[2];
       split8(pv, ph[0], pl[0]);
       split8(pv + 8, ph[1], pl[1]);
       // O^T += V^T P^T
+      auto read_v = [&](int c, int dt) {
+        union { v4s t[2]; v8h v; } vv;
 #pragma unroll
-      for (int c = 0; c < 2; ++c)
+        for (int u = 0; u < 2; ++u) {
+          const int key = 16 * c + 4 * u + vkey;
+          const v4u* p = &vcur[key * CH + ((4 * (ds * NDT + dt) + vch) ^ vswz<CH>(vkey))];
+          vv.t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t)(reinterpret_cast<const v4s*>(p) + (lane & 1)));
+        }
+        return vv.v;
+      };
+      if constexpr (FULL) {
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt) {
-          union { v4s t[2]; v8h v; } vv;
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            const int key = 16 * c + 4 * u + vkey;
-            const v4u* p = &vcur[key * CH + ((4 * (ds * NDT + dt) + vch) ^ vswz<CH>(vkey))];
-            vv.t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t)(reinterpret_cast<const v4s*>(p) + (lane & 1)));
-          }
-          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vv.v, ph[c], o[dt], 0, 0, 0);
-          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vv.v, pl[c], o[dt], 0, 0, 0);
+          const v8h v0 = read_v(0, dt), v1 = read_v(1, dt);
+          v16f r = __builtin_amdgcn_mfma_f32_32x32x16_f16(v0, pl[0], v16f{}, 0, 0, 0);
+          r = __builtin_amdgcn_mfma_f32_32x32x16_f16(v1, pl[1], r, 0, 0, 0);
+          r = __builtin_amdgcn_mfma_f32_32x32x16_f16(v0, ph[0], r, 0, 0, 0);
+          r = __builtin_amdgcn_mfma_f32_32x32x16_f16(v1, ph[1], r, 0, 0, 0);
+          o[dt] += r;
         }
+      } else {
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int dt = 0; dt < NDT; ++dt) {
+            const v8h v = read_v(c, dt);
+            o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, ph[c], o[dt], 0, 0, 0);
+            o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, pl[c], o[dt], 0, 0, 0);
+          }
+      }
     }
     if (Q8 && st + 1 < nstep) store_q(st + 1, knxt, vnxt, scn);
     turn();
@@ -436,7 +489,7 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
       lt += mk == -INFINITY ? 0.f : gl[k][32 * rt + n] * __builtin_amdgcn_exp2f(mk - mx);
     }
     // (a row whose scores are all -inf keeps its 0 / 0)
-    const float f = (m == -INFINITY ? 0.f : Q8 ? pow2(ex - kPExp - mx) : __builtin_amdgcn_exp2f(m - mx)) / lt;
+    const float f = (m == -INFINITY ? 0.f : pow2((Q8 ? ex : m) - kPExp - mx)) / lt;
     auto bank = [&](int w) { return w == 0 ? ks0 : w == 1 ? vs0 : w == 2 ? ks1 : vs1; };
     const int tile = wave / DS;
     float4* dst = reinterpret_cast<float4*>(bank(tile / (KG / 2))) + (tile % (KG / 2)) * (32 * HD / 4);
@@ -467,24 +520,28 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
   }
 }
 
-template <int HD, int RT, int KG, int DS, bool Q8>
+template <int HD, int RT, int KG, int DS, bool Q8, bool FULL>
 hipError_t launch_flash_kv(int group, const AttnArgs& a, hipStream_t s) {
   const int64_t tiles = ((int64_t)a.n_tok * group + 32 * RT - 1) / (32 * RT);
   if (tiles * a.n_kv_heads > INT32_MAX) return hipErrorInvalidValue;
   const dim3 grid((unsigned)(tiles * a.n_kv_heads)), block(RT * KG * DS * 64);
   switch (group) {
-    case 1: hipLaunchKernelGGL((k_flash_rows<HD, 1, RT, KG, DS, Q8>), grid, block, 0, s, a); break;
-    case 2: hipLaunchKernelGGL((k_flash_rows<HD, 2, RT, KG, DS, Q8>), grid, block, 0, s, a); break;
-    case 4: hipLaunchKernelGGL((k_flash_rows<HD, 4, RT, KG, DS, Q8>), grid, block, 0, s, a); break;
-    case 8: hipLaunchKernelGGL((k_flash_rows<HD, 8, RT, KG, DS, Q8>), grid, block, 0, s, a); break;
+    case 1: hipLaunchKernelGGL((k_flash_rows<HD, 1, RT, KG, DS, Q8, FULL>), grid, block, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((k_flash_rows<HD, 2, RT, KG, DS, Q8, FULL>), grid, block, 0, s, a); break;
+    case 4: hipLaunchKernelGGL((k_flash_rows<HD, 4, RT, KG, DS, Q8, FULL>), grid, block, 0, s, a); break;
+    case 8: hipLaunchKernelGGL((k_flash_rows<HD, 8, RT, KG, DS, Q8, FULL>), grid, block, 0, s, a); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
+// The sums' form (FULL above): every int8 launch, and fp16 launches of fewer
+// than kFullRows tokens.
 template <int HD, int RT, int KG, int DS = 1>
 hipError_t launch_flash(int group, int kv_type, const AttnArgs& a, hipStream_t s) {
-  return kv_type ? launch_flash_kv<HD, RT, KG, DS, true>(group, a, s)
-                 : launch_flash_kv<HD, RT, KG, DS, false>(group, a, s);
+  if (kv_type) return launch_flash_kv<HD, RT, KG, DS, true, true>(group, a, s);
+  if constexpr (RT == 1)
+    if (a.n_tok < kFullRows) return launch_flash_kv<HD, RT, KG, DS, false, true>(group, a, s);
+  return launch_flash_kv<HD, RT, KG, DS, false, false>(group, a, s);
 }
 
 }  // namespace
@@ -506,7 +563,7 @@ hipError_t launch_attention_rows(int head_dim, int group, int kv_type, const Att
   if (head_dim == 64) return two_blocks ? launch_flash<64, 1, 2>(group, kv_type, a, s) : launch_flash<64, 1, 4>(group, kv_type, a, s);
   if (head_dim == 128) {
     if (two_blocks) return launch_flash<128, 1, 2>(group, kv_type, a, s);
-    return tiles > kCompute ? launch_flash<128, 2, 4>(group, kv_type, a, s) : launch_flash<128, 1, 4>(group, kv_type, a, s);
+    return tiles > kCompute && (kv_type || a.n_tok >= kFullRows) ? launch_flash<128, 2, 4>(group, kv_type, a, s) : launch_flash<128, 1, 4>(group, kv_type, a, s);
   }
   if (head_dim == 256) return launch_flash<256, 1, 2, 2>(group, kv_type, a, s);   // Gemma
   return hipErrorInvalidValue;
