@@ -71,6 +71,8 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include <type_traits>
+
 #include "ss_device.h"
 #include "ss_kernels.h"
 
@@ -135,6 +137,45 @@ __host__ __device__ constexpr int tile_key(int r) { return (r & 19) | ((r & 4) <
 // 16 places of 256 bytes; the 4 keys of a transposed read take 4 groups of 4
 template <int CH> __device__ __forceinline__ int kswz(int row) { return CH == 8 ? (row >> 1) & 7 : row & 15; }
 template <int CH> __device__ __forceinline__ int vswz(int key) { return CH == 8 ? 2 * (key & 2) : 4 * (key & 3); }
+
+// One query row over positions 0..lim of the fp16 cache by one wave in fp32: 64
+// keys at a time, one per lane, then their V rows, lane l taking dimensions l,
+// l + 64, ... For the rows a tile's products cannot serve: a V that is not
+// finite reaches, as 0 * inf, rows that do not see its position.
+template <int HD>
+__device__ __forceinline__ void one_row(const AttnArgs& a, const float* q, const uint16_t* kc, const uint16_t* vc, int lim,
+                                        float* out) {
+  constexpr int ND = HD / kWave;
+  const int lane = threadIdx.x & 63;
+  float m = -INFINITY, l = 0.f, o[ND] = {};
+#pragma unroll 1
+  for (int k0 = 0; k0 <= lim; k0 += kWave) {
+    float s = -INFINITY;
+    if (k0 + lane <= lim) {
+      const uint16_t* kr = kc + (size_t)(k0 + lane) * HD;
+      s = 0.f;
+#pragma unroll 1
+      for (int i = 0; i < HD; ++i) s = fmaf(q[i], h2f(kr[i]), s);
+      s *= a.scale;
+      if (a.softcap > 0.f) s = softcap(s, a);
+    }
+    const float mn = fmaxf(m, wave_max(s));
+    const float mo = mn == -INFINITY ? 0.f : mn;
+    const float p = expf(s - mo), corr = expf(m - mo);
+    l = l * corr + wave_sum(p);
+#pragma unroll
+    for (int d = 0; d < ND; ++d) o[d] *= corr;
+#pragma unroll 1
+    for (int j = 0; j < kWave && k0 + j <= lim; ++j) {
+      const float pj = __shfl(p, j, kWave);
+#pragma unroll
+      for (int d = 0; d < ND; ++d) o[d] = fmaf(pj, h2f(vc[(size_t)(k0 + j) * HD + lane + kWave * d]), o[d]);
+    }
+    m = mn;
+  }
+#pragma unroll
+  for (int d = 0; d < ND; ++d) out[lane + kWave * d] = o[d] / l;
+}
 
 template <int HD, int G, int RT, int KG, int DS, bool Q8, bool FULL>
 __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs a) {
@@ -321,23 +362,28 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
     const v4u* vcur = vall + g * kGrp;
     v16f acc = v16f{};
     if (kb <= wmax) {
-      v8h kv[NC];
+      auto read_k = [&](int c) {
+        return __builtin_bit_cast(v8h, kcur[n * CH + ((2 * (ds * NC + c) + h) ^ kswz<CH>(n))]);
+      };
+      // slices c0 .. c0 + N - 1 in one chain, the low parts first: what rounds then is the small sum
+      auto chain = [&](auto nc, int c0, v16f d) {
+        constexpr int N = decltype(nc)::value;
+        v8h kv[N];
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        kv[c] = __builtin_bit_cast(v8h, kcur[n * CH + ((2 * (ds * NC + c) + h) ^ kswz<CH>(n))]);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv[c], ql[c], acc, 0, 0, 0);
-      }
-      if constexpr (FULL) {
-        v16f odd = v16f{};
-#pragma unroll
-        for (int c = 0; c < NC; c += 2) {
-          acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv[c], qh[c], acc, 0, 0, 0);
-          odd = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv[c + 1], qh[c + 1], odd, 0, 0, 0);
+        for (int c = 0; c < N; ++c) {
+          kv[c] = read_k(c0 + c);
+          d = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv[c], ql[c0 + c], d, 0, 0, 0);
         }
-        acc += odd;
-      } else {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv[c], qh[c], acc, 0, 0, 0);
+        for (int c = 0; c < N; ++c) d = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv[c], qh[c0 + c], d, 0, 0, 0);
+        return d;
+      };
+      if constexpr (FULL) {
+        constexpr std::integral_constant<int, NC / 2> half;
+        const v16f first = chain(half, 0, v16f{});
+        acc = first + chain(half, NC / 2, v16f{});
+      } else {
+        acc = chain(std::integral_constant<int, NC>{}, 0, v16f{});
       }
     }
     if (DS > 1) {   // the sum of the two waves' shares, the same in both
@@ -500,10 +546,12 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
         dst[n * (HD / 4) + ((8 * (ds * NDT + dt) + 2 * q + h) ^ (n & 15))] =
             make_float4(o[dt][4 * q] * f, o[dt][4 * q + 1] * f, o[dt][4 * q + 2] * f, o[dt][4 * q + 3] * f);
     __syncthreads();
+    static_assert(RT * 32 * (HD / 4) % NT == 0, "every lane of a wave takes each turn");
+    float odd = 0.f;   // NaN: some output of this thread is not finite
     for (int i = tid; i < RT * 32 * (HD / 4); i += NT) {
       const int r = i / (HD / 4), c = i % (HD / 4);
       const int zr = (row0 + r) / G, hr = (row0 + r) % G;
-      if (zr >= a.n_tok) continue;
+      const bool live = zr < a.n_tok;
       float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
       for (int k = 0; k < KG; ++k) {
@@ -515,7 +563,31 @@ __global__ void __launch_bounds__(RT * KG * DS * 64) k_flash_rows(const AttnArgs
         s.z += v.z;
         s.w += v.w;
       }
-      *reinterpret_cast<float4*>(a.out + (size_t)zr * a.tok_o + ((size_t)kvh * G + hr) * HD + 4 * c) = s;
+      if (live) *reinterpret_cast<float4*>(a.out + (size_t)zr * a.tok_o + ((size_t)kvh * G + hr) * HD + 4 * c) = s;
+      // (inf - inf and NaN - NaN are NaN)
+      if (!Q8 && live) odd += (s.x - s.x) + (s.y - s.y) + (s.z - s.z) + (s.w - s.w);
+    }
+    // fp16: rows that are not finite, again, each over the positions it sees
+    // alone (layer_scheduler.c:415-468 reads no others). A row's HD / 4 threads
+    // are neighbours in one wave.
+    if (!Q8 && __ballot(odd != odd)) {
+      vm_drain();   // this wave's stores
+#pragma unroll 1
+      for (int i = tid; i < RT * 32 * (HD / 4); i += NT) {
+        const int r = i / (HD / 4), z = (row0 + r) / G;
+        float* op = a.out + (size_t)z * a.tok_o + ((size_t)kvh * G + (row0 + r) % G) * HD;
+        float d = 0.f;
+        if (z < a.n_tok)
+          for (int k = 0; k < 4; ++k) d += op[4 * (i % (HD / 4)) + k] - op[4 * (i % (HD / 4)) + k];
+        uint64_t bad = __ballot(d != d);
+        while (bad) {
+          const int at = __ffsll((unsigned long long)bad) - 1, rb = __shfl(r, at, kWave);
+          bad &= ~(((HD / 4 < 64 ? 1ull << (HD / 4 % 64) : 0ull) - 1) << (at / (HD / 4) * (HD / 4)));
+          const int zb = (row0 + rb) / G;
+          const size_t head = ((size_t)kvh * G + (row0 + rb) % G) * HD;
+          one_row<HD>(a, a.q + (size_t)zb * a.tok_q + head, kc, vc, a.pos0 + zb, a.out + (size_t)zb * a.tok_o + head);
+        }
+      }
     }
   }
 }
