@@ -718,7 +718,11 @@ __global__ void __launch_bounds__(kSW * 64) k_gemm_rs(const GemmArgs a, int nu) 
   static_assert(RW >= 2 && NS % 4 == 0, "whole turns of the four stages per unit");
   // vector memory instructions of a unit's two loads of codes
   constexpr bool kSumLate = is_wide(QT);   // the block sums at the unit's end (Q4_1, Q5_1: registers)
-  constexpr int kN1 = kTB + (is_kq(QT) ? 1 : 0) + kTB * KCodes<QT>::kQ + (kSumLate ? 0 : SUMS * TT), kN2 = kTB * KCodes<QT>::kQ;
+  // and Q5_1's scales not before its unit begins: with a second set in
+  // registers the accumulators went through scratch memory every unit (14336 x
+  // 4096 at 77 / 200 / 512 tokens: 91, 178 and 320 us)
+  constexpr bool kScaleLate = QT == kQ5_1;
+  constexpr int kN1 = (kScaleLate ? 0 : kTB) + (is_kq(QT) ? 1 : 0) + kTB * KCodes<QT>::kQ + (kSumLate ? 0 : SUMS * TT), kN2 = kTB * KCodes<QT>::kQ;
   constexpr int kStage = 2048;   // 16-byte chunks
   __shared__ v4u s0[kStage], s1[kStage], s2[kStage], s3[kStage];
   __shared__ float rn[TT * kSTok], psum[TT][kSW][kSTok];
@@ -774,7 +778,7 @@ __global__ void __launch_bounds__(kSW * 64) k_gemm_rs(const GemmArgs a, int nu) 
   auto load_first = [&](int it) {
     asm volatile("" ::: "memory");   // the count of wait_loads: not before the loads ahead, not after those behind
     load_codes<QT>(q, wv, unit_of(it + 1), 0);
-    load_scales<QT>(wn, wv, unit_of(it + 1));
+    if constexpr (!kScaleLate) load_scales<QT>(wn, wv, unit_of(it + 1));
     if constexpr (!kSumLate) load_sums(it);
     asm volatile("" ::: "memory");
   };
@@ -881,7 +885,10 @@ __global__ void __launch_bounds__(kSW * 64) k_gemm_rs(const GemmArgs a, int nu) 
     if constexpr (kSumLate) load_sums(it);   // (not among the counted: wait_loads then waits for more)
     load_second(it);
     pipe.finish(acc, w, sum, inv_lds + u * kSTok + 4 * kg, nu * kSTok, live);
-    w = wn;
+    if constexpr (kScaleLate)
+      load_scales<QT>(w, wv, unit_of(it + 1));   // (nor these)
+    else
+      w = wn;
   }
 
   // the column groups' sums of each row tile, added in group order

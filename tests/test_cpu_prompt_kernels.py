@@ -1,0 +1,53 @@
+"""The compiled prompt products (k_gemm_rs in the built library), read from its
+gfx950 code object with the LLVM tools that built it: no GPU."""
+import os
+import re
+import struct
+import subprocess
+
+import pytest
+
+import phonemap_amd as pm
+
+LLVM = "/opt/rocm/llvm/bin/"
+LIB = os.path.join(os.path.dirname(pm.__file__), "libslipstream_hip.so")
+
+
+def _tool(name, *args):
+    if not os.path.exists(LLVM + name):
+        pytest.skip("no " + name)
+    return subprocess.run([LLVM + name, *args], check=True, stdout=subprocess.PIPE, text=True).stdout
+
+
+@pytest.fixture(scope="module")
+def code_object(tmp_path_factory):
+    """The device code of the translation unit that holds k_gemm_rs."""
+    if not os.path.exists(LIB):
+        pytest.skip("library not built")
+    blob = open(LIB, "rb").read()
+    for m in re.finditer(b"__CLANG_OFFLOAD_BUNDLE__", blob):
+        at = m.start() + 32
+        for _ in range(struct.unpack_from("<Q", blob, m.start() + 24)[0]):
+            off, size, n = struct.unpack_from("<QQQ", blob, at)
+            target, at = blob[at + 24:at + 24 + n], at + 24 + n
+            part = blob[m.start() + off:m.start() + off + size]
+            if b"gfx950" in target and b"k_gemm_rs" in part:
+                path = tmp_path_factory.mktemp("co") / "gemm.co"
+                path.write_bytes(part)
+                return str(path)
+    raise AssertionError("no k_gemm_rs in " + LIB)
+
+
+def test_products_keep_their_sums_in_registers(code_object):
+    """Two waves per SIMD have 256 registers each. A few addresses may be
+    spilled (at most 16 bytes per lane), not the 32 accumulators of a wave."""
+    notes = _tool("llvm-readelf", "--notes", code_object)
+    seen = 0
+    for k in notes.split(".name:")[1:]:
+        name = k.split()[0]
+        if "k_gemm_rs" not in name:
+            continue
+        seen += 1
+        scratch = int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", k).group(1))
+        assert scratch <= 16, (name, scratch)
+    assert seen >= 50   # ten block types, three epilogues, two shapes (two types: one)
