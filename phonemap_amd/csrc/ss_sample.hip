@@ -45,6 +45,7 @@ constexpr int kTile = 1024;                    // entries per workgroup of the o
 constexpr int kTileThreads = 256;
 constexpr int kBins = 2048;                    // by key >> 19 (sign 0, exponent, 4 bits of the mantissa): e, p <= 1
 constexpr int kCand = 2048;                    // candidates the top-k path keeps in LDS
+constexpr int kPairs = 288;                    // up to this many are compared each with all, more are sorted
 constexpr int kMaxTopK = 1024;                 // top_k it takes
 constexpr double kFix = 4503599627370496.0;   // 2^52: probabilities (each <= 1, sums <= ~1)
 constexpr double kFixE = 1099511627776.0;     // 2^40: softmax terms (each <= 1, up to 2^18 of them)
@@ -196,31 +197,35 @@ __device__ void put_result(const SampleArgs& a, int idx, uint64_t st) {
   }
 }
 
-// the whole of ss_sample in one workgroup
-__device__ void sample_one_group(const SampleArgs& a, Shared& sh) {
+// The whole of ss_sample in one workgroup. HAVE: the softmax terms are in
+// a.probs already; inv: the factor that makes them probabilities.
+template <bool HAVE>
+__device__ void sample_one_group(const SampleArgs& a, Shared& sh, float inv = 0.f) {
   const int V = a.V, tid = threadIdx.x;
   float* p = a.probs;
-
-  // 1. temperature and softmax (tensor.c:374-381, 154-173)
-  float mx = -FLT_MAX;
-  for (int i = tid; i < V; i += kThreads) {
-    const float l = a.logits[i];
-    const float x = l != l ? -FLT_MAX : l / a.temperature;
-    p[i] = x;
-    mx = fmaxf(mx, x);
-  }
-  mx = block_max(mx, sh);
   uint64_t s = 0;
   int nan_at = 0x7fffffff;
-  for (int i = tid; i < V; i += kThreads) {
-    const float e = expf(p[i] - mx);
-    p[i] = e;
-    s += e > 0.f ? (uint64_t)((double)e * kFixE) : 0ull;   // e <= 1
-    if (e != e) nan_at = min(nan_at, i);
+
+  // 1. temperature and softmax (tensor.c:374-381, 154-173)
+  if constexpr (!HAVE) {
+    float mx = -FLT_MAX;
+    for (int i = tid; i < V; i += kThreads) {
+      const float l = a.logits[i];
+      const float x = l != l ? -FLT_MAX : l / a.temperature;
+      p[i] = x;
+      mx = fmaxf(mx, x);
+    }
+    mx = block_max(mx, sh);
+    for (int i = tid; i < V; i += kThreads) {
+      const float e = expf(p[i] - mx);
+      p[i] = e;
+      s += e > 0.f ? (uint64_t)((double)e * kFixE) : 0ull;   // e <= 1
+      if (e != e) nan_at = min(nan_at, i);
+    }
+    const bool nan_sum = block_min_i(nan_at, sh) != 0x7fffffff;
+    const uint64_t esum = block_sum(s, sh);
+    inv = nan_sum ? NAN : 1.0f / (float)((double)esum / kFixE);
   }
-  const bool nan_sum = block_min_i(nan_at, sh) != 0x7fffffff;
-  const uint64_t esum = block_sum(s, sh);
-  const float inv = nan_sum ? NAN : 1.0f / (float)((double)esum / kFixE);
   for (int i = tid; i < V; i += kThreads) p[i] *= inv;
   __syncthreads();
 
@@ -295,7 +300,7 @@ __device__ void sample_one_group(const SampleArgs& a, Shared& sh) {
 
 __global__ void __launch_bounds__(kThreads) k_sample(const SampleArgs a) {
   __shared__ Shared sh;
-  sample_one_group(a, sh);
+  sample_one_group<false>(a, sh);
 }
 
 // ---- many workgroups ---------------------------------------------------------
@@ -360,6 +365,27 @@ __device__ __forceinline__ bool any_nan(const Work& w, int nb, uint64_t* red) {
   uint64_t v = 0;
   for (int i = threadIdx.x; i < nb; i += W * kWave) v += w.nan[i];
   return group_sum<W>(v, red) != 0;
+}
+// sum of v over the threads of a workgroup of W waves before this one; all: over every thread
+template <int W>
+__device__ __forceinline__ uint64_t sum_before(uint64_t v, uint64_t* red, uint64_t& all) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint64_t incl = v;
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const uint64_t o = __shfl_up(incl, off, kWave);
+    if (lane >= off) incl += o;
+  }
+  __syncthreads();
+  if (lane == 63) red[wave] = incl;
+  __syncthreads();
+  uint64_t before = incl - v;
+  all = 0;
+  for (int i = 0; i < W; ++i) {
+    if (i < wave) before += red[i];
+    all += red[i];
+  }
+  return before;
 }
 __device__ __forceinline__ float inv_of(uint64_t esum) { return 1.0f / (float)((double)esum / kFixE); }
 
@@ -491,77 +517,157 @@ __global__ void __launch_bounds__(kTileThreads) k_smp_gather(const SampleArgs a)
   }
 }
 
+// v[0 .. n - 1], n a power of two up to kCand, in descending order (bitonic).
+// The pairs of a step up to 64 apart lie within one wave's 128 entries, so
+// only wider steps meet at a barrier.
+__device__ void sort_descending(uint64_t* v, int n) {
+  __syncthreads();
+  for (int k = 2; k <= n; k <<= 1)
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      for (int t = threadIdx.x; t < n / 2; t += kThreads) {
+        const int i = ((t & ~(j - 1)) << 1) | (t & (j - 1));
+        const uint64_t x = v[i], y = v[i + j];
+        if ((x < y) == ((i & k) == 0)) {
+          v[i] = y;
+          v[i + j] = x;
+        }
+      }
+      if (j > 64 || (j == 1 && k > 64))   // (after j = 1 the next step's pairs are k apart)
+        __syncthreads();
+      else
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+  __syncthreads();
+}
+__device__ __forceinline__ int pow2_from(int n) {   // the power of two at or above n
+  int p = 2;
+  while (p < n) p <<= 1;
+  return p;
+}
+
 // 4. the k-th largest, the top-p cutoff, the renormalisation and the draw over
-// the candidates, whose order in the list does not matter: each is compared
-// with all others by 8 threads. More than kCand candidates (ties, a flat
-// row): the whole row in this workgroup.
+// the candidates, whose order in the list does not matter. Up to kPairs are each
+// compared with all others by 8 threads, which takes the square of their
+// number. More are sorted, by probability, then what is kept by index, with
+// running sums over each order. Calls over 3000 entries, in pairs and sorted:
+// top_k 200 39 and 46 us, 300 50 and 50, 1000 463 and 66 (one workgroup: 84).
+// More than kCand (ties, a flat row): the whole row in this workgroup, from its
+// softmax terms on; with room for 4096, 3000 equal entries took 100 us, 79 so.
 __global__ void __launch_bounds__(kThreads) k_smp_topk(const SampleArgs a) {
   __shared__ Shared sh;
-  __shared__ int idx[kCand];
-  __shared__ float p[kCand];
+  __shared__ uint64_t ent[kCand];   // probability (its bits) << 32 | index
   __shared__ uint32_t th, cut;
   __shared__ int found;
   const Work w = work_of(a.probs, a.V, nullptr);
   const int tid = threadIdx.x, nb = (a.V + kTile - 1) / kTile;
-  const uint32_t n = *w.count;
-  if (n > (uint32_t)kCand) {
-    sample_one_group(a, sh);
+  const int n = (int)*w.count;
+  const bool nan = any_nan<kWaves>(w, nb, sh.u);
+  const float inv = inv_of(total<kWaves>(w.esum, nb, sh.u));
+  if (n > kCand) {
+    sample_one_group<true>(a, sh, nan ? NAN : inv);
     return;
   }
   const uint64_t st = advance(a.rng), rf = draw_fix(st);
-  const bool nan = any_nan<kWaves>(w, nb, sh.u);
-  const float inv = inv_of(total<kWaves>(w.esum, nb, sh.u));
-  for (int i = tid; i < (int)n; i += kThreads) {
-    idx[i] = __float_as_int(w.list[2 * i]);
-    p[i] = w.list[2 * i + 1] * inv;
-  }
+  const bool topp = a.top_p > 0.f && a.top_p < 1.0f;
+  const uint64_t target = top_p_target(a.top_p);
+  const bool sorted = n > kPairs;
+  const int pn = sorted ? pow2_from(n) : n;
+  for (int i = tid; i < pn; i += kThreads)
+    ent[i] = i < n ? (uint64_t)__float_as_uint(w.list[2 * i + 1] * inv) << 32 | __float_as_uint(w.list[2 * i]) : 0ull;
   if (tid == 0) {
     th = 0;
     cut = 0;
     found = 0x7fffffff;
   }
   __syncthreads();
+  auto p = [&](int i) { return __uint_as_float((uint32_t)(ent[i] >> 32)); };
+  auto idx = [&](int i) { return (int)(uint32_t)ent[i]; };
   const int part = tid & 7;
-  // f(i) for every candidate, by the 8 threads of an aligned group
-  auto each = [&](auto f) {
-    for (int i = tid >> 3; i < (int)n; i += kThreads / 8) f(i);
+  // f(i) for i < m, by the 8 threads of an aligned group
+  auto each = [&](int m, auto f) {
+    for (int i = tid >> 3; i < m; i += kThreads / 8) f(i);
   };
   auto sum8u = [](uint64_t v) {
     v += __shfl_xor(v, 1, kWave);
     v += __shfl_xor(v, 2, kWave);
     return v + __shfl_xor(v, 4, kWave);
   };
-  each([&](int i) {   // the k-th largest p (p >= 0: its bits order like its value)
-    uint64_t c = 0;   // greater ones, and (high half) equal ones
-    for (int j = part; j < (int)n; j += 8) c += p[j] > p[i] ? 1ull : p[j] == p[i] ? 1ull << 32 : 0ull;
-    c = sum8u(c);
-    const uint32_t gt = (uint32_t)c, eq = (uint32_t)(c >> 32);
-    if (part == 0 && gt < (uint32_t)a.top_k && gt + eq >= (uint32_t)a.top_k) th = __float_as_uint(p[i]);
-  });
-  __syncthreads();
-  const float tk = __uint_as_float(th);
-  if (a.top_p > 0.f && a.top_p < 1.0f) {
-    const uint64_t target = top_p_target(a.top_p);
-    each([&](int i) {   // the largest p whose sum with those above it reaches the target
-      uint64_t s = 0;
-      for (int j = part; j < (int)n; j += 8) s += p[j] >= tk && p[j] >= p[i] ? fix(p[j]) : 0ull;
-      s = sum8u(s);
-      if (part == 0 && p[i] >= tk && s >= target) atomicMax(&cut, __float_as_uint(p[i]));
+  // the running sum of v(i) over i < m (at most kCand) in order: f(i, sum through i - 1, v(i))
+  auto running = [&](int m, auto v, auto f) {
+    constexpr int C = kCand / kThreads;
+    uint64_t x[C], s = 0, all;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const int i = C * tid + c;
+      x[c] = i < m ? v(i) : 0ull;
+      s += x[c];
+    }
+    uint64_t before = sum_before<kWaves>(s, sh.u, all);
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      if (C * tid + c < m) f(C * tid + c, before, x[c]);
+      before += x[c];
+    }
+    __syncthreads();
+  };
+  float tk;
+  if (sorted) {
+    sort_descending(ent, pn);
+    tk = n >= a.top_k ? p(a.top_k - 1) : 0.f;
+    if (topp)
+      running(n, [&](int i) { return p(i) >= tk ? fix(p(i)) : 0ull; },
+              [&](int i, uint64_t before, uint64_t v) {   // the first to reach the target
+                if (before < target && before + v >= target) cut = (uint32_t)(ent[i] >> 32);
+              });
+  } else {
+    each(n, [&](int i) {   // the k-th largest p (p >= 0: its bits order like its value)
+      uint64_t c = 0;      // greater ones, and (high half) equal ones
+      for (int j = part; j < n; j += 8) c += p(j) > p(i) ? 1ull : p(j) == p(i) ? 1ull << 32 : 0ull;
+      c = sum8u(c);
+      const uint32_t gt = (uint32_t)c, eq = (uint32_t)(c >> 32);
+      if (part == 0 && gt < (uint32_t)a.top_k && gt + eq >= (uint32_t)a.top_k) th = (uint32_t)(ent[i] >> 32);
+    });
+    __syncthreads();
+    tk = __uint_as_float(th);
+    if (topp) {
+      each(n, [&](int i) {   // the largest p whose sum with those above it reaches the target
+        uint64_t s = 0;
+        for (int j = part; j < n; j += 8) s += p(j) >= tk && p(j) >= p(i) ? fix(p(j)) : 0ull;
+        s = sum8u(s);
+        if (part == 0 && p(i) >= tk && s >= target) atomicMax(&cut, (uint32_t)(ent[i] >> 32));
+      });
+      __syncthreads();
+    }
+  }
+  const float low = fmaxf(tk, __uint_as_float(cut));
+  uint64_t s = 0, kept = 0;
+  for (int i = tid; i < n; i += kThreads) {
+    s += p(i) >= low ? fix(p(i)) : 0ull;
+    kept += p(i) >= low;
+  }
+  s = group_sum<kWaves>(s, sh.u);
+  const float pinv = s > 0 ? 1.0f / (float)((double)s / kFix) : 1.0f;
+  // the first index whose cumulative probability exceeds r; sorted, what is
+  // kept comes first
+  const int m = sorted ? (int)group_sum<kWaves>(kept, sh.u) : n;
+  if (m > kPairs) {
+    const int pm = pow2_from(m);
+    __syncthreads();
+    for (int i = tid; i < pm; i += kThreads) ent[i] = i < m ? ~ent[i] << 32 | ent[i] >> 32 : 0ull;   // ~index, p
+    sort_descending(ent, pm);
+    running(m, [&](int i) { return fix(__uint_as_float((uint32_t)ent[i]) * pinv); },
+            [&](int i, uint64_t before, uint64_t v) {
+              if (rf < before + v) atomicMin(&found, (int)~(uint32_t)(ent[i] >> 32));
+            });
+  } else {
+    each(m, [&](int i) {
+      uint64_t c = 0;
+      for (int j = part; j < m; j += 8) c += p(j) >= low && idx(j) <= idx(i) ? fix(p(j) * pinv) : 0ull;
+      c = sum8u(c);
+      if (part == 0 && p(i) >= low && rf < c) atomicMin(&found, idx(i));
     });
     __syncthreads();
   }
-  const float low = fmaxf(tk, __uint_as_float(cut));
-  uint64_t s = 0;
-  for (int i = tid; i < (int)n; i += kThreads) s += p[i] >= low ? fix(p[i]) : 0ull;
-  s = group_sum<kWaves>(s, sh.u);
-  const float pinv = s > 0 ? 1.0f / (float)((double)s / kFix) : 1.0f;
-  each([&](int i) {   // the first index whose cumulative probability exceeds r
-    uint64_t c = 0;
-    for (int j = part; j < (int)n; j += 8) c += p[j] >= low && idx[j] <= idx[i] ? fix(p[j] * pinv) : 0ull;
-    c = sum8u(c);
-    if (part == 0 && p[i] >= low && rf < c) atomicMin(&found, idx[i]);
-  });
-  __syncthreads();
   if (tid == 0) put_result(a, !nan && found < a.V ? found : a.V - 1, st);
 }
 
@@ -691,29 +797,10 @@ __global__ void __launch_bounds__(kThreads) k_smp_draw(const SampleArgs a) {
   __shared__ uint64_t red[kWaves], base;
   __shared__ int tile, found;
   const Work w = work_of(a.probs, a.V, nullptr);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nb = (a.V + kTile - 1) / kTile;
+  const int tid = threadIdx.x, nb = (a.V + kTile - 1) / kTile;
   const uint64_t st = advance(a.rng), rf = draw_fix(st);
   const bool nan = any_nan<kWaves>(w, nb, red);
   const float low = w.cut[0], pinv = w.cut[1];
-  // exclusive sum of v over the threads before this one; total in all
-  auto scan = [&](uint64_t v, uint64_t& total_out) {
-    uint64_t incl = v;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-      const uint64_t o = __shfl_up(incl, off, kWave);
-      if (lane >= off) incl += o;
-    }
-    __syncthreads();
-    if (lane == 63) red[wave] = incl;
-    __syncthreads();
-    uint64_t before = incl - v;
-    total_out = 0;
-    for (int i = 0; i < kWaves; ++i) {
-      if (i < wave) before += red[i];
-      total_out += red[i];
-    }
-    return before;
-  };
   if (tid == 0) {
     tile = -1;
     found = 0x7fffffff;
@@ -722,7 +809,7 @@ __global__ void __launch_bounds__(kThreads) k_smp_draw(const SampleArgs a) {
   for (int b0 = 0; b0 < nb; b0 += kThreads) {
     const uint64_t v = b0 + tid < nb ? w.psum[b0 + tid] : 0ull;
     uint64_t all;
-    const uint64_t before = done + scan(v, all);
+    const uint64_t before = done + sum_before<kWaves>(v, red, all);
     if (v > 0 && rf >= before && rf < before + v) {
       tile = b0 + tid;
       base = before;
@@ -736,7 +823,7 @@ __global__ void __launch_bounds__(kThreads) k_smp_draw(const SampleArgs a) {
     const float p = w.e[min(i, a.V - 1)];
     const uint64_t v = i < a.V && p >= low ? fix(p * pinv) : 0ull;
     uint64_t all;
-    const uint64_t c = base + scan(v, all) + v;
+    const uint64_t c = base + sum_before<kWaves>(v, red, all) + v;
     if (i < a.V && rf < c) atomicMin(&found, i);
   }
   __syncthreads();

@@ -33,3 +33,25 @@ def test_sample_sizes(hip, V, kind):
             got, got_st = _device_sample(hip, x, T, top_p, top_k, seed)
             assert got_st == want_st and 0 <= got < V
             _check_index(got, want, p, r)
+
+
+@pytest.mark.parametrize("V", [1025, 3000, 70001])
+@pytest.mark.parametrize("top_k", [1, 150, 288, 289, 513, 1000, 1024])
+@pytest.mark.parametrize("kind", ["normal", "ties", "inf"])
+def test_sample_few_and_many_candidates(hip, V, top_k, kind):
+    """Candidates compared in pairs (up to 288 of them) and sorted, with what
+    is kept after top-p on either side too, and ties across the k-th."""
+    print("sample candidates", V, top_k, kind, flush=True)
+    rng = np.random.default_rng(V + top_k)
+    for T, top_p in [(0.7, 1.0), (1.5, 0.99), (0.8, 0.5)]:
+        x = (2.5 * rng.standard_normal(V)).astype(np.float32)
+        if kind == "ties":
+            x = np.round(x * 4) / 4
+        elif kind == "inf":
+            x[rng.permutation(V)[: V - 400]] = -np.inf   # fewer terms than many a top_k
+        for _ in range(3):
+            seed = int(rng.integers(1, 2 ** 63))
+            want, want_st, p, r = oracle.sample(x, T, top_p, top_k, seed)
+            got, got_st = _device_sample(hip, x, T, top_p, top_k, seed)
+            assert got_st == want_st and 0 <= got < V
+            _check_index(got, want, p, r)
