@@ -1474,17 +1474,22 @@ int32_t enqueue_prompt_layer_major(ss_hip_model* m, const int32_t* tokens, int n
 // workgroups and its walk costs 10 us (int8: 16) per 1000 positions and layer,
 // a token's own attention 1.2: at 8000 positions 4 tokens break even with the
 // int8 cache and 8 still run in half the time, so the prefix may grow by 2048
-// positions per token above two. From kPrefillAlways tokens on an fp16 cache
-// any prefix goes (8 tokens over 8000: 871 us against 1790).
+// positions per token above two. At head_dim 256 the walk has half the key
+// groups and twice the elements (31 us per 1000 positions and layer, int8 41)
+// and the prefix may grow by 1024: two layers of 8 heads on 4 break even with
+// the int8 cache at 3000 / 6000 / 12000 / 16000 positions with 5 / 8 / 12 / 16
+// tokens (4 tokens over 4000: 348 us one by one, 500 as products). From
+// kPrefillAlways tokens on an fp16 cache any prefix goes (8 tokens over 8000:
+// 871 us against 1790).
 constexpr int kPrefillChunk = 512;
 constexpr int kPrefillMin = 4, kPrefillAlways = 8;
-constexpr int kPrefillPrefix = 2048;
+constexpr int kPrefillPrefix = 2048, kPrefillPrefix256 = 1024;
 
 bool prompt_as_products(const ss_hip_model* m, int n, int start) {
   if (m->pf_min < 0 || m->token_only) return false;
   if (m->pf_min > 0) return n >= m->pf_min;
   if (m->kv_type == SS_HIP_KV_F16 && n >= kPrefillAlways) return true;
-  return n >= kPrefillMin && start <= (int64_t)kPrefillPrefix * (n - 2);
+  return n >= kPrefillMin && start <= (int64_t)(m->hd == 256 ? kPrefillPrefix256 : kPrefillPrefix) * (n - 2);
 }
 
 int32_t prefill_setup(ss_hip_model* m) {

@@ -19,13 +19,26 @@ def test_where_prompts_become_products(kv, n, start, products):
     """The default rule at its edges: 4 tokens, and 2048 positions of prefix
     per token above two; 8 tokens on an fp16 cache over any prefix (None:
     products with that cache only)."""
-    path = os.path.join(TMP, "ss_test_rule.gguf")
+    _check(64, kv, n, start, products)
+
+
+@pytest.mark.parametrize("kv", ["f16", "int8"])
+@pytest.mark.parametrize("n,start,products", [
+    (4, 0, True), (4, 2048, True), (4, 2049, False), (7, 5120, True), (7, 5121, False), (8, 6145, None), (14, 12288, True),
+])
+def test_where_prompts_become_products_head_dim_256(kv, n, start, products):
+    """At head_dim 256 the prefix may grow by 1024 positions per token above two."""
+    _check(256, kv, n, start, products)
+
+
+def _check(hd, kv, n, start, products):
+    path = os.path.join(TMP, "ss_test_rule_%d.gguf" % hd)
     if not os.path.exists(path):
         api.write_synthetic_gguf(path + ".part", api.SynthSpec(
-            n_layers=1, hidden=64, n_heads=1, n_kv_heads=1, head_dim=64, ffn=64, vocab=64, context_length=16384,
+            n_layers=1, hidden=hd, n_heads=1, n_kv_heads=1, head_dim=hd, ffn=64, vocab=64, context_length=16384,
             seed=5, scale_mode=1))
         os.replace(path + ".part", path)
-    print("rule", kv, n, start, flush=True)
+    print("rule", hd, kv, n, start, flush=True)
     L = api._lib()
 
     def count():
