@@ -896,10 +896,12 @@ struct ss_hip_model {
   int* pos_iota = nullptr;           // device [max_seq]: value i at index i
   float* hid_all = nullptr;          // device [max_seq][d]: residual streams of a prompt
   uint32_t* xr_all = nullptr;        // device [max_seq][xrec_words(d)]: their x records
-  // prompts as matrix products (fp16 KV): up to pf_cap tokens per pass over the
+  // prompts as matrix products: up to pf_cap tokens per pass over the
   // layers, in row-major [token][...] buffers
   int pf_min = 0;                    // shortest prompt evaluated this way (0: the default)
   int pf_cap = 0;                    // chunk capacity (0: not set up)
+  void* pf_base = nullptr;           // their one allocation, of pf_bytes
+  size_t pf_bytes = 0;
   float *pf_h = nullptr, *pf_qkv = nullptr, *pf_att = nullptr, *pf_f = nullptr, *pf_ssq = nullptr;
   float* pf_y = nullptr;   // [chunk][d]: projections before their post norm (Gemma 2)
   uint16_t* pf_xs = nullptr;         // x of a product split into fp16 parts
@@ -1492,9 +1494,13 @@ bool prompt_as_products(const ss_hip_model* m, int n, int start) {
   return n >= kPrefillMin && start <= (int64_t)(m->hd == 256 ? kPrefillPrefix256 : kPrefillPrefix) * (n - 2);
 }
 
-int32_t prefill_setup(ss_hip_model* m) {
-  if (m->pf_cap) return 0;
-  const int cap = std::min(kPrefillChunk, m->max_seq);
+// Buffers for a prompt of n tokens, one allocation: for up to kPrefillFew
+// tokens, which a short prompt needs, or for a whole chunk. The stream is idle.
+constexpr int kPrefillFew = 32;
+
+int32_t prefill_setup(ss_hip_model* m, int n) {
+  const int cap = std::min(n <= kPrefillFew ? kPrefillFew : kPrefillChunk, m->max_seq);
+  if (m->pf_cap >= cap) return 0;
   if (!m->pos_iota) {
     if (int32_t rc = m_alloc(m, (void**)&m->pos_iota, sizeof(int) * m->max_seq, false)) return rc;
     std::vector<int> iota(m->max_seq);
@@ -1502,15 +1508,27 @@ int32_t prefill_setup(ss_hip_model* m) {
     HIP_TRY(hipMemcpy(m->pos_iota, iota.data(), sizeof(int) * m->max_seq, hipMemcpyHostToDevice));
   }
   const size_t c = (size_t)cap;
-  if (int32_t rc = m_alloc(m, (void**)&m->pf_h, sizeof(float) * c * m->d, false)) return rc;
-  if (int32_t rc = m_alloc(m, (void**)&m->pf_qkv, sizeof(float) * c * (m->qdim + 2 * m->kvdim), false)) return rc;
-  if (int32_t rc = m_alloc(m, (void**)&m->pf_att, sizeof(float) * c * m->qdim, false)) return rc;
-  if (int32_t rc = m_alloc(m, (void**)&m->pf_f, sizeof(float) * c * m->ffn, false)) return rc;
-  if (int32_t rc = m_alloc(m, (void**)&m->pf_ssq, sizeof(float) * c, false)) return rc;
-  if (m->any_post)
-    if (int32_t rc = m_alloc(m, (void**)&m->pf_y, sizeof(float) * c * m->d, false)) return rc;
   const int widest = std::max(std::max(m->d, m->qdim), m->ffn);
-  if (int32_t rc = m_alloc(m, (void**)&m->pf_xs, 2 * ssk::gemm_split_elems(cap, widest), false)) return rc;
+  const size_t need[] = {sizeof(float) * c * m->d, sizeof(float) * c * (m->qdim + 2 * m->kvdim), sizeof(float) * c * m->qdim,
+                         sizeof(float) * c * m->ffn, sizeof(float) * c, m->any_post ? sizeof(float) * c * m->d : 0,
+                         2 * ssk::gemm_split_elems(cap, widest)};
+  void** const dst[] = {(void**)&m->pf_h, (void**)&m->pf_qkv, (void**)&m->pf_att, (void**)&m->pf_f, (void**)&m->pf_ssq,
+                        (void**)&m->pf_y, (void**)&m->pf_xs};
+  size_t total = 0;
+  for (size_t b : need) total += round256(b);
+  char* base = nullptr;
+  if (hipMalloc((void**)&base, total) != hipSuccess) {
+    (void)hipGetLastError();   // or the next launch's check would report it
+    return fail(kErrOom, "hipMalloc(%zu) for a prompt of %d tokens failed", total, n);
+  }
+  if (m->pf_base) hipFree(m->pf_base);
+  m->bytes += total - m->pf_bytes;
+  m->pf_base = base;
+  m->pf_bytes = total;
+  for (int i = 0; i < 7; ++i) {
+    *dst[i] = need[i] ? base : nullptr;
+    base += round256(need[i]);
+  }
   m->pf_cap = cap;
   return 0;
 }
@@ -1749,6 +1767,7 @@ void model_release(ss_hip_model* m) {
   if (m->g_full) hipGraphExecDestroy(m->g_full);
   if (m->g_nohead) hipGraphExecDestroy(m->g_nohead);
   for (void* p : m->allocs) hipFree(p);
+  if (m->pf_base) hipFree(m->pf_base);
   for (hipEvent_t e : m->ev_pool) hipEventDestroy(e);
   if (m->h_io) hipHostFree(m->h_io);
   for (hipStream_t cs : {m->copy_stream, m->copy_stream2})
@@ -2072,8 +2091,8 @@ int32_t ss_hip_eval_prompt(ss_hip_model_t* m, const int32_t* tokens, int32_t n, 
   HIP_TRY(hipStreamSynchronize(s));
   HIP_TRY(hipMemcpy(m->tokens + start, tokens, sizeof(int) * n, hipMemcpyHostToDevice));
   HIP_TRY(ssk::launch_set_state(m->dpos, m->tokens, start, tokens[0], s));
-  if (prompt_as_products(m, n, start)) {
-    if (int32_t rc = prefill_setup(m)) return rc;
+  // (without room for its buffers a prompt runs token by token)
+  if (prompt_as_products(m, n, start) && !prefill_setup(m, n)) {
     if (int32_t rc = enqueue_prompt_rows(m, tokens, n, start)) {
       hipStreamSynchronize(s);
       return rc;
@@ -2119,10 +2138,9 @@ int32_t ss_hip_embed(ss_hip_model_t* m, const int32_t* tokens, int32_t n, float*
   HIP_TRY(hipMemsetAsync(m->emb, 0, sizeof(float) * m->d, s));
   m->host_pos = -1;   // the cache holds positions 0..n-1, but no token to continue from
   int32_t rc = 0;
-  if (m->pf_min >= 0 && !m->token_only) {
+  if (m->pf_min >= 0 && !m->token_only && !prefill_setup(m, n)) {
     int T = 0;
-    rc = prefill_setup(m);
-    if (!rc) rc = enqueue_rows(m, n, 0, true, &T);
+    rc = enqueue_rows(m, n, 0, true, &T);
   } else {
     float* ssq = m->emb + 2 * (size_t)m->d;
     HIP_TRY(ssk::launch_set_state(m->dpos, m->tokens, 0, tokens[0], s));
