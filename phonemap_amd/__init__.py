@@ -42,6 +42,7 @@ _PROTOS = {
     "ss_hip_pack_matrix": (_i32, [_vp, _vp, _vp, _i32, _i32, _i32]),
     "ss_hip_matvec": (_i32, [_vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp]),
     "ss_hip_gemm": (_i32, [_vp, _vp, _vp, _vp, _vp, _f32, _i32, _i32, _i32, _i32, _i32, _vp]),
+    "ss_hip_gemm_shape": (_i32, [_i32, _i32, _i32, _i32, _i32, _i32]),
     "ss_hip_matvec_q4_0": (_i32, [_vp, _vp, _vp, _vp, _i32, _i32, _vp]),
     "ss_hip_matvec_q8_0": (_i32, [_vp, _vp, _vp, _vp, _i32, _i32, _vp]),
     "ss_hip_matvec_q4_k": (_i32, [_vp, _vp, _vp, _vp, _i32, _i32, _vp]),

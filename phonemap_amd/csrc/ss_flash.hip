@@ -89,7 +89,6 @@ typedef __attribute__((address_space(3))) v4s* lds_v4s_t;
 typedef __attribute__((address_space(1))) void* gbl_ptr_t;
 
 constexpr int kBlk = 32;            // keys per block, query rows per tile
-constexpr int kCompute = 256;       // compute units
 constexpr int kFullRows = 8;        // fp16 launches of fewer tokens sum in the FULL form
 constexpr float kLog2e = 1.44269504088896340736f, kLog2eLow = 1.92596299e-8f;   // log2 e = their sum
 constexpr float kPExp = 12.0f, kPScale = 4096.0f;   // P is held times 2^12
@@ -623,7 +622,7 @@ hipError_t launch_flash(int group, int kv_type, const AttnArgs& a, hipStream_t s
 hipError_t launch_attention_rows(int head_dim, int group, int kv_type, const AttnArgs& a, hipStream_t s) {
   if (a.n_tok < 1 || a.n_kv_heads < 1 || a.max_seq < 1 || !a.q || !a.out || !a.kc || !a.vc ||
       (kv_type && (!a.ks || !a.vs)) || a.tok_q % 4 ||
-      a.tok_o % 4)
+      a.tok_o % 4 || a.n_cu <= 0)
     return hipErrorInvalidValue;
   // Up to 64 keys: two key groups, one step (32 heads x 32 tokens at head_dim
   // 128: 6.5 us, with four groups 7.8). More row tiles than compute units at
@@ -637,7 +636,7 @@ hipError_t launch_attention_rows(int head_dim, int group, int kv_type, const Att
   if (head_dim == 64) return two_blocks ? launch_flash<64, 1, 2>(group, kv_type, a, s) : launch_flash<64, 1, 4>(group, kv_type, a, s);
   if (head_dim == 128) {
     if (two_blocks) return launch_flash<128, 1, 2>(group, kv_type, a, s);
-    return tiles > kCompute && (kv_type || a.n_tok >= kFullRows) ? launch_flash<128, 2, 4>(group, kv_type, a, s) : launch_flash<128, 1, 4>(group, kv_type, a, s);
+    return tiles > a.n_cu && (kv_type || a.n_tok >= kFullRows) ? launch_flash<128, 2, 4>(group, kv_type, a, s) : launch_flash<128, 1, 4>(group, kv_type, a, s);
   }
   if (head_dim == 256) return launch_flash<256, 1, 2, 2>(group, kv_type, a, s);   // Gemma
   return hipErrorInvalidValue;

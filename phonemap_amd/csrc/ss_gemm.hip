@@ -951,17 +951,6 @@ hipError_t launch_rs(const GemmArgs& a, int nu, hipStream_t s) {
   return hipGetLastError();
 }
 
-int device_cus() {
-  static int n = 0;
-  if (!n) {
-    int dev = 0;
-    hipDeviceProp_t p;
-    if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&p, dev) == hipSuccess) n = p.multiProcessorCount;
-    if (n <= 0) n = 256;
-  }
-  return n;
-}
-
 // The workgroup shape: 1 for k_gemm_ks, else k_gemm_rs's RW. Every shape runs
 // one workgroup per compute unit at a time, so a launch takes its rounds of
 // workgroups times what one round takes: at 4096 columns 10 us (two matrices
@@ -970,25 +959,27 @@ int device_cus() {
 // every token count from 8 to 512 of 4096, 11008 and 1024 rows but for ties
 // (4096 rows, 77 / 128 / 256 / 512 tokens: 25.1, 27.1, 48.8, 89.3 us with 1;
 // 26.3, 27.3, 32.7, 58.3 with 2; 36.8, 37.5, 40.9, 49.7 with 4).
-int pick_shape(int rows, int T, int nmat, int nu, int n_cu) {
+// rw: the most row tiles the type has.
+int pick_shape(int rows, int T, int nmat, int nu, int rw, int n_cu) {
   auto rounds = [&](int r, int t) {
     const long wg = (long)((rows + r - 1) / r) * ((T + t - 1) / t);
     return (wg + n_cu - 1) / n_cu;
   };
   const long c1 = rounds(32, 32) * (nmat == 2 ? 18 : 10);
   const long c2 = rounds(64 / nmat, 64) * 24, c4 = rounds(128 / nmat, 64) * 38;
-  if (nu > kRsUnits || (c1 <= c2 && c1 <= c4)) return 1;
-  return c2 <= c4 ? 2 : 4;
+  if (nu > kRsUnits || (c1 <= c2 && (rw < 4 || c1 <= c4))) return 1;
+  return rw < 4 || c2 <= c4 ? 2 : 4;
 }
+// Q4_1 and Q5_1 (a scale and a minimum of 16 bits per block) would spill with RW 4
+constexpr int most_row_tiles(int qt) { return qt == kQ4_1 || qt == kQ5_1 ? 2 : 4; }
 
 template <int QT, int NMAT, int EPI>
 hipError_t launch_shape(const GemmArgs& a, int nu, hipStream_t s) {
-  switch (pick_shape(a.rows, a.T, NMAT, nu, device_cus())) {
+  constexpr int RW = most_row_tiles(QT);
+  switch (pick_shape(a.rows, a.T, NMAT, nu, RW, a.n_cu)) {
     case 1: return launch_ks<QT, NMAT, EPI>(a, nu, s);
     case 2: return launch_rs<QT, NMAT, EPI, 2>(a, nu, s);
-    default:
-      // Q4_1 and Q5_1 (a scale and a minimum of 16 bits per block) would spill with RW 4
-      return launch_rs<QT, NMAT, EPI, QT == kQ4_1 || QT == kQ5_1 ? 2 : 4>(a, nu, s);
+    default: return launch_rs<QT, NMAT, EPI, RW>(a, nu, s);
   }
 }
 
@@ -1013,6 +1004,10 @@ const int64_t* gemm_launch_counts() {
   return snap;
 }
 
+int gemm_shape(int rows, int T, int nmat, int cols, int type, int n_cu) {
+  return pick_shape(rows, T, nmat, (cols / 32 + kSUnit - 1) / kSUnit, most_row_tiles(dev_type(type)), n_cu);
+}
+
 hipError_t launch_sumsq(const float* x, int cols, int T, float* ssq, hipStream_t s) {
   if (T <= 0 || cols <= 0 || cols % 4) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_sumsq, dim3(T), dim3(256), 0, s, x, cols, cols, ssq);
@@ -1020,7 +1015,8 @@ hipError_t launch_sumsq(const float* x, int cols, int T, float* ssq, hipStream_t
 }
 
 hipError_t launch_gemm(int epi, const GemmArgs& a, hipStream_t s) {
-  if (a.T <= 0 || a.rows <= 0 || a.cols <= 0 || a.cols % 32 || a.ldy < a.rows || a.ldx < a.cols || a.ldx % 4 || !a.xs)
+  if (a.T <= 0 || a.rows <= 0 || a.cols <= 0 || a.cols % 32 || a.ldy < a.rows || a.ldx < a.cols || a.ldx % 4 || !a.xs ||
+      a.n_cu <= 0)
     return hipErrorInvalidValue;
   if (epi != EPI_STORE && epi != EPI_ADD && epi != EPI_SWIGLU) return hipErrorInvalidValue;
   const int t = dev_type(a.type);

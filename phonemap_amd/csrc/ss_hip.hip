@@ -425,6 +425,7 @@ int32_t ss_hip_gemm(ss_hip_ctx_t* c, float* y, const void* w, const float* x, co
   a.cols = cols;
   a.T = n_tokens;
   a.type = type;
+  a.n_cu = c->n_cu;
   HIP_TRY(ssk::launch_gemm(accumulate ? ssk::EPI_ADD : ssk::EPI_STORE, a, s));
   return 0;
 }
@@ -567,6 +568,7 @@ int32_t attention_rows(ss_hip_ctx_t* c, float* out, const float* q, const void* 
   a.n_tok = n_tokens;
   a.pos0 = pos0;
   a.tok_q = a.tok_o = n_heads * head_dim;
+  a.n_cu = c->n_cu;
   HIP_TRY(ssk::launch_attention_rows(head_dim, group, kv_type, a, pick(c, stream)));
   return 0;
 }
@@ -1547,6 +1549,7 @@ ssk::GemmArgs gemm_args(ss_hip_model* m, const void* w, int type, int rows, int 
   a.cols = cols;
   a.T = T;
   a.type = ssk::dev_type(type);
+  a.n_cu = m->ctx->n_cu;
   return a;
 }
 
@@ -1591,6 +1594,7 @@ int32_t enqueue_layer_rows(ss_hip_model* m, int l, const DevLayer& ly, int T, in
   at.part_o = m->att_o;
   at.part_ml = m->att_ml;
   at.n_tok = T;
+  at.n_cu = m->ctx->n_cu;
   at.softcap = m->attn_softcap;   // (:446-448)
   at.softcap_inv = m->attn_softcap > 0.f ? 1.0f / m->attn_softcap : 0.f;
   HIP_TRY(timed(m, PC_OTHER, 0, [&] { return ssk::launch_attention_rows(m->hd, m->group, m->kv_type, at, s); }));
@@ -2017,6 +2021,12 @@ uint64_t ss_hip_model_bytes(const ss_hip_model_t* m) { return m ? m->bytes : 0; 
 uint64_t ss_hip_model_host_bytes(const ss_hip_model_t* m) { return m ? m->host_bytes : 0; }
 
 int32_t ss_hip_model_launch(const ss_hip_model_t* m) { return m ? m->launch : -1; }
+
+// The shape a product of these sizes runs in on a device of n_cu compute units
+// (row tiles per workgroup); tests hold the rule to it. Not in the public header.
+int32_t ss_hip_gemm_shape(int32_t rows, int32_t n_tokens, int32_t two_matrices, int32_t cols, int32_t type, int32_t n_cu) {
+  return ssk::gemm_shape(rows, n_tokens, two_matrices ? 2 : 1, cols, type, n_cu);
+}
 
 int32_t ss_hip_gemm_launch_counts(int64_t* out, int32_t n) {
   if (!out || n < 0) return fail(kErrParams, "gemm_launch_counts: null output");

@@ -107,6 +107,7 @@ struct GemmArgs {
                              // two fp16 parts, with their scales and sums
   int ldx, ldy, rows, cols, T, type;
   int act;                   // EPI_SWIGLU: 0 SiLU, 1 GELU (Gemma's GeGLU)
+  int n_cu;                  // compute units
 };
 // 16-bit words of GemmArgs::xs for T tokens of cols columns
 // (whole tiles of 32 tokens and units of 256 columns: x in two parts, and per
@@ -139,6 +140,7 @@ struct AttnArgs {
   int n_tok;                 // prompt rows (launch_attention_rows): token z at position
   int pos0;                  // pos0 + z,
   int tok_q, tok_o;          // its query at q + z*tok_q, its output at out + z*tok_o
+  int n_cu;                  // compute units
 };
 
 // The attention softcap (layer_scheduler.c:446-448, tensor.c:194-200) of a
@@ -188,6 +190,8 @@ hipError_t launch_gemm(int epi, const GemmArgs& a, hipStream_t s);
 // 1: several): index 2 * epilogue_slot + kernel.
 constexpr int kGemmVariants = 6;
 const int64_t* gemm_launch_counts();
+// The workgroup shape of a product (nmat 2: EPI_SWIGLU): row tiles per workgroup, 1, 2 or 4.
+int gemm_shape(int rows, int T, int nmat, int cols, int type, int n_cu);
 bool attention_supported(int head_dim, int group);
 // positions one attention workgroup covers in one round of loads
 int attn_round_positions(int head_dim, int group);

@@ -1,5 +1,6 @@
-"""The compiled prompt products (k_gemm_rs in the built library), read from its
-gfx950 code object with the LLVM tools that built it: no GPU."""
+"""The prompt products without a GPU: the rule that chooses their workgroups, and
+k_gemm_rs as compiled, read from the built library's gfx950 code object with
+the LLVM tools that built it."""
 import os
 import re
 import struct
@@ -51,3 +52,22 @@ def test_products_keep_their_sums_in_registers(code_object):
         scratch = int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", k).group(1))
         assert scratch <= 16, (name, scratch)
     assert seen >= 50   # ten block types, three epilogues, two shapes (two types: one)
+
+
+def _rounds(rows, T, r, t, n_cu):
+    return -(-(-(-rows // r) * -(-T // t)) // n_cu)
+
+
+@pytest.mark.parametrize("n_cu", [64, 256, 304])
+@pytest.mark.parametrize("two", [0, 1])
+def test_the_shape_is_the_cheapest_one_the_type_has(n_cu, two):
+    """At 4096 columns a round of workgroups takes 10 us with one row tile (18
+    for two matrices), 24 with two, 38 with four; Q4_1 and Q5_1 have no four."""
+    L, m = pm.lib(), 1 + two
+    for qt, most in [(2, 4), (8, 4), (9, 4), (12, 4), (3, 2), (7, 2)]:
+        for rows in (40, 1024, 2816, 4096, 4100, 11008, 14336):
+            for T in (1, 33, 77, 128, 200, 324, 330, 340, 512):
+                cost = {1: _rounds(rows, T, 32, 32, n_cu) * (18 if two else 10), 2: _rounds(rows, T, 64 // m, 64, n_cu) * 24,
+                        4: _rounds(rows, T, 128 // m, 64, n_cu) * 38}
+                got = L.ss_hip_gemm_shape(rows, T, two, 4096, qt, n_cu)
+                assert got <= most and cost[got] == min(c for s, c in cost.items() if s <= most), (qt, rows, T, got, cost)
