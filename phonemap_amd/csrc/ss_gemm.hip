@@ -529,13 +529,14 @@ struct KWork {
 constexpr int kKsUnits = 128;   // units whose inverse scales go through LDS; past them, from memory
 
 template <int QT, int NMAT, int EPI, int TT, int KW>
-__global__ void __launch_bounds__(KW * 64) k_gemm_ks(const GemmArgs a, int nu) {
+__global__ void __launch_bounds__(KW * 64, 2) k_gemm_ks(const GemmArgs a, int nu) {
   constexpr int SUMS = sum_steps<QT>();
   constexpr int KS = KW / NMAT;   // column slices
   constexpr int kThreads = KW * 64, kPer = 1024 / kThreads;   // outputs of a tile per thread
   __shared__ float red[KW][16][kWave];
   __shared__ float rn[TT][kThreads];
-  __shared__ float inv_lds[TT * kKsUnits * kSTok];   // [TT][nu][32]
+  constexpr int kUnits = KW < kSW ? KS : kKsUnits;
+  __shared__ float inv_lds[TT * kUnits * kSTok];   // [TT][nu][32]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int slice = wave % KS;
@@ -601,7 +602,7 @@ __global__ void __launch_bounds__(KW * 64) k_gemm_ks(const GemmArgs a, int nu) {
     const size_t at = (size_t)min(tile0 + tt, ntile - 1) * nu * kSTok;
     float ss = 0.f;
     for (int i = tid; i < nu * kSTok; i += kThreads) {
-      if (nu <= kKsUnits) inv_lds[tt * nu * kSTok + i] = xs.inv[at + i];
+      if (nu <= kUnits) inv_lds[tt * nu * kSTok + i] = xs.inv[at + i];
       ss += xs.ssq[at + i];
     }
     rn[tt][tid] = ss;
@@ -624,7 +625,7 @@ __global__ void __launch_bounds__(KW * 64) k_gemm_ks(const GemmArgs a, int nu) {
     blocks(std::integral_constant<int, 1>{});
     blocks(std::integral_constant<int, 2>{});
     blocks(std::integral_constant<int, 3>{});
-    if (nu <= kKsUnits)
+    if (nu <= kUnits)
       pipe.finish(acc, f.w, f.sum, inv_lds + u * kSTok + 4 * kg, nu * kSTok, true);
     else
       pipe.finish(acc, f.w, f.sum, xs.inv + ((size_t)tile0 * nu + u) * kSTok + 4 * kg, nu * kSTok, true);
@@ -938,7 +939,12 @@ template <int QT, int NMAT, int EPI>
 hipError_t launch_ks(const GemmArgs& a, int nu, hipStream_t s) {
   count_launch<EPI>(0);
   const dim3 grid((a.rows + 31) / 32, (a.T + kSTok - 1) / kSTok);
-  hipLaunchKernelGGL((k_gemm_ks<QT, NMAT, EPI, 1, kSW>), grid, dim3(kSW * 64), 0, s, a, nu);
+  if (nu == 1)
+    hipLaunchKernelGGL((k_gemm_ks<QT, NMAT, EPI, 1, NMAT>), grid, dim3(NMAT * 64), 0, s, a, nu);
+  else if (nu == 2)
+    hipLaunchKernelGGL((k_gemm_ks<QT, NMAT, EPI, 1, 2 * NMAT>), grid, dim3(2 * NMAT * 64), 0, s, a, nu);
+  else
+    hipLaunchKernelGGL((k_gemm_ks<QT, NMAT, EPI, 1, kSW>), grid, dim3(kSW * 64), 0, s, a, nu);
   return hipGetLastError();
 }
 
@@ -960,11 +966,24 @@ hipError_t launch_rs(const GemmArgs& a, int nu, hipStream_t s) {
 // (4096 rows, 77 / 128 / 256 / 512 tokens: 25.1, 27.1, 48.8, 89.3 us with 1;
 // 26.3, 27.3, 32.7, 58.3 with 2; 36.8, 37.5, 40.9, 49.7 with 4).
 // rw: the most row tiles the type has.
+//
+// Up to 512 columns k_gemm_ks has a wave per unit and matrix, so 8 / nu
+// workgroups of one matrix run on a compute unit at a time. One unit: always
+// (Q8_0 8192 x 256, 33 / 512 tokens: 9.3 and 20.4 us; with 8 waves of which one
+// works 14.4, with RW 4 24.8). Two: a round takes 4.5 to 6 us, RW 2's at least
+// as long and RW 4's 6.5 (8192 x 512, 512 tokens: 31.4 us, RW 4 25.6; 4100 x
+// 512, 100 tokens: 10.6 and 14.3).
 int pick_shape(int rows, int T, int nmat, int nu, int rw, int n_cu) {
-  auto rounds = [&](int r, int t) {
-    const long wg = (long)((rows + r - 1) / r) * ((T + t - 1) / t);
-    return (wg + n_cu - 1) / n_cu;
+  auto rounds = [&](int r, int t, int per_cu = 1) {
+    const long wg = (long)((rows + r - 1) / r) * ((T + t - 1) / t), slots = (long)per_cu * n_cu;
+    return (wg + slots - 1) / slots;
   };
+  if (nu == 1) return 1;
+  if (nu == 2) {
+    const long c1 = rounds(32, 32, 4 / nmat) * 50, c2 = rounds(64 / nmat, 64) * 52, c4 = rounds(128 / nmat, 64) * 65;
+    if (c1 <= c2 && (rw < 4 || c1 <= c4)) return 1;
+    return rw < 4 || c2 <= c4 ? 2 : 4;
+  }
   const long c1 = rounds(32, 32) * (nmat == 2 ? 18 : 10);
   const long c2 = rounds(64 / nmat, 64) * 24, c4 = rounds(128 / nmat, 64) * 38;
   if (nu > kRsUnits || (c1 <= c2 && (rw < 4 || c1 <= c4))) return 1;

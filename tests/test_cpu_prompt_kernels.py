@@ -71,3 +71,16 @@ def test_the_shape_is_the_cheapest_one_the_type_has(n_cu, two):
                         4: _rounds(rows, T, 128 // m, 64, n_cu) * 38}
                 got = L.ss_hip_gemm_shape(rows, T, two, 4096, qt, n_cu)
                 assert got <= most and cost[got] == min(c for s, c in cost.items() if s <= most), (qt, rows, T, got, cost)
+
+
+@pytest.mark.parametrize("cols", [32, 256, 288, 512])
+def test_the_shape_with_few_columns(cols):
+    """One unit of 256 columns: always one row tile, a wave per workgroup; two:
+    four row tiles where the smaller workgroups would take two rounds."""
+    L = pm.lib()
+    for T in (1, 130, 330, 512):
+        for rows in (512, 4100, 8192):
+            waves = 4 * 256   # workgroups of a round, two units
+            one = -(-(-(-rows // 32) * -(-T // 32)) // waves) == 1
+            assert L.ss_hip_gemm_shape(rows, T, 0, cols, 8, 256) == (1 if cols <= 256 or one else 4)
+            assert L.ss_hip_gemm_shape(rows, T, 0, cols, 3, 256) == 1

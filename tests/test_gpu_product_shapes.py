@@ -59,8 +59,10 @@ def _check(hip, qtype, rows, cols, T, shape):
 @pytest.mark.parametrize("qtype", TYPES32)
 @pytest.mark.parametrize("rows,cols,T,shape", [
     (17, 32, 2, 1), (40, 2080, 33, 1), (16, 33056, 3, 1),     # one row tile; 130 units
-    (4100, 288, 130, 2),                                       # two row tiles, 2 units for 4 column groups
-    (4100, 1056, 200, 4),                                      # four row tiles, 5 units for 2 column groups
+    (70, 256, 70, 1), (70, 288, 70, 1), (4100, 288, 130, 1),  # a workgroup of one wave, of two
+    (4100, 544, 130, 2),                                       # two row tiles, 3 units for 4 column groups
+    (4100, 288, 330, 4),                                       # four row tiles, 2 units for 2 column groups
+    (4100, 1056, 200, 4),                                      # 5 units for 2 column groups
 ])
 def test_product_shapes_block32(hip, qtype, rows, cols, T, shape):
     if qtype in (Q4_1, Q5_1) and shape == 4:   # not theirs: one row tile beats two here
@@ -70,7 +72,8 @@ def test_product_shapes_block32(hip, qtype, rows, cols, T, shape):
 
 @pytest.mark.parametrize("qtype", TYPES_K)
 @pytest.mark.parametrize("rows,cols,T,shape", [
-    (17, 256, 2, 1), (40, 2304, 33, 1), (4100, 512, 130, 2), (4100, 1280, 200, 4),
+    (17, 256, 2, 1), (70, 512, 70, 1), (40, 2304, 33, 1), (4100, 512, 130, 1), (4100, 768, 130, 2), (4100, 512, 330, 4),
+    (4100, 1280, 200, 4),
 ])
 def test_product_shapes_kquants(hip, qtype, rows, cols, T, shape):
     _check(hip, qtype, rows, cols, T, shape)
