@@ -694,6 +694,10 @@ __global__ void __launch_bounds__(KW * 64, 2) k_gemm_ks(const GemmArgs a, int nu
 // One barrier per stage: past it every wave's loads of the next stage have
 // landed, and every wave has the last of the stage before in registers, so
 // that its array can be refilled.
+// The counts of wait_loads hold only while the compiler
+// issues the code loads counted beside the stages': one more waits for more,
+// one fewer would let x be read before it is here. A test without a GPU reads
+// the compiled loops for it (at most two stages in flight at a barrier).
 //
 // Bound: the vector and matrix instructions of two waves per SIMD. A block of
 // 8 waves takes 0.30 us with nothing but its LDS reads, MFMAs and vector
@@ -806,7 +810,8 @@ __global__ void __launch_bounds__(kSW * 64) k_gemm_rs(const GemmArgs a, int nu) 
     ss += __shfl_xor(ss, 32, kWave);
     if (lane < kSTok) psum[tt][wave][lane] = ss;
   }
-  __syncthreads();   // waits for every load so far, the four stages among them
+  vm_drain();        // every load so far, the four stages among them
+  __syncthreads();
   if (tid < TT * kSTok) {
     float ss = 0.f;
 #pragma unroll

@@ -84,3 +84,91 @@ def test_the_shape_with_few_columns(cols):
             one = -(-(-(-rows // 32) * -(-T // 32)) // waves) == 1
             assert L.ss_hip_gemm_shape(rows, T, 0, cols, 8, 256) == (1 if cols <= 256 or one else 4)
             assert L.ss_hip_gemm_shape(rows, T, 0, cols, 3, 256) == 1
+
+
+# ---- k_gemm_rs's counted waits ------------------------------------------------
+# x comes to LDS by direct loads, four per stage and wave; at a barrier of the
+# loop at most the two youngest stages may still be in flight, outside it none.
+VMEM = re.compile(r"(global|buffer|scratch|flat)_(load|store|atomic)")
+
+
+def _instructions(text):
+    """{kernel: [(address, instruction, branch target or None)]} of a disassembly."""
+    out, cur = {}, None
+    for line in text.splitlines():
+        m = re.match(r"([0-9a-f]+) <(.*)>:", line)
+        if m:
+            base, cur = int(m.group(1), 16), out.setdefault(m.group(2), [])
+        elif cur is not None and "//" in line:
+            ins, rest = line.strip().split("//", 1)
+            to = re.search(r"<[^>+]*(?:\+0x([0-9a-f]+))?>", rest)
+            target = base + int(to.group(1) or "0", 16) if to and "branch" in ins else None
+            cur.append((int(rest.split(":")[0], 16), ins.strip(), target))
+    return out
+
+
+def _in_flight(code):
+    """[(address of a barrier, direct loads to LDS that may be in flight there,
+    whether it is in the main loop)]. Forward data flow: each load with the
+    least number of vector memory instructions after it on any path; a wait for
+    all but N of them ends the loads with N or more."""
+    at = {a: i for i, (a, _, _) in enumerate(code)}
+    loops = [(code[at[t]][0], a) for a, _, t in code if t is not None and t <= a]
+    main = max(loops, key=lambda l: sum("s_barrier" in i and l[0] <= a <= l[1] for a, i, _ in code))
+    joins = {at[t] for _, _, t in code if t is not None}
+    before, work, seen = {0: {}}, [0], {}
+    while work:
+        i = work.pop()
+        state = dict(before[i])
+        while True:
+            a, ins, target = code[i]
+            if VMEM.match(ins):
+                state = {k: min(n + 1, 64) for k, n in state.items()}
+                if "_lds_" in ins:   # an older one of the same instruction keeps its place
+                    for g in (2, 1, 0):
+                        if (a, g) in state:
+                            state[(a, g + 1)] = state.pop((a, g))
+                    state[(a, 0)] = 0
+            m = re.match(r"s_waitcnt.*vmcnt\((\d+)\)", ins)
+            if m:
+                state = {k: n for k, n in state.items() if n < int(m.group(1))}
+            if ins.startswith("s_barrier"):
+                seen[a] = max(seen.get(a, 0), len(state))
+            nxt = [] if ins.startswith(("s_endpgm", "s_branch")) else [i + 1]
+            if target is None and nxt and i + 1 not in joins:
+                i += 1
+                continue
+            for j in nxt + ([at[target]] if target is not None else []):
+                old = before.get(j)
+                new = dict(state) if old is None else {k: min(old.get(k, 99), state.get(k, 99)) for k in {**old, **state}}
+                if new != old:
+                    before[j] = new
+                    work.append(j)
+            break
+    return [(a, n, main[0] <= a <= main[1]) for a, n in sorted(seen.items())]
+
+
+def _too_many(code):
+    return [(a, n) for a, n, loop in _in_flight(code) if n > (8 if loop else 0)]
+
+
+@pytest.fixture(scope="module")
+def products(code_object):
+    text = _tool("llvm-objdump", "-d", "--no-show-raw-insn", code_object)
+    return {k: v for k, v in _instructions(text).items() if "k_gemm_rs" in k}
+
+
+def test_x_has_landed_at_every_barrier(products):
+    assert len(products) >= 50
+    for name, code in products.items():
+        assert sum("_lds_" in i for _, i, _ in code) >= 32, name   # four stages before the loop, four in it
+        assert not _too_many(code), (name, _too_many(code))
+
+
+def test_a_missing_load_would_be_seen(products):
+    """The same reading of a listing without the loop's code loads: the waits
+    then count direct loads in their place."""
+    for name, code in products.items():
+        loop = [a for a, n, inside in _in_flight(code) if inside]
+        fewer = [(a, "s_nop 0" if i.startswith("buffer_load") and a > loop[0] else i, t) for a, i, t in code]
+        assert _too_many(fewer), name
