@@ -298,7 +298,8 @@ int32_t ss_hip_eval_token(ss_hip_model_t *m, int32_t token, int32_t pos, float *
 /* ss_scheduler_prefill (layer_scheduler.h:119). A prompt of at least the
  * batch threshold runs as matrix products over chunks of up to 512 tokens;
  * shorter prompts run token by token. The default threshold is 4 tokens, more
- * over a prefix longer than 4096 positions (up to 8 with the fp16 cache). */
+ * over a prefix longer than 4096 positions (2048 at head_dim 256), up to 8
+ * with the fp16 cache. */
 int32_t ss_hip_eval_prompt(ss_hip_model_t *m, const int32_t *tokens, int32_t n,
                            int32_t start_pos, float *logits_host, int32_t *argmax_out);
 /* Batch threshold of ss_hip_eval_prompt: 0 restores the default, a negative
@@ -308,7 +309,8 @@ int32_t ss_hip_set_prompt_batch(ss_hip_model_t *m, int32_t min_tokens);
 /* ss_scheduler_embed (layer_scheduler.c:805-911): tokens at positions
  * 0..n-1 (the cache is overwritten there), every token's final hidden state
  * through the output norm, mean-pooled and L2-normalised into out_host[hidden].
- * With the fp16 cache the prompt runs as matrix products. */
+ * The prompt runs as matrix products, unless ss_hip_set_prompt_batch was given
+ * a negative value. */
 int32_t ss_hip_embed(ss_hip_model_t *m, const int32_t *tokens, int32_t n, float *out_host);
 /* ss_hip_sample_logits over the logits of the model's last evaluated token
  * (left in HBM by ss_hip_eval_token / ss_hip_eval_prompt, which need not

@@ -994,7 +994,8 @@ int pick_shape(int rows, int T, int nmat, int nu, int rw, int n_cu) {
   if (nu > kRsUnits || (c1 <= c2 && (rw < 4 || c1 <= c4))) return 1;
   return rw < 4 || c2 <= c4 ? 2 : 4;
 }
-// Q4_1 and Q5_1 (a scale and a minimum of 16 bits per block) would spill with RW 4
+// Q4_1 and Q5_1 (a scale and a minimum of 16 bits per block) run with at most
+// RW 2: RW 4 would keep 1040 bytes per lane of Q5_1 in scratch memory
 constexpr int most_row_tiles(int qt) { return qt == kQ4_1 || qt == kQ5_1 ? 2 : 4; }
 
 template <int QT, int NMAT, int EPI>

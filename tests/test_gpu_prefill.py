@@ -126,8 +126,9 @@ def test_embed_prompt_matches_oracle(mode):
 # oracle's prompt takes seconds.
 W70 = dict(n_layers=2, hidden=8192, n_heads=64, n_kv_heads=8, head_dim=128, ffn=28672, vocab=512,
            context_length=1024, seed=71, scale_mode=1)
-# ss_hip_gemm_launch_counts slots: 2 * epilogue (store, add, SwiGLU) + rows per wave - 1
-ADD_RG2 = 3
+# ss_hip_gemm_launch_counts slots: 2 * epilogue (store, add, SwiGLU) + kernel
+# (0: one row tile per workgroup, 1: several)
+ADD_SEVERAL = 3
 
 
 def _gemm_counts():
@@ -145,8 +146,8 @@ def test_prompt_at_70b_layer_width():
     oracle's prefill / forward (layer_scheduler.c:681-803, :571-679), the
     argmax equal, and the model responding to its input (the step-to-step
     guard of the full-shape tests). At d = 8192 and 512 tokens the Wo and
-    down products run with two row groups per wave (k_gemm_h EPI_ADD, RG 2),
-    which no smaller shape selects; the launch counters show that they ran."""
+    down products run with several row tiles per workgroup (k_gemm_rs EPI_ADD);
+    the launch counters show that they ran."""
     from tests.test_gpu_fullshape import Trace
     path = _model_file("w70", **W70)
     rng = np.random.default_rng(700)
@@ -169,6 +170,6 @@ def test_prompt_at_70b_layer_width():
             tok, pos = am, pos + 1
     om.close()
     tr.done()
-    ran = after[ADD_RG2] - before[ADD_RG2]
-    print("k_gemm_h EPI_ADD RG=2 launches during the prompt:", ran, flush=True)
+    ran = after[ADD_SEVERAL] - before[ADD_SEVERAL]
+    print("k_gemm_rs EPI_ADD launches during the prompt:", ran, flush=True)
     assert ran >= 2 * W70["n_layers"], (before, after)

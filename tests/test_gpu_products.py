@@ -10,9 +10,11 @@ cover a ragged token tile, one token, rows not a multiple of 16 and a
 Whole models (Q4_K layers with a Q6_K head as Q4_K_M files have, Q6_K,
 Q3_K, Q5_1 with Q4_1 / Q8_1 tables) evaluate a 300-token prompt as products,
 against the oracle's token-serial prefill, then decode: logits within 1e-3
-(fp16 cache; 5e-2 int8) of the oracle's at every step, with the distance to
-the fp64 model of tests/ref_model.py printed beside it (OracleBar; measured
-worst against the oracle 2.4e-4).
+(fp16 cache) of the oracle's at every step, with the distance to the fp64 model
+of tests/ref_model.py printed beside it (OracleBar; measured worst against the
+oracle 2.4e-4). With the int8 cache 8e-3: a value on the edge between two codes
+may fall either way, which moves one position by 1/127 of its scale (measured
+worst 9.5e-4).
 """
 import ctypes as C
 
@@ -88,22 +90,29 @@ SPECS = {
 KNOWN = {}
 
 
+def _launches():
+    out = (C.c_int64 * 6)()
+    assert api._lib().ss_hip_gemm_launch_counts(out, 6) == 0
+    return sum(out)
+
+
 @pytest.mark.parametrize("kv", ["f16", "int8"])
 @pytest.mark.parametrize("spec", sorted(SPECS))
 def test_long_prompt_as_products(tmp_path, spec, kv):
-    """A 300-token prompt in one chunk of products (fp16 cache), or token by
-    token (int8 cache, where the products do not run), then decode steps."""
+    """A 300-token prompt in one chunk of products, then decode steps."""
     print("products model", spec, kv, flush=True)
     path = str(tmp_path / (spec + ".gguf"))
     api.write_synthetic_gguf(path, api.SynthSpec(**SPECS[spec]))
     prompt = np.random.default_rng(9).integers(3, 900, 300).tolist()
     om = oracle.Model(path, 400, kv)
     rm = RefModel(path, 400, kv)
-    tol = TOL if kv == "f16" else 5e-2
+    tol = TOL if kv == "f16" else 8e-3
     bar = OracleBar("products %s %s" % (spec, kv), tol,
                     {k[2]: v for k, v in KNOWN.items() if k[:2] == (spec, kv)})
     with api.Model(path, max_context=400, kv=kv) as m:
+        before = _launches()
         lg, am = m.eval_prompt(prompt, 0)
+        assert _launches() - before == 4 * SPECS[spec]["n_layers"]   # four products a layer
         olg = om.prefill(prompt, 0)
         bar.check("prompt", lg, olg, rm.prefill(prompt, 0))
         assert am == oracle.argmax(olg)
