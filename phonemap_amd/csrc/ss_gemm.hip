@@ -61,29 +61,15 @@ typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 template <int QT>
 struct PQ {
   static constexpr int kLay = code_bytes_of(QT) == 16 ? 2 : 8;
-  static constexpr bool kGroups = QT == kQ2K || QT == kQ3K || QT == kQ6K;
-  static constexpr bool kMin =
-      QT == kQ4_1 || QT == kQ5_1 || QT == kQ2K || QT == kQ3K || QT == kQ4K || QT == kQ5K;
 };
 
-// (A_g, B_g) of a block from its scale entry e (16 bits, or 32 for Q4_1 /
-// Q5_1 / Q8_1) and, for the K-quants, its super-block word sup.
+// A of a block from its scale entry e (16 bits, or 32 for Q4_1 / Q5_1 / Q8_1)
 template <int QT>
-__device__ __forceinline__ void block_affine(uint32_t e, uint32_t sup, float (&A)[2], float (&B)[2]) {
-  if constexpr (QT == 2 || QT == 8) {
-    A[0] = A[1] = h2f((uint16_t)e);
-    B[0] = B[1] = 0.f;
-  } else if constexpr (QT == kQ4_1 || QT == kQ5_1) {
-    A[0] = A[1] = h2f((uint16_t)(e & 0xffffu));
-    B[0] = B[1] = -h2f((uint16_t)(e >> 16));
-  } else if constexpr (QT == kQ8_1) {
-    A[0] = A[1] = __uint_as_float(e);
-    B[0] = B[1] = 0.f;
-  } else {
-    kq_affine<QT>(e, sup, A, B);
-  }
+__device__ __forceinline__ float block_scale(uint32_t e) {
+  static_assert(!is_kq(QT), "the K-quants' scales: kq_affine, int_scale");
+  if constexpr (QT == kQ8_1) return __uint_as_float(e);
+  return h2f((uint16_t)(e & 0xffffu));
 }
-
 
 // Sum of squares of each token's x (one workgroup per token), for the
 // embedding's RMSNorm scale.
@@ -432,7 +418,7 @@ struct Pipe {
       codes(qn, wn, 0, n0, n1);
     if constexpr (QT == kQ6K) {   // one scale per 16-weight group
       float S[2], Z[2];
-      block_affine<QT>(w.entry(BLK), w.su, S, Z);
+      kq_affine<QT>(w.entry(BLK), w.su, S, Z);
 #pragma unroll
       for (int tt = 0; tt < TT; ++tt) {
         v16f q = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[tt][0], c0, v16f{}, 0, 0, 0);
@@ -456,12 +442,11 @@ struct Pipe {
         for (int tt = 0; tt < TT; ++tt) part[tt] = q[tt];
       } else {
         if constexpr (BLK > 0) add_last<BLK>();
-        float S[2], Z[2];
-        block_affine<QT>(w.entry(BLK), 0u, S, Z);
+        const float S = block_scale<QT>(w.entry(BLK));
 #pragma unroll
-        for (int tt = 0; tt + 1 < TT; ++tt) part[tt] = BLK > 0 ? fma16(S[0], q[tt], part[tt]) : q[tt] * S[0];
+        for (int tt = 0; tt + 1 < TT; ++tt) part[tt] = BLK > 0 ? fma16(S, q[tt], part[tt]) : q[tt] * S;
         p = q[TT - 1];
-        A = S[0];
+        A = S;
       }
     }
     c0 = n0;
@@ -528,15 +513,15 @@ struct KWork {
 // before; Q4_K at 77 tokens 58 -> 26.5 us).
 constexpr int kKsUnits = 128;   // units whose inverse scales go through LDS; past them, from memory
 
-template <int QT, int NMAT, int EPI, int TT, int KW>
+template <int QT, int NMAT, int EPI, int KW>
 __global__ void __launch_bounds__(KW * 64, 2) k_gemm_ks(const GemmArgs a, int nu) {
   constexpr int SUMS = sum_steps<QT>();
   constexpr int KS = KW / NMAT;   // column slices
   constexpr int kThreads = KW * 64, kPer = 1024 / kThreads;   // outputs of a tile per thread
   __shared__ float red[KW][16][kWave];
-  __shared__ float rn[TT][kThreads];
+  __shared__ float rn[kThreads];
   constexpr int kUnits = KW < kSW ? KS : kKsUnits;
-  __shared__ float inv_lds[TT * kUnits * kSTok];   // [TT][nu][32]
+  __shared__ float inv_lds[kUnits * kSTok];   // [nu][32]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int slice = wave % KS;
@@ -544,51 +529,40 @@ __global__ void __launch_bounds__(KW * 64, 2) k_gemm_ks(const GemmArgs a, int nu
   const int ntk = ((a.cols >> 5) + kTB - 1) / kTB;
   const int ngroups = (a.rows + kRG - 1) / kRG;
   const int row0 = blockIdx.x * 32;
-  const int tile0 = blockIdx.y * TT, ntile = (a.T + kSTok - 1) / kSTok;
+  const int tile = blockIdx.y, ntile = (a.T + kSTok - 1) / kSTok;
   const KsView xs = ks_view(a.xs, ntile, nu);
 
   KView<QT> wv;
   wv.init(NMAT == 2 && wave >= KS ? a.w2 : a.w, row0 / kRG, ngroups, ntk, n, kg);
 
-  // this workgroup's token tiles as buffer views: a lane whose token is past
-  // T has an offset past the view and reads zero without touching memory
-  __amdgpu_buffer_rsrc_t xr[TT], sr[TT];
-  uint32_t xo[TT];
-#pragma unroll
-  for (int tt = 0; tt < TT; ++tt) {
-    const size_t at = (size_t)min(tile0 + tt, ntile - 1) * nu;
-    xr[tt] = __builtin_amdgcn_make_buffer_rsrc(xs.x + at * kSUnit * 4 * kWave, (short)0, nu * kSUnit * 4096, kBufferFlags);
-    if constexpr (SUMS > 0)
-      sr[tt] = __builtin_amdgcn_make_buffer_rsrc(xs.sum + at * SUMS * kWave, (short)0, nu * SUMS * 1024, kBufferFlags);
-    xo[tt] = (tile0 + tt) * kSTok + n < a.T ? lane * 16u : 0x7fffff00u;
-  }
+  // this workgroup's token tile as buffer views: a lane whose token is past T
+  // has an offset past the view and reads zero without touching memory
+  const size_t at = (size_t)tile * nu;
+  const __amdgpu_buffer_rsrc_t xr =
+      __builtin_amdgcn_make_buffer_rsrc(xs.x + at * kSUnit * 4 * kWave, (short)0, nu * kSUnit * 4096, kBufferFlags);
+  __amdgpu_buffer_rsrc_t sr;
+  if constexpr (SUMS > 0) sr = __builtin_amdgcn_make_buffer_rsrc(xs.sum + at * SUMS * kWave, (short)0, nu * SUMS * 1024, kBufferFlags);
+  const uint32_t xo = tile * kSTok + n < a.T ? lane * 16u : 0x7fffff00u;
   struct Frags {
-    v8h v[TT][4];   // (step, part) fragments of one block
+    v8h v[1][4];   // (step, part) fragments of one block
   };
   auto load_x = [&](Frags& f, int blk) {
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        f.v[tt][i] = __builtin_bit_cast(v8h, __builtin_amdgcn_raw_buffer_load_b128(xr[tt], xo[tt] + i * 1024, blk * 4096, 0));
+    for (int i = 0; i < 4; ++i)
+      f.v[0][i] = __builtin_bit_cast(v8h, __builtin_amdgcn_raw_buffer_load_b128(xr, xo + i * 1024, blk * 4096, 0));
   };
   // two units of codes, used in turn: each is refilled with the unit two
   // turns on as soon as it is used up
-  KWork<QT, TT> wa, wb;
-  auto load_w = [&](KWork<QT, TT>& f, int u) {
+  KWork<QT, 1> wa, wb;
+  auto load_w = [&](KWork<QT, 1>& f, int u) {
     u = min(u, nu - 1);   // past the end: reloaded, not used
     load_scales<QT>(f.w, wv, u);
     load_codes<QT>(f.q, wv, u, -1);
 #pragma unroll
     for (int s = 0; s < SUMS; ++s)
-#pragma unroll
-      for (int tt = 0; tt < TT; ++tt)
-        f.sum[s][tt] =
-            __builtin_bit_cast(v8h, __builtin_amdgcn_raw_buffer_load_b128(sr[tt], xo[tt], (u * SUMS + s) * 1024, 0));
+      f.sum[s][0] = __builtin_bit_cast(v8h, __builtin_amdgcn_raw_buffer_load_b128(sr, xo, (u * SUMS + s) * 1024, 0));
   };
-  v16f acc[TT];
-#pragma unroll
-  for (int tt = 0; tt < TT; ++tt) acc[tt] = v16f{};
+  v16f acc[1] = {v16f{}};
   Frags xa, xb;   // blocks of even and odd index
   const int u0 = min(slice, nu - 1);
   load_w(wa, u0);
@@ -597,20 +571,18 @@ __global__ void __launch_bounds__(KW * 64, 2) k_gemm_ks(const GemmArgs a, int nu
   load_w(wb, u0 + KS);
   // while those are in flight: the inverse scales into LDS, and each token's
   // sum of squares (thread: token tid % 32, units tid / 32, + KW * 2, ...)
-#pragma unroll
-  for (int tt = 0; tt < TT; ++tt) {
-    const size_t at = (size_t)min(tile0 + tt, ntile - 1) * nu * kSTok;
+  {
     float ss = 0.f;
     for (int i = tid; i < nu * kSTok; i += kThreads) {
-      if (nu <= kUnits) inv_lds[tt * nu * kSTok + i] = xs.inv[at + i];
-      ss += xs.ssq[at + i];
+      if (nu <= kUnits) inv_lds[i] = xs.inv[at * kSTok + i];
+      ss += xs.ssq[at * kSTok + i];
     }
-    rn[tt][tid] = ss;
+    rn[tid] = ss;
   }
   __syncthreads();
-  Pipe<QT, TT> pipe;
+  Pipe<QT, 1> pipe;
   pipe.init(wa.q, wa.w);
-  auto unit = [&](int u, KWork<QT, TT>& f, const KWork<QT, TT>& next) {
+  auto unit = [&](int u, KWork<QT, 1>& f, const KWork<QT, 1>& next) {
     const int un = min(u + KS, nu - 1);
     auto blocks = [&](auto kc) {   // blocks 2k and 2k + 1, then the x two on
       constexpr int k = 2 * decltype(kc)::value;
@@ -626,9 +598,9 @@ __global__ void __launch_bounds__(KW * 64, 2) k_gemm_ks(const GemmArgs a, int nu
     blocks(std::integral_constant<int, 2>{});
     blocks(std::integral_constant<int, 3>{});
     if (nu <= kUnits)
-      pipe.finish(acc, f.w, f.sum, inv_lds + u * kSTok + 4 * kg, nu * kSTok, true);
+      pipe.finish(acc, f.w, f.sum, inv_lds + u * kSTok + 4 * kg, 0, true);
     else
-      pipe.finish(acc, f.w, f.sum, xs.inv + ((size_t)tile0 * nu + u) * kSTok + 4 * kg, nu * kSTok, true);
+      pipe.finish(acc, f.w, f.sum, xs.inv + (at + u) * kSTok + 4 * kg, 0, true);
     load_w(f, u + 2 * KS);
   };
   int u = slice;
@@ -639,48 +611,39 @@ __global__ void __launch_bounds__(KW * 64, 2) k_gemm_ks(const GemmArgs a, int nu
   }
   if (u < nu) unit(u, wa, wb);
 
-  // the slices' partial sums, tile by tile, added in slice order: output
-  // tid + kThreads k of a tile is register j = wave + KW k, lane `lane`
-  float v[NMAT][TT][kPer];
+  // the slices' partial sums, added in slice order: output tid + kThreads k of
+  // the tile is register j = wave + KW k, lane `lane`
 #pragma unroll
-  for (int tt = 0; tt < TT; ++tt) {
-    if (tt) __syncthreads();
+  for (int j = 0; j < 16; ++j) red[wave][j][lane] = acc[0][j];
+  __syncthreads();
 #pragma unroll
-    for (int j = 0; j < 16; ++j) red[wave][j][lane] = acc[tt][j];
-    __syncthreads();
+  for (int k = 0; k < kPer; ++k) {
+    const int j = wave + KW * k;
+    float v[NMAT];
 #pragma unroll
-    for (int m = 0; m < NMAT; ++m)
+    for (int m = 0; m < NMAT; ++m) {
+      v[m] = 0.f;
 #pragma unroll
-      for (int k = 0; k < kPer; ++k) {
-        float s = 0.f;
-#pragma unroll
-        for (int q = 0; q < KS; ++q) s += red[m * KS + q][wave + KW * k][lane];
-        v[m][tt][k] = s;
-      }
-  }
-#pragma unroll
-  for (int tt = 0; tt < TT; ++tt)
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-      const int j = wave + KW * k;
-      const int tok = 8 * (j >> 2) + 4 * kg + (j & 3), t = (tile0 + tt) * kSTok + tok, row = row0 + n;
-      if (t >= a.T || row >= a.rows) continue;
-      float scale = 1.f;   // the RMSNorm scale of tensor.c:114-131
-      if (a.nw) {
-        float ss = 0.f;
-#pragma unroll
-        for (int q = 0; q < 2 * KW; ++q) ss += rn[tt][q * kSTok + tok];
-        scale = 1.0f / sqrtf(ss / (float)a.cols + a.eps);
-      }
-      float* yp = a.y + (size_t)t * a.ldy + row;
-      const float y = v[0][tt][k] * scale;
-      if constexpr (EPI == EPI_SWIGLU)
-        *yp = v[NMAT - 1][tt][k] * scale * (a.act == 1 ? gelu_tanh(y) : silu(y));   // layer_scheduler.c:529-547
-      else if constexpr (EPI == EPI_ADD)
-        *yp += y;
-      else
-        *yp = y;
+      for (int q = 0; q < KS; ++q) v[m] += red[m * KS + q][j][lane];
     }
+    const int tok = 8 * (j >> 2) + 4 * kg + (j & 3), t = tile * kSTok + tok, row = row0 + n;
+    if (t >= a.T || row >= a.rows) continue;
+    float scale = 1.f;   // the RMSNorm scale of tensor.c:114-131
+    if (a.nw) {
+      float ss = 0.f;
+#pragma unroll
+      for (int q = 0; q < 2 * KW; ++q) ss += rn[q * kSTok + tok];
+      scale = 1.0f / sqrtf(ss / (float)a.cols + a.eps);
+    }
+    float* yp = a.y + (size_t)t * a.ldy + row;
+    const float y = v[0] * scale;
+    if constexpr (EPI == EPI_SWIGLU)
+      *yp = v[NMAT - 1] * scale * (a.act == 1 ? gelu_tanh(y) : silu(y));   // layer_scheduler.c:529-547
+    else if constexpr (EPI == EPI_ADD)
+      *yp += y;
+    else
+      *yp = y;
+  }
 }
 
 // ---- longer prompts: x shared through LDS -----------------------------------
@@ -693,11 +656,13 @@ __global__ void __launch_bounds__(KW * 64, 2) k_gemm_ks(const GemmArgs a, int nu
 // named at compile time, three of them in flight ahead of the one in use.
 // One barrier per stage: past it every wave's loads of the next stage have
 // landed, and every wave has the last of the stage before in registers, so
-// that its array can be refilled.
-// The counts of wait_loads hold only while the compiler
-// issues the code loads counted beside the stages': one more waits for more,
-// one fewer would let x be read before it is here. A test without a GPU reads
-// the compiled loops for it (at most two stages in flight at a barrier).
+// that its array can be refilled. The counts of wait_loads hold only while the
+// compiler issues the code loads counted beside the stages': one more waits
+// for more, one fewer would let x be read before it is here. A test without a
+// GPU reads the compiled loops for it (at most two stages in flight at a
+// barrier). With RW 4 the compiler waits for everything once per unit besides,
+// where the next unit's scales are first used: no counted wait comes between
+// their load and that.
 //
 // Bound: the vector and matrix instructions of two waves per SIMD. A block of
 // 8 waves takes 0.30 us with nothing but its LDS reads, MFMAs and vector
@@ -945,11 +910,11 @@ hipError_t launch_ks(const GemmArgs& a, int nu, hipStream_t s) {
   count_launch<EPI>(0);
   const dim3 grid((a.rows + 31) / 32, (a.T + kSTok - 1) / kSTok);
   if (nu == 1)
-    hipLaunchKernelGGL((k_gemm_ks<QT, NMAT, EPI, 1, NMAT>), grid, dim3(NMAT * 64), 0, s, a, nu);
+    hipLaunchKernelGGL((k_gemm_ks<QT, NMAT, EPI, NMAT>), grid, dim3(NMAT * 64), 0, s, a, nu);
   else if (nu == 2)
-    hipLaunchKernelGGL((k_gemm_ks<QT, NMAT, EPI, 1, 2 * NMAT>), grid, dim3(2 * NMAT * 64), 0, s, a, nu);
+    hipLaunchKernelGGL((k_gemm_ks<QT, NMAT, EPI, 2 * NMAT>), grid, dim3(2 * NMAT * 64), 0, s, a, nu);
   else
-    hipLaunchKernelGGL((k_gemm_ks<QT, NMAT, EPI, 1, kSW>), grid, dim3(kSW * 64), 0, s, a, nu);
+    hipLaunchKernelGGL((k_gemm_ks<QT, NMAT, EPI, kSW>), grid, dim3(kSW * 64), 0, s, a, nu);
   return hipGetLastError();
 }
 
@@ -1023,10 +988,8 @@ hipError_t launch_type(int epi, const GemmArgs& a, hipStream_t s) {
 
 }  // namespace
 
-const int64_t* gemm_launch_counts() {
-  static int64_t snap[kGemmVariants];
-  for (int i = 0; i < kGemmVariants; ++i) snap[i] = g_gemm_launches[i].load(std::memory_order_relaxed);
-  return snap;
+void gemm_launch_counts(int64_t* out, int n) {
+  for (int i = 0; i < n && i < kGemmVariants; ++i) out[i] = g_gemm_launches[i].load(std::memory_order_relaxed);
 }
 
 int gemm_shape(int rows, int T, int nmat, int cols, int type, int n_cu) {

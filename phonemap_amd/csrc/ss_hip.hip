@@ -2030,8 +2030,7 @@ int32_t ss_hip_gemm_shape(int32_t rows, int32_t n_tokens, int32_t two_matrices, 
 
 int32_t ss_hip_gemm_launch_counts(int64_t* out, int32_t n) {
   if (!out || n < 0) return fail(kErrParams, "gemm_launch_counts: null output");
-  const int64_t* c = ssk::gemm_launch_counts();
-  for (int i = 0; i < n && i < ssk::kGemmVariants; ++i) out[i] = c[i];
+  ssk::gemm_launch_counts(out, n);
   return 0;
 }
 

@@ -189,7 +189,7 @@ hipError_t launch_gemm(int epi, const GemmArgs& a, hipStream_t s);
 // (EPI_STORE, EPI_ADD, EPI_SWIGLU) and kernel (0: one row tile per workgroup,
 // 1: several): index 2 * epilogue_slot + kernel.
 constexpr int kGemmVariants = 6;
-const int64_t* gemm_launch_counts();
+void gemm_launch_counts(int64_t* out, int n);
 // The workgroup shape of a product (nmat 2: EPI_SWIGLU): row tiles per workgroup, 1, 2 or 4.
 int gemm_shape(int rows, int T, int nmat, int cols, int type, int n_cu);
 bool attention_supported(int head_dim, int group);
