@@ -555,7 +555,9 @@ __device__ __forceinline__ int pow2_from(int n) {   // the power of two at or ab
 // softmax terms on; with room for 4096, 3000 equal entries took 100 us, 79 so.
 __global__ void __launch_bounds__(kThreads) k_smp_topk(const SampleArgs a) {
   __shared__ Shared sh;
-  __shared__ uint64_t ent[kCand];   // probability (its bits) << 32 | index
+  __shared__ uint64_t ent[kCand];   // sorted: probability (its bits) << 32 | index
+  __shared__ float p[kPairs];       // in pairs
+  __shared__ int idx[kPairs];
   __shared__ uint32_t th, cut;
   __shared__ int found;
   const Work w = work_of(a.probs, a.V, nullptr);
@@ -572,16 +574,23 @@ __global__ void __launch_bounds__(kThreads) k_smp_topk(const SampleArgs a) {
   const uint64_t target = top_p_target(a.top_p);
   const bool sorted = n > kPairs;
   const int pn = sorted ? pow2_from(n) : n;
-  for (int i = tid; i < pn; i += kThreads)
-    ent[i] = i < n ? (uint64_t)__float_as_uint(w.list[2 * i + 1] * inv) << 32 | __float_as_uint(w.list[2 * i]) : 0ull;
+  for (int i = tid; i < pn; i += kThreads) {
+    const float q = i < n ? w.list[2 * i + 1] * inv : 0.f;
+    const uint32_t at = i < n ? __float_as_uint(w.list[2 * i]) : 0u;
+    if (sorted) {
+      ent[i] = (uint64_t)__float_as_uint(q) << 32 | at;
+    } else {
+      p[i] = q;
+      idx[i] = (int)at;
+    }
+  }
   if (tid == 0) {
     th = 0;
     cut = 0;
     found = 0x7fffffff;
   }
   __syncthreads();
-  auto p = [&](int i) { return __uint_as_float((uint32_t)(ent[i] >> 32)); };
-  auto idx = [&](int i) { return (int)(uint32_t)ent[i]; };
+  auto ep = [&](int i) { return __uint_as_float((uint32_t)(ent[i] >> 32)); };
   const int part = tid & 7;
   // f(i) for i < m, by the 8 threads of an aligned group
   auto each = [&](int m, auto f) {
@@ -610,64 +619,78 @@ __global__ void __launch_bounds__(kThreads) k_smp_topk(const SampleArgs a) {
     }
     __syncthreads();
   };
-  float tk;
-  if (sorted) {
-    sort_descending(ent, pn);
-    tk = n >= a.top_k ? p(a.top_k - 1) : 0.f;
-    if (topp)
-      running(n, [&](int i) { return p(i) >= tk ? fix(p(i)) : 0ull; },
-              [&](int i, uint64_t before, uint64_t v) {   // the first to reach the target
-                if (before < target && before + v >= target) cut = (uint32_t)(ent[i] >> 32);
-              });
-  } else {
+  // what is left of m of them in pairs, given the least that stays and the
+  // factor: the first index whose cumulative probability exceeds r
+  auto draw_pairs = [&](int m, float low, float pinv) {
+    each(m, [&](int i) {
+      uint64_t c = 0;
+      for (int j = part; j < m; j += 8) c += p[j] >= low && idx[j] <= idx[i] ? fix(p[j] * pinv) : 0ull;
+      c = sum8u(c);
+      if (part == 0 && p[i] >= low && rf < c) atomicMin(&found, idx[i]);
+    });
+  };
+  auto factor = [&](uint64_t s) {
+    s = group_sum<kWaves>(s, sh.u);
+    return s > 0 ? 1.0f / (float)((double)s / kFix) : 1.0f;
+  };
+  uint64_t s = 0;
+  if (!sorted) {
     each(n, [&](int i) {   // the k-th largest p (p >= 0: its bits order like its value)
       uint64_t c = 0;      // greater ones, and (high half) equal ones
-      for (int j = part; j < n; j += 8) c += p(j) > p(i) ? 1ull : p(j) == p(i) ? 1ull << 32 : 0ull;
+      for (int j = part; j < n; j += 8) c += p[j] > p[i] ? 1ull : p[j] == p[i] ? 1ull << 32 : 0ull;
       c = sum8u(c);
       const uint32_t gt = (uint32_t)c, eq = (uint32_t)(c >> 32);
-      if (part == 0 && gt < (uint32_t)a.top_k && gt + eq >= (uint32_t)a.top_k) th = (uint32_t)(ent[i] >> 32);
+      if (part == 0 && gt < (uint32_t)a.top_k && gt + eq >= (uint32_t)a.top_k) th = __float_as_uint(p[i]);
     });
     __syncthreads();
-    tk = __uint_as_float(th);
+    const float tk = __uint_as_float(th);
     if (topp) {
       each(n, [&](int i) {   // the largest p whose sum with those above it reaches the target
-        uint64_t s = 0;
-        for (int j = part; j < n; j += 8) s += p(j) >= tk && p(j) >= p(i) ? fix(p(j)) : 0ull;
-        s = sum8u(s);
-        if (part == 0 && p(i) >= tk && s >= target) atomicMax(&cut, (uint32_t)(ent[i] >> 32));
+        uint64_t v = 0;
+        for (int j = part; j < n; j += 8) v += p[j] >= tk && p[j] >= p[i] ? fix(p[j]) : 0ull;
+        v = sum8u(v);
+        if (part == 0 && p[i] >= tk && v >= target) atomicMax(&cut, __float_as_uint(p[i]));
       });
       __syncthreads();
     }
-  }
-  const float low = fmaxf(tk, __uint_as_float(cut));
-  uint64_t s = 0, kept = 0;
-  for (int i = tid; i < n; i += kThreads) {
-    s += p(i) >= low ? fix(p(i)) : 0ull;
-    kept += p(i) >= low;
-  }
-  s = group_sum<kWaves>(s, sh.u);
-  const float pinv = s > 0 ? 1.0f / (float)((double)s / kFix) : 1.0f;
-  // the first index whose cumulative probability exceeds r; sorted, what is
-  // kept comes first
-  const int m = sorted ? (int)group_sum<kWaves>(kept, sh.u) : n;
-  if (m > kPairs) {
-    const int pm = pow2_from(m);
-    __syncthreads();
-    for (int i = tid; i < pm; i += kThreads) ent[i] = i < m ? ~ent[i] << 32 | ent[i] >> 32 : 0ull;   // ~index, p
-    sort_descending(ent, pm);
-    running(m, [&](int i) { return fix(__uint_as_float((uint32_t)ent[i]) * pinv); },
-            [&](int i, uint64_t before, uint64_t v) {
-              if (rf < before + v) atomicMin(&found, (int)~(uint32_t)(ent[i] >> 32));
-            });
+    const float low = fmaxf(tk, __uint_as_float(cut));
+    for (int i = tid; i < n; i += kThreads) s += p[i] >= low ? fix(p[i]) : 0ull;
+    draw_pairs(n, low, factor(s));
   } else {
-    each(m, [&](int i) {
-      uint64_t c = 0;
-      for (int j = part; j < m; j += 8) c += p(j) >= low && idx(j) <= idx(i) ? fix(p(j) * pinv) : 0ull;
-      c = sum8u(c);
-      if (part == 0 && p(i) >= low && rf < c) atomicMin(&found, idx(i));
-    });
-    __syncthreads();
+    sort_descending(ent, pn);
+    const float tk = n >= a.top_k ? ep(a.top_k - 1) : 0.f;
+    if (topp)
+      running(n, [&](int i) { return ep(i) >= tk ? fix(ep(i)) : 0ull; },
+              [&](int i, uint64_t before, uint64_t v) {   // the first to reach the target
+                if (before < target && before + v >= target) cut = (uint32_t)(ent[i] >> 32);
+              });
+    const float low = fmaxf(tk, __uint_as_float(cut));
+    uint64_t kept = 0;
+    for (int i = tid; i < n; i += kThreads) {
+      s += ep(i) >= low ? fix(ep(i)) : 0ull;
+      kept += ep(i) >= low;
+    }
+    const float pinv = factor(s);
+    const int m = (int)group_sum<kWaves>(kept, sh.u);   // they come first
+    if (m > kPairs) {
+      const int pm = pow2_from(m);
+      __syncthreads();
+      for (int i = tid; i < pm; i += kThreads) ent[i] = i < m ? ~ent[i] << 32 | ent[i] >> 32 : 0ull;   // ~index, p
+      sort_descending(ent, pm);
+      running(m, [&](int i) { return fix(__uint_as_float((uint32_t)ent[i]) * pinv); },
+              [&](int i, uint64_t before, uint64_t v) {
+                if (rf < before + v) atomicMin(&found, (int)~(uint32_t)(ent[i] >> 32));
+              });
+    } else {
+      if (tid < m) {
+        p[tid] = ep(tid);
+        idx[tid] = (int)(uint32_t)ent[tid];
+      }
+      __syncthreads();
+      draw_pairs(m, low, pinv);
+    }
   }
+  __syncthreads();
   if (tid == 0) put_result(a, !nan && found < a.V ? found : a.V - 1, st);
 }
 
@@ -829,6 +852,7 @@ __global__ void __launch_bounds__(kThreads) k_smp_draw(const SampleArgs a) {
   __syncthreads();
   if (tid == 0) put_result(a, !nan && found < a.V ? found : a.V - 1, st);
 }
+static_assert(kPairs <= kThreads, "k_smp_topk: a thread per pair's end");
 static_assert(kTile == kThreads, "k_smp_draw: one entry per thread");
 
 }  // namespace
