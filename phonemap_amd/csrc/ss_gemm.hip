@@ -8,7 +8,7 @@
 // fp16 integers from a magic number (bits 0x6400 | u are 1024 + u; the
 // subtraction of the offset is exact), x is split into two fp16 parts under a
 // power-of-two scale per token and 256 columns (the largest |x s| in [2^13,
-// 2^14), so xh + xl is within 2^-22 |x| of x), every block's fp32 result is
+// 2^14), so xh + xl is within 2^-23 |x| of x), every block's fp32 result is
 // scaled by its A into fp32 accumulators. The RMSNorm scale 1/rms of each
 // token multiplies its outputs (tensor.c:114-131 applies it to x).
 //
