@@ -195,3 +195,14 @@ def test_long_prompt_as_products(tmp_path, spec):
             tok, pos = am, pos + 1
     om.close()
     bar.report()
+
+
+@pytest.mark.parametrize("kv", ["f16", "int8"])
+@pytest.mark.parametrize("n", [4, 7])
+@pytest.mark.parametrize("spec", sorted(SPECS))
+def test_short_prompt_as_products(tmp_path, spec, n, kv):
+    """4 and 7 tokens run as products (the rows' attention in the form that
+    sums as single tokens do, softcapped too), then decode steps."""
+    print("gemma short prompt", spec, n, kv, flush=True)
+    prompt = np.random.default_rng(n).integers(3, SPECS[spec]["vocab"], n).tolist()
+    _run(_file(tmp_path, spec), kv, "graph", prompt, 3, spec=spec)
