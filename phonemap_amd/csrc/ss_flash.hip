@@ -142,7 +142,8 @@ template <int CH> __device__ __forceinline__ int vswz(int key) { return CH == 8 
 // l + 64, ... For the rows a tile's products cannot serve: a V that is not
 // finite reaches, as 0 * inf, rows that do not see its position. (Finite
 // launches pay one test per output: 180 shapes take 0.999 of what they took
-// without, geometric mean.)
+// without, geometric mean. 512 tokens over 1536 that all see a NaN, 32 heads on
+// 8, head_dim 128: 2.1 ms.)
 template <int HD>
 __device__ __forceinline__ void one_row(const AttnArgs& a, const float* q, const uint16_t* kc, const uint16_t* vc, int lim,
                                         float* out) {
@@ -156,7 +157,11 @@ __device__ __forceinline__ void one_row(const AttnArgs& a, const float* q, const
       const uint16_t* kr = kc + (size_t)(k0 + lane) * HD;
       s = 0.f;
 #pragma unroll 1
-      for (int i = 0; i < HD; ++i) s = fmaf(q[i], h2f(kr[i]), s);
+      for (int i = 0; i < HD; i += 8) {
+        const v8h kv = *reinterpret_cast<const v8h*>(kr + i);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) s = fmaf(q[i + k], (float)kv[k], s);
+      }
       s *= a.scale;
       if (a.softcap > 0.f) s = softcap(s, a);
     }
@@ -166,11 +171,23 @@ __device__ __forceinline__ void one_row(const AttnArgs& a, const float* q, const
     l = l * corr + wave_sum(p);
 #pragma unroll
     for (int d = 0; d < ND; ++d) o[d] *= corr;
+    const int nk = min(kWave, lim + 1 - k0);
 #pragma unroll 1
-    for (int j = 0; j < kWave && k0 + j <= lim; ++j) {
-      const float pj = __shfl(p, j, kWave);
+    for (int j = 0; j < nk; j += 8) {   // (past the last: the last again, not added)
+      float pj[8], v[8][ND];
 #pragma unroll
-      for (int d = 0; d < ND; ++d) o[d] = fmaf(pj, h2f(vc[(size_t)(k0 + j) * HD + lane + kWave * d]), o[d]);
+      for (int u = 0; u < 8; ++u) {
+        const int ju = min(j + u, nk - 1);
+        pj[u] = __shfl(p, ju, kWave);
+#pragma unroll
+        for (int d = 0; d < ND; ++d) v[u][d] = h2f(vc[(size_t)(k0 + ju) * HD + lane + kWave * d]);
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (j + u < nk) {
+#pragma unroll
+          for (int d = 0; d < ND; ++d) o[d] = fmaf(pj[u], v[u][d], o[d]);
+        }
     }
     m = mn;
   }
