@@ -1464,8 +1464,8 @@ int32_t enqueue_prompt_layer_major(ss_hip_model* m, const int32_t* tokens, int n
 // The reference evaluates a prompt layer by layer, each layer's matvecs once
 // per token. Here a chunk of up to kPrefillChunk tokens goes through each
 // layer as MFMA products of the quantised matrices with the chunk's rows
-// (ss_gemm.hip), one RoPE + cache append kernel and one attention launch
-// over all rows (ss_flash.hip; each token attends to positions 0..its own, the
+// (ss_gemm.h), one RoPE + cache append kernel and one attention launch
+// over all rows (ss_flash.h; each token attends to positions 0..its own, the
 // chunk's K/V having been appended first). Later chunks read the earlier
 // chunks' cache. Both caches take it: token by token, 64 tokens of a
 // 22-layer TinyLlama with the int8 cache took 40.5 ms, as products 1.6.

@@ -177,7 +177,7 @@ hipError_t launch_attention(int head_dim, int group, int kv_type, const AttnArgs
 hipError_t launch_attention_merge(int head_dim, int group, const AttnArgs& a, hipStream_t s);
 // Causal attention of a.n_tok prompt rows (token z: query a.q + z*a.tok_q,
 // positions 0..a.pos0 + z, output a.out + z*a.tok_o), fp16
-// or int8 cache, head_dim 64, 128 or 256, on MFMA (ss_flash.hip).
+// or int8 cache, head_dim 64, 128 or 256, on MFMA (ss_flash.h).
 hipError_t launch_attention_rows(int head_dim, int group, int kv_type, const AttnArgs& a, hipStream_t s);
 // ssq[t] = sum of x[t][c]^2 (x [T][cols])
 hipError_t launch_sumsq(const float* x, int cols, int T, float* ssq, hipStream_t s);
